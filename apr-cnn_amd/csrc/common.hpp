@@ -158,6 +158,8 @@ int get_tiles(aprnet_plan* plan, int level_delta, int TZ, int TX, TileList* out,
 bool stream_is_capturing(hipStream_t st);
 int get_lists(aprnet_plan* plan, int level_delta, int code, const TileList& tl, WinLists* out, hipStream_t st, bool dx = false);
 void free_lists(WinLists& wl);
+// an idle second stream of `device` (the current device), owned by the caller until its plan is destroyed
+int side_stream_acquire(int device, hipStream_t* out);
 int get_face_lists(aprnet_plan* plan, int level_delta, int code, FaceLists* out, hipStream_t st);
 void free_face_lists(FaceLists& fl);
 int get_need_lists(aprnet_plan* plan, int level_delta, int code, const WinLists& wl, NeedLists* out, hipStream_t st);

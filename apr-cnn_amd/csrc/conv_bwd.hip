@@ -321,7 +321,7 @@ static int fork_side(aprnet_plan* p, hipStream_t st, hipStream_t* side) {
     *side = st;
     if (!backward_overlap()) return 0;
     if (!p->side) {
-        APRNET_HIP_CHECK(hipStreamCreateWithFlags(&p->side, hipStreamNonBlocking));
+        if (int rc = side_stream_acquire(p->device, &p->side)) return rc;
         APRNET_HIP_CHECK(hipEventCreateWithFlags(&p->ev_fork, hipEventDisableTiming));
         APRNET_HIP_CHECK(hipEventCreateWithFlags(&p->ev_join, hipEventDisableTiming));
     }

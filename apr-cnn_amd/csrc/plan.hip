@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <mutex>
 #include <thread>
 
 namespace aprnet {
@@ -141,6 +142,36 @@ bool stream_is_capturing(hipStream_t st) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) != hipSuccess) { (void)hipGetLastError(); return false; }
     return cs != hipStreamCaptureStatusNone;
+}
+
+// Second streams of the convolution backward (aprnet_plan::side).  A training program makes a plan per APR and drops it
+// after a few steps; streams are taken from and given back to a free list per device instead of being created and
+// destroyed with every plan, and no event is left that was recorded on a destroyed stream: with the stream destroyed first,
+// host memory was seen changed after it had been freed and handed out again (the y_vec of an APR built after the plans of
+// others were destroyed; the sanitizers find nothing in this library or the builder).  At most SIDE_KEPT idle streams
+// are kept per device.
+constexpr size_t SIDE_KEPT = 16;
+static std::mutex g_side_mutex;
+static std::map<int, std::vector<hipStream_t>>& side_free() { static auto* m = new std::map<int, std::vector<hipStream_t>>(); return *m; }
+
+int side_stream_acquire(int device, hipStream_t* out) {
+    {
+        std::lock_guard<std::mutex> lock(g_side_mutex);
+        auto& v = side_free()[device];
+        if (!v.empty()) { *out = v.back(); v.pop_back(); return 0; }
+    }
+    APRNET_HIP_CHECK(hipStreamCreateWithFlags(out, hipStreamNonBlocking));
+    return 0;
+}
+
+static void side_stream_release(int device, hipStream_t s) {
+    (void)hipStreamSynchronize(s);                       // the next owner finds it idle
+    {
+        std::lock_guard<std::mutex> lock(g_side_mutex);
+        auto& v = side_free()[device];
+        if (v.size() < SIDE_KEPT) { v.push_back(s); return; }
+    }
+    (void)hipStreamDestroy(s);
 }
 
 void plan_scratch_done(aprnet_plan* p, hipStream_t st) {
@@ -283,10 +314,12 @@ void aprnet_plan_destroy(aprnet_plan* p) {
     for (auto& kv : p->lists) free_lists(kv.second);
     for (auto& kv : p->faces) free_face_lists(kv.second);
     for (auto& kv : p->need) free_need_lists(kv.second);
-    if (p->side) { (void)hipStreamSynchronize(p->side); (void)hipStreamDestroy(p->side); }
+    // (a stream is handed on only after the events that were recorded on it are gone)
+    if (p->side) (void)hipStreamSynchronize(p->side);
     if (p->ev_fork) (void)hipEventDestroy(p->ev_fork);
     if (p->ev_join) (void)hipEventDestroy(p->ev_join);
     if (p->ev_scratch) (void)hipEventDestroy(p->ev_scratch);
+    if (p->side) side_stream_release(p->device, p->side);
     delete p;
 }
 

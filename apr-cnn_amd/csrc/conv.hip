@@ -238,7 +238,7 @@ int fill_tree_for_conv(const aprnet_plan* p, int d, const double* x, int64_t ldx
 // fill is switched off or its lists cannot be had (no window lists, first call under stream capture, no memory): the
 // caller then fills every node.  The kernels stage exactly what the window lists name, so either fill gives the same result.
 static std::atomic<int> g_need_fill{1};      // 1: the tree fill before a forward convolution covers the nodes that are read, 0: all nodes
-static const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& tl, hipStream_t st, NeedLists* store) {
+const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& tl, hipStream_t st, NeedLists* store) {
     if (!g_need_fill || !g_use_lists || g_conv_path == 1 || !conv_mfma_supported(code) || tl.n == 0) return nullptr;
     WinLists wl;
     if (get_lists(p, d, code, tl, &wl, st) != 0) { (void)hipGetLastError(); return nullptr; }

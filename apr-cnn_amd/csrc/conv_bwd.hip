@@ -237,6 +237,8 @@ int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
 int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st);
 int conv_path();
+// the tree nodes the forward window lists name, null: fill every node (conv.hip)
+const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& tl, hipStream_t st, NeedLists* store);
 // points a at the plan's window lists (conv.hip); leaves a.tile_win null when they are off or unavailable
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st);
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st);
@@ -356,14 +358,17 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
     if (nt > 0 && (!tree_ws || ldt < nt || (gx && (!gtree_ws || ldgt < nt))))
         return fail(APRNET_ERR_INVALID_ARGUMENT, "conv_backward: tree work space too small");
     APRNET_HIP_CHECK(hipSetDevice(p->device));
-    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, nullptr)) return rc;
+    const bool flat = (kz == 1);
+    TileList tl;
+    if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &tl, st)) return rc;
+    // the weight gradient on the matrix cores stages what the forward pass stages: the same tree nodes
+    NeedLists need_store;
+    const NeedLists* need = sizeof(T) == 4 ? needed_nodes(p, d, code, tl, st, &need_store) : nullptr;
+    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, need)) return rc;
     if (gx) {
         fill2d<T>(gx, ldgx, p->number_parts(d), Cin, (T)0, st);
         fill2d<T>(gtree_ws, ldgt, nt, Cin, (T)0, st);
     }
-    const bool flat = (kz == 1);
-    TileList tl;
-    if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &tl, st)) return rc;
     if (tl.n > 0) {
         ConvArgs<T> a{};
         a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.n_tiles = tl.n;
@@ -412,14 +417,16 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
     if ((gx && (!gx32_ws || ldgx32 < np)) || (nt > 0 && (!tree_ws || ldt < nt || (gx && (!gtree_ws || ldgt < nt)))))
         return fail(APRNET_ERR_INVALID_ARGUMENT, "conv_backward: work space too small");
     APRNET_HIP_CHECK(hipSetDevice(p->device));
-    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, nullptr)) return rc;
+    const bool flat = (kz == 1);
+    TileList tl, near;
+    if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &tl, st)) return rc;
+    NeedLists need_store;            // (a regrouped copy carries the unfilled nodes along unread)
+    const NeedLists* need = needed_nodes(p, d, code, tl, st, &need_store);
+    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, need)) return rc;
     if (gx) {
         fill2d<float>(gx32_ws, ldgx32, np, Cin, 0.f, st);
         fill2d<float>(gtree_ws, ldgt, nt, Cin, 0.f, st);
     }
-    const bool flat = (kz == 1);
-    TileList tl, near;
-    if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &tl, st)) return rc;
     if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &near, st, 1)) return rc;
     if (tl.n > 0) {
         ConvArgs<bf16_t> a{};

@@ -160,8 +160,10 @@ int fill_tree_mean_g8(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx,
             hipLaunchKernelGGL(fill_tree_level_g8_kernel, dim3((unsigned)((e - b + GTB - 1) / GTB)), dim3(GTB), 0, st, p->d_children,
                                p->n_tree, b, e, x, ldx, tree, ldt, from_x ? p->tree_offset(Lc) : 0, from_x, from_x && !particles_first, G);
     }
+    int l_read = p->tree.level_min;          // with a need list: down to the coarsest level that is read (see fill_tree_mean_needed)
+    if (need) while (l_read <= l_coarse && need->cnt[l_read] == 0) ++l_read;
     GCoarse lv{};
-    for (int l = l_coarse; l >= p->tree.level_min; --l)
+    for (int l = l_coarse; l >= l_read; --l)
         if (p->tree.level_end(l) > p->tree.level_begin(l)) { lv.begin[lv.n] = p->tree.level_begin(l); lv.end[lv.n] = p->tree.level_end(l); ++lv.n; }
     if (lv.n > 0)
         hipLaunchKernelGGL(fill_tree_coarse_g8_kernel, dim3((unsigned)G), dim3(GTB), 0, st, p->d_children, p->n_tree, lv, x, ldx, tree, ldt);

@@ -497,13 +497,16 @@ int fill_tree_mean_needed(const aprnet_plan* p, int d, const NeedLists& need, co
                                need.cnt[l], x, ldx, C, tree, ldt, from_x ? p->tree_offset(Lc) : 0, from_x, from_x, cpt);
         }
     }
+    // The coarse levels (a few thousand nodes together) are filled whole, in one launch, down to the coarsest one that is
+    // read: levels without particles are never read, and on most APRs those are all of them (a launch of 14 to 20 us, for
+    // one workgroup per four channels walks the levels one after the other, in front of every convolution).
+    int l_read = l_coarse + 1;
+    for (int l = p->tree.level_min; l <= l_coarse; ++l)
+        if (need.cnt[l] > 0) { l_read = l; break; }
     CoarseLevels lv{};
-    bool any = false;
-    for (int l = l_coarse; l >= p->tree.level_min; --l) {
+    for (int l = l_coarse; l >= l_read; --l)
         if (p->tree.level_end(l) > p->tree.level_begin(l)) { lv.begin[lv.n] = p->tree.level_begin(l); lv.end[lv.n] = p->tree.level_end(l); ++lv.n; }
-        any = any || need.cnt[l] > 0;
-    }
-    if (lv.n > 0 && any)          // the coarse levels (a few thousand nodes together) are filled whole, in one launch
+    if (lv.n > 0)
         hipLaunchKernelGGL(fill_tree_coarse_kernel<T>, dim3((unsigned)((C + CPT_COARSE - 1) / CPT_COARSE)), dim3(TB), 0, st, p->d_children, p->n_tree,
                            lv, x, ldx, C, tree, ldt);
     APRNET_LAUNCH_CHECK("fill_tree kernels (needed nodes)");

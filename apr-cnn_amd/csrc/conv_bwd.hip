@@ -253,6 +253,10 @@ int bf16_math();
 int bwd_deterministic();
 int launch_face_dx(const FaceLists& fl, const float* gy, int64_t ldy, const float* w, int S_exp, int Cout, int Cin, int K, int Lc,
                    float* gx, int64_t ldgx, hipStream_t st);
+size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout);
+int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
+                      const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl, float* part,
+                      float* gw, hipStream_t st);
 int conv_dw_partial_blocks(int code, int Cout, int Cin);
 size_t conv_dw_partial_bytes(int code, int Cout, int Cin);
 // Points the weight-gradient kernels at their partial-sum slots, `off` bytes into the plan's scratch buffer (behind
@@ -447,28 +451,41 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         // everything that can allocate or fail on the host comes before the fork
         if (near.n > 0 && bf16_math())
             if (int rc = set_conv_dx_lists(p, d, code, near, b, st)) return rc;
-        const size_t wbytes = (conv_packed_bf16_bytes(code, S_exp, Cin, Cout) + 255) / 256 * 256;
-        const size_t ng = (size_t)(Cout + 7) / 8, ibytes = ng * (size_t)np * 16;
-        const bool regroup = bf16_regroup() && np < (1ll << 28) && ibytes <= ((size_t)32 << 30);
-        size_t need = 0;
-        if (near.n > 0) need = b.tile_win ? wbytes + (regroup ? ibytes : 0) : conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float);
-        need = (need + 255) / 256 * 256;
-        const size_t pbytes = bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+        // Both halves stage from copies grouped by eight channels behind the packed weights in the scratch buffer: the output
+        // gradient (read by both), the features and their tree (weight gradient).
+        auto align = [](size_t v) { return (v + 255) / 256 * 256; };
+        const size_t ngo = (size_t)(Cout + 7) / 8, ngi = (size_t)(Cin + 7) / 8;
+        const size_t wbytes = near.n > 0 ? align(conv_packed_bf16_bytes(code, S_exp, Cin, Cout)) : 0;
+        const size_t gybytes = align(ngo * (size_t)np * 16), xbytes = align(ngi * (size_t)np * 16), tbytes = align(ngi * (size_t)nt * 16);
+        const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
+        const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
+        WinLists wl;
+        const bool dw_g8 = regroup_gy && bwd_deterministic() && a.tile_win && gybytes + xbytes + tbytes <= ((size_t)48 << 30) &&
+                           get_lists(p, d, code, tl, &wl, st, false) == 0;
+        const bool dx_g8 = near.n > 0 && b.tile_win && regroup_gy;
+        size_t need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
+        if (near.n > 0 && !b.tile_win) need = std::max(need, conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
+        need = align(need);
+        const size_t pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join
         if (need + pbytes) if (int rc = lease.acquire(p, need + pbytes, st)) return rc;
-        if (pbytes) set_dw_partials(p, need, code, a);
+        if (pbytes && !dw_g8) set_dw_partials(p, need, code, a);
+        bf16_t* gyi = (bf16_t*)((char*)p->d_scratch + wbytes);
+        if (dw_g8 || dx_g8) if (int rc = interleave8_bf16(gy, ldy, nullptr, 0, Cout, Cout, np, gyi, st)) return rc;
         hipStream_t side = st;
         if (near.n > 0) if (int rc = fork_side(p, st, &side)) return rc;
         SideJoin guard(p, st, side);
-        if (int rc = launch_conv_dw_mfma(code, a, tl, p->apr.level_min, side)) return rc;
+        if (dw_g8) {
+            bf16_t* xi = (bf16_t*)((char*)gyi + gybytes);
+            bf16_t* ti = (bf16_t*)((char*)xi + xbytes);
+            if (int rc = interleave8_bf16(x, ldx, nullptr, 0, Cin, Cin, np, xi, side)) return rc;
+            if (int rc = interleave8_bf16(tree_ws, ldt, nullptr, 0, Cin, Cin, nt, ti, side)) return rc;
+            if (int rc = launch_conv_dw_g8(code, xi, np, np, ti, nt, nt, gyi, np, np, Cin, Cout, S_exp, a.Lc, wl,
+                                           (float*)((char*)p->d_scratch + need), gw, side)) return rc;
+        } else if (int rc = launch_conv_dw_mfma(code, a, tl, p->apr.level_min, side)) return rc;
         if (near.n > 0 && b.tile_win) {
-            // the output gradient regrouped as [Cout / 8][particles][8] behind the packed weights, as in the forward pass
             if (int rc = pack_conv_weights_bf16(code, w, S_exp, Cin, Cout, p->d_scratch, st, true)) return rc;
-            if (regroup) {
-                bf16_t* gyi = (bf16_t*)((char*)p->d_scratch + wbytes);
-                if (int rc = interleave8_bf16(gy, ldy, nullptr, 0, Cout, Cout, np, gyi, st)) return rc;
-                b.xi = gyi; b.ti = nullptr; b.xi_ld = np; b.ti_ld = 0;
-            }
+            if (dx_g8) { b.xi = gyi; b.ti = nullptr; b.xi_ld = np; b.ti_ld = 0; }
             b.w = (const float*)p->d_scratch;
             if (int rc = launch_conv_dx_mfma_bf16(code, b, near.n, st)) return rc;
         } else if (near.n > 0) {

@@ -1,0 +1,49 @@
+"""The backward pass of the stencil convolutions on copies grouped by eight channels (bfloat16 features): sizes at the
+edges of the kernels' blocks (16 input / 16 or 32 output channels, 32 columns per product, 256 columns per staged group)."""
+import pytest
+import torch
+
+import apr_cases
+from oracle import oracle
+from pyapr import _native
+from pyapr.aprnet import _ops
+from test_gpu_parity import _conv_case
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+# full windows of a uniformly fine image (more than one staged group of columns), sparse 3-D and 2-D ones, level deltas
+CASES = [([("3d_dense", 0)], (3, 3, 3)), ([("3d_t", 0), ("3d_a", 1)], (3, 3, 3)), ([("2d_t", 0), ("2d_s", 1)], (1, 5, 5)),
+         ([("2d_t", 0)], (1, 3, 3)), ([("3d_s", 1)], (1, 3, 3))]
+
+
+@pytest.fixture(autouse=True)
+def dense_case(monkeypatch):
+    get = apr_cases.get
+    monkeypatch.setattr(apr_cases, "get", lambda n: apr_cases.random_apr((12, 13, 150), 21, 0.6, 1) if n == "3d_dense" else get(n))
+
+
+@pytest.mark.parametrize("cin,cout", [(1, 16), (8, 17), (16, 16), (24, 48), (40, 33)])
+@pytest.mark.parametrize("bt,ksize", CASES, ids=["333-dense", "333", "155-2d", "133-2d", "133-3d"])
+def test_weight_gradient_blocks(bt, ksize, cin, cout):
+    """Against the oracle on the same bfloat16-representable values (the tree means it reads are rounded to bfloat16 on the
+    GPU: 2^-9 per value, 1e-2 of the largest element as in the other bfloat16 tests), against the kernel on channel planes,
+    which multiplies the same bfloat16 values exactly (fp32 sums in another order: 1e-5), and bit for bit on a second run."""
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, cin, cout, torch.float32)
+    xb = x.to(torch.bfloat16)
+    gob = torch.randn(x.size(0), cout, x.size(2), generator=torch.Generator().manual_seed(5)).to(torch.bfloat16)
+    _, gw_ref = oracle.conv_backward(aprs, xb.float(), w_exp, gob.float(), ld)
+    wd = w_exp.permute(1, 2, 0, 3, 4, 5).contiguous().to(DEV)
+    xd, gd = xb.to(DEV), gob.to(DEV)
+    gw = _ops.conv_backward(aprs, xd, wd, gd, ld)[1]
+    again = _ops.conv_backward(aprs, xd, wd, gd, ld)[1]
+    lib = _native.hip()
+    assert lib.aprnet_set_conv_path(9) == 0
+    try:
+        planes = _ops.conv_backward(aprs, xd, wd, gd, ld)[1]
+    finally:
+        lib.aprnet_set_conv_path(8)
+    assert torch.equal(gw, again)
+    scale = float(planes.abs().max())
+    assert float((gw - planes).abs().max()) <= 1e-5 * scale
+    assert float((gw.permute(2, 0, 1, 3, 4, 5).cpu() - gw_ref).abs().max()) <= 1e-2 * float(gw_ref.abs().max())

@@ -477,20 +477,52 @@ __device__ __forceinline__ void store_items16(const ItemRegs16<G, IPT>& R, int n
 }
 
 // out[q][i][c] = channel 8 q + c of element i; channels from c_split on come from x2 (null: all from x), channels
-// past C read as zeros.  One thread per (element, group): eight 2-byte reads along the planes, one 16-byte write.
-__global__ void interleave8_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ x2, int64_t ldx2, int c_split,
-                                   int C, int64_t count, bf16_t* __restrict__ out) {
+// past C read as zeros.  A streaming pass: a thread takes four consecutive elements of a group with eight 8-byte reads along
+// the planes (element-aligned: planes start wherever `ldx` puts them), transposes them in registers, and the block's
+// 16-byte results go out through LDS so that a wave writes whole lines.  All reads are unconditional and issued before the
+// first is used (a read under "channel exists" is waited for before the next is issued): 64 channels of 15.4 M elements
+// 2.85 -> 0.68 ms, 5.8 TB/s.  (Written straight from the registers, 64 bytes apart: 0.92 ms; one or two elements per thread
+// with 2-byte reads: 0.69 ms alone, but 3 ms next to the convolution kernels of a backward pass.)
+constexpr int IL_E = 4, IL_TB = 256;
+__global__ void __launch_bounds__(IL_TB)
+interleave8_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ x2, int64_t ldx2, int c_split,
+                   int C, int64_t count, bf16_t* __restrict__ out) {
+    typedef unsigned uintx2u __attribute__((ext_vector_type(2), aligned(2)));
+    __shared__ uint4 buf[IL_TB * IL_E];
     const int q = blockIdx.y;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
-        unsigned v[BF_CIB];
+    const int64_t b0 = (int64_t)blockIdx.x * (IL_TB * IL_E), i = b0 + threadIdx.x * IL_E;
+    // the last elements of a plane: the read is moved back so that it stays inside, and the words shifted into place
+    const int64_t at = max(min(i, count - IL_E), (int64_t)0);
+    uintx2u v[BF_CIB];
 #pragma unroll
-        for (int c = 0; c < BF_CIB; ++c) {
-            const int ch = q * BF_CIB + c;
-            v[c] = 0u;
-            if (ch < C) v[c] = (x2 != nullptr && ch >= c_split) ? x2[(int64_t)(ch - c_split) * ldx2 + i].bits : x[(int64_t)ch * ldx + i].bits;
+    for (int c = 0; c < BF_CIB; ++c) {
+        const int ch = min(q * BF_CIB + c, C - 1);
+        const bf16_t* p = (x2 != nullptr && ch >= c_split) ? x2 + (int64_t)(ch - c_split) * ldx2 : x + (int64_t)ch * ldx;
+        if (count >= IL_E) v[c] = *reinterpret_cast<const uintx2u*>(p + at);
+        else {                                                        // (fewer than four elements in all)
+            unsigned s[IL_E];
+#pragma unroll
+            for (int e = 0; e < IL_E; ++e) s[e] = p[min((int64_t)e, count - 1)].bits;
+            v[c] = uintx2u{s[0] | (s[1] << 16), s[2] | (s[3] << 16)};
         }
-        reinterpret_cast<uint4*>(out)[(int64_t)q * count + i] = make_uint4(v[0] | (v[1] << 16), v[2] | (v[3] << 16), v[4] | (v[5] << 16), v[6] | (v[7] << 16));
     }
+#pragma unroll
+    for (int c = 0; c < BF_CIB; ++c)
+        if (q * BF_CIB + c >= C) v[c] = uintx2u{0u, 0u};              // uniform
+    const int shift = (int)(i - at);                                  // elements past the end are not written
+#pragma unroll
+    for (int e = 0; e < IL_E; ++e) {
+        unsigned w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)           // halves e % 2 of words e / 2 of two planes
+            w[k] = __builtin_amdgcn_perm(v[2 * k + 1][e >> 1], v[2 * k][e >> 1], (e & 1) ? 0x07060302u : 0x05040100u);
+        if (e >= shift) buf[threadIdx.x * IL_E + e - shift] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    __syncthreads();
+    uint4* dst = reinterpret_cast<uint4*>(out) + (int64_t)q * count + b0;
+#pragma unroll
+    for (int e = 0; e < IL_E; ++e)
+        if (b0 + e * IL_TB + threadIdx.x < count) dst[e * IL_TB + threadIdx.x] = buf[e * IL_TB + threadIdx.x];
 }
 
 // MODE 0: forward.  MODE 1: input gradient (items = output gradient, results added atomically in fp32 to the place
@@ -857,8 +889,8 @@ int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, h
 int interleave8_bf16(const bf16_t* x, int64_t ldx, const bf16_t* x2, int64_t ldx2, int c_split, int C, int64_t count, bf16_t* out,
                      hipStream_t st) {
     if (count <= 0 || C <= 0) return 0;
-    dim3 grid((unsigned)std::min<int64_t>((count + 255) / 256, 1 << 20), (unsigned)((C + BF_CIB - 1) / BF_CIB));
-    hipLaunchKernelGGL(interleave8_kernel, grid, dim3(256), 0, st, x, ldx, x2, ldx2, c_split, C, count, out);
+    dim3 grid((unsigned)((count + IL_TB * IL_E - 1) / (IL_TB * IL_E)), (unsigned)((C + BF_CIB - 1) / BF_CIB));
+    hipLaunchKernelGGL(interleave8_kernel, grid, dim3(IL_TB), 0, st, x, ldx, x2, ldx2, c_split, C, count, out);
     APRNET_LAUNCH_CHECK("interleave8_kernel");
     return 0;
 }

@@ -47,3 +47,22 @@ def test_weight_gradient_blocks(bt, ksize, cin, cout):
     scale = float(planes.abs().max())
     assert float((gw - planes).abs().max()) <= 1e-5 * scale
     assert float((gw.permute(2, 0, 1, 3, 4, 5).cpu() - gw_ref).abs().max()) <= 1e-2 * float(gw_ref.abs().max())
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 2), (1, 1, 3), (1, 2, 3), (2, 3, 3), (1, 1, 1030), (3, 5, 137)])
+def test_grouped_copy_of_any_length(shape):
+    """The grouped copy the kernels stage from: fewer particles than one thread takes (four), remainders of four and of a
+    block's 1024.  Same products in the same order as the kernel that gathers from the planes: bit-identical."""
+    apr = apr_cases.random_apr(shape, 3, 0.5, 1)
+    n = apr.total_number_particles()
+    x = torch.randn(1, 9, n, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16).to(DEV)
+    w = torch.randn(apr.level_max() - apr.level_min() + 1, 5, 9, 1, 3, 3, generator=torch.Generator().manual_seed(1)).to(DEV)
+    ld = torch.zeros(1, dtype=torch.int32)
+    y = _ops.conv_forward([apr], x, w, ld)
+    lib = _native.hip()
+    assert lib.aprnet_set_conv_path(9) == 0
+    try:
+        planes = _ops.conv_forward([apr], x, w, ld)
+    finally:
+        lib.aprnet_set_conv_path(8)
+    assert torch.equal(y, planes)

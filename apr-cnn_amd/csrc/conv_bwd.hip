@@ -210,8 +210,8 @@ using W555 = ConvGeom<5, 5, 5, 2, 4, 256>;
 
 int fill_tree_for_conv(const aprnet_plan* p, int d, const float* x, int64_t ldx, int C, float* tree, int64_t ldt, hipStream_t st, const NeedLists* need);
 int fill_tree_for_conv(const aprnet_plan* p, int d, const double* x, int64_t ldx, int C, double* tree, int64_t ldt, hipStream_t st, const NeedLists* need);
-int fill_tree_bwd_for_conv(const aprnet_plan* p, int d, float* gx, int64_t ldx, int C, float* gt, int64_t ldt, hipStream_t st);
-int fill_tree_bwd_for_conv(const aprnet_plan* p, int d, double* gx, int64_t ldx, int C, double* gt, int64_t ldt, hipStream_t st);
+int fill_tree_bwd_for_conv(const aprnet_plan* p, int d, float* gx, int64_t ldx, int C, float* gt, int64_t ldt, hipStream_t st, const NeedLists* need);
+int fill_tree_bwd_for_conv(const aprnet_plan* p, int d, double* gx, int64_t ldx, int C, double* gt, int64_t ldt, hipStream_t st, const NeedLists* need);
 
 template <typename T, class GX, int XCIB, class GW, int WCIB, int WCOB>
 static int launch_bwd(ConvArgs<T>& a, hipStream_t st) {
@@ -392,7 +392,7 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
         }
         if (rc) return rc;
     }
-    return gx ? fill_tree_bwd_for_conv(p, d, gx, ldgx, Cin, gtree_ws, ldgt, st) : 0;
+    return gx ? fill_tree_bwd_for_conv(p, d, gx, ldgx, Cin, gtree_ws, ldgt, st, need) : 0;
 }
 
 __global__ void round_to_bf16_kernel(const float* __restrict__ src, int64_t lds, bf16_t* __restrict__ dst, int64_t ldd, int64_t n) {
@@ -425,8 +425,8 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
     TileList tl, near;
     if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &tl, st)) return rc;
     NeedLists need_store;            // (a regrouped copy carries the unfilled nodes along unread)
-    const NeedLists* need = needed_nodes(p, d, code, tl, st, &need_store);
-    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, need)) return rc;
+    const NeedLists* nodes = needed_nodes(p, d, code, tl, st, &need_store);
+    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, nodes)) return rc;
     if (gx) {
         fill2d<float>(gx32_ws, ldgx32, np, Cin, 0.f, st);
         fill2d<float>(gtree_ws, ldgt, nt, Cin, 0.f, st);
@@ -497,7 +497,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         if (int rc = guard.join()) return rc;
     }
     if (!gx) return 0;
-    if (int rc = fill_tree_bwd_for_conv(p, d, gx32_ws, ldgx32, Cin, gtree_ws, ldgt, st)) return rc;
+    if (int rc = fill_tree_bwd_for_conv(p, d, gx32_ws, ldgx32, Cin, gtree_ws, ldgt, st, nodes)) return rc;
     if (np > 0) {
         dim3 grid((unsigned)std::min<int64_t>((np + 255) / 256, 4096), (unsigned)Cin);
         hipLaunchKernelGGL(round_to_bf16_kernel, grid, dim3(256), 0, st, gx32_ws, ldgx32, gx, ldgx, np);

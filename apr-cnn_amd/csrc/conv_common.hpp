@@ -269,6 +269,7 @@ __device__ __attribute__((noinline)) void scan_window_impl(const ScanArgs a, Con
 //            those box sums.  Only at the far faces of the image, where some of the cells do not exist, it
 //            takes one column per cell.
 constexpr unsigned COL_CELL = 0x0fffu;
+constexpr unsigned COL_SOLE = 0x2000u;    // input gradient: no other column, of this window or another, adds to this place
 constexpr unsigned COL_BOX = 0x4000u;
 constexpr unsigned COL_TREE = 0x8000u;
 
@@ -329,7 +330,10 @@ __device__ __attribute__((noinline)) void scan_window_dx_impl(const ScanArgs a, 
                         const int rank = __popcll(m & below_me);
                         const bool to_tree = src == 2 && !tree_from_x;
                         sh.col_idx[base + rank] = i + ((src == 2 && tree_from_x) ? (int)a.tree_off : 0);
-                        sh.col_pos[base + rank] = (unsigned short)((r * G::RS + (yy[g] - lo)) | (to_tree ? COL_TREE : 0u));
+                        // a place is a centre cell of one window of its own level; further columns come from windows one
+                        // level finer, which see it as a coarser particle: none above the finest level, none for a tree node
+                        sh.col_pos[base + rank] = (unsigned short)((r * G::RS + (yy[g] - lo)) | (to_tree ? COL_TREE : 0u) |
+                                                                   (to_tree || tree_from_x ? COL_SOLE : 0u));
                     }
                 }
             } else {

@@ -17,17 +17,36 @@
 
 namespace aprnet {
 
+// Streaming passes over the rows of the work space: a thread handles STREAM_V consecutive values with 16-byte accesses
+// (element-aligned: rows start wherever the leading dimension puts them), STREAM_R times a block's width apart, all loads
+// of a thread ahead of its first store.
+constexpr int STREAM_TB = 256, STREAM_V = 4, STREAM_R = 4, STREAM_BLOCK = STREAM_TB * STREAM_V * STREAM_R;
+
+// Bound by the stores.  One 4-byte store per lane and turn of a grid-stride loop filled the two
+// work spaces of 64 channels (5.2 GB) in 1.69 ms; that and round_to_bf16_kernel below: 1x5x5 64 -> 64 forward and backward
+// on 15.4 M particles 25.9 -> 24.7 ms, training step on 5.5 M particles 21.4 -> 20.8 ms.
 template <typename T>
-__global__ void fill_kernel(T* __restrict__ p, int64_t ld, int64_t n, T v) {
+__global__ void __launch_bounds__(STREAM_TB) fill_kernel(T* __restrict__ p, int64_t ld, int64_t n, T v) {
+    constexpr int V = 16 / sizeof(T);
+    typedef T vec __attribute__((ext_vector_type(V), aligned(sizeof(T))));
     T* row = p + (int64_t)blockIdx.y * ld;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) row[i] = v;
+    vec w;
+#pragma unroll
+    for (int e = 0; e < V; ++e) w[e] = v;
+#pragma unroll
+    for (int r = 0; r < STREAM_R; ++r) {
+        const int64_t i = ((int64_t)blockIdx.x * STREAM_R + r) * (STREAM_TB * V) + threadIdx.x * V;
+        if (i + V <= n) *reinterpret_cast<vec*>(row + i) = w;
+        else
+            for (int64_t k = i; k < n; ++k) row[k] = v;
+    }
 }
 
 template <typename T>
 static void fill2d(T* p, int64_t ld, int64_t n, int rows, T v, hipStream_t st) {
     if (n <= 0 || rows <= 0) return;
-    dim3 grid((unsigned)std::min<int64_t>((n + 255) / 256, 4096), (unsigned)rows);
-    hipLaunchKernelGGL(fill_kernel<T>, grid, dim3(256), 0, st, p, ld, n, v);
+    constexpr int64_t per = STREAM_TB * (16 / sizeof(T)) * STREAM_R;
+    hipLaunchKernelGGL(fill_kernel<T>, dim3((unsigned)((n + per - 1) / per), (unsigned)rows), dim3(STREAM_TB), 0, st, p, ld, n, v);
 }
 
 // Transpose of stage_values: add the gradient patch back to its sources, item by item.
@@ -395,10 +414,30 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
     return gx ? fill_tree_bwd_for_conv(p, d, gx, ldgx, Cin, gtree_ws, ldgt, st, need) : 0;
 }
 
-__global__ void round_to_bf16_kernel(const float* __restrict__ src, int64_t lds, bf16_t* __restrict__ dst, int64_t ldd, int64_t n) {
+// Bound by memory (6 bytes per value).  One value per lane and turn of a grid-stride loop took 1.47 ms
+// for 64 channels of 15.4 M particles, 4.0 TB/s (gain: see fill_kernel).
+__global__ void __launch_bounds__(STREAM_TB)
+round_to_bf16_kernel(const float* __restrict__ src, int64_t lds, bf16_t* __restrict__ dst, int64_t ldd, int64_t n) {
+    typedef float vecf __attribute__((ext_vector_type(STREAM_V), aligned(4)));
+    typedef unsigned vech __attribute__((ext_vector_type(STREAM_V / 2), aligned(2)));
     const float* s = src + (int64_t)blockIdx.y * lds;
     bf16_t* d = dst + (int64_t)blockIdx.y * ldd;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) d[i] = float_to_bf16(s[i]);
+    const int64_t i0 = (int64_t)blockIdx.x * STREAM_BLOCK + threadIdx.x * STREAM_V;
+    if ((int64_t)(blockIdx.x + 1) * STREAM_BLOCK <= n) {                    // uniform
+        vecf v[STREAM_R];
+#pragma unroll
+        for (int r = 0; r < STREAM_R; ++r) v[r] = *reinterpret_cast<const vecf*>(s + i0 + r * (STREAM_TB * STREAM_V));
+#pragma unroll
+        for (int r = 0; r < STREAM_R; ++r) {
+            vech w;
+#pragma unroll
+            for (int e = 0; e < STREAM_V / 2; ++e)
+                w[e] = (unsigned)float_to_bf16(v[r][2 * e]).bits | ((unsigned)float_to_bf16(v[r][2 * e + 1]).bits << 16);
+            *reinterpret_cast<vech*>(d + i0 + r * (STREAM_TB * STREAM_V)) = w;
+        }
+        return;
+    }
+    for (int64_t i = (int64_t)blockIdx.x * STREAM_BLOCK + threadIdx.x; i < n; i += STREAM_TB) d[i] = float_to_bf16(s[i]);   // last block
 }
 
 // bfloat16 features and output gradient; weights, weight gradient and all accumulation in fp32 (the fp32
@@ -499,8 +538,8 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
     if (!gx) return 0;
     if (int rc = fill_tree_bwd_for_conv(p, d, gx32_ws, ldgx32, Cin, gtree_ws, ldgt, st, nodes)) return rc;
     if (np > 0) {
-        dim3 grid((unsigned)std::min<int64_t>((np + 255) / 256, 4096), (unsigned)Cin);
-        hipLaunchKernelGGL(round_to_bf16_kernel, grid, dim3(256), 0, st, gx32_ws, ldgx32, gx, ldgx, np);
+        dim3 grid((unsigned)((np + STREAM_BLOCK - 1) / STREAM_BLOCK), (unsigned)Cin);
+        hipLaunchKernelGGL(round_to_bf16_kernel, grid, dim3(STREAM_TB), 0, st, gx32_ws, ldgx32, gx, ldgx, np);
         APRNET_LAUNCH_CHECK("round_to_bf16_kernel");
     }
     return 0;

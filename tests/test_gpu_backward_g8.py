@@ -73,8 +73,9 @@ def test_grouped_copy_of_any_length(shape):
                                                      ((9, 12, 1), 2, (1, 3, 3), (0,))])
 def test_tree_gradient_of_the_nodes_with_outputs(shape, drop, ksize, deltas, dtype):
     """Handing the tree's gradient down from the nodes the forward lists name against handing it down from every node
-    (levels walked in one launch, level by level from a list, whole): small whole numbers, so that the sums of the
-    convolution do not depend on their order, hence bit-identical."""
+    (levels walked in one launch, level by level from a list, whole), and the stored lists (plain stores where one column
+    writes a place) against the kernel that scans and adds every column atomically.  Small whole numbers, so that the sums
+    of the convolution do not depend on their order, hence bit-identical."""
     apr = apr_cases.random_apr(shape, 5, 0.01 if drop > 2 else 0.1, drop)
     gen = torch.Generator().manual_seed(3)
     lib = _native.hip()
@@ -85,11 +86,12 @@ def test_tree_gradient_of_the_nodes_with_outputs(shape, drop, ksize, deltas, dty
         gy = torch.randint(-3, 4, (1, 18, n), generator=gen).to(dtype).to(DEV)
         w = torch.randint(-2, 3, (apr.level_max() - apr.level_min() + 1, 18, 5) + ksize, generator=gen).float().to(DEV)
         got = _ops.conv_backward([apr], x, w, gy, ld)
-        assert lib.aprnet_set_conv_path(17) == 0
-        try:
-            ref = _ops.conv_backward([apr], x, w, gy, ld)
-        finally:
-            lib.aprnet_set_conv_path(16)
-        assert float(ref[0].float().abs().max()) > 0
-        assert torch.equal(got[0], ref[0])
-        assert float((got[1] - ref[1]).abs().max()) <= 1e-5 * float(ref[1].abs().max())
+        for off, on in ((17, 16), (5, 4)):
+            assert lib.aprnet_set_conv_path(off) == 0
+            try:
+                ref = _ops.conv_backward([apr], x, w, gy, ld)
+            finally:
+                lib.aprnet_set_conv_path(on)
+            assert float(ref[0].float().abs().max()) > 0
+            assert torch.equal(got[0], ref[0])
+            assert float((got[1] - ref[1]).abs().max()) <= 1e-5 * float(ref[1].abs().max())

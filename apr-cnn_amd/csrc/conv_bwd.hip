@@ -499,15 +499,27 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
         const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
         WinLists wl;
-        const bool dw_g8 = regroup_gy && bwd_deterministic() && a.tile_win && gybytes + xbytes + tbytes <= ((size_t)48 << 30) &&
-                           get_lists(p, d, code, tl, &wl, st, false) == 0;
+        bool dw_g8 = regroup_gy && bwd_deterministic() && a.tile_win && gybytes + xbytes + tbytes <= ((size_t)48 << 30) &&
+                     get_lists(p, d, code, tl, &wl, st, false) == 0;
         const bool dx_g8 = near.n > 0 && b.tile_win && regroup_gy;
-        size_t need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
-        if (near.n > 0 && !b.tile_win) need = std::max(need, conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
-        need = align(need);
-        const size_t pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+        size_t need = 0, pbytes = 0;
+        auto layout = [&]() {
+            need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
+            if (near.n > 0 && !b.tile_win) need = std::max(need, conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
+            need = align(need);
+            pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+            return need + pbytes;
+        };
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join
-        if (need + pbytes) if (int rc = lease.acquire(p, need + pbytes, st)) return rc;
+        if (layout()) {
+            int rc = lease.acquire(p, need + pbytes, st);
+            if (rc && dw_g8) {   // no room for the copies, or a capture that may not grow the buffer: the kernel on channel planes
+                (void)hipGetLastError();
+                dw_g8 = false;
+                rc = layout() ? lease.acquire(p, need + pbytes, st) : 0;
+            }
+            if (rc) return rc;
+        }
         if (pbytes && !dw_g8) set_dw_partials(p, need, code, a);
         bf16_t* gyi = (bf16_t*)((char*)p->d_scratch + wbytes);
         if (dw_g8 || dx_g8) if (int rc = interleave8_bf16(gy, ldy, nullptr, 0, Cout, Cout, np, gyi, st)) return rc;

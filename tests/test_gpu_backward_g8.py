@@ -95,3 +95,29 @@ def test_tree_gradient_of_the_nodes_with_outputs(shape, drop, ksize, deltas, dty
             assert float(ref[0].float().abs().max()) > 0
             assert torch.equal(got[0], ref[0])
             assert float((got[1] - ref[1]).abs().max()) <= 1e-5 * float(ref[1].abs().max())
+
+
+def test_weight_gradient_without_room_for_the_copies():
+    """A capture must not grow the plan's scratch buffer: when the copies do not fit what is there, the kernel on channel planes
+    runs as it did for the eager call that sized the buffer (same kernel, same order of summation: bit-identical)."""
+    apr = apr_cases.random_apr((70, 90, 110), 5, 0.01, 4)
+    gen = torch.Generator().manual_seed(7)
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    x = torch.randn(1, 5, n, generator=gen).to(torch.bfloat16).to(DEV)
+    gy = torch.randn(1, 18, n, generator=gen).to(torch.bfloat16).to(DEV)
+    w = torch.randn(apr.level_max() - apr.level_min() + 1, 18, 5, 3, 3, 3, generator=gen).to(DEV)
+    lib = _native.hip()
+    assert lib.aprnet_set_conv_path(9) == 0
+    try:
+        planes = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1]
+    finally:
+        lib.aprnet_set_conv_path(8)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1]
+    for _ in range(3):
+        captured.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured, planes)

@@ -494,7 +494,9 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         // gradient (read by both), the features and their tree (weight gradient).
         auto align = [](size_t v) { return (v + 255) / 256 * 256; };
         const size_t ngo = (size_t)(Cout + 7) / 8, ngi = (size_t)(Cin + 7) / 8;
-        const size_t wbytes = near.n > 0 ? align(conv_packed_bf16_bytes(code, S_exp, Cin, Cout)) : 0;
+        // the image of the weights that the input gradient below packs: fp32 ones where it has no lists (twice the bfloat16 size)
+        const size_t wbytes = near.n == 0 ? 0 : align(b.tile_win ? conv_packed_bf16_bytes(code, S_exp, Cin, Cout)
+                                                                 : conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
         const size_t gybytes = align(ngo * (size_t)np * 16), xbytes = align(ngi * (size_t)np * 16), tbytes = align(ngi * (size_t)nt * 16);
         const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
         const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
@@ -505,8 +507,6 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         size_t need = 0, pbytes = 0;
         auto layout = [&]() {
             need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
-            if (near.n > 0 && !b.tile_win) need = std::max(need, conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
-            need = align(need);
             pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
             return need + pbytes;
         };

@@ -121,3 +121,37 @@ def test_weight_gradient_without_room_for_the_copies():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(captured, planes)
+
+
+@pytest.mark.parametrize("cin,cout", [(5, 18), (32, 32)])
+def test_grouped_weight_gradient_next_to_an_input_gradient_without_lists(cin, cout):
+    """Forward lists there, input-gradient lists not: the weight gradient reads its grouped copies on the side stream while the
+    input gradient packs fp32 weights, twice the size of the bfloat16 image, at the front of the same scratch buffer.  Reached
+    by a capture: the 1x3x3 backward has built the row groups that 1x5x5 shares, the 1x5x5 lists of the input gradient would
+    have to be built.  Weight gradient: same kernel, lists and order as the eager call without an input gradient, hence
+    bit-identical.  Input gradient: fp32 products in place of bfloat16 ones on weights rounded to bfloat16 (2^-9 each)."""
+    apr = apr_cases.random_apr((1, 300, 411), 5, 0.02, 5)
+    gen = torch.Generator().manual_seed(11)
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    levels = apr.level_max() - apr.level_min() + 1
+    x = torch.randn(1, cin, n, generator=gen).to(torch.bfloat16).to(DEV)
+    gy = torch.randn(1, cout, n, generator=gen).to(torch.bfloat16).to(DEV)
+    w3 = torch.randn(levels, cout, cin, 1, 3, 3, generator=gen).to(DEV)
+    w5 = torch.randn(levels, cout, cin, 1, 5, 5, generator=gen).to(DEV)
+    lib = _native.hip()
+    assert lib.aprnet_plan_reserve(apr.plan(0), 256 << 20, None) == 0
+    _ops.conv_backward([apr], x, w3, gy, ld)
+    gw = _ops.conv_backward([apr], x, w5, gy, ld, need_input_grad=False)[1]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = _ops.conv_backward([apr], x, w5, gy, ld)
+    eager = _ops.conv_backward([apr], x, w5, gy, ld)
+    assert torch.equal(eager[1], gw)
+    for _ in range(5):
+        for t in captured:
+            t.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(captured[1], gw)
+        assert float((captured[0].float() - eager[0].float()).abs().max()) <= 1e-2 * float(eager[0].float().abs().max())

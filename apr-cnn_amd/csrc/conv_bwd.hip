@@ -272,7 +272,7 @@ int bf16_math();
 int bwd_deterministic();
 int launch_face_dx(const FaceLists& fl, const float* gy, int64_t ldy, const float* w, int S_exp, int Cout, int Cin, int K, int Lc,
                    float* gx, int64_t ldgx, hipStream_t st);
-size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout);
+size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl);
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
                       const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl, float* part,
                       float* gw, hipStream_t st);
@@ -507,7 +507,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         size_t need = 0, pbytes = 0;
         auto layout = [&]() {
             need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
-            pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+            pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout, S_exp, a.Lc, wl) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
             return need + pbytes;
         };
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join

@@ -290,6 +290,7 @@ using DG133 = ConvGeom<1, 3, 3, 1, 8, 512>;
 using DG155 = ConvGeom<1, 5, 5, 1, 8, 512>;
 
 static int dwg_taps(int code) { return code == 333 ? 27 : code == 133 ? 9 : 25; }
+static int64_t dwg_slot_bytes(int code, const DwG8Args& a) { return (int64_t)dwg_taps(code) * a.CinP * a.CoutP * (int64_t)sizeof(float); }
 static int dwg_nco(int Cout) { return Cout <= 16 ? 1 : 2; }
 // Workgroups of a launch: about two rounds of the 512 that the chip holds (windows differ in work), fewer for layers with
 // several channel blocks, whose every window is visited once per block.
@@ -297,9 +298,32 @@ static int dwg_blocks_x(int Cin, int Cout) {
     const int per = ((Cin + 15) / 16) * ((Cout + 16 * dwg_nco(Cout) - 1) / (16 * dwg_nco(Cout)));
     return std::max(64, 1024 / per);
 }
-size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout) {
-    const int nco = dwg_nco(Cout), CinP = (Cin + 15) / 16 * 16, CoutP = (Cout + 16 * nco - 1) / (16 * nco) * 16 * nco;
-    return (size_t)(dwg_blocks_x(Cin, Cout) + MAX_LEVELS) * dwg_taps(code) * CinP * CoutP * sizeof(float);
+// Channels rounded up to the kernel's blocks and the workgroups of every stencil index (level Lc - s has index s, every level
+// from S_exp - 1 on the last one), from the windows there are.  A workgroup's slot is as large as the gradient of one
+// stencil index: 3x3x3 512 -> 512 has slots of 28 MB, so the slots are held to 512 MiB, or to one per stencil index where
+// that is more.  Wide layers fill the chip with their channel blocks alone (512 of them at 512 -> 512): with 18 slots
+// instead of 66 that layer on 95 k particles takes 6.65 instead of 7.38 ms; up to 256 -> 256 the limit does not bind.
+static void dwg_table(int code, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl, DwG8Args& a) {
+    const int nco = dwg_nco(Cout);
+    a.Cin = Cin; a.Cout = Cout;
+    a.CinP = (Cin + 15) / 16 * 16; a.CoutP = (Cout + 16 * nco - 1) / (16 * nco) * 16 * nco;
+    a.n_s = 0;
+    for (int k = 0; k < wl.n_lv; ++k) {                    // finest level first: stencil indices ascend
+        const int s = std::min(S_exp - 1, Lc - wl.lv_level[k]);
+        const int w0 = wl.lv_first[k], w1 = k + 1 < wl.n_lv ? wl.lv_first[k + 1] : wl.n_win;
+        if (a.n_s > 0 && a.s_of[a.n_s - 1] == s) { a.nwin[a.n_s - 1] = w1 - a.win0[a.n_s - 1]; continue; }
+        a.s_of[a.n_s] = s; a.win0[a.n_s] = w0; a.nwin[a.n_s] = w1 - w0; ++a.n_s;
+    }
+    const int64_t slots = ((int64_t)512 << 20) / dwg_slot_bytes(code, a);
+    const int64_t bx = std::min<int64_t>(dwg_blocks_x(Cin, Cout), std::max<int64_t>(0, slots - a.n_s));
+    a.blk0[0] = 0;
+    for (int k = 0; k < a.n_s; ++k)                        // (together at most bx + n_s)
+        a.blk0[k + 1] = a.blk0[k] + (int)std::max<int64_t>(1, std::min<int64_t>(a.nwin[k], bx * a.nwin[k] / wl.n_win));
+}
+size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl) {
+    DwG8Args a{};
+    dwg_table(code, Cin, Cout, S_exp, Lc, wl, a);
+    return (size_t)a.blk0[a.n_s] * dwg_slot_bytes(code, a);
 }
 
 template <class G>
@@ -315,30 +339,17 @@ static int launch_dw_g8_g(const DwG8Args& a, float* gw, hipStream_t st) {
 }
 
 // gw += weight gradient; xi / ti / gyi grouped copies, fewer than 2^28 particles (32-bit byte offsets); `part` holds
-// conv_dw_g8_part_bytes.  One launch for all stencil indices (level Lc - s has index s, every level from S_exp - 1 on the
-// last one) plus one for the sums.
+// conv_dw_g8_part_bytes.  One launch for all stencil indices plus one for the sums.
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
                       const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl, float* part,
                       float* gw, hipStream_t st) {
     if (wl.n_win <= 0) return 0;
     DwG8Args a{};
     a.xi = xi; a.xi_ld = xi_ld; a.x_count = x_count; a.ti = ti; a.ti_ld = ti_ld; a.t_count = t_count;
-    a.gyi = gyi; a.gy_ld = gy_ld; a.gy_count = gy_count; a.Cin = Cin; a.Cout = Cout;
-    const int nco = dwg_nco(Cout);
-    a.CinP = (Cin + 15) / 16 * 16; a.CoutP = (Cout + 16 * nco - 1) / (16 * nco) * 16 * nco;
+    a.gyi = gyi; a.gy_ld = gy_ld; a.gy_count = gy_count;
+    dwg_table(code, Cin, Cout, S_exp, Lc, wl, a);
     a.win = wl.d_win; a.item_idx = wl.d_item_idx; a.item_pos = wl.d_item_pos; a.col_idx = wl.d_col_idx; a.col_pos = wl.d_col_pos;
     a.part = part;
-    for (int k = 0; k < wl.n_lv; ++k) {                    // finest level first: stencil indices ascend
-        const int s = std::min(S_exp - 1, Lc - wl.lv_level[k]);
-        const int w0 = wl.lv_first[k], w1 = k + 1 < wl.n_lv ? wl.lv_first[k + 1] : wl.n_win;
-        if (a.n_s > 0 && a.s_of[a.n_s - 1] == s) { a.nwin[a.n_s - 1] = w1 - a.win0[a.n_s - 1]; continue; }
-        a.s_of[a.n_s] = s; a.win0[a.n_s] = w0; a.nwin[a.n_s] = w1 - w0; ++a.n_s;
-    }
-    const int bx = dwg_blocks_x(Cin, Cout);
-    for (int k = 0; k < a.n_s; ++k) {
-        const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(a.nwin[k], (int64_t)bx * a.nwin[k] / wl.n_win));
-        a.blk0[k + 1] = a.blk0[k] + nb;
-    }
     switch (code) {
         case 333: return launch_dw_g8_g<DG333>(a, gw, st);
         case 133: return launch_dw_g8_g<DG133>(a, gw, st);

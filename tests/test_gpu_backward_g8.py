@@ -155,3 +155,33 @@ def test_grouped_weight_gradient_next_to_an_input_gradient_without_lists(cin, co
         torch.cuda.synchronize()
         assert torch.equal(captured[1], gw)
         assert float((captured[0].float() - eager[0].float()).abs().max()) <= 1e-2 * float(eager[0].float().abs().max())
+
+
+def _memory_outside_torch():
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free - torch.cuda.memory_reserved()
+
+
+def test_partial_sums_of_a_wide_layer_stay_within_512_mib():
+    """3x3x3 512 -> 512: a slot of the partial sums holds 28 MB, and one per workgroup of a narrow layer's grid would be
+    2.2 GB.  What the call keeps besides them: the copies of 2 x 512 channels and the plan's lists."""
+    apr = apr_cases.random_apr((40, 36, 44), 9, 0.02)
+    apr.init_cuda()
+    gen = torch.Generator().manual_seed(2)
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    x = torch.randn(1, 512, n, generator=gen).to(torch.bfloat16).to(DEV)
+    gy = torch.randn(1, 512, n, generator=gen).to(torch.bfloat16).to(DEV)
+    w = torch.randn(2, 512, 512, 3, 3, 3, device=DEV)
+    before = _memory_outside_torch()
+    gw = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1]
+    grown = _memory_outside_torch() - before
+    copies = 2 * 512 * (2 * n + apr.total_number_tree_particles())
+    assert grown <= (512 << 20) + copies + (32 << 20)
+    lib = _native.hip()
+    assert lib.aprnet_set_conv_path(9) == 0
+    try:
+        planes = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1]
+    finally:
+        lib.aprnet_set_conv_path(8)
+    assert float((gw - planes).abs().max()) <= 1e-5 * float(planes.abs().max())

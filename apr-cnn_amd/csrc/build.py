@@ -15,7 +15,7 @@ HIP_SOURCES = ["plan.hip", "lists.hip", "faces.hip", "need.hip", "tree_ops.hip",
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-fno-gpu-rdc",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
              "-Wno-unused-command-line-argument", "-Wno-unknown-attributes"]
-HEADERS = ["common.hpp", "conv_common.hpp", os.path.join("..", "..", "include", "aprnet_hip.h")]
+HEADERS = ["common.hpp", "conv_common.hpp", "sum_slots.hpp", os.path.join("..", "..", "include", "aprnet_hip.h")]
 
 
 def _newer(target, deps):

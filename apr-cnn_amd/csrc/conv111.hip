@@ -4,6 +4,7 @@
 // with the stencil index s = min(S-1, Lc-level) constant per segment.  One launch per segment keeps
 // the weights wave-uniform (scalar loads); x is read once per block of COB output channels.
 #include "common.hpp"
+#include "sum_slots.hpp"
 
 namespace aprnet {
 
@@ -184,7 +185,7 @@ bool try_conv111_mfma<float>(const float* src, int64_t lds, int Csrc, const floa
 
 // gw[co][ci] += sum_i gy[co][i] * x[ci][i] over [begin, end): 8x8 register tile per thread, block
 // reduction through LDS; then one atomic per (co, ci) and block, or - with `part` - the block's sum goes to
-// part[blockIdx.x][co][ci] for conv111_dw_reduce_kernel to add up in a fixed order (same bits on every run).
+// part[blockIdx.x][co][ci] for sum_slots_kernel to add up in a fixed order (same bits on every run).
 template <typename T>
 __global__ void __launch_bounds__(TB1)
 conv111_dw_kernel(const T* __restrict__ x, int64_t ldx, int Cin, const T* __restrict__ gy, int64_t ldy, int Cout,
@@ -233,20 +234,6 @@ conv111_dw_kernel(const T* __restrict__ x, int64_t ldx, int Cin, const T* __rest
     }
 }
 
-// gw[e] += sum of part[b][e] over the blocks: a wave per element, lane l adds blocks l, l + 64, ..., then a fixed tree over
-// the lanes.  (One thread per element walked up to 256 blocks in a chain of dependent loads: 6 to 22 us per
-// launch on average in a training step, 4 us now.)
-template <typename A>
-__global__ void __launch_bounds__(64)
-conv111_dw_reduce_kernel(const A* __restrict__ part, int nblocks, int n, A* __restrict__ gw) {
-    const int e = blockIdx.x;
-    A s = 0;
-    for (int b = threadIdx.x; b < nblocks; b += 64) s += part[(int64_t)b * n + e];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
-    if (threadIdx.x == 0) gw[e] += s;
-}
-
 int bwd_deterministic();
 
 // the weight gradient of one segment, by partial sums per workgroup (default) or by atomic additions
@@ -264,9 +251,8 @@ static int launch_conv111_dw(aprnet_plan* p, const T* x, int64_t ldx, int Cin, c
     if (int rc = lease.acquire(p, (size_t)g2.x * Cout * Cin * sizeof(A), st)) return rc;
     A* part = (A*)p->d_scratch;
     hipLaunchKernelGGL(conv111_dw_kernel<T>, g2, dim3(TB1), 0, st, x, ldx, Cin, gy, ldy, Cout, gw, part, begin, end);
-    hipLaunchKernelGGL(conv111_dw_reduce_kernel<A>, dim3((unsigned)(Cout * Cin)), dim3(64), 0, st, part, (int)g2.x,
-                       Cout * Cin, gw);
-    return 0;
+    APRNET_LAUNCH_CHECK("conv111_dw_kernel");
+    return launch_sum_slots<A>(part, (int64_t)Cout * Cin, (int)g2.x, (int64_t)Cout * Cin, gw, st);
 }
 
 struct Segment { int64_t begin, end; int stencil; };

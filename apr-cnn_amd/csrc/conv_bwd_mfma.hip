@@ -18,6 +18,7 @@
 // stencil index); they are added to the result with one atomic per element at the end.  The patch rows are 67 words
 // apart so that the 27 tap offsets of a B read fall into 27 different LDS banks.
 #include "conv_common.hpp"
+#include "sum_slots.hpp"
 
 namespace aprnet {
 
@@ -514,40 +515,6 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const int s_idx) {
     }
 }
 
-// gw[e] += sum of part[slot][e] over the slots, in an order that is fixed by the slot count alone: wave w of the block adds
-// slots w, w + RED_W, ... (eight loads in flight), the RED_W sums of an element meet in LDS and are added in wave order.
-// Bound by the latency of the chain of loads when one thread walks all slots of an element (27 k elements fill a tenth of
-// the chip): 128 us on average over the launches of a training step of the 16-32-64 network on 5.5 M particles, 48 us with
-// RED_W waves per 64 elements.
-constexpr int RED_W = 16;
-__global__ void __launch_bounds__(64 * RED_W) dw_reduce_kernel(const float* __restrict__ part, int64_t ld, int slots, int64_t n, float* __restrict__ gw) {
-    __shared__ float sums[RED_W][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t e = (int64_t)blockIdx.x * 64 + lane;
-    const float* src = part + (e < n ? e : n - 1);
-    float s[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) s[i] = 0.f;
-    int k = w;
-    for (; k + 7 * RED_W < slots; k += 8 * RED_W)
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s[i] += src[(int64_t)(k + i * RED_W) * ld];
-    for (; k < slots; k += RED_W) s[0] += src[(int64_t)k * ld];
-    sums[w][lane] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
-    __syncthreads();
-    if (w == 0 && e < n) {
-        float t = 0.f;
-#pragma unroll
-        for (int i = 0; i < RED_W; ++i) t += sums[i][lane];
-        gw[e] += t;
-    }
-}
-int launch_dw_reduce(const float* part, int64_t ld, int slots, int64_t n, float* gw, hipStream_t st) {
-    hipLaunchKernelGGL(dw_reduce_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64 * RED_W), 0, st, part, ld, slots, n, gw);
-    APRNET_LAUNCH_CHECK("dw_reduce_kernel");
-    return 0;
-}
-
 // Workgroups of one weight-gradient launch when its partial sums go to a buffer: at most 512, fewer for very wide
 // layers so that the buffer (two slots per workgroup) stays within 512 MiB.
 int conv_dw_partial_blocks(int code, int Cout, int Cin) {
@@ -582,7 +549,7 @@ static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, int level_min, h
         // the partial sums of this launch, added up in slot order (every slot of the grid is written in full)
         auto reduce = [&]() -> int {
             if (!a.gw_part) return 0;
-            return launch_dw_reduce((const float*)a.gw_part, a.gw_part_ld, 2 * (int)grid.x, n_el, (float*)a.gw + (int64_t)s * n_el, st);
+            return launch_sum_slots((const float*)a.gw_part, a.gw_part_ld, 2 * (int)grid.x, n_el, (float*)a.gw + (int64_t)s * n_el, st);
         };
         if constexpr (std::is_same<T, bf16_t>::value) {
             if (bf16_math()) {      // bfloat16 matrix instructions; the fp32 ones below when those are asked for

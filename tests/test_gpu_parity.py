@@ -573,6 +573,25 @@ def test_conv111_backward_bf16(cin, cout, S):
         _ops.conv_backward(aprs, xb.to(DEV), w.permute(1, 2, 0, 3, 4, 5).contiguous().to(DEV), gob.float().to(DEV), ld)
 
 
+@pytest.mark.parametrize("cin,cout,dtype", [(8192, 8192, torch.float32), (300, 520, torch.bfloat16), (130, 70, torch.float64), (1, 1, torch.float32)],
+                         ids=["8192x8192-f32", "300x520-bf16", "130x70-f64", "1x1-f32"])
+def test_conv111_weight_gradient_of_any_width(cin, cout, dtype):
+    """The slots of the workgroups are added 64 elements to a workgroup (a wave per element needs 2^32 threads for 8192 x
+    8192 channels, more than a launch can have).  Against the product in 64 bits; n terms of size <= 1 each, so fp32 sums
+    differ by at most n 2^-24 of the sum of magnitudes."""
+    apr = apr_cases.get("1d_a" if cin > 1000 else "3d_t")
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    x = (2 * torch.rand(1, cin, n, device=DEV, generator=gen) - 1).to(dtype)
+    gy = (2 * torch.rand(1, cout, n, device=DEV, generator=gen) - 1).to(dtype)
+    w = torch.zeros(1, cout, cin, 1, 1, 1, device=DEV, dtype=torch.float32 if dtype == torch.bfloat16 else dtype)
+    gw = _ops.conv_backward([apr], x, w, gy, ld)[1].view(cout, cin)
+    x, gy = x[0].double(), gy[0].double()
+    ref, size = gy @ x.T, gy.abs() @ x.abs().T
+    eps = 2.0 ** -53 if dtype == torch.float64 else 2.0 ** -24
+    assert bool(((gw.double() - ref).abs() <= 2 * n * eps * size).all())
+
+
 # ------------------------------------------------------------------------- fused forward (ReLU, second input)
 @pytest.mark.parametrize("path", [0, 1], ids=["mfma", "valu"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16], ids=["f32", "f64", "bf16"])

@@ -121,6 +121,7 @@ struct aprnet_plan {
     int64_t n_tree = 0, n_apr = 0;
     std::map<std::tuple<int, int, int, int>, aprnet::TileList> tiles;   // (level_delta, TZ, TX, halo) -> row groups
     void* d_scratch = nullptr; size_t scratch_bytes = 0;          // re-laid-out weights of the call in flight
+    size_t scratch_refused = 0;                                   // a size that could not be allocated (0: none)
     bool scratch_in_graph = false;                                // the buffer was handed out while its stream was capturing
     std::vector<void*> retired;                                   // outgrown buffers that a captured graph may address: freed at destroy
     // Hand-over of the buffer between streams: the last call that used it recorded ev_scratch behind its kernels, and a
@@ -169,7 +170,9 @@ void free_need_lists(NeedLists& nl);
 // with APRNET_ERR_UNSUPPORTED (reserve first: aprnet_plan_reserve, or run the call once outside the capture).  A call on
 // another stream than the previous one first waits for that stream, so that two streams cannot overwrite each other's
 // packed weights (under capture the caller must have ordered the streams, as for any input of the graph).
-int plan_scratch(aprnet_plan* plan, size_t bytes, hipStream_t st);
+// `optional`: the caller has a way to go on with less.  Such a request is refused, without touching the buffer there is,
+// when the device has no room for it or an equal one failed before: a program short of memory repeats it in every call.
+int plan_scratch(aprnet_plan* plan, size_t bytes, hipStream_t st, bool optional = false);
 // Records "this call is done with the scratch buffer" on `st` (after the last kernel that reads it was launched).
 void plan_scratch_done(aprnet_plan* plan, hipStream_t st);
 // A call's hold on the scratch buffer: acquire() is plan_scratch(); the destructor records the hand-over event, on every
@@ -177,8 +180,8 @@ void plan_scratch_done(aprnet_plan* plan, hipStream_t st);
 // its destructor runs last.
 struct ScratchLease {
     aprnet_plan* plan = nullptr; hipStream_t st = nullptr;
-    int acquire(aprnet_plan* p, size_t bytes, hipStream_t s) {
-        const int rc = plan_scratch(p, bytes, s);
+    int acquire(aprnet_plan* p, size_t bytes, hipStream_t s, bool optional = false) {
+        const int rc = plan_scratch(p, bytes, s, optional);
         if (!rc) { plan = p; st = s; }
         return rc;
     }

@@ -512,7 +512,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         };
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join
         if (layout()) {
-            int rc = lease.acquire(p, need + pbytes, st);
+            int rc = lease.acquire(p, need + pbytes, st, dw_g8);
             if (rc && dw_g8) {   // no room for the copies, or a capture that may not grow the buffer: the kernel on channel planes
                 (void)hipGetLastError();
                 dw_g8 = false;

@@ -185,7 +185,7 @@ void plan_scratch_done(aprnet_plan* p, hipStream_t st) {
     if (!p->scratch_event_recorded) { (void)hipGetLastError(); (void)hipStreamSynchronize(st); }
 }
 
-int plan_scratch(aprnet_plan* p, size_t bytes, hipStream_t st) {
+int plan_scratch(aprnet_plan* p, size_t bytes, hipStream_t st, bool optional) {
     const bool capturing = stream_is_capturing(st);
     // a second stream takes the buffer over only after the first is done with it: a device-side wait for the event
     // that the previous call recorded behind its kernels
@@ -196,6 +196,13 @@ int plan_scratch(aprnet_plan* p, size_t bytes, hipStream_t st) {
         if (capturing)
             return fail(APRNET_ERR_UNSUPPORTED, "the plan's scratch buffer would have to grow while the stream is capturing: call "
                                                 "aprnet_plan_reserve, or run this call once, before the capture");
+        if (optional) {
+            const char* none = "no device memory for a scratch buffer of this size";
+            if (p->scratch_refused && bytes >= p->scratch_refused) return fail(APRNET_ERR_UNSUPPORTED, none);
+            size_t free_bytes = 0, total = 0;
+            APRNET_HIP_CHECK(hipMemGetInfo(&free_bytes, &total));
+            if (bytes > free_bytes + (p->scratch_in_graph ? 0 : p->scratch_bytes)) return fail(APRNET_ERR_UNSUPPORTED, none);
+        }
         if (p->d_scratch) {
             if (p->scratch_in_graph) p->retired.push_back(p->d_scratch);     // a graph may replay into it: keep it until destroy
             else {
@@ -206,8 +213,13 @@ int plan_scratch(aprnet_plan* p, size_t bytes, hipStream_t st) {
             }
         }
         p->d_scratch = nullptr; p->scratch_bytes = 0; p->scratch_in_graph = false;
-        APRNET_HIP_CHECK(hipMalloc(&p->d_scratch, bytes));
+        if (hipError_t e = hipMalloc(&p->d_scratch, bytes); e != hipSuccess) {
+            p->d_scratch = nullptr;
+            p->scratch_refused = p->scratch_refused ? std::min(p->scratch_refused, bytes) : bytes;
+            return fail(APRNET_ERR_HIP, std::string("scratch buffer: ") + hipGetErrorString(e));
+        }
         p->scratch_bytes = bytes;
+        if (bytes >= p->scratch_refused) p->scratch_refused = 0;
     }
     if (capturing) p->scratch_in_graph = true;
     return 0;

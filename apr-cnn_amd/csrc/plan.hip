@@ -146,10 +146,11 @@ bool stream_is_capturing(hipStream_t st) {
 
 // Second streams of the convolution backward (aprnet_plan::side).  A training program makes a plan per APR and drops it
 // after a few steps; streams are taken from and given back to a free list per device instead of being created and
-// destroyed with every plan, and no event is left that was recorded on a destroyed stream: with the stream destroyed first,
-// host memory was seen changed after it had been freed and handed out again (the y_vec of an APR built after the plans of
-// others were destroyed; the sanitizers find nothing in this library or the builder).  At most SIDE_KEPT idle streams
-// are kept per device.
+// destroyed with every plan (at most SIDE_KEPT idle ones are kept per device), and a stream is handed on, or destroyed, only
+// after the events that the plan recorded on it are gone.  An earlier form destroyed the stream with the plan, and its
+// events after it; host memory was then seen changed after it had been freed and handed out again (the y_vec of the next
+// APR, refused by plan_create).  That this order was the cause is inferred from its going away, not shown: HIP allows an
+// event to outlive its stream, and the plan's host code is clean under the sanitizers on a stand-in of the runtime.
 constexpr size_t SIDE_KEPT = 16;
 static std::mutex g_side_mutex;
 static std::map<int, std::vector<hipStream_t>>& side_free() { static auto* m = new std::map<int, std::vector<hipStream_t>>(); return *m; }

@@ -66,6 +66,8 @@ const char* aprnet_last_error(void);
  * the host (row table non-decreasing and within n_particles, level_xz_vec consistent with z_num * x_num, y strictly
  * ascending per row and below y_num): APRNET_ERR_INVALID_ARGUMENT names the first violation. */
 int aprnet_plan_create(const aprnet_access_desc* apr, const aprnet_access_desc* tree, int device, aprnet_plan** out);
+/* Frees the device arrays (waits for the work that uses them).  The plan holds events that its calls recorded on the
+ * streams they were given: where a program can choose, it destroys a plan before those streams. */
 void aprnet_plan_destroy(aprnet_plan* plan);
 
 /* No counterpart in the reference.  The convolutions keep re-laid-out weights (and, for bfloat16 features, a regrouped

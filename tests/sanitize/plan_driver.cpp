@@ -103,6 +103,56 @@ static void* build(int zn, int xn, int yn, unsigned seed) {
 
 using namespace aprnet;
 
+// what a backward call does to its plan: scratch, side stream, fork and join
+static void backward(aprnet_plan* p, hipStream_t st) {
+    TileList tl;
+    CHECK(get_tiles(p, 0, 2, 4, &tl, st) == 0 && tl.n > 0);
+    ScratchLease lease;
+    CHECK(lease.acquire(p, 4096, st) == 0);
+    std::memset(p->d_scratch, 1, 4096);
+    if (!p->side) {
+        CHECK(side_stream_acquire(p->device, &p->side) == 0);
+        CHECK(hipEventCreateWithFlags(&p->ev_fork, 0) == hipSuccess && hipEventCreateWithFlags(&p->ev_join, 0) == hipSuccess);
+    }
+    CHECK(hipEventRecord(p->ev_fork, st) == hipSuccess && hipStreamWaitEvent(p->side, p->ev_fork, 0) == hipSuccess);
+    CHECK(hipEventRecord(p->ev_join, p->side) == hipSuccess && hipStreamWaitEvent(st, p->ev_join, 0) == hipSuccess);
+}
+
+// plans that come and go: the arrays of the APRs stay as they were built, side streams are shared by the plans that
+// follow each other, nothing is left behind
+static void plans_come_and_go() {
+    hipStream_t st = nullptr;
+    CHECK(hipStreamCreateWithFlags(&st, 0) == hipSuccess);
+    g_streams_made = 0;
+    for (int round = 0; round < 20; ++round) {
+        void* h = build(9 + round, 21, 17 + 3 * round, 7u + (unsigned)round);
+        Access apr(h, 0), tree(h, 1);
+        aprcore_destroy(h);
+        const std::vector<uint16_t> y0 = apr.yv, t0 = tree.yv;
+        aprnet_plan* p[3] = {};
+        for (auto& q : p) {
+            CHECK(aprnet_plan_create(&apr.d, &tree.d, 0, &q) == 0);
+            backward(q, st);
+            std::vector<int32_t> children((size_t)8 * q->n_tree);
+            CHECK(aprnet_plan_children(q, children.data()) == 0);
+        }
+        for (auto& q : p) aprnet_plan_destroy(q);
+        CHECK(apr.yv == y0 && tree.yv == t0);
+        CHECK(g_events.empty() && g_mem.empty());
+    }
+    CHECK(g_streams_made == 3 && g_streams_destroyed == 0);
+    // more plans at once than idle streams are kept: the rest are destroyed, after their events
+    void* h = build(9, 21, 17, 3u);
+    Access apr(h, 0), tree(h, 1);
+    aprcore_destroy(h);
+    std::vector<aprnet_plan*> many(20, nullptr);
+    for (auto& q : many) { CHECK(aprnet_plan_create(&apr.d, &tree.d, 0, &q) == 0); backward(q, st); }
+    for (auto& q : many) aprnet_plan_destroy(q);
+    CHECK(g_streams_made == 20 && g_streams_destroyed == 4);
+    CHECK(g_events.empty() && g_mem.empty());
+    CHECK(hipStreamDestroy(st) == hipSuccess);
+}
+
 // a request that the caller can do without costs nothing when it cannot be met
 static void optional_scratch() {
     void* h = build(9, 21, 17, 5u);
@@ -153,6 +203,7 @@ static void optional_scratch() {
 
 int main() {
     optional_scratch();
+    plans_come_and_go();
     std::printf("OK\n");
     return 0;
 }

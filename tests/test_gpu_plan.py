@@ -89,3 +89,26 @@ def test_growth_and_first_use_during_capture_are_refused():
         eager_wide = _ops.conv_forward([apr], x48, w_wide, ld)
         assert torch.equal(y_wide, eager_wide)
         assert torch.equal(_ops.conv_forward([apr], x4, w_small, ld), eager_small)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_aprs_built_beside_plans_that_come_and_go(dtype):
+    """Plans dropped after a backward pass (its side stream and events with them) while further APRs are built: the arrays of
+    the new APRs are those of the same APR built before any plan was destroyed, and stay so while their own plans run."""
+    shapes = [(21 + k, 19, 25 + 7 * k) for k in range(5)]
+    want = [[a.copy() for a in apr_cases.random_apr(s, 31 + k, density=0.03).get_state()[4:]] for k, s in enumerate(shapes)]
+    ld, g = torch.zeros(1, dtype=torch.int32), torch.Generator().manual_seed(0)
+    side = torch.cuda.Stream()
+    for turn in range(4):
+        for k, s in enumerate(shapes):
+            apr = apr_cases.random_apr(s, 31 + k, density=0.03)
+            n, levels = apr.total_number_particles(), apr.level_max() - apr.level_min() + 1
+            x, gy = torch.randn(1, 8, n, generator=g).to(dtype).to(DEV), torch.randn(1, 20, n, generator=g).to(dtype).to(DEV)
+            side.wait_stream(torch.cuda.current_stream())
+            with torch.cuda.stream(side if turn % 2 else torch.cuda.current_stream()):
+                gx, gw = _ops.conv_backward([apr], x, _weights(levels, 20, 8, k), gy, ld)
+            torch.cuda.synchronize()
+            assert torch.isfinite(gx.float()).all() and torch.isfinite(gw).all()
+            for a, b in zip(apr.get_state()[4:], want[k]):
+                assert (a == b).all()
+            del apr

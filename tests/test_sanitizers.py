@@ -36,7 +36,8 @@ def test_aprcore_and_oracle_run_clean_under_asan_and_ubsan(tmp_path):
 
 @pytest.mark.timeout(600)
 def test_plan_management_under_asan_and_ubsan(tmp_path):
-    """csrc/plan.hip (host code only) on a stand-in of the HIP runtime (tests/sanitize/plan_driver.cpp)."""
+    """csrc/plan.hip (host code only) on a stand-in of the HIP runtime (tests/sanitize/plan_driver.cpp): scratch requests that a
+    call can do without, and plans made and destroyed in turn with their side streams and events."""
     gxx, rocm = shutil.which("g++"), os.environ.get("ROCM_PATH", "/opt/rocm")
     if gxx is None or not os.path.exists(os.path.join(rocm, "include", "hip", "hip_runtime.h")):
         pytest.skip("no g++ or no HIP headers")

@@ -12,7 +12,8 @@
 // A workgroup owns 16 input channels, 16 * NCO output channels and a contiguous range of windows of one stencil index; its
 // eight waves are WT groups of taps x WK shares of the columns.  The sums stay in registers over all windows, the WK
 // shares meet in LDS at the end, and every workgroup writes its sums to a slot of its own (added up in slot order by
-// dw_g8_reduce_kernel: the same bits on every run).
+// dw_g8_reduce_kernel).  Calls on one plan give the same bits; the lists of another plan of the same APR may hold a window's
+// columns in another order (their places are taken with an atomic counter when the lists are built), and with it the sums.
 //
 // What bounds it: the LDS reads (7 taps: 9 KB per wave and 32 columns against 14 matrix instructions of 16 cycles) at
 // two workgroups per CU.  The kernel before it read one channel per lane: eight 2-byte LDS reads per operand and a gather of
@@ -129,7 +130,7 @@ conv_dw_g8_kernel(const DwG8Args a) {
     };
     intx4g gv[NCO];
     auto load_gy = [&](int cidx, int ng) {
-        const int off = gc < ng ? cidx * 16 : (int)BUF_OOB;
+        const int off = (int)(gc < ng ? (unsigned)cidx * 16u : BUF_OOB);         // (unsigned: up to 2^28 particles)
 #pragma unroll
         for (int h = 0; h < NCO; ++h) {
             const int q = p0 + gp + 2 * h;                              // wave-uniform
@@ -173,7 +174,7 @@ conv_dw_g8_kernel(const DwG8Args a) {
 #pragma unroll
             for (int k = 0; k < S::IPT; ++k) {
                 if (k * G::NT >= nitem) break;                          // uniform
-                const int off = tid + k * G::NT < nitem ? sl.idx[k] * 16 : (int)BUF_OOB;
+                const int off = (int)(tid + k * G::NT < nitem ? (unsigned)sl.idx[k] * 16u : BUF_OOB);
                 if (sl.pos[k] & (int)ITEM_TREE) {
                     v0[k] = __builtin_amdgcn_raw_buffer_load_b128(rt0, off, 0, 0);
                     if (two) v1[k] = __builtin_amdgcn_raw_buffer_load_b128(rt1, off, 0, 0);

@@ -124,6 +124,35 @@ def test_spots16k_whole_image_identity_adjoint_and_grouped_equals_planes():
         assert float((got[0, ch].float() - ref8[0, ch]).abs().max()) <= 1e-2 * float(ref8[0, ch].abs().max())
 
 
+def test_spots16k_whole_image_weight_gradient_of_grouped_copies():
+    """More than 2^27 particles: the byte offsets of the grouped weight gradient (16 per particle) pass 2^31.  Against the
+    kernel on channel planes, the same products in another order.  Features and gradients in {-1, 0, 1} keep the sums far
+    below 2^24, so that only the sums with tree means (multiples of 1/4, rounded to bfloat16) round at all."""
+    _need(60)
+    apr, _ = make_config("spots16k")
+    apr.init_cuda()
+    n = apr.total_number_particles()
+    assert 1 << 27 < n < 1 << 28
+    levels = apr.level_max() - apr.level_min() + 1
+    ld = torch.zeros(1, dtype=torch.int32)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = torch.empty(1, 10, n, device=DEV, dtype=torch.bfloat16)
+    gy = torch.empty(1, 8, n, device=DEV, dtype=torch.bfloat16)
+    for t in (x, gy):
+        for c in range(t.size(1)):
+            t[0, c] = torch.randint(-1, 2, (n,), device=DEV, generator=g, dtype=torch.int8)
+    w = torch.zeros(levels, 8, 10, 1, 3, 3, device=DEV)
+    got = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1]
+    lib = _ops._lib()
+    assert lib.aprnet_set_conv_path(9) == 0
+    try:
+        planes = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1]
+    finally:
+        lib.aprnet_set_conv_path(8)
+    assert float(planes.abs().max()) > 0
+    assert float((got - planes).abs().max()) <= 1e-5 * float(planes.abs().max())
+
+
 def test_nuclei1024_whole_volume_conv_matches_the_oracle():
     """configs[3], whole 1024^3 volume (844 M particles): with few channels the CPU oracle finishes in seconds at this
     size too, so the three forward kernel families are compared with it on EVERY particle of the full-size APR -

@@ -274,8 +274,8 @@ int launch_face_dx(const FaceLists& fl, const float* gy, int64_t ldy, const floa
                    float* gx, int64_t ldgx, hipStream_t st);
 size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl);
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
-                      const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl, float* part,
-                      float* gw, hipStream_t st);
+                      const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int ci0, int CinW, int Cout, int S_exp, int Lc,
+                      const WinLists& wl, float* part, float* gw, hipStream_t st);
 int conv_dw_partial_blocks(int code, int Cout, int Cin);
 size_t conv_dw_partial_bytes(int code, int Cout, int Cin);
 // Points the weight-gradient kernels at their partial-sum slots, `off` bytes into the plan's scratch buffer (behind
@@ -440,6 +440,23 @@ round_to_bf16_kernel(const float* __restrict__ src, int64_t lds, bf16_t* __restr
     for (int64_t i = (int64_t)blockIdx.x * STREAM_BLOCK + threadIdx.x; i < n; i += STREAM_TB) d[i] = float_to_bf16(s[i]);   // last block
 }
 
+// Input channels of the features and tree that the grouped weight gradient copies at a time (whole blocks of the kernel, 16
+// channels).  The scratch buffer stays with the plan, so a program with a plan per APR pays for it on each: beside the
+// output gradient's copy these may take what the forward pass of the layer has needed for its own copies anyway, plus
+// 256 MiB; wider layers on larger APRs copy a part of their channels at a time, in equal parts.  Next to the input gradient,
+// which fills the ends of the parts' launches, that costs no time (1x5x5 64 -> 64 on 15.4 M particles, four parts: 25.0 ->
+// 24.4 ms forward and backward; 3x3x3 64 -> 64 on 23 M 38.3 -> 38.5 ms backward).  Without an input gradient it
+// would (128 -> 64 on 5.4 M 9.9 -> 10.5 ms), and the call then has no fp32 work spaces, which are larger than the
+// copies: all channels at once.
+static int dw_copy_channels(int Cin, int64_t np, int64_t nt, size_t gybytes) {
+    const size_t blk = (size_t)(np + nt) * 32, all = (size_t)((Cin + 7) / 8) * (size_t)(np + nt) * 16;
+    const int nb = (Cin + 15) / 16;
+    const size_t room = std::max(all, gybytes) - gybytes + ((size_t)256 << 20);
+    const int most = (int)std::min<size_t>(nb, std::max<size_t>(1, room / std::max<size_t>(blk, 1)));
+    const int parts = (nb + most - 1) / most;
+    return 16 * ((nb + parts - 1) / parts);
+}
+
 // bfloat16 features and output gradient; weights, weight gradient and all accumulation in fp32 (the fp32
 // matrix-core kernels with 16-bit loads).  gx32_ws [Cin][ldgx32] and gtree_ws [Cin][ldgt] are fp32 work space:
 // the input gradient is accumulated there and rounded to bfloat16 at the end.
@@ -497,17 +514,19 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         // the image of the weights that the input gradient below packs: fp32 ones where it has no lists (twice the bfloat16 size)
         const size_t wbytes = near.n == 0 ? 0 : align(b.tile_win ? conv_packed_bf16_bytes(code, S_exp, Cin, Cout)
                                                                  : conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
-        const size_t gybytes = align(ngo * (size_t)np * 16), xbytes = align(ngi * (size_t)np * 16), tbytes = align(ngi * (size_t)nt * 16);
+        const size_t gybytes = align(ngo * (size_t)np * 16);
+        const int chunk = gx ? dw_copy_channels(Cin, np, nt, gybytes) : (Cin + 15) / 16 * 16;
+        const size_t ngc = std::min<size_t>(ngi, chunk / 8), xbytes = align(ngc * (size_t)np * 16), tbytes = align(ngc * (size_t)nt * 16);
         const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
         const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
         WinLists wl;
-        bool dw_g8 = regroup_gy && bwd_deterministic() && a.tile_win && gybytes + xbytes + tbytes <= ((size_t)48 << 30) &&
+        bool dw_g8 = regroup_gy && bwd_deterministic() && a.tile_win && gybytes + ngi * (size_t)(np + nt) * 16 <= ((size_t)48 << 30) &&
                      get_lists(p, d, code, tl, &wl, st, false) == 0;
         const bool dx_g8 = near.n > 0 && b.tile_win && regroup_gy;
         size_t need = 0, pbytes = 0;
         auto layout = [&]() {
             need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
-            pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, Cin, Cout, S_exp, a.Lc, wl) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+            pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, std::min(Cin, chunk), Cout, S_exp, a.Lc, wl) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
             return need + pbytes;
         };
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join
@@ -529,10 +548,13 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         if (dw_g8) {
             bf16_t* xi = (bf16_t*)((char*)gyi + gybytes);
             bf16_t* ti = (bf16_t*)((char*)xi + xbytes);
-            if (int rc = interleave8_bf16(x, ldx, nullptr, 0, Cin, Cin, np, xi, side)) return rc;
-            if (int rc = interleave8_bf16(tree_ws, ldt, nullptr, 0, Cin, Cin, nt, ti, side)) return rc;
-            if (int rc = launch_conv_dw_g8(code, xi, np, np, ti, nt, nt, gyi, np, np, Cin, Cout, S_exp, a.Lc, wl,
-                                           (float*)((char*)p->d_scratch + need), gw, side)) return rc;
+            for (int c0 = 0; c0 < Cin; c0 += chunk) {
+                const int c = std::min(chunk, Cin - c0);
+                if (int rc = interleave8_bf16(x + (int64_t)c0 * ldx, ldx, nullptr, 0, c, c, np, xi, side)) return rc;
+                if (int rc = interleave8_bf16(tree_ws + (int64_t)c0 * ldt, ldt, nullptr, 0, c, c, nt, ti, side)) return rc;
+                if (int rc = launch_conv_dw_g8(code, xi, np, np, ti, nt, nt, gyi, np, np, c, c0, Cin, Cout, S_exp, a.Lc, wl,
+                                               (float*)((char*)p->d_scratch + need), gw, side)) return rc;
+            }
         } else if (int rc = launch_conv_dw_mfma(code, a, tl, p->apr.level_min, side)) return rc;
         if (near.n > 0 && b.tile_win) {
             if (int rc = pack_conv_weights_bf16(code, w, S_exp, Cin, Cout, p->d_scratch, st, true)) return rc;

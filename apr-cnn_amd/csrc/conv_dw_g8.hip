@@ -32,13 +32,14 @@ struct DwG8Args {
     const bf16_t* xi; const bf16_t* ti; const bf16_t* gyi;     // [C / 8][count][8]: features, mean tree, output gradient
     int64_t xi_ld, ti_ld, gy_ld;                               // particles between two groups
     int64_t x_count, t_count, gy_count;
-    int Cin, Cout, CinP, CoutP;                                // channels, and rounded up to the kernel's blocks
+    int Cin, Cout, CinP, CoutP;                                // channels of the copies, and rounded up to the kernel's blocks
     const int4* win;
     const int* item_idx; const unsigned short* item_pos; const int* col_idx; const unsigned short* col_pos;
     float* part;                                               // [blocks][K][CoutP][CinP]
     int n_s;                                                   // stencil indices that have windows
     int s_of[MAX_LEVELS], win0[MAX_LEVELS], nwin[MAX_LEVELS];  // their index, first window and windows
     int blk0[MAX_LEVELS + 1];                                  // their first workgroup (blockIdx.x)
+    int ci0, CinW;                                             // first of these channels in the layer, its input channels
 };
 
 constexpr int DWG_COLS = 256;             // columns whose output gradient is staged at a time
@@ -282,7 +283,7 @@ dw_g8_reduce_kernel(const DwG8Args a, int K, float* __restrict__ gw) {
         float v = 0.f;
 #pragma unroll
         for (int i = 0; i < DWG_RED_W; ++i) v += sums[i][lane];
-        gw[(((int64_t)a.s_of[si] * a.Cout + co) * a.Cin + ci) * K + t] += v;
+        gw[(((int64_t)a.s_of[si] * a.Cout + co) * a.CinW + a.ci0 + ci) * K + t] += v;
     }
 }
 
@@ -339,16 +340,18 @@ static int launch_dw_g8_g(const DwG8Args& a, float* gw, hipStream_t st) {
     return 0;
 }
 
-// gw += weight gradient; xi / ti / gyi grouped copies, fewer than 2^28 particles (32-bit byte offsets); `part` holds
-// conv_dw_g8_part_bytes.  One launch for all stencil indices plus one for the sums.
+// gw (of CinW input channels) += weight gradient of the input channels ci0 .. ci0 + Cin - 1, which are those of xi and ti;
+// xi / ti / gyi grouped copies, fewer than 2^28 particles (32-bit byte offsets); `part` holds conv_dw_g8_part_bytes of Cin
+// channels.  One launch for all stencil indices plus one for the sums.
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
-                      const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl, float* part,
-                      float* gw, hipStream_t st) {
+                      const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int ci0, int CinW, int Cout, int S_exp, int Lc,
+                      const WinLists& wl, float* part, float* gw, hipStream_t st) {
     if (wl.n_win <= 0) return 0;
     DwG8Args a{};
     a.xi = xi; a.xi_ld = xi_ld; a.x_count = x_count; a.ti = ti; a.ti_ld = ti_ld; a.t_count = t_count;
     a.gyi = gyi; a.gy_ld = gy_ld; a.gy_count = gy_count;
     dwg_table(code, Cin, Cout, S_exp, Lc, wl, a);
+    a.ci0 = ci0; a.CinW = CinW;
     a.win = wl.d_win; a.item_idx = wl.d_item_idx; a.item_pos = wl.d_item_pos; a.col_idx = wl.d_col_idx; a.col_pos = wl.d_col_pos;
     a.part = part;
     switch (code) {

@@ -15,9 +15,10 @@
 // dw_g8_reduce_kernel).  Calls on one plan give the same bits; the lists of another plan of the same APR may hold a window's
 // columns in another order (their places are taken with an atomic counter when the lists are built), and with it the sums.
 //
-// What bounds it: the LDS reads (7 taps: 9 KB per wave and 32 columns against 14 matrix instructions of 16 cycles) at
-// two workgroups per CU.  The kernel before it read one channel per lane: eight 2-byte LDS reads per operand and a gather of
-// 2-byte values from the channel planes: 1x5x5 64 -> 64 on 15.4 M particles 24.2 ms, 5.8 ms here (3.15 TFLOP).
+// What bounds it: waiting.  1x5x5 64 -> 64 on 15.4 M particles, alone: the waves wait 62 % of their resident cycles
+// (the gather and the three barriers of a window, which every one of its 4 x 2 channel blocks stages anew), LDS is busy
+// 42 % of the launch (a third of that with bank conflicts), the matrix pipes 25 %.  The kernel before it read one channel per lane: eight 2-byte LDS reads per operand and a gather of
+// 2-byte values from the channel planes: 24.2 ms, 5.9 ms here (3.15 TFLOP).
 #include "conv_common.hpp"
 
 namespace aprnet {

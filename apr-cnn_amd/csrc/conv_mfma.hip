@@ -481,7 +481,7 @@ __device__ __forceinline__ void store_items16(const ItemRegs16<G, IPT>& R, int n
 // the planes (element-aligned: planes start wherever `ldx` puts them), transposes them in registers, and the block's
 // 16-byte results go out through LDS so that a wave writes whole lines.  All reads are unconditional and issued before the
 // first is used (a read under "channel exists" is waited for before the next is issued): 64 channels of 15.4 M elements
-// 2.85 -> 0.68 ms, 5.8 TB/s.  (Written straight from the registers, 64 bytes apart: 0.92 ms; one or two elements per thread
+// 2.85 -> 0.68 to 0.72 ms, 5.5 to 5.8 TB/s.  (Written straight from the registers, 64 bytes apart: 0.92 ms; one or two elements per thread
 // with 2-byte reads: 0.69 ms alone, but 3 ms next to the convolution kernels of a backward pass.)
 constexpr int IL_E = 4, IL_TB = 256;
 __global__ void __launch_bounds__(IL_TB)

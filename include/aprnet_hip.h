@@ -70,8 +70,12 @@ int aprnet_plan_create(const aprnet_access_desc* apr, const aprnet_access_desc* 
  * streams they were given: where a program can choose, it destroys a plan before those streams. */
 void aprnet_plan_destroy(aprnet_plan* plan);
 
-/* No counterpart in the reference.  The convolutions keep re-laid-out weights (and, for bfloat16 features, a regrouped
- * copy of their input) in one scratch buffer of the plan that grows to the largest call seen.  Growth allocates, so it is
+/* No counterpart in the reference.  The convolutions keep re-laid-out weights, the partial sums of weight gradients and, for
+ * bfloat16 features, copies grouped by eight channels (16 bytes per particle and eight channels: input and mean tree in
+ * the forward pass; output gradient, input and mean tree in the backward pass, the latter two a part of the channels at a
+ * time in large layers) in one scratch buffer of the plan that grows to the largest call seen.  The copies are left out, and
+ * slower kernels on the channel planes run, from 2^28 particles on, beyond 32 GiB of them in the forward pass and 48 GiB in
+ * the backward pass, and in the backward pass where there is no room for them.  Growth allocates, so it is
  * refused with APRNET_ERR_UNSUPPORTED while `stream` is capturing into a graph, and so is the first convolution at a
  * level delta (it builds the plan's tile and window lists).  Call this - or run the network once - before a capture;
  * a buffer that a captured graph may address is kept until aprnet_plan_destroy.  Calls that share a plan use one
@@ -107,19 +111,20 @@ int aprnet_profile_enable(int on);
  * use and keeps (about 20 bytes of device memory per particle and level delta; default), 5 = scan the access arrays
  * in every call (also the fallback when the lists cannot be allocated); and for the backward matrix-core kernels:
  * 6 = the weight gradient runs on a second stream of the plan next to the input gradient, forked from and joined
- * to the caller's stream with events (default), 7 = both on the caller's stream; and for the bfloat16 forward
- * kernel: 8 = stage from a copy of the input regrouped as [Cin / 8][particles][8] in the plan's scratch buffer, one
- * 16-byte load per item and 8 channels (default; 16 bytes per particle and 8 channels of device memory, made by one
- * streaming pass per call), 9 = gather from the channel planes; and for the weight gradient of the matrix-core
+ * to the caller's stream with events (default), 7 = both on the caller's stream; and for the bfloat16 kernels on
+ * channel planes, forward and backward: 8 = stage from copies of their inputs regrouped as [C / 8][particles][8] in the
+ * plan's scratch buffer, one 16-byte load per item and 8 channels (default; made by one streaming pass per call), 9 = gather
+ * from the channel planes; and for the weight gradient of the matrix-core
  * kernels: 10 = every workgroup writes the sums of its tiles to its own slots of the plan's scratch buffer and a second
- * kernel adds the slots in a fixed order (default: the gradient repeats bit for bit from call to call; at most 512 MiB
+ * kernel adds the slots in a fixed order (default: the gradient repeats bit for bit from call to call on a plan; at most 512 MiB
  * of scratch, for very wide layers 32 times the gradient of one stencil, or the gradient itself where bfloat16 features
  * are staged from grouped copies), 11 = atomic additions; and for forward layers of 1 to 3 input channels (bound by memory, not by the
  * contraction): 12 = the pipelined kernel with the (tap, channel) axis flattened (default), 13 = the general kernel;
  * and for the bfloat16 forward kernel on grouped tensors: 14 = 32-bit byte offsets where a group holds fewer than 2^28
  * elements, 64-bit addresses beyond (default), 15 = 64-bit addresses always; and for the tree fill that precedes a
- * forward stencil convolution: 16 = fill the nodes that the kernel's window lists read, and their descendants (default;
- * the node lists are built with the window lists and kept in the plan, 4 bytes per needed node), 17 = fill every node.
+ * stencil convolution, forward or backward, and the hand-down of the tree's gradient that follows a backward one: 16 = the
+ * nodes that the forward kernel's window lists read, and their descendants (default; the node lists are built with the
+ * window lists and kept in the plan, 4 bytes per needed node), 17 = every node.
  * All are HIP kernels; the switch
  * exists so that tests can cover them and memory-bound callers can do without the lists. */
 int aprnet_set_conv_path(int path);

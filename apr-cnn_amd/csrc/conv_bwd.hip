@@ -275,7 +275,7 @@ int launch_face_dx(const FaceLists& fl, const float* gy, int64_t ldy, const floa
 size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl);
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
                       const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int ci0, int CinW, int Cout, int S_exp, int Lc,
-                      const WinLists& wl, float* part, float* gw, hipStream_t st);
+                      const WinLists& wl, float* part, size_t part_bytes, float* gw, hipStream_t st);
 int conv_dw_partial_blocks(int code, int Cout, int Cin);
 size_t conv_dw_partial_bytes(int code, int Cout, int Cin);
 // Points the weight-gradient kernels at their partial-sum slots, `off` bytes into the plan's scratch buffer (behind
@@ -526,7 +526,9 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         size_t need = 0, pbytes = 0;
         auto layout = [&]() {
             need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
-            pbytes = dw_g8 ? conv_dw_g8_part_bytes(code, std::min(Cin, chunk), Cout, S_exp, a.Lc, wl) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+            const int last = Cin - (Cin - 1) / chunk * chunk;              // channels of the last part
+            pbytes = dw_g8 ? std::max(conv_dw_g8_part_bytes(code, std::min(Cin, chunk), Cout, S_exp, a.Lc, wl),
+                                      conv_dw_g8_part_bytes(code, last, Cout, S_exp, a.Lc, wl)) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
             return need + pbytes;
         };
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join
@@ -553,7 +555,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
                 if (int rc = interleave8_bf16(x + (int64_t)c0 * ldx, ldx, nullptr, 0, c, c, np, xi, side)) return rc;
                 if (int rc = interleave8_bf16(tree_ws + (int64_t)c0 * ldt, ldt, nullptr, 0, c, c, nt, ti, side)) return rc;
                 if (int rc = launch_conv_dw_g8(code, xi, np, np, ti, nt, nt, gyi, np, np, c, c0, Cin, Cout, S_exp, a.Lc, wl,
-                                               (float*)((char*)p->d_scratch + need), gw, side)) return rc;
+                                               (float*)((char*)p->d_scratch + need), pbytes, gw, side)) return rc;
             }
         } else if (int rc = launch_conv_dw_mfma(code, a, tl, p->apr.level_min, side)) return rc;
         if (near.n > 0 && b.tile_win) {

@@ -323,6 +323,7 @@ static void dwg_table(int code, int Cin, int Cout, int S_exp, int Lc, const WinL
     for (int k = 0; k < a.n_s; ++k)                        // (together at most bx + n_s)
         a.blk0[k + 1] = a.blk0[k] + (int)std::max<int64_t>(1, std::min<int64_t>(a.nwin[k], bx * a.nwin[k] / wl.n_win));
 }
+// (not monotonous in the channels: the workgroups are rounded down)
 size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout, int S_exp, int Lc, const WinLists& wl) {
     DwG8Args a{};
     dwg_table(code, Cin, Cout, S_exp, Lc, wl, a);
@@ -342,16 +343,18 @@ static int launch_dw_g8_g(const DwG8Args& a, float* gw, hipStream_t st) {
 }
 
 // gw (of CinW input channels) += weight gradient of the input channels ci0 .. ci0 + Cin - 1, which are those of xi and ti;
-// xi / ti / gyi grouped copies, fewer than 2^28 particles (32-bit byte offsets); `part` holds conv_dw_g8_part_bytes of Cin
-// channels.  One launch for all stencil indices plus one for the sums.
+// xi / ti / gyi grouped copies, fewer than 2^28 particles (32-bit byte offsets); `part` holds part_bytes, at least
+// conv_dw_g8_part_bytes of Cin channels.  One launch for all stencil indices plus one for the sums.
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
                       const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int ci0, int CinW, int Cout, int S_exp, int Lc,
-                      const WinLists& wl, float* part, float* gw, hipStream_t st) {
+                      const WinLists& wl, float* part, size_t part_bytes, float* gw, hipStream_t st) {
     if (wl.n_win <= 0) return 0;
     DwG8Args a{};
     a.xi = xi; a.xi_ld = xi_ld; a.x_count = x_count; a.ti = ti; a.ti_ld = ti_ld; a.t_count = t_count;
     a.gyi = gyi; a.gy_ld = gy_ld; a.gy_count = gy_count;
     dwg_table(code, Cin, Cout, S_exp, Lc, wl, a);
+    if ((size_t)a.blk0[a.n_s] * dwg_slot_bytes(code, a) > part_bytes)
+        return fail(APRNET_ERR_INVALID_ARGUMENT, "weight gradient: the buffer for partial sums is too small");
     a.ci0 = ci0; a.CinW = CinW;
     a.win = wl.d_win; a.item_idx = wl.d_item_idx; a.item_pos = wl.d_item_pos; a.col_idx = wl.d_col_idx; a.col_pos = wl.d_col_pos;
     a.part = part;

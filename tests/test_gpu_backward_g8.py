@@ -188,22 +188,25 @@ def test_partial_sums_of_a_wide_layer_stay_within_512_mib():
     assert float((gw - planes).abs().max()) <= 1e-5 * float(planes.abs().max())
 
 
-def test_copies_of_a_large_layer_are_made_in_parts():
-    """40 -> 33 on 7 M particles: features and tree are copied 16, 16 and 8 channels at a time, so that the scratch buffer holds
-    the copies of the output gradient and of one part (at most 256 MiB more than the forward pass needs).  Against the
-    kernel on channel planes (the same products; fp32 sums of 7 M terms in another order) and a second run."""
+@pytest.mark.parametrize("cin,cout", [(40, 33), (80, 32)])
+def test_copies_of_a_large_layer_are_made_in_parts(cin, cout):
+    """Features and tree of 7 M particles are copied 16, 16 and 8 channels at a time (40 -> 33), 48 and 32 (80 -> 32, where the
+    smaller part has more slots of partial sums in all), so that the scratch buffer holds the copies of the output gradient
+    and of one part (at most 256 MiB more than the forward pass needs).  Against the kernel on channel planes (the same
+    products; fp32 sums of 7 M terms in another order) and a second run."""
     apr, _ = make_config("blobs512", scale=0.68)
     gen = torch.Generator(device=DEV).manual_seed(3)
     n, nt, ld = apr.total_number_particles(), _ops.tree_parts(apr, 0), torch.zeros(1, dtype=torch.int32)
-    x = torch.randn(1, 40, n, device=DEV, generator=gen).to(torch.bfloat16)
-    gy = torch.randn(1, 33, n, device=DEV, generator=gen).to(torch.bfloat16)
-    w = torch.randn(2, 33, 40, 3, 3, 3, device=DEV, generator=gen)
+    x = torch.randn(1, cin, n, device=DEV, generator=gen).to(torch.bfloat16)
+    gy = torch.randn(1, cout, n, device=DEV, generator=gen).to(torch.bfloat16)
+    w = torch.randn(2, cout, cin, 3, 3, 3, device=DEV, generator=gen)
     _ops.conv_backward([apr], x[:, :1].contiguous(), w[:, :1, :1].contiguous(), gy[:, :1].contiguous(), ld)      # the plan's lists
     torch.cuda.empty_cache()
     before = _memory_outside_torch()
     gw = _ops.conv_backward([apr], x, w, gy, ld)[1]
     grown = _memory_outside_torch() - before
-    assert 16 * 5 * n <= grown <= max(16 * 5 * (n + nt), 16 * 5 * n) + (256 << 20) + (128 << 20)    # ... and the sums' slots
+    gi, go = (cin + 7) // 8, (cout + 7) // 8
+    assert 16 * go * n <= grown <= 16 * max(gi * (n + nt), go * n) + (256 << 20) + (128 << 20)    # ... and the sums' slots
     assert torch.equal(gw, _ops.conv_backward([apr], x, w, gy, ld)[1])
     lib = _native.hip()
     assert lib.aprnet_set_conv_path(9) == 0

@@ -5,19 +5,17 @@
 
 namespace aprnet {
 
-// out[e] += sum of part[slot][e] over the slots, in an order that is fixed by the slot count alone: wave w of the block's W (at
-// most RED_W, no more than there are slots) adds slots w, w + W, ... (eight loads in flight), the W sums of an element
-// meet in LDS and are added in wave order.  A wave reads 64 neighbouring elements of a slot, whole lines: with a wave per
-// element, whose lanes read one element of 64 slots, the 1x1x1 backward of 512 -> 512 channels took 9.80 ms on 103 k
-// particles and 2.63 ms on 4 k, now 9.59 and 2.40 ms.
+// out[e] += sum of part[slot][e] over the slots, in an order that is fixed by the slot count alone: wave w of the block's W adds
+// slots w, w + W, ... (eight loads in flight), the W sums of an element meet in LDS and are added in wave order.
+// A wave reads 64 neighbouring elements of a slot, whole lines: with a wave per element, whose lanes read one element of 64
+// slots, the 1x1x1 backward of 512 -> 512 channels took 9.80 ms on 103 k particles and 2.63 ms on 4 k, now 9.59 and 2.40 ms.
 // Bound by the latency of the chain of loads when one thread walks all slots of an element (27 k elements fill a tenth of
 // the chip): 128 us on average over the launches of a training step of the 16-32-64 network on 5.5 M particles, 48 us with
-// RED_W waves per 64 elements.
-constexpr int RED_W = 16;
-template <typename A>
-__global__ void __launch_bounds__(64 * RED_W) sum_slots_kernel(const A* __restrict__ part, int64_t ld, int slots, int64_t n, A* __restrict__ out) {
-    __shared__ A sums[RED_W][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, W = blockDim.x >> 6;
+// 16 waves per 64 elements.
+template <typename A, int W>
+__global__ void __launch_bounds__(64 * W) sum_slots_kernel(const A* __restrict__ part, int64_t ld, int slots, int64_t n, A* __restrict__ out) {
+    __shared__ A sums[W][64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int64_t e = (int64_t)blockIdx.x * 64 + lane;
     const A* src = part + (e < n ? e : n - 1);
     A s[8];
@@ -32,15 +30,19 @@ __global__ void __launch_bounds__(64 * RED_W) sum_slots_kernel(const A* __restri
     __syncthreads();
     if (w == 0 && e < n) {
         A t = 0;
+#pragma unroll
         for (int i = 0; i < W; ++i) t += sums[i][lane];
         out[e] += t;
     }
 }
 
+// 16 waves, 4 where there are fewer slots than that (1x1x1 256 -> 512 on 4 k particles, 3 slots: 2.54 instead of 2.55 ms)
 template <typename A>
 int launch_sum_slots(const A* part, int64_t ld, int slots, int64_t n, A* out, hipStream_t st) {
     if (n <= 0 || slots <= 0) return 0;
-    hipLaunchKernelGGL(sum_slots_kernel<A>, dim3((unsigned)((n + 63) / 64)), dim3(64u * (slots < RED_W ? slots : RED_W)), 0, st, part, ld, slots, n, out);
+    const dim3 grid((unsigned)((n + 63) / 64));
+    if (slots < 16) hipLaunchKernelGGL((sum_slots_kernel<A, 4>), grid, dim3(64 * 4), 0, st, part, ld, slots, n, out);
+    else hipLaunchKernelGGL((sum_slots_kernel<A, 16>), grid, dim3(64 * 16), 0, st, part, ld, slots, n, out);
     APRNET_LAUNCH_CHECK("sum_slots_kernel");
     return 0;
 }

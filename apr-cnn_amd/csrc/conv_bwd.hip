@@ -249,9 +249,9 @@ static int launch_bwd(ConvArgs<T>& a, hipStream_t st) {
 // matrix-core kernels (conv_mfma.hip, conv_bwd_mfma.hip)
 bool conv_mfma_supported(int code);
 int launch_conv_dx_mfma(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
-int launch_conv_dw_mfma(int code, const ConvArgs<float>& a, const TileList& tl, int level_min, hipStream_t st);
+int launch_conv_dw_mfma(int code, const ConvArgs<float>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st);
 int launch_conv_dx_mfma(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
-int launch_conv_dw_mfma(int code, const ConvArgs<bf16_t>& a, const TileList& tl, int level_min, hipStream_t st);
+int launch_conv_dw_mfma(int code, const ConvArgs<bf16_t>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st);
 int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx, int C, bf16_t* tree, int64_t ldt, hipStream_t st, const NeedLists* need);
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
 int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st);
@@ -276,15 +276,13 @@ size_t conv_dw_g8_part_bytes(int code, int Cin, int Cout, int S_exp, int Lc, con
 int launch_conv_dw_g8(int code, const bf16_t* xi, int64_t xi_ld, int64_t x_count, const bf16_t* ti, int64_t ti_ld, int64_t t_count,
                       const bf16_t* gyi, int64_t gy_ld, int64_t gy_count, int Cin, int ci0, int CinW, int Cout, int S_exp, int Lc,
                       const WinLists& wl, float* part, size_t part_bytes, float* gw, hipStream_t st);
-int conv_dw_partial_blocks(int code, int Cout, int Cin);
-size_t conv_dw_partial_bytes(int code, int Cout, int Cin);
+size_t conv_dw_partial_bytes(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists* wl);
 // Points the weight-gradient kernels at their partial-sum slots, `off` bytes into the plan's scratch buffer (behind
 // whatever the input gradient keeps there: the two run side by side).
 template <typename T>
 static void set_dw_partials(aprnet_plan* p, size_t off, int code, ConvArgs<T>& a) {
     a.gw_part = (float*)((char*)p->d_scratch + off);
     a.gw_part_ld = (int64_t)a.Cout * a.Cin * (code == 333 ? 27 : code == 133 ? 9 : 25);
-    a.gw_part_blocks = conv_dw_partial_blocks(code, a.Cout, a.Cin);
 }
 
 template <typename T> static int try_mfma_bwd(aprnet_plan*, const ConvArgs<T>&, const TileList&, int, int, hipStream_t, bool*) { return 0; }
@@ -304,6 +302,9 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     // weight gradient on the side stream (when there is an input gradient to run next to)
     ConvArgs<float> c = a;
     if (int rc = set_conv_lists(p, d, code, tl, c, st)) return rc;
+    WinLists lists;
+    const WinLists* wl = c.tile_win && get_lists(p, d, code, tl, &lists, st) == 0 ? &lists : nullptr;
+    if (!wl) c.tile_win = nullptr;
     // everything that can allocate or fail on the host comes before the fork
     TileList near;
     FaceLists faces;
@@ -311,14 +312,14 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     if (a.gx) if (int rc = get_tiles(p, d, code == 333 ? 2 : 1, code == 333 ? 4 : 8, &near, st, 1)) return rc;
     if (split_faces) if (int rc = get_face_lists(p, d, code, &faces, st)) return rc;
     const size_t wbytes = a.gx ? (conv_packed_floats(code, a.S_exp, a.Cin, a.Cout, true) * sizeof(float) + 255) / 256 * 256 : 0;
-    const size_t pbytes = bwd_deterministic() ? conv_dw_partial_bytes(code, a.Cout, a.Cin) : 0;
+    const size_t pbytes = bwd_deterministic() ? conv_dw_partial_bytes(code, a.Cout, a.Cin, a.S_exp, a.Lc, wl) : 0;
     ScratchLease lease;          // before the join guard below: its hand-over event is recorded after the join
     if (wbytes + pbytes) if (int rc = lease.acquire(p, wbytes + pbytes, st)) return rc;
     if (pbytes) set_dw_partials(p, wbytes, code, c);
     hipStream_t side = st;
     if (a.gx) if (int rc = fork_side(p, st, &side)) return rc;
     SideJoin guard(p, st, side);
-    if (int rc = launch_conv_dw_mfma(code, c, tl, p->apr.level_min, side)) return rc;
+    if (int rc = launch_conv_dw_mfma(code, c, tl, wl, p->apr.level_min, side)) return rc;
     if (a.gx) {
         // input gradient: the forward kernel on the output gradient with the transposed, flipped stencil;
         // every row group within one row of an output takes part
@@ -520,15 +521,16 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
         const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
         WinLists wl;
-        bool dw_g8 = regroup_gy && bwd_deterministic() && a.tile_win && gybytes + ngi * (size_t)(np + nt) * 16 <= ((size_t)48 << 30) &&
-                     get_lists(p, d, code, tl, &wl, st, false) == 0;
+        const bool listed = a.tile_win && get_lists(p, d, code, tl, &wl, st, false) == 0;
+        if (!listed) a.tile_win = nullptr;
+        bool dw_g8 = regroup_gy && bwd_deterministic() && listed && gybytes + ngi * (size_t)(np + nt) * 16 <= ((size_t)48 << 30);
         const bool dx_g8 = near.n > 0 && b.tile_win && regroup_gy;
         size_t need = 0, pbytes = 0;
         auto layout = [&]() {
             need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
             const int last = Cin - (Cin - 1) / chunk * chunk;              // channels of the last part
             pbytes = dw_g8 ? std::max(conv_dw_g8_part_bytes(code, std::min(Cin, chunk), Cout, S_exp, a.Lc, wl),
-                                      conv_dw_g8_part_bytes(code, last, Cout, S_exp, a.Lc, wl)) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin) : 0;
+                                      conv_dw_g8_part_bytes(code, last, Cout, S_exp, a.Lc, wl)) : bwd_deterministic() ? conv_dw_partial_bytes(code, Cout, Cin, S_exp, a.Lc, listed ? &wl : nullptr) : 0;
             return need + pbytes;
         };
         ScratchLease lease;      // before the join guard below: its hand-over event is recorded after the join
@@ -557,7 +559,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
                 if (int rc = launch_conv_dw_g8(code, xi, np, np, ti, nt, nt, gyi, np, np, c, c0, Cin, Cout, S_exp, a.Lc, wl,
                                                (float*)((char*)p->d_scratch + need), pbytes, gw, side)) return rc;
             }
-        } else if (int rc = launch_conv_dw_mfma(code, a, tl, p->apr.level_min, side)) return rc;
+        } else if (int rc = launch_conv_dw_mfma(code, a, tl, listed ? &wl : nullptr, p->apr.level_min, side)) return rc;
         if (near.n > 0 && b.tile_win) {
             if (int rc = pack_conv_weights_bf16(code, w, S_exp, Cin, Cout, p->d_scratch, st, true)) return rc;
             if (dx_g8) { b.xi = gyi; b.ti = nullptr; b.xi_ld = np; b.ti_ld = 0; }

@@ -14,8 +14,8 @@
 //
 // A block owns 16 input channels (four staged chunks of 4) and 32 output channels.  Wave w takes input
 // channel w%4 of every chunk and half of the columns (w/4), so it holds four accumulators, and keeps them
-// in registers while the (persistent) block walks over many tiles of one stencil index (one launch per
-// stencil index); they are added to the result with one atomic per element at the end.  The patch rows are 67 words
+// in registers while the (persistent) block walks over many windows of one stencil index (one launch
+// for all of them, see DwWork); its sums go to slots of its own, which sum_slots.hpp adds up in a fixed order.  The patch rows are 67 words
 // apart so that the 27 tap offsets of a B read fall into 27 different LDS banks.
 #include "conv_common.hpp"
 #include "sum_slots.hpp"
@@ -34,6 +34,15 @@ constexpr int DW_NCH = 4;          // chunks per block
 constexpr int DW_GB = 256;         // columns of gY staged at a time
 constexpr int DW_KB = 8;          // MFMAs issued back to back between operand phases (16 would spill registers)
 constexpr int DW_GLD = 33;         // words per column of gyl (32 output channels + 1 against bank conflicts)
+
+// Work of a launch on the plan's window lists: workgroups blk0[k] .. blk0[k + 1] - 1 (grid.x) take the windows of stencil
+// index s_of[k] in turn.  One launch covers all stencil indices: with one launch each, whose coarse levels have fewer windows than
+// the chip has places, a training step of the 16-32-64-128 network on two APRs of 338 k particles spent LAUNCHES_BEFORE
+struct DwWork {
+    int n_s;
+    int s_of[MAX_LEVELS + 1], win0[MAX_LEVELS + 1], nwin[MAX_LEVELS + 1], blk0[MAX_LEVELS + 2];
+    int first_coarse;              // windows from here on may stage tree nodes (below the finest level of the call)
+};
 
 // Lists of the plan carry patch cells for rows of 64 words; this kernel's rows are RS words apart.
 template <class G> __device__ __forceinline__ unsigned restride(unsigned pos) {
@@ -228,7 +237,7 @@ __device__ __forceinline__ void dw_window16(const ConvArgs<T>& a, const Lists& s
 
 template <typename T, class G, int CIB, int NCH, bool LISTS>
 __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
-conv_dw16_mfma_kernel(const ConvArgs<T> a, const int s_idx) {
+conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
     static_assert(G::NWAVE == 8 && CIB == 4, "wave w owns input channel w%4 and column half w/4");
     __shared__ float patch[CIB * G::CH_STRIDE];
     __shared__ float gyl[DW_GB * DW_GLD16];
@@ -254,20 +263,25 @@ conv_dw16_mfma_kernel(const ConvArgs<T> a, const int s_idx) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[q][tile][r] = 0.f;
 
-    for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
-        const ConvTile tile = a.tiles[ti];
-        const int L = tile.level;
-        const bool tree_items = L < a.Lc;
-        if constexpr (LISTS) {
-            const int wb = a.tile_win[ti], we = a.tile_win[ti + 1];
-            for (int w = wb; w < we; ++w) {
-                const int4 hd = a.win[w];
-                const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-                const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
-                                     a.l_col_pos + (unsigned)hd.z};
-                dw_window16<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, bl, kh, wave, lane, patch, gyl, cpl, acc);
-            }
-        } else {
+    int s_idx = s_arg;
+    if constexpr (LISTS) {
+        int si = 0;
+        while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
+        s_idx = wk.s_of[si];
+        const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si];
+        for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
+            const int4 hd = a.win[w];
+            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+            const bool tree_items = w >= wk.first_coarse;
+            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
+                                 a.l_col_pos + (unsigned)hd.z};
+            dw_window16<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, bl, kh, wave, lane, patch, gyl, cpl, acc);
+        }
+    } else {
+        for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
+            const ConvTile tile = a.tiles[ti];
+            const int L = tile.level;
+            const bool tree_items = L < a.Lc;
             __shared__ ConvShared<G> sh;
             const int yn = a.apr.y_num[L];
             const bool out_tree = (L == a.Lc) && (L < a.apr.level_max);
@@ -375,7 +389,7 @@ __device__ __forceinline__ void dw_window_bf16(const ConvArgs<bf16_t>& a, const 
 
 template <class G, int CIB, int NCH, bool LISTS>
 __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
-conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const int s_idx) {
+conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const DwWork wk, const int s_arg) {
     static_assert(G::NWAVE == 8 && CIB == 4, "wave w owns input channel w%4 and column half w/4");
     static_assert(G::CH_STRIDE % 2 == 0 && DW_LDG16 % 8 == 0, "dword fill of the patch, 16-byte rows of gyl");
     __shared__ __attribute__((aligned(16))) unsigned short patch[CIB * G::CH_STRIDE];
@@ -397,20 +411,25 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const int s_idx) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
 
-    for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
-        const ConvTile tile = a.tiles[ti];
-        const int L = tile.level;
-        const bool tree_items = L < a.Lc;
-        if constexpr (LISTS) {
-            const int wb = a.tile_win[ti], we = a.tile_win[ti + 1];
-            for (int w = wb; w < we; ++w) {
-                const int4 hd = a.win[w];
-                const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-                const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
-                                     a.l_col_pos + (unsigned)hd.z};
-                dw_window_bf16<G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, acc);
-            }
-        } else {
+    int s_idx = s_arg;
+    if constexpr (LISTS) {
+        int si = 0;
+        while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
+        s_idx = wk.s_of[si];
+        const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si];
+        for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
+            const int4 hd = a.win[w];
+            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+            const bool tree_items = w >= wk.first_coarse;
+            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
+                                 a.l_col_pos + (unsigned)hd.z};
+            dw_window_bf16<G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, acc);
+        }
+    } else {
+        for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
+            const ConvTile tile = a.tiles[ti];
+            const int L = tile.level;
+            const bool tree_items = L < a.Lc;
             __shared__ ConvShared<G> sh;
             const int yn = a.apr.y_num[L];
             const bool out_tree = (L == a.Lc) && (L < a.apr.level_max);
@@ -447,7 +466,7 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const int s_idx) {
 // LISTS: the windows come from the plan's lists; otherwise the block scans the access arrays.
 template <typename T, class G, int CIB, int NCH, bool LISTS>
 __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
-conv_dw_mfma_kernel(const ConvArgs<T> a, const int s_idx) {
+conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
     static_assert(G::NWAVE == 8 && CIB == 4, "wave w owns input channel w%4 and column half w/4");
     __shared__ float patch[CIB * G::CH_STRIDE];
     __shared__ float gyl[DW_GB * DW_GLD];
@@ -469,20 +488,25 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const int s_idx) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
 
-    for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
-        const ConvTile tile = a.tiles[ti];
-        const int L = tile.level;
-        const bool tree_items = L < a.Lc;
-        if constexpr (LISTS) {
-            const int wb = a.tile_win[ti], we = a.tile_win[ti + 1];
-            for (int w = wb; w < we; ++w) {
-                const int4 hd = a.win[w];
-                const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-                const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
-                                     a.l_col_pos + (unsigned)hd.z};
-                dw_window<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, ap, acc);
-            }
-        } else {
+    int s_idx = s_arg;
+    if constexpr (LISTS) {
+        int si = 0;
+        while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
+        s_idx = wk.s_of[si];
+        const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si];
+        for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
+            const int4 hd = a.win[w];
+            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+            const bool tree_items = w >= wk.first_coarse;
+            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
+                                 a.l_col_pos + (unsigned)hd.z};
+            dw_window<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, ap, acc);
+        }
+    } else {
+        for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
+            const ConvTile tile = a.tiles[ti];
+            const int L = tile.level;
+            const bool tree_items = L < a.Lc;
             __shared__ ConvShared<G> sh;
             const int yn = a.apr.y_num[L];
             const bool out_tree = (L == a.Lc) && (L < a.apr.level_max);
@@ -515,23 +539,81 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const int s_idx) {
     }
 }
 
-// Workgroups of one weight-gradient launch when its partial sums go to a buffer: at most 512, fewer for very wide
-// layers so that the buffer (two slots per workgroup) stays within 512 MiB.
-int conv_dw_partial_blocks(int code, int Cout, int Cin) {
-    const int64_t e = (int64_t)Cout * Cin * (code == 333 ? 27 : code == 133 ? 9 : 25);
-    const int64_t cap = ((int64_t)512 << 20) / (8 * e);
-    return (int)std::max<int64_t>(16, std::min<int64_t>(512, cap));
+static int dw_taps(int code) { return code == 333 ? 27 : code == 133 ? 9 : 25; }
+// a narrow input (the first layer of a network) fits one chunk: no staging and products of empty chunks
+static int dw_chunks(int Cin) { return Cin <= DW_CIB ? 1 : DW_NCH; }
+// Workgroups along grid.x: two rounds of the 512 that the chip holds, fewer for layers with several channel blocks, whose every
+// window is visited once per block, and for very wide layers, so that the partial sums (two slots per workgroup) stay
+// within 512 MiB.
+static int dw_blocks_x(int code, int Cout, int Cin) {
+    const int nci = DW_CIB * dw_chunks(Cin), per = ((Cin + nci - 1) / nci) * ((Cout + 31) / 32);
+    const int64_t cap = ((int64_t)512 << 20) / (8 * (int64_t)Cout * Cin * dw_taps(code));
+    return (int)std::max<int64_t>(16, std::min<int64_t>(std::max(64, 1024 / per), cap));
 }
-size_t conv_dw_partial_bytes(int code, int Cout, int Cin) {
-    const int64_t e = (int64_t)Cout * Cin * (code == 333 ? 27 : code == 133 ? 9 : 25);
-    return (size_t)(2 * conv_dw_partial_blocks(code, Cout, Cin)) * e * sizeof(float);
+// The stencil indices that have windows, and a share of the workgroups for each by its windows.
+static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists& wl) {
+    DwWork k{};
+    k.first_coarse = (wl.n_lv > 0 && wl.lv_level[0] == Lc) ? (wl.n_lv > 1 ? wl.lv_first[1] : wl.n_win) : 0;
+    for (int i = 0; i < wl.n_lv; ++i) {                    // finest level first: stencil indices ascend
+        const int s = std::min(S_exp - 1, Lc - wl.lv_level[i]);
+        const int w0 = wl.lv_first[i], w1 = i + 1 < wl.n_lv ? wl.lv_first[i + 1] : wl.n_win;
+        if (k.n_s > 0 && k.s_of[k.n_s - 1] == s) { k.nwin[k.n_s - 1] = w1 - k.win0[k.n_s - 1]; continue; }
+        k.s_of[k.n_s] = s; k.win0[k.n_s] = w0; k.nwin[k.n_s] = w1 - w0; ++k.n_s;
+    }
+    const int64_t bx = dw_blocks_x(code, Cout, Cin);
+    for (int i = 0; i < k.n_s; ++i)                        // (together at most bx + n_s)
+        k.blk0[i + 1] = k.blk0[i] + (int)std::max<int64_t>(1, std::min<int64_t>(k.nwin[i], bx * k.nwin[i] / wl.n_win));
+    return k;
+}
+// wl null: the kernels scan
+size_t conv_dw_partial_bytes(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists* wl) {
+    const int blocks = wl ? [&] { const DwWork k = dw_work(code, Cout, Cin, S_exp, Lc, *wl); return k.blk0[k.n_s]; }() : dw_blocks_x(code, Cout, Cin);
+    return (size_t)(2 * blocks) * Cout * Cin * dw_taps(code) * sizeof(float);
 }
 
-// Weight gradient; a.gw is accumulated into (the caller zeroes it).
-// One launch per stencil index: level Lc - s for s < S_exp - 1, every coarser level for the last one
-// (adjacent in the tile list, which is sorted finest level first).
+template <typename T, class G, bool LISTS>
+static int launch_dw_kernel(const ConvArgs<T>& a, const DwWork& k, int s, int blocks, hipStream_t st) {
+    const int nch = dw_chunks(a.Cin);
+    dim3 grid((unsigned)blocks, (unsigned)((a.Cin + DW_CIB * nch - 1) / (DW_CIB * nch)), (unsigned)((a.Cout + 31) / 32));
+    if constexpr (std::is_same<T, bf16_t>::value) {
+        if (bf16_math()) {      // bfloat16 matrix instructions; the fp32 ones below when those are asked for
+            if (nch == 1) hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, 1, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
+            else hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, DW_NCH, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
+            APRNET_LAUNCH_CHECK("conv_dw_bf16_kernel");
+            return 0;
+        }
+    }
+    if (a.Cout <= 16) {         // 16-row form
+        if (nch == 1) hipLaunchKernelGGL((conv_dw16_mfma_kernel<T, G, DW_CIB, 1, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
+        else hipLaunchKernelGGL((conv_dw16_mfma_kernel<T, G, DW_CIB, DW_NCH, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
+        APRNET_LAUNCH_CHECK("conv_dw16_mfma_kernel");
+        return 0;
+    }
+    if (nch == 1) hipLaunchKernelGGL((conv_dw_mfma_kernel<T, G, DW_CIB, 1, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
+    else hipLaunchKernelGGL((conv_dw_mfma_kernel<T, G, DW_CIB, DW_NCH, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
+    APRNET_LAUNCH_CHECK("conv_dw_mfma_kernel");
+    return 0;
+}
+
+// Weight gradient; a.gw is accumulated into (the caller zeroes it).  The partial sums of a launch are added up in slot order
+// (every slot of the grid is written in full).
 template <typename T, class G>
-static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, int level_min, hipStream_t st) {
+static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st) {
+    const int code = G::KZ * 100 + G::KX * 10 + G::KY;
+    const int64_t n_el = (int64_t)a0.Cout * a0.Cin * G::K;
+    if (a0.tile_win && wl) {
+        if (wl->n_win <= 0) return 0;
+        const DwWork k = dw_work(code, a0.Cout, a0.Cin, a0.S_exp, a0.Lc, *wl);
+        if (int rc = launch_dw_kernel<T, G, true>(a0, k, 0, k.blk0[k.n_s], st)) return rc;
+        if (!a0.gw_part) return 0;
+        SlotGroups g{};
+        g.n = k.n_s;
+        for (int i = 0; i < k.n_s; ++i) { g.first[i] = 2 * k.blk0[i]; g.out[i] = k.s_of[i]; }
+        g.first[k.n_s] = 2 * k.blk0[k.n_s];
+        return launch_sum_slot_groups((const float*)a0.gw_part, a0.gw_part_ld, g, n_el, (float*)a0.gw, st);
+    }
+    // scanning kernels: one launch per stencil index, level Lc - s for s < S_exp - 1, every coarser level for the last one
+    // (adjacent in the tile list, which is sorted finest level first)
     for (int s = 0; s < a0.S_exp; ++s) {
         const int l_hi = a0.Lc - s, l_lo = (s == a0.S_exp - 1) ? level_min : l_hi;
         if (l_hi < level_min) break;
@@ -540,64 +622,28 @@ static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, int level_min, h
         if (n == 0) continue;
         ConvArgs<T> a = a0;
         a.tiles = tl.d_tiles + tl.level_begin[l_hi]; a.n_tiles = n;
-        if (a.tile_win) a.tile_win += tl.level_begin[l_hi];
-        // a narrow input (the first layer of a network) fits one chunk: no staging and products of empty chunks
-        const int nch = a.Cin <= DW_CIB ? 1 : DW_NCH;
-        const int gmax = a.gw_part ? a.gw_part_blocks : 512;
-        dim3 grid((unsigned)std::min(n, gmax), (unsigned)((a.Cin + DW_CIB * nch - 1) / (DW_CIB * nch)), (unsigned)((a.Cout + 31) / 32));
-        const int64_t n_el = (int64_t)a.Cout * a.Cin * G::K;
-        // the partial sums of this launch, added up in slot order (every slot of the grid is written in full)
-        auto reduce = [&]() -> int {
-            if (!a.gw_part) return 0;
-            return launch_sum_slots((const float*)a.gw_part, a.gw_part_ld, 2 * (int)grid.x, n_el, (float*)a.gw + (int64_t)s * n_el, st);
-        };
-        if constexpr (std::is_same<T, bf16_t>::value) {
-            if (bf16_math()) {      // bfloat16 matrix instructions; the fp32 ones below when those are asked for
-                if (nch == 1) {
-                    if (a.tile_win) hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, 1, true>), grid, dim3(G::NT), 0, st, a, s);
-                    else hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, 1, false>), grid, dim3(G::NT), 0, st, a, s);
-                } else if (a.tile_win) hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, DW_NCH, true>), grid, dim3(G::NT), 0, st, a, s);
-                else hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, DW_NCH, false>), grid, dim3(G::NT), 0, st, a, s);
-                APRNET_LAUNCH_CHECK("conv_dw_bf16_kernel");
-                if (int rc = reduce()) return rc;
-                continue;
-            }
-        }
-        if (a.Cout <= 16) {         // 16-row form
-            if (nch == 1) {
-                if (a.tile_win) hipLaunchKernelGGL((conv_dw16_mfma_kernel<T, G, DW_CIB, 1, true>), grid, dim3(G::NT), 0, st, a, s);
-                else hipLaunchKernelGGL((conv_dw16_mfma_kernel<T, G, DW_CIB, 1, false>), grid, dim3(G::NT), 0, st, a, s);
-            } else if (a.tile_win) hipLaunchKernelGGL((conv_dw16_mfma_kernel<T, G, DW_CIB, DW_NCH, true>), grid, dim3(G::NT), 0, st, a, s);
-            else hipLaunchKernelGGL((conv_dw16_mfma_kernel<T, G, DW_CIB, DW_NCH, false>), grid, dim3(G::NT), 0, st, a, s);
-            APRNET_LAUNCH_CHECK("conv_dw16_mfma_kernel");
-            if (int rc = reduce()) return rc;
-            continue;
-        }
-        if (nch == 1) {
-            if (a.tile_win) hipLaunchKernelGGL((conv_dw_mfma_kernel<T, G, DW_CIB, 1, true>), grid, dim3(G::NT), 0, st, a, s);
-            else hipLaunchKernelGGL((conv_dw_mfma_kernel<T, G, DW_CIB, 1, false>), grid, dim3(G::NT), 0, st, a, s);
-        } else if (a.tile_win) hipLaunchKernelGGL((conv_dw_mfma_kernel<T, G, DW_CIB, DW_NCH, true>), grid, dim3(G::NT), 0, st, a, s);
-        else hipLaunchKernelGGL((conv_dw_mfma_kernel<T, G, DW_CIB, DW_NCH, false>), grid, dim3(G::NT), 0, st, a, s);
-        APRNET_LAUNCH_CHECK("conv_dw_mfma_kernel");
-        if (int rc = reduce()) return rc;
+        const int blocks = std::min(n, a.gw_part ? dw_blocks_x(code, a.Cout, a.Cin) : 512);
+        if (int rc = launch_dw_kernel<T, G, false>(a, DwWork{}, s, blocks, st)) return rc;
+        if (a.gw_part)
+            if (int rc = launch_sum_slots((const float*)a.gw_part, a.gw_part_ld, 2 * blocks, n_el, (float*)a.gw + (int64_t)s * n_el, st)) return rc;
     }
     return 0;
 }
 
 template <typename T>
-static int launch_dw_code(int code, const ConvArgs<T>& a, const TileList& tl, int level_min, hipStream_t st) {
+static int launch_dw_code(int code, const ConvArgs<T>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st) {
     switch (code) {
-        case 333: return launch_dw<T, W333M>(a, tl, level_min, st);
-        case 133: return launch_dw<T, W133M>(a, tl, level_min, st);
-        case 155: return launch_dw<T, W155M>(a, tl, level_min, st);
+        case 333: return launch_dw<T, W333M>(a, tl, wl, level_min, st);
+        case 133: return launch_dw<T, W133M>(a, tl, wl, level_min, st);
+        case 155: return launch_dw<T, W155M>(a, tl, wl, level_min, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }
-int launch_conv_dw_mfma(int code, const ConvArgs<float>& a, const TileList& tl, int level_min, hipStream_t st) {
-    return launch_dw_code<float>(code, a, tl, level_min, st);
+int launch_conv_dw_mfma(int code, const ConvArgs<float>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st) {
+    return launch_dw_code<float>(code, a, tl, wl, level_min, st);
 }
-int launch_conv_dw_mfma(int code, const ConvArgs<bf16_t>& a, const TileList& tl, int level_min, hipStream_t st) {
-    return launch_dw_code<bf16_t>(code, a, tl, level_min, st);
+int launch_conv_dw_mfma(int code, const ConvArgs<bf16_t>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st) {
+    return launch_dw_code<bf16_t>(code, a, tl, wl, level_min, st);
 }
 
 }  // namespace aprnet

@@ -54,9 +54,9 @@ struct ConvArgs {
     const T* gy; typename Num<T>::acc* gx; int64_t ldgx; typename Num<T>::acc* gtree; int64_t ldgt;
     typename Num<T>::acc* gw; int n_tiles;
     // Weight gradient without atomics: every persistent workgroup writes the sums of its tiles to two slots (one per
-    // half of the columns) of gw_part [2 * gw_part_blocks][gw_part_ld], which a second kernel adds up in slot order and
+    // half of the columns) of gw_part [2 * workgroups][gw_part_ld], which a second kernel adds up in slot order and
     // adds to gw, so the result does not depend on scheduling (null: atomic additions to gw).
-    typename Num<T>::acc* gw_part; int64_t gw_part_ld; int gw_part_blocks;
+    typename Num<T>::acc* gw_part; int64_t gw_part_ld;
     // input-gradient scan: leave out the coarser particles that stick out of a far face of the level (some of the
     // cells they would cover do not exist); a separate kernel adds their gradient (faces.hip)
     int dx_skip_faces;

@@ -13,7 +13,7 @@ namespace aprnet {
 // the chip): 128 us on average over the launches of a training step of the 16-32-64 network on 5.5 M particles, 48 us with
 // 16 waves per 64 elements.
 template <typename A, int W>
-__global__ void __launch_bounds__(64 * W) sum_slots_kernel(const A* __restrict__ part, int64_t ld, int slots, int64_t n, A* __restrict__ out) {
+__device__ __forceinline__ void sum_slots_body(const A* __restrict__ part, int64_t ld, int slots, int64_t n, A* __restrict__ out) {
     __shared__ A sums[W][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int64_t e = (int64_t)blockIdx.x * 64 + lane;
@@ -34,6 +34,25 @@ __global__ void __launch_bounds__(64 * W) sum_slots_kernel(const A* __restrict__
         for (int i = 0; i < W; ++i) t += sums[i][lane];
         out[e] += t;
     }
+}
+template <typename A, int W>
+__global__ void __launch_bounds__(64 * W) sum_slots_kernel(const A* __restrict__ part, int64_t ld, int slots, int64_t n, A* __restrict__ out) {
+    sum_slots_body<A, W>(part, ld, slots, n, out);
+}
+
+// Several sums in one launch: slots first[k] .. first[k + 1] - 1 are added to out + out[k] * n.
+struct SlotGroups { int n; int first[MAX_LEVELS + 2], out[MAX_LEVELS + 1]; };
+template <typename A>
+__global__ void __launch_bounds__(1024) sum_slot_groups_kernel(const A* __restrict__ part, int64_t ld, const SlotGroups g, int64_t n, A* __restrict__ out) {
+    const int k = blockIdx.y;
+    sum_slots_body<A, 16>(part + (int64_t)g.first[k] * ld, ld, g.first[k + 1] - g.first[k], n, out + (int64_t)g.out[k] * n);
+}
+template <typename A>
+int launch_sum_slot_groups(const A* part, int64_t ld, const SlotGroups& g, int64_t n, A* out, hipStream_t st) {
+    if (n <= 0 || g.n <= 0) return 0;
+    hipLaunchKernelGGL(sum_slot_groups_kernel<A>, dim3((unsigned)((n + 63) / 64), (unsigned)g.n), dim3(1024), 0, st, part, ld, g, n, out);
+    APRNET_LAUNCH_CHECK("sum_slot_groups_kernel");
+    return 0;
 }
 
 // 16 waves, 4 where there are fewer slots than that (1x1x1 256 -> 512 on 4 k particles, 3 slots: 2.54 instead of 2.55 ms)

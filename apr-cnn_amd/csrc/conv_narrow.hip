@@ -90,9 +90,11 @@ __global__ void pack_weights_narrow_bf16_kernel(const float* __restrict__ w, int
 
 // two workgroups of eight waves per CU (three, at 80 registers with a few spills, ran slower: 2.0 against 1.25 ms)
 constexpr int NARROW_WAVES = 4;
+constexpr int NARROW_BOTH = 8;          // windows per workgroup from which on every workgroup takes windows of both kinds
 struct NarrowArgs {
-    int win0;                           // first window of this launch
-    int n_win;                          // windows of this launch (stored windows of the plan's lists, finest level first)
+    int n_win, n_fine;                  // stored windows of the plan's lists, finest level first; the first n_fine hold no tree items
+    int fine_blocks;                    // workgroups (grid.x) 0 .. fine_blocks - 1 share out the first n_fine windows,
+    int coarse_block0;                  // workgroups coarse_block0 .. the others; a workgroup may have a share of both
     int n_lv;                           // levels with windows
     int lv_first[MAX_LEVELS];           // first window of the k-th such level
     int lv_level[MAX_LEVELS];
@@ -102,27 +104,19 @@ struct NarrowArgs {
 // it the tree loads, a third of a window's load instructions, are not issued at all
 // BM: the bfloat16 matrix instruction described above (bfloat16 features, CIN 1, 3x3x3)
 typedef __bf16 bf16x8n __attribute__((ext_vector_type(8)));
-template <typename T, class G, int CIN, int COH, bool TREE, bool BM = false>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(NARROW_WAVES, NARROW_WAVES)))
-conv_narrow_kernel(const ConvArgs<T> a, const NarrowArgs na) {
+template <typename T, class G, int CIN, int COH, bool TREE, bool BM>
+__device__ __forceinline__ void narrow_windows(const ConvArgs<T>& a, const NarrowArgs& na, const int wb, const int we, float* __restrict__ patch,
+                                               float* __restrict__ Wl, uint4* __restrict__ Wl16, const float* __restrict__ bias_l) {
     static_assert(!BM || (std::is_same<T, bf16_t>::value && CIN == 1 && G::KZ == 3 && G::KX == 3 && G::KY == 3), "see narrow_bf16_tap");
     typedef NarrowShape<G, CIN> NS;
     constexpr int IPT = NS::IPT, NBW = ((G::MAXCOL + 15) / 16 + G::NWAVE - 1) / G::NWAVE;
     constexpr int PATCH = CIN * G::CH_STRIDE;
     static_assert((G::MAXCOL + 15) / 16 <= G::NWAVE * NBW, "a window must fit the accumulators of the block");
-    __shared__ __attribute__((aligned(16))) float patch[3 * PATCH];
-    __shared__ float Wl[BM ? 1 : NS::STEPS * COH * 64];
-    __shared__ __attribute__((aligned(16))) uint4 Wl16[BM ? COH * 64 : 1];
-    __shared__ float bias_l[16 * COH];
+    if (wb >= we) return;
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int co0 = blockIdx.y * 16 * COH;
-    const int wb = na.win0 + (int)((int64_t)na.n_win * blockIdx.x / gridDim.x), we = na.win0 + (int)((int64_t)na.n_win * (blockIdx.x + 1) / gridDim.x);
-    if (wb >= we) return;
-
-    if (threadIdx.x < 16 * COH)
-        bias_l[threadIdx.x] = (a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
     for (int i = threadIdx.x; i < 3 * PATCH; i += G::NT) patch[i] = 0.f;
 
     // per-lane part of the B address: unit u = 4 q + lane / 16 of a stencil row -> channel plane and y-tap
@@ -144,7 +138,7 @@ conv_narrow_kernel(const ConvArgs<T> a, const NarrowArgs na) {
         runC = (g < 3 ? row_off(3 * g + 2) : row_off(8) + 2) - G::TAP0;
     }
 
-    const __amdgpu_buffer_rsrc_t r_hdr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int4*>(a.win), 0, (na.win0 + na.n_win) * 16, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r_hdr = __builtin_amdgcn_make_buffer_rsrc(const_cast<int4*>(a.win), 0, na.n_win * 16, 0x00020000);
     __amdgpu_buffer_rsrc_t rx[CIN], rt[CIN];
 #pragma unroll
     for (int c = 0; c < CIN; ++c) {
@@ -405,6 +399,30 @@ conv_narrow_kernel(const ConvArgs<T> a, const NarrowArgs na) {
     if (nc > 0) store_outputs(c0, we - 1, nc);
 }
 
+// The windows without and with tree items in one launch: as two launches, the second waited for the first one's last
+// workgroups (1 -> 16 channels on 680 k particles: 36 + 13 us, now 43 us; 338 k 24 + 9 us, now 25 us; 23 M 1.11 ms, now 1.09 ms).
+template <typename T, class G, int CIN, int COH, bool BM = false>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(NARROW_WAVES, NARROW_WAVES)))
+conv_narrow_kernel(const ConvArgs<T> a, const NarrowArgs na) {
+    typedef NarrowShape<G, CIN> NS;
+    __shared__ __attribute__((aligned(16))) float patch[3 * CIN * G::CH_STRIDE];
+    __shared__ float Wl[BM ? 1 : NS::STEPS * COH * 64];
+    __shared__ __attribute__((aligned(16))) uint4 Wl16[BM ? COH * 64 : 1];
+    __shared__ float bias_l[16 * COH];
+    const int co0 = blockIdx.y * 16 * COH, blk = blockIdx.x;
+    if (threadIdx.x < 16 * COH)
+        bias_l[threadIdx.x] = (a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
+    if (blk < na.fine_blocks)
+        narrow_windows<T, G, CIN, COH, false, BM>(a, na, (int)((int64_t)na.n_fine * blk / na.fine_blocks), (int)((int64_t)na.n_fine * (blk + 1) / na.fine_blocks),
+                                                  patch, Wl, Wl16, bias_l);
+    if (blk >= na.coarse_block0) {
+        __syncthreads();                // the patch and the weights are written anew
+        const int n = na.n_win - na.n_fine, k = blk - na.coarse_block0, nb = gridDim.x - na.coarse_block0;
+        narrow_windows<T, G, CIN, COH, true, BM>(a, na, na.n_fine + (int)((int64_t)n * k / nb), na.n_fine + (int)((int64_t)n * (k + 1) / nb), patch, Wl,
+                                                 Wl16, bias_l);
+    }
+}
+
 using N333 = ConvGeom<3, 3, 3, 2, 4, 512, 64, 16>;
 using N133 = ConvGeom<1, 3, 3, 1, 8, 512, 64, 16>;
 using N155 = ConvGeom<1, 5, 5, 1, 8, 512, 64, 16>;
@@ -452,36 +470,33 @@ static int launch_narrow_cin(const ConvArgs<T>& a, const NarrowArgs& na, hipStre
     // two persistent workgroups per CU; short lists get one workgroup per window
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-    // the windows of the call's finest level hold no tree items (they come first in the list): their launch skips the tree loads
-    const int n_fine = (na.n_lv > 0 && na.lv_level[0] == a.Lc) ? (na.n_lv > 1 ? na.lv_first[1] : na.n_win) : 0;
-    for (int part = 0; part < 2; ++part) {
-        NarrowArgs nb = na;
-        nb.win0 = part == 0 ? 0 : n_fine;
-        nb.n_win = part == 0 ? n_fine : na.n_win - n_fine;
-        if (nb.n_win <= 0) continue;
-        dim3 grid((unsigned)std::max(1, std::min(nb.n_win, 2 * cus)), (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
-        if constexpr (std::is_same<T, bf16_t>::value && CIN == 1 && G::KZ == 3) {
-            if (conv_narrow_bf16_math(333, 1)) {
-                if (part == 0) {
-                    if (coh == 1) hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 1, false, true>), grid, dim3(G::NT), 0, st, a, nb);
-                    else hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 2, false, true>), grid, dim3(G::NT), 0, st, a, nb);
-                } else {
-                    if (coh == 1) hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 1, true, true>), grid, dim3(G::NT), 0, st, a, nb);
-                    else hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 2, true, true>), grid, dim3(G::NT), 0, st, a, nb);
-                }
-                APRNET_LAUNCH_CHECK("conv_narrow_kernel");
-                continue;
-            }
-        }
-        if (part == 0) {
-            if (coh == 1) hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 1, false>), grid, dim3(G::NT), 0, st, a, nb);
-            else hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 2, false>), grid, dim3(G::NT), 0, st, a, nb);
-        } else {
+    NarrowArgs nb = na;
+    // the windows of the call's finest level hold no tree items (they come first in the list): they skip the tree loads
+    nb.n_fine = (na.n_lv > 0 && na.lv_level[0] == a.Lc) ? (na.n_lv > 1 ? na.lv_first[1] : na.n_win) : 0;
+    const int blocks = std::max(1, std::min(na.n_win, 2 * cus)), n_coarse = na.n_win - nb.n_fine;
+    // Many windows per workgroup: each takes a share of both kinds, which keeps the shares equal in work (a coarse window has
+    // fewer columns).  Few: a workgroup takes one kind, and the three round trips before a kind's first window only once.
+    if (na.n_win >= NARROW_BOTH * blocks) { nb.fine_blocks = nb.n_fine > 0 ? blocks : 0; nb.coarse_block0 = n_coarse > 0 ? 0 : blocks; }
+    else {
+        nb.fine_blocks = (int)((int64_t)blocks * nb.n_fine / na.n_win);
+        if (nb.n_fine > 0 && nb.fine_blocks == 0) nb.fine_blocks = 1;
+        if (n_coarse > 0 && nb.fine_blocks == blocks && blocks > 1) --nb.fine_blocks;
+        nb.coarse_block0 = n_coarse > 0 && nb.fine_blocks == blocks ? 0 : nb.fine_blocks;      // (a single workgroup takes both)
+    }
+    dim3 grid((unsigned)blocks, (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
+    bool bm = false;
+    if constexpr (std::is_same<T, bf16_t>::value && CIN == 1 && G::KZ == 3) {
+        bm = conv_narrow_bf16_math(333, 1);
+        if (bm) {
             if (coh == 1) hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 1, true>), grid, dim3(G::NT), 0, st, a, nb);
             else hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 2, true>), grid, dim3(G::NT), 0, st, a, nb);
         }
-        APRNET_LAUNCH_CHECK("conv_narrow_kernel");
     }
+    if (!bm) {
+        if (coh == 1) hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 1>), grid, dim3(G::NT), 0, st, a, nb);
+        else hipLaunchKernelGGL((conv_narrow_kernel<T, G, CIN, 2>), grid, dim3(G::NT), 0, st, a, nb);
+    }
+    APRNET_LAUNCH_CHECK("conv_narrow_kernel");
     return 0;
 }
 template <typename T, class G>

@@ -118,13 +118,60 @@ fill_tree_list_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, c
 constexpr int G_MAX_COARSE = 12;
 struct GCoarse { int n; int64_t begin[G_MAX_COARSE], end[G_MAX_COARSE]; };
 
-// the coarse levels in one launch, finest first, one workgroup per channel group (see fill_tree_coarse_kernel)
-__global__ void __launch_bounds__(GTB)
-fill_tree_coarse_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, const GCoarse lv, const bf16_t* x, int64_t ldx,
-                           bf16_t* tree, int64_t ldt) {
+// the coarse levels in one launch, finest first, two workgroups per channel group; tables and values of all levels are read first
+// and the levels meet in LDS (see fill_tree_coarse_kernel): 9.2 -> 6.9 us on a 700 k-particle APR
+constexpr int G_COARSE_NODES = 2048, G_COARSE_TB = 1024, G_COARSE_J = G_COARSE_NODES / G_COARSE_TB;
+__global__ void __launch_bounds__(G_COARSE_TB)
+fill_tree_coarse_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, const GCoarse lv, const bf16_t* __restrict__ x, int64_t ldx,
+                           bf16_t* __restrict__ tree, int64_t ldt) {
+    __shared__ uint2 mean[G_COARSE_NODES];
+    const int64_t t0 = lv.begin[lv.n - 1], t1 = lv.end[0];
+    const int q = blockIdx.x >> 1, half = blockIdx.x & 1;              // half a group per workgroup: the values fit the registers
+    int32_t ch[G_COARSE_J][8];
+    uint2 raw[G_COARSE_J][8];
+#pragma unroll
+    for (int j = 0; j < G_COARSE_J; ++j)
+#pragma unroll
+        for (int s = 0; s < 8; ++s) ch[j][s] = children[(int64_t)s * n_tree + min(t0 + (int64_t)(j * G_COARSE_TB + threadIdx.x), t1 - 1)];
+#pragma unroll
+    for (int j = 0; j < G_COARSE_J; ++j)
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            const int32_t c = ch[j][s];
+            const bool node = c < 0 && c != NO_CHILD, outer = node && (int64_t)~c >= t1;
+            raw[j][s] = reinterpret_cast<const uint2*>(g8_at(outer ? (const bf16_t*)tree : x, outer ? ldt : ldx, q, c >= 0 ? (int64_t)c : outer ? (int64_t)~c : 0))[half];
+        }
+    auto add4 = [](uint2 r, float (&sum)[4]) {
+        sum[0] += __builtin_bit_cast(float, r.x << 16); sum[1] += __builtin_bit_cast(float, r.x & 0xffff0000u);
+        sum[2] += __builtin_bit_cast(float, r.y << 16); sum[3] += __builtin_bit_cast(float, r.y & 0xffff0000u);
+    };
     for (int i = 0; i < lv.n; ++i) {
-        for (int64_t t = lv.begin[i] + threadIdx.x; t < lv.end[i]; t += GTB)
-            fill_node_g8(children, n_tree, t, x, ldx, tree, ldt, 0, 0, 0, blockIdx.x);
+#pragma unroll
+        for (int j = 0; j < G_COARSE_J; ++j) {
+            const int64_t t = t0 + j * G_COARSE_TB + threadIdx.x;
+            if (t < lv.begin[i] || t >= lv.end[i]) continue;
+            float sum[4] = {0.f, 0.f, 0.f, 0.f};
+            int cnt = 0;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                cnt += ch[j][s] != NO_CHILD;
+                if (ch[j][s] >= 0) add4(raw[j][s], sum);
+            }
+#pragma unroll
+            for (int s = 0; s < 8; ++s)
+                if (ch[j][s] < 0 && ch[j][s] != NO_CHILD) {
+                    uint2 r = raw[j][s];
+                    if ((int64_t)~ch[j][s] < t1) r = mean[~ch[j][s] - t0];
+                    add4(r, sum);
+                }
+            const float scale = 1.0f / (float)max(cnt, 1);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sum[c] *= scale;
+            const uint2 m = make_uint2((unsigned)float_to_bf16(sum[0]).bits | ((unsigned)float_to_bf16(sum[1]).bits << 16),
+                                       (unsigned)float_to_bf16(sum[2]).bits | ((unsigned)float_to_bf16(sum[3]).bits << 16));
+            mean[t - t0] = m;
+            reinterpret_cast<uint2*>(g8_at(tree, ldt, q, t))[half] = m;
+        }
         __syncthreads();
     }
 }
@@ -144,7 +191,7 @@ int fill_tree_mean_g8(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx,
     int l_coarse = p->tree.level_min - 1;
     while (l_coarse + 1 < l_top && l_coarse + 1 - p->tree.level_min < G_MAX_COARSE) {
         nodes += p->tree.level_end(l_coarse + 1) - p->tree.level_begin(l_coarse + 1);
-        if (nodes > 2048) break;
+        if (nodes > G_COARSE_NODES) break;
         ++l_coarse;
     }
     for (int l = l_top; l > l_coarse; --l) {
@@ -166,7 +213,7 @@ int fill_tree_mean_g8(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx,
     for (int l = l_coarse; l >= l_read; --l)
         if (p->tree.level_end(l) > p->tree.level_begin(l)) { lv.begin[lv.n] = p->tree.level_begin(l); lv.end[lv.n] = p->tree.level_end(l); ++lv.n; }
     if (lv.n > 0)
-        hipLaunchKernelGGL(fill_tree_coarse_g8_kernel, dim3((unsigned)G), dim3(GTB), 0, st, p->d_children, p->n_tree, lv, x, ldx, tree, ldt);
+        hipLaunchKernelGGL(fill_tree_coarse_g8_kernel, dim3((unsigned)(2 * G)), dim3(G_COARSE_TB), 0, st, p->d_children, p->n_tree, lv, x, ldx, tree, ldt);
     APRNET_LAUNCH_CHECK("fill_tree g8 kernels");
     return 0;
 }

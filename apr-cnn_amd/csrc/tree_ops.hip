@@ -9,7 +9,7 @@
 namespace aprnet {
 
 constexpr int TB = 256;
-constexpr int CPT_COARSE = 4;   // channels per workgroup of the coarse-level kernels
+constexpr int COARSE_C = 2;     // channels per workgroup of the coarse-level kernels
 constexpr int NB = 4;           // channels of one batch: all loads of a batch are issued before its first store
 
 // Channels per thread of a launch over n nodes: up to 16 (32 for 2-byte features), halved while fewer than 2^20
@@ -172,20 +172,61 @@ fill_tree_list_kernel(const int32_t* __restrict__ children, int64_t n_tree, cons
 }
 
 // The coarse levels of the tree hold a few nodes each: one launch walks them all, finest first, one workgroup per
-// group of CPT_COARSE channels (a level's parents read only values of the same channels, so a workgroup barrier between
+// group of COARSE_C channels (a level's parents read only values of the same channels, so a workgroup barrier between
 // levels is enough).  Tree children come from the tree itself (none of these levels sits directly under the features),
 // particle children from the feature vector as always.
+// Bound by latency.  With a level's child tables and values read after the barrier behind the level before it, a level cost
+// two memory round trips: 18 us for four levels of a 338 k-particle APR, in front of every convolution.  Now every thread
+// reads the tables and values of its nodes of all levels first and the levels meet in LDS: 11 us.
 constexpr int MAX_COARSE = 12;
-struct CoarseLevels { int n; int64_t begin[MAX_COARSE], end[MAX_COARSE]; };
-constexpr int64_t COARSE_NODES = 2048;      // levels are merged while they hold at most this many nodes together
+struct CoarseLevels { int n; int64_t begin[MAX_COARSE], end[MAX_COARSE]; };      // adjacent ranges of nodes
+constexpr int COARSE_NODES = 2048;          // levels are merged while they hold at most this many nodes together
+constexpr int COARSE_TB = 1024, COARSE_J = COARSE_NODES / COARSE_TB;     // a thread holds COARSE_J nodes
 
 template <typename T>
-__global__ void __launch_bounds__(TB)
-fill_tree_coarse_kernel(const int32_t* __restrict__ children, int64_t n_tree, const CoarseLevels lv, const T* x, int64_t ldx,
-                        int C, T* tree, int64_t ldt) {
+__global__ void __launch_bounds__(COARSE_TB)
+fill_tree_coarse_kernel(const int32_t* __restrict__ children, int64_t n_tree, const CoarseLevels lv, const T* __restrict__ x, int64_t ldx,
+                        int C, T* __restrict__ tree, int64_t ldt) {
+    typedef typename Num<T>::acc A;
+    __shared__ A mean[COARSE_C][COARSE_NODES];
+    const int64_t t0 = lv.begin[lv.n - 1], t1 = lv.end[0];
+    const int c0 = blockIdx.x * COARSE_C;
+    Kids kd[COARSE_J];
+    A v[COARSE_J][COARSE_C][8];
+#pragma unroll
+    for (int j = 0; j < COARSE_J; ++j) kd[j].read(children, n_tree, min(t0 + (int64_t)(j * COARSE_TB + threadIdx.x), t1 - 1));
+#pragma unroll
+    for (int j = 0; j < COARSE_J; ++j)
+#pragma unroll
+        for (int c = 0; c < COARSE_C; ++c) {
+            const int cc = min(c0 + c, C - 1);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const bool inner = kd[j].tree(s) && kd[j].off[s] < t1;         // a node of this launch: its value comes through LDS
+                const T* p = (kd[j].tree(s) && !inner ? tree + (int64_t)cc * ldt : x + (int64_t)cc * ldx) + (inner ? 0 : kd[j].off[s]);
+                v[j][c][s] = Num<T>::ld(*p);
+            }
+        }
     for (int i = 0; i < lv.n; ++i) {
-        for (int64_t t = lv.begin[i] + threadIdx.x; t < lv.end[i]; t += TB)
-            fill_node<T>(children, n_tree, t, x, ldx, C, tree, ldt, 0, 0, 0, blockIdx.x * CPT_COARSE, CPT_COARSE);
+#pragma unroll
+        for (int j = 0; j < COARSE_J; ++j) {
+            const int64_t t = t0 + j * COARSE_TB + threadIdx.x;
+            if (t < lv.begin[i] || t >= lv.end[i]) continue;
+            const A scale = (A)(1.0f / (float)max(kd[j].count(), 1));
+#pragma unroll
+            for (int c = 0; c < COARSE_C; ++c) {
+                A sum = 0;
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    if (kd[j].has(s) && !kd[j].tree(s)) sum += v[j][c][s];
+#pragma unroll
+                for (int s = 0; s < 8; ++s)
+                    if (kd[j].tree(s)) sum += kd[j].off[s] < t1 ? mean[c][kd[j].off[s] - t0] : v[j][c][s];
+                const T m = Num<T>::st(sum * scale);
+                mean[c][t - t0] = Num<T>::ld(m);
+                if (c0 + c < C) tree[(int64_t)(c0 + c) * ldt + t] = m;
+            }
+        }
         __syncthreads();
     }
 }
@@ -239,14 +280,56 @@ fill_tree_bwd_list_kernel(const int32_t* __restrict__ children, int64_t n_tree, 
     if (i < count) fill_node_bwd<T>(children, n_tree, nodes[i], gx, ldx, C, gtree, ldt, tree_off, tree_child_in_x, blockIdx.y * cpt, cpt);
 }
 
-// the coarse levels in one launch, coarsest first (a parent's share must have arrived before it is handed down)
+// the coarse levels in one launch, coarsest first (a parent's share must have arrived before it is handed down); as above, what
+// the children hold is read ahead and the levels meet in LDS: 34 -> 17 us
 template <typename T>
-__global__ void __launch_bounds__(TB)
-fill_tree_bwd_coarse_kernel(const int32_t* __restrict__ children, int64_t n_tree, const CoarseLevels lv, T* gx, int64_t ldx,
-                            int C, T* gtree, int64_t ldt) {
+__global__ void __launch_bounds__(COARSE_TB)
+fill_tree_bwd_coarse_kernel(const int32_t* __restrict__ children, int64_t n_tree, const CoarseLevels lv, T* __restrict__ gx, int64_t ldx,
+                            int C, T* __restrict__ gtree, int64_t ldt) {
+    typedef typename Num<T>::acc A;
+    __shared__ A g[COARSE_C][COARSE_NODES];
+    const int64_t t0 = lv.begin[0], t1 = lv.end[lv.n - 1];
+    const int c0 = blockIdx.x * COARSE_C;
+    Kids kd[COARSE_J];
+    A v[COARSE_J][COARSE_C][8];
+#pragma unroll
+    for (int j = 0; j < COARSE_J; ++j) kd[j].read(children, n_tree, min(t0 + (int64_t)(j * COARSE_TB + threadIdx.x), t1 - 1));
+#pragma unroll
+    for (int j = 0; j < COARSE_J; ++j)
+#pragma unroll
+        for (int c = 0; c < COARSE_C; ++c) {
+            const int cc = min(c0 + c, C - 1);
+            const int64_t t = t0 + j * COARSE_TB + threadIdx.x;
+            if (t < t1) g[c][t - t0] = Num<T>::ld(gtree[(int64_t)cc * ldt + t]);
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                const bool inner = kd[j].tree(s) && kd[j].off[s] < t1;
+                const T* p = (kd[j].tree(s) && !inner ? gtree + (int64_t)cc * ldt : gx + (int64_t)cc * ldx) + (inner ? 0 : kd[j].off[s]);
+                v[j][c][s] = Num<T>::ld(*p);
+            }
+        }
+    __syncthreads();
     for (int i = 0; i < lv.n; ++i) {
-        for (int64_t t = lv.begin[i] + threadIdx.x; t < lv.end[i]; t += TB)
-            fill_node_bwd<T>(children, n_tree, t, gx, ldx, C, gtree, ldt, 0, 0, blockIdx.x * CPT_COARSE, CPT_COARSE);
+#pragma unroll
+        for (int j = 0; j < COARSE_J; ++j) {
+            const int64_t t = t0 + j * COARSE_TB + threadIdx.x;
+            if (t < lv.begin[i] || t >= lv.end[i]) continue;
+            const A scale = (A)(1.0f / (float)max(kd[j].count(), 1));
+#pragma unroll
+            for (int c = 0; c < COARSE_C; ++c) {
+                if (c0 + c >= C) break;
+                const A gt = g[c][t - t0];
+                if (t >= lv.end[0]) gtree[(int64_t)(c0 + c) * ldt + t] = Num<T>::st(gt);        // (the coarsest level's are as they were)
+#pragma unroll
+                for (int s = 0; s < 8; ++s) {
+                    if (!kd[j].has(s)) continue;
+                    if (kd[j].tree(s) && kd[j].off[s] < t1) {
+                        A& d = g[c][kd[j].off[s] - t0];                       // (a node has one parent)
+                        d = Num<T>::ld(Num<T>::st(d + gt * scale));
+                    } else (kd[j].tree(s) ? gtree + (int64_t)(c0 + c) * ldt : gx + (int64_t)(c0 + c) * ldx)[kd[j].off[s]] = Num<T>::st(v[j][c][s] + gt * scale);
+                }
+            }
+        }
         __syncthreads();
     }
 }
@@ -474,7 +557,7 @@ int fill_tree_mean(const aprnet_plan* p, int d, const T* x, int64_t ldx, int C, 
     for (int l = l_coarse; l >= p->tree.level_min; --l)
         if (p->tree.level_end(l) > p->tree.level_begin(l)) { lv.begin[lv.n] = p->tree.level_begin(l); lv.end[lv.n] = p->tree.level_end(l); ++lv.n; }
     if (lv.n > 0)
-        hipLaunchKernelGGL(fill_tree_coarse_kernel<T>, dim3((unsigned)((C + CPT_COARSE - 1) / CPT_COARSE)), dim3(TB), 0, st, p->d_children, p->n_tree,
+        hipLaunchKernelGGL(fill_tree_coarse_kernel<T>, dim3((unsigned)((C + COARSE_C - 1) / COARSE_C)), dim3(COARSE_TB), 0, st, p->d_children, p->n_tree,
                            lv, x, ldx, C, tree, ldt);
     APRNET_LAUNCH_CHECK("fill_tree kernels");
     return 0;
@@ -516,7 +599,7 @@ int fill_tree_mean_needed(const aprnet_plan* p, int d, const NeedLists& need, co
     for (int l = l_coarse; l >= l_read; --l)
         if (p->tree.level_end(l) > p->tree.level_begin(l)) { lv.begin[lv.n] = p->tree.level_begin(l); lv.end[lv.n] = p->tree.level_end(l); ++lv.n; }
     if (lv.n > 0)
-        hipLaunchKernelGGL(fill_tree_coarse_kernel<T>, dim3((unsigned)((C + CPT_COARSE - 1) / CPT_COARSE)), dim3(TB), 0, st, p->d_children, p->n_tree,
+        hipLaunchKernelGGL(fill_tree_coarse_kernel<T>, dim3((unsigned)((C + COARSE_C - 1) / COARSE_C)), dim3(COARSE_TB), 0, st, p->d_children, p->n_tree,
                            lv, x, ldx, C, tree, ldt);
     APRNET_LAUNCH_CHECK("fill_tree kernels (needed nodes)");
     return 0;
@@ -543,7 +626,7 @@ int fill_tree_mean_bwd(const aprnet_plan* p, int d, T* gx, int64_t ldx, int C, T
     for (int l = l_first; l <= l_coarse; ++l)
         if (p->tree.level_end(l) > p->tree.level_begin(l)) { lv.begin[lv.n] = p->tree.level_begin(l); lv.end[lv.n] = p->tree.level_end(l); ++lv.n; }
     if (lv.n > 0)
-        hipLaunchKernelGGL(fill_tree_bwd_coarse_kernel<T>, dim3((unsigned)((C + CPT_COARSE - 1) / CPT_COARSE)), dim3(TB), 0, st, p->d_children,
+        hipLaunchKernelGGL(fill_tree_bwd_coarse_kernel<T>, dim3((unsigned)((C + COARSE_C - 1) / COARSE_C)), dim3(COARSE_TB), 0, st, p->d_children,
                            p->n_tree, lv, gx, ldx, C, gtree, ldt);
     for (int l = std::max(l_coarse + 1, l_first); l <= l_top; ++l) {
         const int64_t b = p->tree.level_begin(l), e = p->tree.level_end(l);

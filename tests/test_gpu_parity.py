@@ -1010,3 +1010,46 @@ def test_conv_forward_fills_only_the_tree_nodes_it_reads(ksize, cin, dtype):
         assert torch.equal(trees[0][filled], trees[1][filled])
         untouched += int((~filled).sum())
     assert untouched > 0
+
+
+def _coarse_nodes(apr, d):
+    """Nodes of the tree levels that the coarse-level kernels walk in one launch (at most 2048, not the level under the features)."""
+    t = apr.tree_iterator()
+    n, top = 0, min(apr.level_max() - d - 1, t.level_max())
+    for lv in range(t.level_min(), top):
+        k = t.particles_level_end(lv) - t.particles_level_begin(lv)
+        if n + k > 2048:
+            break
+        n += k
+    return n
+
+
+@pytest.mark.parametrize("shape,seed,density", [((36, 40, 44), 21, 0.02), ((48, 60, 64), 22, 0.03), ((64, 64, 64), 23, 0.3), ((1, 256, 230), 24, 0.05)])
+@pytest.mark.parametrize("channels", [1, 3, 4])
+def test_coarse_tree_levels_in_one_launch(shape, seed, density, channels):
+    """Tree means and their gradient where the levels that one launch walks hold fewer and more nodes than a workgroup has threads
+    (one and two nodes per thread) and the channels end inside a workgroup's group: bit for bit the oracle's means, its gradient
+    to the rounding of a sum of one share per level (at most ten: 10 * 2^-24 of the largest)."""
+    apr = apr_cases.random_apr(shape, seed, density)
+    apr.init_cuda()
+    n, nt = oracle.number_parts(apr, 0), oracle.tree_parts(apr, 0)
+    assert 8 < _coarse_nodes(apr, 0) <= 2048
+    g = torch.Generator().manual_seed(seed)
+    x, gt = torch.randn(channels, n, generator=g), torch.randn(channels, nt, generator=g)
+    lib, plan, st = _native.hip(), apr.plan(0), torch.cuda.current_stream().cuda_stream
+    xd, tree = x.to(DEV), torch.full((channels, nt), float("nan"), device=DEV)
+    assert lib.aprnet_fill_tree_mean_f32(plan, 0, xd.data_ptr(), n, channels, tree.data_ptr(), nt, st) == 0
+    gx, gtd = torch.zeros(channels, n, device=DEV), gt.to(DEV)
+    assert lib.aprnet_fill_tree_mean_bwd_f32(plan, 0, gx.data_ptr(), n, channels, gtd.data_ptr(), nt, st) == 0
+    for c in range(channels):
+        assert torch.equal(tree[c].cpu(), oracle.fill_tree_mean(apr, x[c], 0))
+        ref = oracle.fill_tree_mean_backward(apr, gt[c], n, 0)
+        assert float((gx[c].cpu() - ref).abs().max()) <= 10 * 2.0 ** -24 * float(ref.abs().max())
+    # grouped bfloat16 features: the means of the planes
+    xb = torch.randn(1, 8 * channels, n, generator=g).to(torch.bfloat16).to(DEV)
+    planes, grp = torch.empty(8 * channels, nt, dtype=torch.bfloat16, device=DEV), torch.empty(channels, nt, 8, dtype=torch.bfloat16, device=DEV)
+    xg = torch.empty(channels, n, 8, dtype=torch.bfloat16, device=DEV)
+    assert lib.aprnet_regroup8_bf16(xb.data_ptr(), n, 8 * channels, n, xg.data_ptr(), n, st) == 0
+    assert lib.aprnet_fill_tree_mean_bf16(plan, 0, xb.data_ptr(), n, 8 * channels, planes.data_ptr(), nt, st) == 0
+    assert lib.aprnet_fill_tree_mean_bf16g(plan, 0, xg.data_ptr(), n, 8 * channels, grp.data_ptr(), nt, st) == 0
+    assert torch.equal(grp.permute(0, 2, 1).reshape(8 * channels, nt), planes)

@@ -255,18 +255,26 @@ static int launch_conv111_dw(aprnet_plan* p, const T* x, int64_t ldx, int Cin, c
     return launch_sum_slots<A>(part, (int64_t)Cout * Cin, (int)g2.x, (int64_t)Cout * Cin, gw, st);
 }
 
+// Runs of features with one stencil index.  Levels follow each other in the feature vector (downsampled particles behind the
+// particles of their level), so the levels that share the last stencil are one run, and so are the particles and the
+// downsampled particles of level Lc: two runs instead of up to six launches with the two stencils of a network.
 struct Segment { int64_t begin, end; int stencil; };
 
 static std::vector<Segment> segments(const aprnet_plan* p, int d, int S) {
     std::vector<Segment> segs;
+    auto add = [&](int64_t b, int64_t e, int s) {
+        if (e <= b) return;
+        if (!segs.empty() && segs.back().stencil == s && segs.back().begin == e) segs.back().begin = b;
+        else if (!segs.empty() && segs.back().stencil == s && segs.back().end == b) segs.back().end = e;
+        else segs.push_back({b, e, s});
+    };
     const int Lc = p->lc(d);
     for (int l = Lc; l >= p->apr.level_min; --l) {
         const int s = std::min(S - 1, Lc - l);
-        if (p->apr.level_end(l) > p->apr.level_begin(l)) segs.push_back({p->apr.level_begin(l), p->apr.level_end(l), s});
+        add(p->apr.level_begin(l), p->apr.level_end(l), s);
         if (l == Lc && Lc < p->apr.level_max) {
             const int64_t off = p->tree_offset(Lc);
-            if (p->tree.level_end(Lc) > p->tree.level_begin(Lc))
-                segs.push_back({p->tree.level_begin(Lc) + off, p->tree.level_end(Lc) + off, s});
+            add(p->tree.level_begin(Lc) + off, p->tree.level_end(Lc) + off, s);
         }
     }
     return segs;

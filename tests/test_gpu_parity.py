@@ -1053,3 +1053,21 @@ def test_coarse_tree_levels_in_one_launch(shape, seed, density, channels):
     assert lib.aprnet_fill_tree_mean_bf16(plan, 0, xb.data_ptr(), n, 8 * channels, planes.data_ptr(), nt, st) == 0
     assert lib.aprnet_fill_tree_mean_bf16g(plan, 0, xg.data_ptr(), n, 8 * channels, grp.data_ptr(), nt, st) == 0
     assert torch.equal(grp.permute(0, 2, 1).reshape(8 * channels, nt), planes)
+
+
+@pytest.mark.parametrize("cin,cout,shape,density", [(512, 500, (64, 64, 64), 0.3), (33, 31, (64, 64, 64), 0.3), (1, 1, (9, 17, 12), 0.05), (8, 40, (1, 1, 63), 0.1)])
+def test_conv111_weight_gradient_bf16_strips(cin, cout, shape, density):
+    """The matrix-core form of the 1x1x1 weight gradient: several strips per wave with the accumulators set aside, a last strip that
+    ends inside eight positions, channels that end inside a block of 32, runs of features with two stencils.  Against the
+    product in 64 bits: products exact, fp32 sums of n terms differ by at most n 2^-24 of the sum of magnitudes."""
+    apr = apr_cases.random_apr(shape, 23, density)
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    x = (2 * torch.rand(1, cin, n, device=DEV, generator=gen) - 1).to(torch.bfloat16)
+    gy = (2 * torch.rand(1, cout, n, device=DEV, generator=gen) - 1).to(torch.bfloat16)
+    gw = _ops.conv_backward([apr], x, torch.zeros(2, cout, cin, 1, 1, 1, device=DEV), gy, ld)[1].view(2, cout, cin)
+    b = apr.iterator().particles_level_begin(apr.level_max())
+    for s, part in ((0, slice(b, n)), (1, slice(0, b))):
+        xs, gs = x[0, :, part].double(), gy[0, :, part].double()
+        ref, size = gs @ xs.T, gs.abs() @ xs.abs().T
+        assert bool(((gw[s].double() - ref).abs() <= n * 2.0 ** -24 * size).all())

@@ -525,8 +525,13 @@ interleave8_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __re
         if (b0 + e * IL_TB + threadIdx.x < count) dst[e * IL_TB + threadIdx.x] = buf[e * IL_TB + threadIdx.x];
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+
 // MODE 0: forward.  MODE 1: input gradient (items = output gradient, results added in fp32 onto the place each column
-// names; no pooled columns).
+// names; the columns of a coarser particle summed across lanes first).
 // IL: the input comes regrouped (a.xi, a.ti), see above
 // HEAD: the 1x1x1 convolution of the result follows here (see ConvArgs::head_w); head_a holds the A operands of the
 // head's weights for this tile's level (per lane: bfloat16 heads, then bfloat16 remainders), head_b4 its bias
@@ -656,6 +661,25 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
                     if (k < a.head_C) a.head_y[(int64_t)k * a.head_ld + oh] = float_to_bf16(hacc[k] + head_b4[k]);
             }
             continue;
+        }
+        if constexpr (MODE == 1) {
+            // The columns of a coarser particle (COL_BOX, see dx_group) are added up across lanes and the first one takes the sum:
+            // one addition per coarser particle instead of one per cell: training step on 3.4 M particles 19.2 -> 17.8 ms (16 outputs
+            // 895 -> 738 us, 32 715 -> 592 us); an image with hardly any coarser particle next to finer ones as before.
+            const bool boxed = col < nc && (sh.col_pos[col] & COL_BOX) != 0;
+            if (__ballot(boxed)) {
+#pragma unroll
+                for (int h = 0; h < COH; ++h)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        float s = acc[j][h][r];
+                        s += dpp_f32<0xb1>(s);                                       // lanes 1, 0, 3, 2 of each four
+                        s += dpp_f32<0x4e>(s);                                       // lanes 2, 3, 0, 1
+                        if constexpr (dx_group<G>() == 8) s += dpp_f32<0x141>(s);    // the eight mirrored
+                        acc[j][h][r] = boxed ? s : acc[j][h][r];
+                    }
+            }
+            if (boxed && (lane & (dx_group<G>() - 1)) != 0) continue;
         }
         if (col >= nc) continue;
         int64_t o;

@@ -11,7 +11,7 @@
 
 namespace aprnet {
 
-// DX: lists of the input gradient (scan_window_dx without pooled columns) over the tiles within one row of an
+// DX: lists of the input gradient (scan_window_dx, the columns of a coarser particle in groups) over the tiles within one row of an
 // output; windows without an output position are not stored.
 //
 // Forward lists keep the items that some output position of the window can reach through the stencil.  The scan
@@ -38,10 +38,11 @@ build_lists_kernel(const ConvArgs<float> a, const int pass, int4* __restrict__ t
     open_segments<G, float>(a, L, tile.z0, tile.x0, sh);
     __syncthreads();
     for (int y0 = 0; y0 < yn; y0 += G::TY) {
-        if constexpr (DX) scan_window_dx<G, float>(a, L, tile.z0, tile.x0, y0, out_tree, sh, false);
+        if constexpr (DX) scan_window_dx<G, float>(a, L, tile.z0, tile.x0, y0, out_tree, sh, false, true);
         else scan_window<G, float>(a, L, y0, out_tree, sh);
         __syncthreads();
-        const int nc = sh.ncol, nitem = sh.nitem;
+        const int nsum = DX ? dx_group<G>() * sh.nbox : 0;                   // columns of coarser particles, summed in groups: first
+        const int nc = nsum + sh.ncol, nitem = sh.nitem;
         if (nc > 0 && (!DX || nitem > 0)) {
             // list offsets are unsigned 32-bit numbers stored in the int fields of the header
             const unsigned ib = (unsigned)off.y + (unsigned)ni, cb = (unsigned)off.z + (unsigned)ncl;
@@ -88,7 +89,10 @@ build_lists_kernel(const ConvArgs<float> a, const int pass, int4* __restrict__ t
             }
             if (pass == 1) {
                 if (threadIdx.x == 0) win[off.x + nwin] = make_int4((int)ib, nkeep, (int)cb, nc);
-                for (int i = threadIdx.x; i < nc; i += G::NT) { col_idx[(size_t)cb + i] = sh.col_idx[i]; col_pos[(size_t)cb + i] = sh.col_pos[i]; }
+                for (int i = threadIdx.x; i < nc; i += G::NT) {
+                    const int at = DX && i >= nsum ? G::MAXCOL - 1 - (i - nsum) : i;
+                    col_idx[(size_t)cb + i] = sh.col_idx[at]; col_pos[(size_t)cb + i] = sh.col_pos[at];
+                }
             }
             ++nwin; ni += nkeep; ncl += nc;
         }

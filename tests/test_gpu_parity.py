@@ -1071,3 +1071,28 @@ def test_conv111_weight_gradient_bf16_strips(cin, cout, shape, density):
         xs, gs = x[0, :, part].double(), gy[0, :, part].double()
         ref, size = gs @ xs.T, gs.abs() @ xs.abs().T
         assert bool(((gw[s].double() - ref).abs() <= n * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("shape,ksize", [((32, 48, 64), (3, 3, 3)), ((33, 47, 61), (3, 3, 3)), ((1, 128, 250), (1, 5, 5)), ((1, 95, 127), (1, 3, 3))])
+@pytest.mark.parametrize("cin,cout", [(16, 16), (40, 24)])
+def test_conv_backward_bf16_groups_of_coarser_particles(shape, ksize, cin, cout):
+    """The bfloat16 input gradient sums the cells of a coarser particle across lanes before it adds them: level boundaries in every
+    row group, even sizes (all such particles in groups: the gradient then repeats bit for bit, two additions per element)
+    and odd ones (some stick out of the far faces and are added cell by cell).  Against the oracle in float64 on the rounded
+    operands: products exact, at most 8 * K * cout terms in fp32, one rounding to bfloat16."""
+    apr = apr_cases.random_apr(shape, 31, 0.03)
+    apr.init_cuda()
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    g = torch.Generator().manual_seed(5)
+    x, go = (torch.randn(1, c, n, generator=g).to(torch.bfloat16) for c in (cin, cout))
+    w = torch.randn(apr.level_max() - apr.level_min() + 1, cout, cin, *ksize, generator=g).to(torch.bfloat16).float()
+    run = lambda: _ops.conv_backward([apr], x.to(DEV), w.to(DEV), go.to(DEV), ld)[0]
+    gx = run()
+    wo = w.permute(2, 0, 1, 3, 4, 5).contiguous().double()
+    ref = oracle.conv_backward([apr], x.double(), wo, go.double(), ld)[0]
+    terms = oracle.conv_backward([apr], x.double().abs(), wo.abs(), go.double().abs(), ld)[0]
+    bound = 2.0 ** -8 * ref.abs() + 8 * int(np.prod(ksize)) * cout * 2.0 ** -24 * terms
+    assert bool(((gx.double().cpu() - ref).abs() <= bound).all())
+    if all(s % 2 == 0 for s in shape[1:]) and all(v % 2 == 0 or v == 1 for lv in range(apr.level_min() + 1, apr.level_max() + 1)
+                                                 for v in (apr.iterator().z_num(lv), apr.iterator().x_num(lv), apr.iterator().y_num(lv))):
+        assert all(torch.equal(gx, run()) for _ in range(3))

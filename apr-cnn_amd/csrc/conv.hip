@@ -150,6 +150,13 @@ int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
 int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st);
 
+size_t split_mark_bytes();
+size_t conv_packed_split_bytes(int code, int S_exp, int Cout, int Cin);
+int pack_conv_weights_split(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, int* marks, hipStream_t st);
+int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st);
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
+static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
+
 bool conv_narrow_supported(int code, int Cin);
 size_t conv_narrow_packed_floats(int code, int S_exp, int Cout, int Cin, bool bf16m);
 bool conv_narrow_bf16_math(int code, int Cin);
@@ -211,20 +218,53 @@ static int try_narrow(aprnet_plan* p, const ConvArgs<T>& a, int code, int d, con
     return launch_conv_narrow(code, b, wl, st);
 }
 
-template <typename T> static int try_mfma(aprnet_plan*, const ConvArgs<T>&, int, int, const TileList&, int, hipStream_t, bool*) { return 0; }
+// Work space of the forward pass on products of bfloat16 pieces: packed weights, the input and its mean tree in groups of four
+// channels.  0: the layer does not take that path.
+//  - fewer than SPLIT_MIN_CIN input channels: with 8 it is no faster (8 -> 16 channels on 320 k particles 0.080 against 0.078 ms,
+//    copies included), and with 5 the fp32 instructions' short sums have the smaller error (2.07 against 2.28 of 1e-7).
+//  - 1x3x3: two steps of eight taps for nine, less than the copies cost (64 -> 64 channels on 70 k particles 107 against 98 us,
+//    on 320 k 346 against 352).
+//  - little work: the copies and launches take 8 us (3x3x3, split against fp32; 16 outputs: 70 k particles 52 and 47 us, 320 k
+//    96 and 107; 32 outputs: 13 k particles x 16 channels 43 and 39, x 32 49 and 55, 2 k x 32 39 and 34; 64 outputs:
+//    2 k x 64 46 and 53 us).
+//  - the 16-byte items are reached with 32-bit offsets: fewer than 2^28 particles.
+constexpr int SPLIT_MIN_CIN = 16;
+static size_t split_align(size_t v) { return (v + 255) / 256 * 256; }
+static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx, int64_t nt) {
+    if (!g_f32_split || g_conv_path == 1 || (code != 333 && code != 155) || Cin < SPLIT_MIN_CIN || nx >= (1ll << 28) || nt >= (1ll << 28)) return 0;
+    if (g_f32_split == 1 && (double)nx * Cin * ((Cout + 15) / 16 * 16) < (Cout <= 16 ? 1 << 26 : 1 << 23)) return 0;
+    if (conv_packed_split_bytes(code, S_exp, Cout, Cin) / 48 >= (1u << 29)) return 0;               // elements the packing kernel counts in 32 bits
+    return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cout, Cin)) + (size_t)(Cin + 3) / 4 * (size_t)(nx + nt) * 16;
+}
+
+template <typename T> static int try_mfma(aprnet_plan*, const ConvArgs<T>&, int, int, const TileList&, int, hipStream_t, bool*, void*, int64_t) { return 0; }
 template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int code, int d, const TileList& tl, int n_tiles,
-                                hipStream_t st, bool* done) {
+                                hipStream_t st, bool* done, void* ws, int64_t ws_bytes) {
     if (g_conv_path == 1 || !conv_mfma_supported(code)) return 0;
     if (int rc = try_narrow<float>(p, a, code, d, tl, st, done)) return rc;
     if (*done) return 0;
     *done = true;
+    ConvArgs<float> b = a;
+    if (int rc = set_lists(p, d, code, tl, b, st)) return rc;
+    const size_t need = b.tile_win ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
+    if (need > 0 && ws && ws_bytes >= 0 && (size_t)ws_bytes >= need) {
+        // products of bfloat16 pieces on copies in groups of four channels, all in the caller's work space
+        const size_t wbytes = split_align(conv_packed_split_bytes(code, a.S_exp, a.Cout, a.Cin)), ng = (size_t)(a.Cin + 3) / 4;
+        char* image = (char*)ws + split_mark_bytes();
+        float* xi = (float*)(image + wbytes), *ti = xi + ng * (size_t)a.x_count * 4;
+        if (int rc = pack_conv_weights_split(code, a.w, a.S_exp, a.Cout, a.Cin, image, (int*)ws, st)) return rc;
+        if (int rc = group4_f32(a.x, a.ldx, a.x2, a.ldx2, a.c_split, a.Cin, a.x_count, xi, st)) return rc;
+        if (int rc = group4_f32(a.tree_data, a.ldt, nullptr, 0, a.Cin, a.Cin, a.t_count, ti, st)) return rc;
+        b.w_raw = a.w; b.w = (const float*)image; b.redo = (int*)ws;
+        b.xi = xi; b.ti = ti; b.xi_ld = a.x_count; b.ti_ld = a.t_count;
+        TimedLaunch timed(st);
+        return launch_conv_split(code, b, n_tiles, st);
+    }
     // plan-owned scratch for the re-laid-out weights, grown on demand
     ScratchLease lease;
     if (int rc = lease.acquire(p, conv_packed_floats(code, a.S_exp, a.Cout, a.Cin, false) * sizeof(float), st)) return rc;
     if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cout, a.Cin, false, (float*)p->d_scratch, st)) return rc;
-    ConvArgs<float> b = a;
     b.w = (const float*)p->d_scratch;
-    if (int rc = set_lists(p, d, code, tl, b, st)) return rc;
     TimedLaunch timed(st);
     return launch_conv_mfma(code, b, n_tiles, st);
 }
@@ -267,7 +307,7 @@ static int read_fusion(const aprnet_conv_fusion* f, Fusion<T>* out) {
 template <typename T>
 int conv_fwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, int64_t ldx, int C1, const T* w,
              int S_exp, int Cout, const T* bias, T* y, int64_t ldy, T* tree_ws, int64_t ldt, hipStream_t st,
-             const Fusion<T>& fu = Fusion<T>{}) {
+             const Fusion<T>& fu = Fusion<T>{}, void* ws = nullptr, int64_t ws_bytes = 0) {
     aprnet_plan* p = const_cast<aprnet_plan*>(cp);
     if (int rc = check_level_delta(p, d, "conv_forward")) return rc;
     if (int rc = check_plane_size(p, d, sizeof(*x), "conv_forward")) return rc;
@@ -298,7 +338,7 @@ int conv_fwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
     a.tree_data = tree_ws; a.ldt = ldt; a.Lc = p->lc(d); a.tree_off = p->tree_offset(a.Lc);
     a.x_count = p->number_parts(d); a.t_count = p->tree_parts(d);
     bool done = false;
-    if (int rc = try_mfma<T>(p, a, code, d, tl, tl.n, st, &done)) return rc;
+    if (int rc = try_mfma<T>(p, a, code, d, tl, tl.n, st, &done, ws, ws_bytes)) return rc;
     if (done) return 0;
     // few output channels per thread keep the wave-uniform weights within the scalar register file;
     // wider layers run more blocks along grid.y (each re-stages its patch)
@@ -528,6 +568,19 @@ int aprnet_conv_fwd_fused_f32(const aprnet_plan* p, int d, int kz, int kx, int k
     APRNET_FUSED_111(float)
     return conv_fwd<float>(p, d, kz, kx, ky, x, ldx, Cin, w, S_exp, Cout, bias, y, ldy, tree_ws, ldt, (hipStream_t)st, fu);
 }
+int64_t aprnet_conv_ws_bytes_f32(const aprnet_plan* p, int d, int kz, int kx, int ky, int Cin, int S_exp, int Cout) {
+    if (!p || d < 0 || d >= p->tree.level_max + 1 || Cin <= 0 || S_exp <= 0 || Cout <= 0) return 0;
+    return (int64_t)split_fwd_bytes(kz * 100 + kx * 10 + ky, Cin, S_exp, Cout, p->number_parts(d), p->tree_parts(d));
+}
+int aprnet_conv_fwd_ws_f32(const aprnet_plan* p, int d, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
+                           const float* w, int S_exp, int Cout, const float* bias, float* y, int64_t ldy, float* tree_ws,
+                           int64_t ldt, const aprnet_conv_fusion* fusion, void* ws, int64_t ws_bytes, void* st) {
+    Fusion<float> fu;
+    if (int rc = read_fusion(fusion, &fu)) return rc;
+    APRNET_FUSED_111(float)
+    if (((uintptr_t)ws & 15) != 0) return fail(APRNET_ERR_INVALID_ARGUMENT, "conv_forward: the work space is not aligned to 16 bytes");
+    return conv_fwd<float>(p, d, kz, kx, ky, x, ldx, Cin, w, S_exp, Cout, bias, y, ldy, tree_ws, ldt, (hipStream_t)st, fu, ws, ws_bytes);
+}
 int aprnet_conv_fwd_fused_f64(const aprnet_plan* p, int d, int kz, int kx, int ky, const double* x, int64_t ldx, int Cin,
                               const double* w, int S_exp, int Cout, const double* bias, double* y, int64_t ldy, double* tree_ws,
                               int64_t ldt, const aprnet_conv_fusion* fusion, void* st) {
@@ -551,13 +604,15 @@ int aprnet_set_conv_path(int path) {
     if (path == 12 || path == 13) { g_narrow = path == 12; return 0; }
     if (path == 14 || path == 15) { g_big_addr = path == 15; return 0; }
     if (path == 16 || path == 17) { g_need_fill = path == 16; return 0; }
+    if (path >= 18 && path <= 20) { g_f32_split = path == 18 ? 1 : path == 19 ? 0 : 2; return 0; }
     if (path != 0 && path != 1)
         return fail(APRNET_ERR_INVALID_ARGUMENT, "set_conv_path: 0 (auto), 1 (VALU only), 2 / 3 (bfloat16 features: bfloat16 / fp32 "
                                                  "matrix math), 4 / 5 (forward: window lists of the plan / scan per call), 6 / 7 (backward on two streams / one), "
                                                  "8 / 9 (bfloat16 forward: regrouped copy of the input / channel planes), 10 / 11 (weight gradient: "
                                                  "fixed-order partial sums / atomic additions), 12 / 13 (1 to 3 input channels: pipelined kernel / general kernel), "
                                                  "14 / 15 (grouped bfloat16 forward: 32-bit offsets where they suffice / 64-bit addresses always), "
-                                                 "16 / 17 (tree fill before a forward convolution: the nodes it reads / every node)");
+                                                 "16 / 17 (tree fill before a forward convolution: the nodes it reads / every node), "
+                                                 "18 / 19 (fp32 features: products of bfloat16 pieces where a work space is given / fp32 matrix instructions)");
     g_conv_path = path;
     return 0;
 }

@@ -32,6 +32,8 @@ struct ConvArgs {
     // the result can be clamped at zero after the bias
     const T* x2; int64_t ldx2; int c_split; int relu;
     const typename Num<T>::acc* w; int S_exp; int Cout;     // [S_exp][Cout][Cin][K]; fp32 for bfloat16 features
+    const typename Num<T>::acc* w_raw;                      // the weights as the caller gave them (kernels whose `w` is a packed image)
+    int* redo;                                              // conv_split.hip: marks of the tiles to compute again
     const typename Num<T>::acc* bias;                       // [Cout] or null
     T* y; int64_t ldy;
     const T* tree_data; int64_t ldt;
@@ -583,6 +585,36 @@ __device__ __forceinline__ void store_items(const ItemRegs<G, T, CIB, NR>& R, in
     }
 }
 
+// ---- items of 16 bytes (a group of channels of one particle next to each other) -------------------------------
+typedef int intx4 __attribute__((ext_vector_type(4)));
+template <class G, int IPT>
+struct ItemRegs16 { intx4 v[IPT]; unsigned off[IPT]; unsigned short pos[IPT]; };
+
+// BIG: tensors of 2^28 elements and more per group, whose 16-byte items lie past 32-bit byte offsets: R.off keeps the
+// element index and the loads take 64-bit addresses (a lane without an item reads element 0; its value is never stored)
+template <class G, int IPT, bool BIG = false, class Lists>
+__device__ __forceinline__ void fetch_slots16(const Lists& sh, int nitem, ItemRegs16<G, IPT>& R) {
+    // unconditional buffer loads, results touched only after every round is issued (see fetch_slots)
+    const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(sh.item_idx), 0, nitem * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(sh.item_pos), 0, nitem * 2, 0x00020000);
+    int idx[IPT], pos[IPT];
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));                       // offsets formed per call, not kept (and spilled) across the window loop
+#pragma unroll
+    for (int k = 0; k < IPT; ++k) {
+        idx[k] = 0; pos[k] = 0;
+        if (k * G::NT >= nitem) continue;               // wave-uniform
+        const int it = tid + k * G::NT;
+        idx[k] = __builtin_amdgcn_raw_buffer_load_b32(ri, it * 4, 0, 0);
+        pos[k] = (int)__builtin_amdgcn_raw_buffer_load_b16(rp, it * 2, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < IPT; ++k) {
+        const bool valid = (int)threadIdx.x + k * G::NT < nitem;
+        R.pos[k] = valid ? (unsigned short)pos[k] : (unsigned short)0xffffu;
+        R.off[k] = BIG ? (valid ? (unsigned)idx[k] : 0u) : (valid ? (unsigned)idx[k] * 16u : BUF_OOB);
+    }
+}
 // Gather of one channel chunk into the patch.  Cells that no item covers keep the zeros written once
 // per window (outside the image, or inside a particle two or more levels coarser, which a stencil of
 // half-width <= 2 never reads on a 2:1-balanced APR); covered cells are overwritten by every chunk.

@@ -399,35 +399,6 @@ __device__ __forceinline__ void store_items_bf16(const ItemRegs<G, bf16_t, BF_CI
 // of a group next to each other an item is ONE 16-byte load per round of staging instead of eight 2-byte loads
 // through eight descriptors: an eighth of the load instructions, a quarter of the value registers, two
 // descriptors instead of sixteen.  The regrouping is one streaming pass over the input (interleave8_kernel).
-typedef int intx4 __attribute__((ext_vector_type(4)));
-template <class G, int IPT>
-struct ItemRegs16 { intx4 v[IPT]; unsigned off[IPT]; unsigned short pos[IPT]; };
-
-// BIG: tensors of 2^28 elements and more per group, whose 16-byte items lie past 32-bit byte offsets: R.off keeps the
-// element index and the loads take 64-bit addresses (a lane without an item reads element 0; its value is never stored)
-template <class G, int IPT, bool BIG = false, class Lists>
-__device__ __forceinline__ void fetch_slots16(const Lists& sh, int nitem, ItemRegs16<G, IPT>& R) {
-    // unconditional buffer loads, results touched only after every round is issued (see fetch_slots)
-    const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(sh.item_idx), 0, nitem * 4, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(sh.item_pos), 0, nitem * 2, 0x00020000);
-    int idx[IPT], pos[IPT];
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));                       // offsets formed per call, not kept (and spilled) across the window loop
-#pragma unroll
-    for (int k = 0; k < IPT; ++k) {
-        idx[k] = 0; pos[k] = 0;
-        if (k * G::NT >= nitem) continue;               // wave-uniform
-        const int it = tid + k * G::NT;
-        idx[k] = __builtin_amdgcn_raw_buffer_load_b32(ri, it * 4, 0, 0);
-        pos[k] = (int)__builtin_amdgcn_raw_buffer_load_b16(rp, it * 2, 0, 0);
-    }
-#pragma unroll
-    for (int k = 0; k < IPT; ++k) {
-        const bool valid = (int)threadIdx.x + k * G::NT < nitem;
-        R.pos[k] = valid ? (unsigned short)pos[k] : (unsigned short)0xffffu;
-        R.off[k] = BIG ? (valid ? (unsigned)idx[k] : 0u) : (valid ? (unsigned)idx[k] * 16u : BUF_OOB);
-    }
-}
 template <class G, int IPT, bool BIG = false>
 __device__ __forceinline__ void load_values16(const ConvArgs<bf16_t>& a, int ci0, int nitem, bool tree_items, ItemRegs16<G, IPT>& R) {
     const int q = ci0 / BF_CIB;

@@ -1,0 +1,473 @@
+// Stencil convolution of fp32 features on the bfloat16 matrix instructions, gfx950: every fp32 operand as three bfloat16
+// pieces.
+//
+// An fp32 value is the exact sum of three bfloat16 numbers: x = x1 + x2 + x3 with x1 = bf16(x), x2 = bf16(x - x1),
+// x3 = x - x1 - x2 (8 significant bits each, round to nearest even).  Of the nine products of two such sums the six that
+// reach 2^-24 of the whole are formed, x1 w1, x1 w2, x2 w1, x2 w2, x1 w3, x3 w1: a product of two bfloat16 numbers is
+// exact in fp32, what is left out is below 2^-25 of |x w|, half of one rounding of an fp32 product, and all sums are fp32.
+// v_mfma_f32_16x16x32_bf16 does 16 times the multiply-adds per cycle of v_mfma_f32_16x16x4_f32, so six products per
+// multiply-add leave a factor of 2.7, and the bfloat16 instructions do not occupy the vector ALU the staging needs.
+//
+// A chunk of four input channels lies in LDS as three patches of 8 bytes per cell, one per piece; the 32 k of an instruction are
+// 4 pairs of taps x 4 channels, so both operands are pieces as they lie there and a step of eight taps takes six instructions.  (With
+// 16-byte cells {x1, x2} and weights {w1, w1}, {w2, w2}, {w3, w1} a step of four taps takes three, one eighth fewer over
+// the 27 taps, but the doubled weights cost 24 register moves per step and wave: 10.1 against 9.1 ms for 32 -> 32 channels
+// on 23 M particles.)  Values come from copies in groups of four channels, one 16-byte load per item; a value is split when it is
+// written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
+//
+// Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.5 (12.5) ms, 16 -> 16
+// channels 3.4 (4.1) ms; 320 k particles, 64 -> 64 channels 0.51 (0.78) ms.
+// Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: matrix pipes busy 46 %,
+// vector ALU 15 %, LDS 56 % of the cycles.
+// Error against 64 bits (2-norm, 16 to 128 channels): 0.37 to 0.40 of the fp32 instructions' with N(0, 1) features, 0.44 to 0.49
+// with those after a ReLU.
+//
+// Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
+// NaN), and a value within 2^-9 of the largest fp32 number has an infinite first piece.  A result that comes out infinite
+// or NaN is therefore not stored: the tile is marked, and conv_split_redo_kernel computes the marked tiles again from the fp32
+// values.  (As a call inside this kernel it cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart.)  Values below
+// 2^-110 lose low pieces to the end of the exponent range (an absolute error below 2^-133).
+#include "conv_common.hpp"
+
+namespace aprnet {
+
+typedef float floatx4s __attribute__((ext_vector_type(4)));
+typedef int intx4s __attribute__((ext_vector_type(4)));
+typedef unsigned uintx2s __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4s __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x2s __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8s __attribute__((ext_vector_type(8)));
+
+constexpr int SP_CIB = 4;                      // input channels of a staged chunk
+// The 32 k of an instruction are 4 pairs of taps x 4 channels: lane group g = lane / 16 supplies pair 4 step + g.  Pairs are
+// neighbours along y where the stencil's rows have them (dy 0 and 1, dy 2 and 3), the last taps of the rows among themselves.
+// An LDS read of 8 bytes per lane goes out for two lane groups at a time, sixteen neighbouring cells each (256 bytes, every bank
+// once) if the two groups' cells do not fall on the same banks: the order below was searched for that (27 taps: 10 of 16
+// reads without conflict, in index order 2; 16 -> 16 on 23 M particles 3.27 -> 3.09 ms).  -1: no tap, zero weights.
+template <int K> struct SplitTaps;
+template <> struct SplitTaps<27> {
+    static constexpr int STEPS = 4;
+    static constexpr signed char tap[32] = {20, 26, 18, 19, 24, 25, 12, 13, 11, 2, 0, 1, 15, 16, 17, 14, 5, -1, 3, 4, 23, 8, 6, 7, 9, 10, -1, -1, 21, 22, -1, -1};
+};
+template <> struct SplitTaps<25> {
+    static constexpr int STEPS = 4;
+    static constexpr signed char tap[32] = {-1, -1, 7, 8, 0, 1, 2, 3, 17, 18, 15, 16, 12, 13, 10, 11, 22, 23, 20, 21, 14, 19, 4, -1, 24, 9, -1, -1, -1, -1, 5, 6};
+};
+template <class G> constexpr int split_steps() { return SplitTaps<G::K>::STEPS; }
+
+// two fp32 numbers -> their bfloat16 roundings, the first in the low half (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ unsigned split_round(float a, float b) {
+    const bf16x2s h = {(__bf16)a, (__bf16)b};
+    return __builtin_bit_cast(unsigned, h);
+}
+__device__ __forceinline__ float split_lo(unsigned p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float split_hi(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// two fp32 numbers -> three words with their pieces
+__device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsigned& p2, unsigned& p3) {
+    p1 = split_round(a, b);
+    const float ra = a - split_lo(p1), rb = b - split_hi(p1);
+    p2 = split_round(ra, rb);
+    p3 = split_round(ra - split_lo(p2), rb - split_hi(p2));
+}
+
+// Marks of a launch: word 0 = any, the others one per tile and block of output channels, several of them to a word where there are more
+// (all of these are then computed again).
+constexpr unsigned SPLIT_MARKS = 4096;
+__device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit % (SPLIT_MARKS - 1); }
+
+// packed[s][cb][q][step][piece][h][lane] (16 bytes: two taps of four channels), cb = block of 16 * COH output channels, q = chunk
+// of four input channels.  The marks of the launch are cleared on the way.
+template <int K>
+__global__ void pack_weights_split_kernel(const float* __restrict__ w, int S_exp, int Cout, int Cin, int COH, uint4* __restrict__ out,
+                                          int* __restrict__ marks) {
+    constexpr int nstep = SplitTaps<K>::STEPS;
+    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < SPLIT_MARKS; i += gridDim.x * blockDim.x) marks[i] = 0;
+    const int ncb = (Cout + 16 * COH - 1) / (16 * COH), nq = (Cin + SP_CIB - 1) / SP_CIB;
+    const unsigned n = (unsigned)S_exp * ncb * nq * nstep * COH * 64;          // (the host checks that it fits)
+    for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
+        unsigned r = e;
+        const int lane = (int)(r % 64u); r /= 64u;
+        const int h = (int)(r % (unsigned)COH); r /= (unsigned)COH;
+        const int step = (int)(r % (unsigned)nstep); r /= (unsigned)nstep;
+        const int q = (int)(r % (unsigned)nq); r /= (unsigned)nq;
+        const int cb = (int)(r % (unsigned)ncb); r /= (unsigned)ncb;
+        const int s = (int)r;
+        const int cm = (cb * COH + h) * 16 + (lane & 15);
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int t = SplitTaps<K>::tap[2 * (4 * step + (lane >> 4)) + (j >> 2)], ck = q * SP_CIB + (j & 3);
+            v[j] = 0.f;
+            if (t >= 0 && cm < Cout && ck < Cin) v[j] = w[(((int64_t)s * Cout + cm) * Cin + ck) * K + t];
+        }
+        uint4 p[3];
+        split_pair(v[0], v[1], p[0].x, p[1].x, p[2].x);
+        split_pair(v[2], v[3], p[0].y, p[1].y, p[2].y);
+        split_pair(v[4], v[5], p[0].z, p[1].z, p[2].z);
+        split_pair(v[6], v[7], p[0].w, p[1].w, p[2].w);
+        const unsigned base = (((s * ncb + cb) * nq + q) * nstep + step) * 3u;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) out[((base + k) * COH + h) * 64 + lane] = p[k];
+    }
+}
+
+// ---- input in groups of four channels: [Cin / 4][count][4] ---------------------------------------------------
+// out[q][i][c] = channel 4 q + c of element i; channels from c_split on come from x2 (null: all from x), channels past C
+// are zeros.  A streaming pass (8 bytes per value), four elements per thread, all reads issued before the first is used.
+constexpr int IG_TB = 256, IG_E = 4;
+__global__ void __launch_bounds__(IG_TB)
+group4_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict__ x2, int64_t ldx2, int c_split, int C, int64_t count,
+              float4* __restrict__ out) {
+    const int q = blockIdx.y;
+    const int64_t i0 = (int64_t)blockIdx.x * (IG_TB * IG_E) + threadIdx.x;
+    float v[SP_CIB][IG_E];
+#pragma unroll
+    for (int c = 0; c < SP_CIB; ++c) {
+        const int ch = min(q * SP_CIB + c, C - 1);
+        const float* p = (x2 != nullptr && ch >= c_split) ? x2 + (int64_t)(ch - c_split) * ldx2 : x + (int64_t)ch * ldx;
+#pragma unroll
+        for (int e = 0; e < IG_E; ++e) v[c][e] = p[min(i0 + e * IG_TB, count - 1)];
+    }
+#pragma unroll
+    for (int c = 0; c < SP_CIB; ++c)
+        if (q * SP_CIB + c >= C) {                  // uniform
+#pragma unroll
+            for (int e = 0; e < IG_E; ++e) v[c][e] = 0.f;
+        }
+    float4* dst = out + (int64_t)q * count;
+#pragma unroll
+    for (int e = 0; e < IG_E; ++e)
+        if (i0 + e * IG_TB < count) dst[i0 + e * IG_TB] = make_float4(v[0][e], v[1][e], v[2][e], v[3][e]);
+}
+
+template <class G> struct SplitItems : ItemRegs16<G, (G::MAXITEM + G::NT - 1) / G::NT> {
+    static constexpr int IPT = (G::MAXITEM + G::NT - 1) / G::NT;
+};
+template <class G>
+__device__ __forceinline__ void load_values_split(const ConvArgs<float>& a, int q, int nitem, bool tree_items, SplitItems<G>& R) {
+    const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.xi + (int64_t)q * a.xi_ld * SP_CIB), 0,
+                                                                        (int)(a.x_count * 16), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.ti + (int64_t)q * a.ti_ld * SP_CIB), 0,
+                                                                        tree_items ? (int)(a.t_count * 16) : 0, 0x00020000);
+#pragma unroll
+    for (int k = 0; k < SplitItems<G>::IPT; ++k) {
+        if (k * G::NT >= nitem) break;                  // wave-uniform
+        const bool from_tree = (R.pos[k] & ITEM_TREE) != 0 && R.pos[k] != 0xffffu;
+        if (tree_items) {
+            if (from_tree) {
+                R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rt, (int)R.off[k], 0, 0);
+                asm volatile("" ::: "memory");          // keeps the two branches from being merged into one load with a per-lane descriptor
+            } else {
+                R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)R.off[k], 0, 0);
+            }
+        } else {
+            R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)R.off[k], 0, 0);
+        }
+    }
+}
+template <class G, int COH>
+struct SplitShared {
+    uint4 w[split_steps<G>() * 3 * COH * 64];
+    uint2 patch[3][G::CH_STRIDE];  // the three pieces of four channels, 8 bytes per cell
+    float bias[16 * COH];
+    int4 hdr[16];                  // headers of sixteen windows: one round trip instead of one per window
+    int2 toff[split_steps<G>() * 4];
+};
+template <class G, int COH>
+__device__ __forceinline__ void store_items_split(const SplitItems<G>& R, int nitem, SplitShared<G, COH>& sh) {
+#pragma unroll
+    for (int k = 0; k < SplitItems<G>::IPT; ++k) {
+        if (k * G::NT >= nitem) break;                  // wave-uniform
+        if (R.pos[k] == 0xffffu) continue;
+        uint2 p[3];
+        split_pair(__builtin_bit_cast(float, (int)R.v[k][0]), __builtin_bit_cast(float, (int)R.v[k][1]), p[0].x, p[1].x, p[2].x);
+        split_pair(__builtin_bit_cast(float, (int)R.v[k][2]), __builtin_bit_cast(float, (int)R.v[k][3]), p[0].y, p[1].y, p[2].y);
+        const int c = R.pos[k] & ITEM_CELL;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) sh.patch[i][c] = p[i];
+        if (R.pos[k] & ITEM_PAIR) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) sh.patch[i][c + 1] = p[i];
+        }
+    }
+}
+
+template <class G, int COH, int NB>
+__device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, int nc, int nitem, bool tree_items, int first,
+                                             const uint4* __restrict__ wl, const WindowLists& gl, int* __restrict__ mark, SplitShared<G, COH>& sh) {
+    constexpr int NSTEP = split_steps<G>(), NBA = NB > 0 ? NB : 1;
+    const int lane = lane_id();
+    int cell[NBA];
+    // unconditional loads (columns past the end read zero) that travel together with the list loads below
+    const __amdgpu_buffer_rsrc_t rcp = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(gl.col_pos), 0, nc * 2, 0x00020000);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) cell[j] = (int)__builtin_amdgcn_raw_buffer_load_b16(rcp, (((first + G::NWAVE * j) << 4) + (lane & 15)) * 2, 0, 0);
+    floatx4s acc[NBA][COH];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int h = 0; h < COH; ++h) acc[j][h] = floatx4s{0.f, 0.f, 0.f, 0.f};
+
+    constexpr int W16 = NSTEP * 3 * COH * 64;                    // 16-byte elements of a weight chunk
+    constexpr int WPT = (W16 + G::NT - 1) / G::NT;
+    SplitItems<G> R;
+    intx4s wr[WPT];                    // unconditional buffer loads, see the fp32 kernel
+    auto load_weights = [&](int q) {
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint4*>(wl + (int64_t)q * W16), 0, W16 * 16, 0x00020000);
+#pragma unroll
+        for (int k = 0; k < WPT; ++k) wr[k] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(threadIdx.x + k * G::NT) * 16, 0, 0);
+    };
+    fetch_slots16<G, SplitItems<G>::IPT>(gl, nitem, R);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int col = ((first + G::NWAVE * j) << 4) + (lane & 15);
+        cell[j] = col < nc ? ((cell[j] & (int)COL_CELL) - G::TAP0) * 8 : 0;
+    }
+    load_values_split<G>(a, 0, nitem, tree_items, R);
+    load_weights(0);
+    for (int i = threadIdx.x; i < 3 * G::CH_STRIDE / 2; i += G::NT) reinterpret_cast<uint4*>(sh.patch)[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int ci0 = 0; ci0 < a.Cin; ci0 += SP_CIB) {
+        __syncthreads();
+        store_items_split<G, COH>(R, nitem, sh);
+#pragma unroll
+        for (int k = 0; k < WPT; ++k) {
+            const int i = threadIdx.x + k * G::NT;
+            if (i < W16) reinterpret_cast<intx4s*>(sh.w)[i] = wr[k];
+        }
+        __syncthreads();
+        if (ci0 + SP_CIB < a.Cin) {
+            load_values_split<G>(a, ci0 / SP_CIB + 1, nitem, tree_items, R);
+            load_weights(ci0 / SP_CIB + 1);
+        }
+        if constexpr (NB > 0) {
+            const uintx4s* wa = reinterpret_cast<const uintx4s*>(sh.w) + lane;
+            const int2* to = sh.toff + (lane >> 4);
+            constexpr int PL = G::CH_STRIDE * 8;                 // bytes of a piece's patch
+            const char* p0 = reinterpret_cast<const char*>(sh.patch);
+            // one step at a time where the weights of a step fill the registers (32 outputs); all of them with 16 outputs
+            constexpr int UNROLL = COH == 1 ? NSTEP : 1;
+#pragma unroll UNROLL
+            for (int st = 0; st < NSTEP; ++st) {
+                bf16x8s a1[COH], a2[COH], a3[COH];
+#pragma unroll
+                for (int h = 0; h < COH; ++h) {
+                    a1[h] = __builtin_bit_cast(bf16x8s, wa[((st * 3 + 0) * COH + h) * 64]);
+                    a2[h] = __builtin_bit_cast(bf16x8s, wa[((st * 3 + 1) * COH + h) * 64]);
+                    a3[h] = __builtin_bit_cast(bf16x8s, wa[((st * 3 + 2) * COH + h) * 64]);
+                }
+                const int2 off = to[st * 4];
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const char* qa = p0 + (cell[j] + off.x);
+                    const char* qb = p0 + (cell[j] + off.y);
+                    bf16x8s b[3];
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) {
+                        const uintx2s u = *reinterpret_cast<const uintx2s*>(qa + i * PL), v = *reinterpret_cast<const uintx2s*>(qb + i * PL);
+                        b[i] = __builtin_bit_cast(bf16x8s, uintx4s{u.x, u.y, v.x, v.y});
+                    }
+                    // the five products below 2^-8 of the first among themselves: the sum so far is rounded twice per step and not six
+                    // times (error 0.45 instead of 1.15 of the fp32 instructions' with ReLU's zeros among the features; 32 -> 32
+                    // channels on 23 M particles 9.5 instead of 9.2 ms).  All six apart: 0.32 and 9.9 ms.
+                    floatx4s t[COH];
+#define APRNET_PRODUCT(C, A, B) _Pragma("unroll") for (int h = 0; h < COH; ++h) t[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[h], B, C, 0, 0, 0);
+                    APRNET_PRODUCT((floatx4s{0.f, 0.f, 0.f, 0.f}), a3, b[0]) APRNET_PRODUCT(t[h], a1, b[2]) APRNET_PRODUCT(t[h], a2, b[1])
+                    APRNET_PRODUCT(t[h], a2, b[0]) APRNET_PRODUCT(t[h], a1, b[1])
+#pragma unroll
+                    for (int h = 0; h < COH; ++h) acc[j][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[h], b[0], acc[j][h], 0, 0, 0) + t[h];
+#undef APRNET_PRODUCT
+                }
+            }
+        }
+    }
+    if constexpr (NB > 0) {
+        const __amdgpu_buffer_rsrc_t rci = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(gl.col_idx), 0, nc * 4, 0x00020000);
+        int ocol[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) ocol[j] = __builtin_amdgcn_raw_buffer_load_b32(rci, (((first + G::NWAVE * j) << 4) + (lane & 15)) * 4, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const int col = ((first + G::NWAVE * j) << 4) + (lane & 15);
+            if (col >= nc) continue;
+            float t = 0.f;              // stays 0 unless one of the sums is infinite or NaN
+#pragma unroll
+            for (int h = 0; h < COH; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) t = fmaf(acc[j][h][r], 0.f, t);
+            if (t != 0.f) mark[0] = mark[split_mark(blockIdx.y * gridDim.x + blockIdx.x)] = 1;
+            float* dst = a.y + ocol[j];
+#pragma unroll
+            for (int h = 0; h < COH; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int cl = h * 16 + 4 * (lane >> 4) + r;
+                    if (co0 + cl >= a.Cout) continue;
+                    float v = acc[j][h][r] + sh.bias[cl];
+                    if (a.relu) v = v < 0.f ? 0.f : v;
+                    dst[(int64_t)(co0 + cl) * a.ldy] = v;
+                }
+        }
+    }
+}
+
+// three workgroups per CU for at most 16 outputs (80 registers), two for 32
+template <class G, int COH>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(COH == 1 ? 6 : 4, COH == 1 ? 6 : 4)))
+conv_split_kernel(const ConvArgs<float> a) {
+    constexpr int NBW = 4, NSTEP = split_steps<G>();
+    static_assert((G::MAXCOL + 15) / 16 <= G::NWAVE * NBW, "a window must fit the accumulators of the block");
+    static_assert(G::RS == 64, "the plan's lists carry cells of rows of 64");
+    __shared__ SplitShared<G, COH> sh;
+    const ConvTile tile = a.tiles[blockIdx.x];
+    const int L = tile.level;
+    const int co0 = blockIdx.y * 16 * COH;
+    const int s_idx = min(a.S_exp - 1, a.Lc - L);
+    const int nq = (a.Cin + SP_CIB - 1) / SP_CIB;
+    const uint4* __restrict__ wl = reinterpret_cast<const uint4*>(a.w) +
+                                   ((int64_t)s_idx * gridDim.y + blockIdx.y) * nq * (NSTEP * 3 * COH * 64);
+    const int wave = threadIdx.x >> 6;
+    const bool tree_items = L < a.Lc;
+
+    if (threadIdx.x < 16 * COH)
+        sh.bias[threadIdx.x] = (a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
+    if (threadIdx.x < NSTEP * 4) {
+        int o[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            int t = SplitTaps<G::K>::tap[2 * threadIdx.x + h];
+            if (t < 0) t = max((int)SplitTaps<G::K>::tap[2 * (threadIdx.x ^ 1) + h], 0);       // no tap (zero weights): the other group's cells
+            o[h] = (((t / (G::KX * G::KY)) * G::RX + (t / G::KY) % G::KX) * G::RS + t % G::KY) * 8;
+        }
+        sh.toff[threadIdx.x] = make_int2(o[0], o[1]);
+    }
+    const int wb = a.tile_win[blockIdx.x], we = a.tile_win[blockIdx.x + 1];
+    for (int w = wb; w < we; ++w) {
+        const int win = w - wb;
+        if ((win & 15) == 0) {                // every wave is past the previous window's last barrier
+            if (threadIdx.x < 16 && w + (int)threadIdx.x < we) sh.hdr[threadIdx.x] = a.win[w + threadIdx.x];
+            __syncthreads();
+        }
+        const int4 hd = sh.hdr[win & 15];
+        const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+        const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
+        const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
+        const int nblk = (nc + 15) >> 4;
+        const int first = (wave - (int)blockIdx.x - win) & (G::NWAVE - 1);
+        const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
+        switch (__builtin_amdgcn_readfirstlane(nb)) {
+            case 0: split_window<G, COH, 0>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 1: split_window<G, COH, 1>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 2: split_window<G, COH, 2>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 3: split_window<G, COH, 3>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            default: split_window<G, COH, 4>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+        }
+        __syncthreads();        // the next window rewrites the patch
+    }
+}
+
+// The marked tiles from the fp32 values: one thread per column, one channel of the input staged at a time.  Rare and slow; a
+// block that finds no mark set ends at once.
+template <class G>
+__global__ void __launch_bounds__(G::NT)
+conv_split_redo_kernel(const ConvArgs<float> a, int n_tiles, int n_cb, int per) {
+    static_assert(G::MAXCOL <= G::NT, "one thread per column");
+    __shared__ float patch[G::CH_STRIDE];
+    if (a.redo[0] == 0) return;
+    for (int u = blockIdx.x; u < n_tiles * n_cb; u += gridDim.x) {          // uniform
+        if (a.redo[split_mark(u)] == 0) continue;
+        const int tile = u % n_tiles, co0 = u / n_tiles * per, co1 = min(co0 + per, a.Cout);
+        const float* __restrict__ w = a.w_raw + (int64_t)min(a.S_exp - 1, a.Lc - a.tiles[tile].level) * a.Cout * a.Cin * G::K;
+        for (int win = a.tile_win[tile]; win < a.tile_win[tile + 1]; ++win) {
+            const int4 hd = a.win[win];
+            const WindowLists l{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z, a.l_col_pos + (unsigned)hd.z};
+            const int col = threadIdx.x, nc = hd.w;
+            const int cell = (col < nc ? (int)(l.col_pos[col] & COL_CELL) : G::TAP0) - G::TAP0;
+#pragma unroll 1
+            for (int m0 = co0; m0 < co1; m0 += 8) {
+                float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+                for (int ci = 0; ci < a.Cin; ++ci) {
+                    __syncthreads();
+                    for (int i = threadIdx.x; i < G::CH_STRIDE; i += G::NT) patch[i] = 0.f;
+                    __syncthreads();
+                    const float* plane = (a.x2 && ci >= a.c_split) ? a.x2 + (int64_t)(ci - a.c_split) * a.ldx2 : a.x + (int64_t)ci * a.ldx;
+                    for (int i = threadIdx.x; i < hd.y; i += G::NT) {
+                        const unsigned pos = l.item_pos[i];
+                        const float v = (pos & ITEM_TREE) ? a.tree_data[(int64_t)ci * a.ldt + l.item_idx[i]] : plane[l.item_idx[i]];
+                        patch[pos & ITEM_CELL] = v;
+                        if (pos & ITEM_PAIR) patch[(pos & ITEM_CELL) + 1] = v;
+                    }
+                    __syncthreads();
+#pragma unroll 1
+                    for (int t = 0; t < G::K; ++t) {
+                        const float v = patch[cell + ((t / (G::KX * G::KY)) * G::RX + (t / G::KY) % G::KX) * G::RS + t % G::KY];
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) acc[k] += w[((int64_t)min(m0 + k, a.Cout - 1) * a.Cin + ci) * G::K + t] * v;
+                    }
+                }
+                if (col >= nc) continue;
+                const int64_t o = l.col_idx[col];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    if (m0 + k >= co1) continue;
+                    float v = acc[k] + (a.bias ? a.bias[m0 + k] : 0.f);
+                    if (a.relu) v = v < 0.f ? 0.f : v;
+                    a.y[(int64_t)(m0 + k) * a.ldy + o] = v;
+                }
+            }
+        }
+    }
+}
+
+using S333 = ConvGeom<3, 3, 3, 2, 4, 512, 64, 16>;
+using S155 = ConvGeom<1, 5, 5, 1, 8, 512, 64, 16>;
+
+static int split_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
+static int split_nstep(int code) { return code == 333 ? split_steps<S333>() : split_steps<S155>(); }
+
+template <class G>
+static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+    const int coh = split_coh(a.Cout), n_cb = (a.Cout + 16 * coh - 1) / (16 * coh);
+    dim3 grid((unsigned)n_tiles, (unsigned)n_cb);
+    if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1>), grid, dim3(G::NT), 0, st, a);
+    else hipLaunchKernelGGL((conv_split_kernel<G, 2>), grid, dim3(G::NT), 0, st, a);
+    APRNET_LAUNCH_CHECK("conv_split_kernel");
+    hipLaunchKernelGGL(conv_split_redo_kernel<G>, dim3((unsigned)std::min(n_tiles * n_cb, 256)), dim3(G::NT), 0, st, a, n_tiles, n_cb, 16 * coh);
+    APRNET_LAUNCH_CHECK("conv_split_redo_kernel");
+    return 0;
+}
+// a.w = image of pack_conv_weights_split, a.w_raw = the weights it was made from, a.redo = the marks that it cleared,
+// a.xi / a.ti = copies of group4_f32 of what a.x, a.x2 and a.tree_data hold, a.tile_win ... the forward lists of the plan
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+    switch (code) {
+        case 333: return launch_split<S333>(a, n_tiles, st);
+        case 155: return launch_split<S155>(a, n_tiles, st);
+    }
+    return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
+}
+// x (and x2 from channel c_split on) -> out[(C + 3) / 4][count][4]
+int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st) {
+    if (count <= 0 || C <= 0) return 0;
+    dim3 grid((unsigned)((count + IG_TB * IG_E - 1) / (IG_TB * IG_E)), (unsigned)((C + SP_CIB - 1) / SP_CIB));
+    hipLaunchKernelGGL(group4_kernel, grid, dim3(IG_TB), 0, st, x, ldx, x2, ldx2, c_split, C, count, (float4*)out);
+    APRNET_LAUNCH_CHECK("group4_kernel");
+    return 0;
+}
+size_t split_mark_bytes() { return SPLIT_MARKS * sizeof(int); }
+size_t conv_packed_split_bytes(int code, int S_exp, int Cout, int Cin) {
+    const int coh = split_coh(Cout);
+    return (size_t)S_exp * ((Cout + 16 * coh - 1) / (16 * coh)) * ((Cin + SP_CIB - 1) / SP_CIB) * split_nstep(code) * 3 * coh * 64 * sizeof(uint4);
+}
+int pack_conv_weights_split(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, int* marks, hipStream_t st) {
+    const size_t n = conv_packed_split_bytes(code, S_exp, Cout, Cin) / (3 * sizeof(uint4));
+    if (n >= ((size_t)1 << 29)) return fail(APRNET_ERR_UNSUPPORTED, "packed weight image of 2^31 elements or more");
+    dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 2048));
+#define APRNET_PACK(K) hipLaunchKernelGGL(pack_weights_split_kernel<K>, grid, dim3(256), 0, st, w, S_exp, Cout, Cin, split_coh(Cout), (uint4*)packed, marks)
+    if (code == 333) APRNET_PACK(27); else APRNET_PACK(25);
+#undef APRNET_PACK
+    APRNET_LAUNCH_CHECK("pack_weights_split_kernel");
+    return 0;
+}
+
+}  // namespace aprnet

@@ -118,6 +118,10 @@ def hip():
     for t in ("f32", "f64", "bf16"):      # ..., tree_ws, ld_tree, const aprnet_conv_fusion*, stream
         getattr(lib, f"aprnet_conv_fwd_fused_{t}").argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, vp, i32, i32, vp, vp, i64,
                                                                 vp, i64, vp, vp]
+    lib.aprnet_conv_ws_bytes_f32.argtypes = [vp, i32, i32, i32, i32, i32, i32, i32]
+    lib.aprnet_conv_ws_bytes_f32.restype = i64
+    # aprnet_conv_fwd_fused_f32 with an optional work space in front of the stream
+    lib.aprnet_conv_fwd_ws_f32.argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, vp, i32, i32, vp, vp, i64, vp, i64, vp, vp, i64, vp]
     lib.aprnet_conv111_fwd_bf16.argtypes = [vp, i32, vp, i64, i32, vp, i32, i32, vp, vp, i64, vp]
     lib.aprnet_conv111_bwd_bf16.argtypes = [vp, i32, vp, i64, i32, vp, i32, i32, vp, i64, vp, i64, vp, vp]
     lib.aprnet_fill_tree_mean_bf16.argtypes = [vp, i32, vp, i64, i32, vp, i64, vp]

@@ -137,13 +137,27 @@ class _Fusion(C.Structure):
                 ("x2_coarse", C.c_void_p), ("ld_coarse", C.c_int64)]
 
 
-def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None):
+def _workspace(nbytes, device):
+    """Optional work space of a call: (tensor, bytes), or (None, 0) when none is asked for or there is no memory for it (the
+    call then runs without)."""
+    if nbytes <= 0:
+        return None, 0
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
+    except torch.cuda.OutOfMemoryError:
+        return None, 0
+
+
+def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, pieces=True):
     """conv333_forward / conv111_forward (wrap_conv_gpu.hpp:32-66, 170-193) for any supported stencil.
     weights: [S_exp, Cout, Cin, kz, kx, ky] (for 1x1x1: [S, Cout, Cin, 1, 1, 1], not expanded).
     bias ([Cout], optional) is added inside the kernel instead of in a separate pass over the output.
     relu: the result is clamped at zero in the kernel (the ReLU of BasicBlock, unet_parts.py:17-26).
     x2 ([B, C2, N], optional): the kernel reads its channels after those of x, which stands for
-    conv(torch.cat([x, x2], dim=1)) (unet_parts.py:82) without writing the concatenated tensor."""
+    conv(torch.cat([x, x2], dim=1)) (unet_parts.py:82) without writing the concatenated tensor.
+    pieces: fp32 features may be multiplied as bfloat16 pieces (smaller error, another order of the sums).  A forward pass that is
+    recorded for a backward one does without: a sign or pooled maximum that tips over moves whole gradients, and the sums of
+    training runs stay those of the fp32 instructions bit for bit (a training step of a U-Net gains 2 % from it, its inference 25 %)."""
     _check_input(x, "input")
     _check_input(weights, "weights")
     c2 = 0
@@ -186,7 +200,17 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None):
     sfx = _sfx(x, bf16=True)
     with torch.cuda.device(x.device):
         st = _stream()
-        if fused:
+        if sfx == "f32" and pieces and (kz, kx, ky) != (1, 1, 1):
+            ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
+            tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
+            ws, ws_bytes = _workspace(max(_lib().aprnet_conv_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout) for b in range(B)), x.device)
+            for b in range(B):
+                fu = _Fusion(_ptr(x2[b]) if x2 is not None else None, N, c2, 1 if relu else 0)
+                rc = _lib().aprnet_conv_fwd_ws_f32(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, c1, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N,
+                                                   _ptr(tree_ws), ld_tree, C.byref(fu) if fused else None, _optr(ws), ws_bytes, st)
+                if rc:
+                    _raise(rc, "conv_forward failed")
+        elif fused:
             ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
             tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             fn = getattr(_lib(), "aprnet_conv_fwd_fused_" + sfx)

@@ -33,7 +33,7 @@ def _from_device_layout(w, layout):
 
 class ConvFunction(Function):
     @staticmethod
-    def forward(ctx, inputs, weights, bias, aprs, level_deltas, layout):
+    def forward(ctx, inputs, weights, bias, aprs, level_deltas, layout, recorded=True):
         ctx.aprs = aprs
         ctx.layout = layout
         ctx.param_dtypes = (weights.dtype, None if bias is None else bias.dtype)
@@ -51,7 +51,7 @@ class ConvFunction(Function):
         inputs = inputs.contiguous()
         ctx.save_for_backward(inputs, w, bias, level_deltas.clone())
         # the bias add of conv.py:101 is fused into the kernel's store
-        return _ops.conv_forward(aprs, inputs, w, level_deltas, None if bias is None else bias.contiguous())
+        return _ops.conv_forward(aprs, inputs, w, level_deltas, None if bias is None else bias.contiguous(), pieces=not recorded)
 
     @staticmethod
     def backward(ctx, grad_output):
@@ -65,7 +65,7 @@ class ConvFunction(Function):
         grad_w = _from_device_layout(grad_w, ctx.layout).to(ctx.param_dtypes[0])     # fp32 sums for bfloat16 features
         if grad_bias is not None:
             grad_bias = grad_bias.to(ctx.param_dtypes[1])
-        return grad_input, grad_w, grad_bias, None, None, None
+        return grad_input, grad_w, grad_bias, None, None, None, None
 
 
 def conv_inference(inputs, weights, bias, aprs, level_deltas, layout, relu=False, inputs2=None, kept_stencils=None):

@@ -47,7 +47,7 @@ class APRConv(nn.Module):
             init.uniform_(self.bias, -bound, bound)
 
     def forward(self, input_features, aprs, level_deltas):
-        return ConvFunction.apply(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout)
+        return ConvFunction.apply(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout, torch.is_grad_enabled())
 
     def forward_fused(self, input_features, aprs, level_deltas, relu=False, second_input=None):
         """Inference-only forward (no autograd record): optionally clamps the result at zero inside the kernel and

@@ -125,6 +125,8 @@ int aprnet_profile_enable(int on);
  * stencil convolution, forward or backward, and the hand-down of the tree's gradient that follows a backward one: 16 = the
  * nodes that the forward kernel's window lists read, and their descendants (default; the node lists are built with the
  * window lists and kept in the plan, 4 bytes per needed node), 17 = every node.
+ * And for fp32 features where the caller gives a work space (aprnet_conv_fwd_ws_f32): 18 = products of bfloat16 pieces
+ * where that is faster (default), 19 = fp32 matrix instructions, 20 = products of pieces at any size.
  * All are HIP kernels; the switch
  * exists so that tests can cover them and memory-bound callers can do without the lists. */
 int aprnet_set_conv_path(int path);
@@ -233,6 +235,18 @@ typedef struct aprnet_conv_fusion {
 
 APRNET_DECL(float, f32)
 APRNET_DECL(double, f64)
+
+/* No counterpart in the reference.  Stencil convolutions of fp32 features with an optional work space of the caller, in which the
+ * forward pass keeps its packed weights and copies of its input and mean tree in groups of four channels: with at least
+ * aprnet_conv_ws_bytes_f32() bytes (16-byte aligned, contents irrelevant before and after) it multiplies pieces of the fp32 values on the
+ * bfloat16 matrix instructions (every value as the exact sum of three bfloat16 numbers, all products above 2^-25 of the result,
+ * fp32 sums: an error no larger than that of the fp32 instructions); with less, or NULL, it is aprnet_conv_fwd_fused_f32.
+ * aprnet_conv_ws_bytes_f32: Cin counts both inputs; 0 where the layer does not take that path (fewer than 16 input channels, little
+ * work, 2^28 particles and more, 1x3x3, 5x5x5 and 1x1x1 stencils). */
+int64_t aprnet_conv_ws_bytes_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, int Cin, int S_exp, int Cout);
+int aprnet_conv_fwd_ws_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
+                           const float* w, int S_exp, int Cout, const float* bias, float* y, int64_t ldy, float* tree_ws,
+                           int64_t ld_tree, const aprnet_conv_fusion* fusion, void* ws, int64_t ws_bytes, void* stream);
 
 /* bfloat16 features (uint16_t bit patterns; no counterpart in the reference, which has no 16-bit path).
  * Values are widened to fp32 on load, accumulated in fp32 and rounded to nearest even on store.  Weights

@@ -1,0 +1,155 @@
+"""Stencil convolution of fp32 features on products of bfloat16 pieces, against the oracle in float64, the fp32 matrix
+instructions and the scanning kernels."""
+
+import pytest
+import torch
+
+from oracle import oracle
+from pyapr import _native
+from pyapr.aprnet import _ops
+from test_gpu_parity import DEV, _conv_case, close
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def path():
+    lib = _native.hip()
+    yield lambda p: lib.aprnet_set_conv_path(p)
+    for p in (18, 4, 0):
+        lib.aprnet_set_conv_path(p)
+
+
+def layer(w_exp):
+    return w_exp.permute(1, 2, 0, 3, 4, 5).contiguous().to(DEV)          # -> [S, Cout, Cin, k]
+
+
+def error(got, ref):
+    return float((got.cpu().double() - ref).norm() / ref.norm())
+
+
+# 16 and 17 outputs: either side of a block of output channels; 18 and 19 inputs: incomplete groups of four
+@pytest.mark.parametrize("cin,cout", [(16, 1), (18, 16), (19, 17), (32, 33), (64, 64)])
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 5, 5)], ids=["k333", "k155"])
+@pytest.mark.parametrize("bt", [[("3d_s", 0), ("3d_t", 1)], [("3d_c", 2)], [("2d_a", 1), ("2d_s", 0)]], ids=["3d", "3d_coarse", "2d"])
+def test_against_float64(path, bt, ksize, cin, cout):
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, cin, cout, torch.float32)
+    ref = oracle.conv_forward(aprs, x.double(), w_exp.double(), ld)
+    xd, wd = x.to(DEV), layer(w_exp)
+    path(19)
+    fp32 = _ops.conv_forward(aprs, xd, wd, ld)
+    path(20)
+    got = _ops.conv_forward(aprs, xd, wd, ld)
+    assert not torch.equal(got, fp32)                                    # the other kernel ran
+    close(got, ref.float(), torch.float32)
+    # six products of pieces leave out less than 2^-25 of |x w| and a sum is rounded twice per 32 products, not once per product: no
+    # larger an error than that of the fp32 products
+    assert error(got, ref) <= error(fp32, ref)
+    assert torch.equal(got, _ops.conv_forward(aprs, xd, wd, ld))         # no atomics
+    # the input in two tensors, bias and ReLU
+    b = torch.linspace(-1, 1, cout)
+    c1 = cin - 5
+    y = _ops.conv_forward(aprs, xd[:, :c1].contiguous(), wd, ld, b.to(DEV), relu=True, x2=xd[:, c1:].contiguous())
+    for i, a in enumerate(aprs):
+        n = oracle.number_parts(a, int(ld[i]))
+        assert torch.equal(y[i, :, :n], (got[i, :, :n] + b.to(DEV)[:, None]).relu())
+
+
+@pytest.mark.parametrize("cout", [3, 32, 40])
+@pytest.mark.parametrize("where", ["features", "weights"])
+def test_infinities_and_nan(path, where, cout):
+    """A result that is not finite is computed again from the fp32 values: infinities and NaN where IEEE arithmetic has
+    them, and nowhere else; values whose first bfloat16 piece is infinite give the finite result."""
+    x, aprs, ld, w_exp = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, cout, torch.float32)
+    w_exp = w_exp * 1e-3
+    inf = float("inf")
+    if where == "features":
+        n = oracle.number_parts(aprs[0], 0)
+        for i, v in enumerate((inf, -inf, float("nan"), 3.4e38, -3.4e38)):
+            x[0, 3 * i, (n * (i + 1)) // 7] = v
+        w_exp[0] = 0.0                                                   # infinity times zero
+    else:
+        w_exp[2, 0, 1, 0, 1, 2], w_exp[5, -1, 0, 1, 1, 1], w_exp[7, 0, 2, 2, 2, 2] = inf, float("nan"), 3.4e38
+        x[:, 7] *= 1e-6
+    ref = oracle.conv_forward(aprs, x.double(), w_exp.double(), ld)
+    path(20)
+    got = _ops.conv_forward(aprs, x.to(DEV), layer(w_exp), ld).cpu()
+    assert torch.equal(got.isnan(), ref.isnan())
+    assert torch.equal(got[ref.isinf()].double(), ref[ref.isinf()])
+    fin = ref.isfinite()
+    assert fin.any() and not fin.all()
+    # 432 products of size |x| max |w|, one rounding (2^-24) each
+    big = float(x[x.isfinite()].abs().max()) * float(w_exp[w_exp.isfinite()].abs().max())
+    assert bool(got[fin].isfinite().all())
+    assert float((got[fin].double() - ref[fin]).abs().max()) <= 432 * 2.0 ** -24 * min(big, 3.4e38)
+
+
+def test_route_by_work_space(path):
+    """Little work, the 1x3x3 stencil and few channels ask for no work space; with too small a one, none, or lists switched off the
+    call is the fp32 kernel's, bit for bit."""
+    lib = _native.hip()
+    x, aprs, ld, w_exp = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
+    xd, wd, a = x.to(DEV), layer(w_exp), aprs[0]
+    a.init_cuda()
+    S, n = wd.size(0), x.size(2)
+    need = lambda kz, k, cin, cout: lib.aprnet_conv_ws_bytes_f32(a.plan(0), 0, kz, k, k, cin, S, cout)
+    assert need(3, 3, 16, 16) == 0 and need(3, 3, 64, 32) == 0 and need(3, 3, 64, 4096) > 0
+    path(20)
+    assert need(1, 3, 64, 64) == 0 and need(5, 5, 64, 64) == 0 and need(3, 3, 15, 64) == 0
+    nb = need(3, 3, 16, 32)
+    assert nb > 0
+    ldt = max(_ops.tree_parts(a, 0), 1)
+
+    def run(nbytes):
+        ws = torch.empty(max(nbytes, 1) + 16, dtype=torch.uint8, device=DEV)
+        tree, y = torch.empty(16, ldt, device=DEV), torch.empty(32, n, device=DEV)
+        rc = lib.aprnet_conv_fwd_ws_f32(a.plan(0), 0, 3, 3, 3, xd.data_ptr(), n, 16, wd.data_ptr(), S, 32, None, y.data_ptr(), n, tree.data_ptr(), ldt,
+                                        None, ws.data_ptr() if nbytes else None, nbytes, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, lib.aprnet_last_error()
+        return y
+    split = run(nb)
+    path(19)
+    fp32 = run(nb)
+    path(20)
+    assert not torch.equal(split, fp32)
+    assert torch.equal(run(nb - 1), fp32) and torch.equal(run(0), fp32)
+    path(5)
+    assert torch.equal(run(nb), fp32)
+
+
+def test_under_capture(path):
+    """Recorded into a graph and replayed on new features, with eager calls in between."""
+    x, aprs, ld, w_exp = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
+    xs, wd = x.to(DEV), layer(w_exp)
+    path(20)
+    _ops.conv_forward(aprs, xs, wd, ld)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = _ops.conv_forward(aprs, xs, wd, ld)
+    for i in range(4):
+        xs.copy_(x.to(DEV) * (i + 1))
+        if i == 2:
+            xs[0, 0, 5] = float("inf")
+        want = _ops.conv_forward(aprs, xs, wd, ld)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(torch.nan_to_num(y), torch.nan_to_num(want)) and torch.equal(y.isnan(), want.isnan())
+
+
+def test_recorded_pass_keeps_the_fp32_products(path):
+    """A forward pass that a backward pass may follow is the fp32 instructions', as are its gradients."""
+    from pyapr import aprnet
+    x, aprs, ld, _ = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
+    conv, xd = aprnet.cuda.APRConv(16, 32, nstencils=2).to(DEV), x.to(DEV)
+    out = {}
+    for p in (19, 20):
+        path(p)
+        with torch.no_grad():
+            out[p, "inference"] = conv(xd, aprs, ld)
+        xg = xd.clone().requires_grad_(True)
+        out[p, "training"] = conv(xg, aprs, ld)
+        out[p, "grads"] = torch.autograd.grad(out[p, "training"].square().sum(), (conv.weight, conv.bias))
+    assert torch.equal(out[19, "training"], out[20, "training"]) and torch.equal(out[19, "inference"], out[19, "training"])
+    assert all(torch.equal(a, b) for a, b in zip(out[19, "grads"], out[20, "grads"]))
+    assert not torch.equal(out[20, "inference"], out[20, "training"])

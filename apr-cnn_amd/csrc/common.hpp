@@ -157,7 +157,7 @@ int fail(int code, const std::string& msg);
 int get_tiles(aprnet_plan* plan, int level_delta, int TZ, int TX, TileList* out, hipStream_t st, int halo = 0);
 // true while `st` records into a graph (allocation, synchronous copies and stream synchronisation are not allowed then)
 bool stream_is_capturing(hipStream_t st);
-int get_lists(aprnet_plan* plan, int level_delta, int code, const TileList& tl, WinLists* out, hipStream_t st, bool dx = false);
+int get_lists(aprnet_plan* plan, int level_delta, int code, const TileList& tl, WinLists* out, hipStream_t st, int dx = 0);
 void free_lists(WinLists& wl);
 // an idle second stream of `device` (the current device), owned by the caller until its plan is destroyed
 int side_stream_acquire(int device, hipStream_t* out);

@@ -148,11 +148,11 @@ static std::atomic<int> g_bf16_regroup{1};   // bfloat16 forward: 1 = stage from
 int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx, int C, bf16_t* tree, int64_t ldt, hipStream_t st,
                        const NeedLists* need);
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
-int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st);
+int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const int* when = nullptr);
 
 size_t split_mark_bytes();
-size_t conv_packed_split_bytes(int code, int S_exp, int Cout, int Cin);
-int pack_conv_weights_split(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, int* marks, hipStream_t st);
+size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
+int pack_conv_weights_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, hipStream_t st);
 int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st);
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
@@ -181,7 +181,7 @@ int bwd_deterministic() { return g_bwd_deterministic; }
 // Points the kernel at the plan's window lists.  When the lists are switched off, or cannot be built (no device
 // memory for them, too many entries), a.tile_win stays null and the kernel scans the access arrays itself.
 template <typename T>
-static int set_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<T>& a, hipStream_t st, bool dx = false) {
+static int set_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<T>& a, hipStream_t st, int dx = 0) {
     a.tile_win = nullptr;
     if (!g_use_lists) return 0;
     WinLists wl;
@@ -194,7 +194,9 @@ static int set_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvAr
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st) { return set_lists(p, d, code, tl, a, st); }
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st) { return set_lists(p, d, code, tl, a, st); }
 // the input-gradient lists (tl: the tile list with a halo of one row)
-int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st) { return set_lists(p, d, code, tl, a, st, true); }
+int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st) { return set_lists(p, d, code, tl, a, st, 1); }
+// without the particles on far faces
+int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st) { return set_lists(p, d, code, tl, a, st, 2); }
 
 // Channel-aware dispatch: a layer with 1 to 3 input channels is bound by memory (4 (Cin + Cout) bytes for 2 K Cin Cout
 // flops per particle) and goes to the pipelined kernel of conv_narrow.hip, which needs the plan's window lists and a
@@ -237,6 +239,18 @@ static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx
     return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cout, Cin)) + (size_t)(Cin + 3) / 4 * (size_t)(nx + nt) * 16;
 }
 
+// The same of the input gradient: packed weights and the output gradient in groups of four channels.
+// Next to the weight gradient, which bounds many of these calls, it takes more work to gain by it (whole backward pass, split against
+// fp32: 3x3x3 16 -> 16 channels on 70 k particles 224 and 220 us, on 320 k 384 and 418; 32 -> 32 on 70 k 434 and 435, on 320 k
+// 868 and 976; 64 -> 64 on 14 k 614 and 626; 1x5x5 32 -> 32 on 70 k 409 and 410, 64 -> 64 879 and 937; at 16 input channels
+// the fp32 kernel's staging of the small stencil is the faster one, 320 k 355 and 343).
+size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n) {
+    if (!g_f32_split || !g_use_lists || g_conv_path == 1 || (code != 333 && code != 155) || Cout < SPLIT_MIN_CIN || n >= (1ll << 28)) return 0;
+    if (g_f32_split == 1 && ((code == 155 && Cin <= 16) || (double)n * Cout * ((Cin + 15) / 16 * 16) < (code == 155 ? 1 << 28 : 1 << 26))) return 0;
+    if (conv_packed_split_bytes(code, S_exp, Cin, Cout) / 48 >= (1u << 29)) return 0;
+    return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cin, Cout)) + (size_t)(Cout + 3) / 4 * (size_t)n * 16;
+}
+
 template <typename T> static int try_mfma(aprnet_plan*, const ConvArgs<T>&, int, int, const TileList&, int, hipStream_t, bool*, void*, int64_t) { return 0; }
 template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int code, int d, const TileList& tl, int n_tiles,
                                 hipStream_t st, bool* done, void* ws, int64_t ws_bytes) {
@@ -252,7 +266,7 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
         const size_t wbytes = split_align(conv_packed_split_bytes(code, a.S_exp, a.Cout, a.Cin)), ng = (size_t)(a.Cin + 3) / 4;
         char* image = (char*)ws + split_mark_bytes();
         float* xi = (float*)(image + wbytes), *ti = xi + ng * (size_t)a.x_count * 4;
-        if (int rc = pack_conv_weights_split(code, a.w, a.S_exp, a.Cout, a.Cin, image, (int*)ws, st)) return rc;
+        if (int rc = pack_conv_weights_split(code, a.w, a.S_exp, a.Cout, a.Cin, false, image, (int*)ws, st)) return rc;
         if (int rc = group4_f32(a.x, a.ldx, a.x2, a.ldx2, a.c_split, a.Cin, a.x_count, xi, st)) return rc;
         if (int rc = group4_f32(a.tree_data, a.ldt, nullptr, 0, a.Cin, a.Cin, a.t_count, ti, st)) return rc;
         b.w_raw = a.w; b.w = (const float*)image; b.redo = (int*)ws;

@@ -254,7 +254,7 @@ int launch_conv_dx_mfma(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStr
 int launch_conv_dw_mfma(int code, const ConvArgs<bf16_t>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st);
 int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx, int C, bf16_t* tree, int64_t ldt, hipStream_t st, const NeedLists* need);
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
-int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st);
+int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const int* when = nullptr);
 int conv_path();
 // the tree nodes the forward window lists name, null: fill every node (conv.hip)
 const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& tl, hipStream_t st, NeedLists* store);
@@ -262,6 +262,14 @@ const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& t
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st);
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st);
 int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st);
+int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st);
+size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n);
+size_t split_mark_bytes();
+size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
+int pack_conv_weights_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, hipStream_t st);
+int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st);
+int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
+int split_clear(const int* mark, float* gx, int64_t ldgx, int64_t n, float* gtree, int64_t ldgt, int64_t nt, int C, hipStream_t st);
 int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
 size_t conv_packed_bf16_bytes(int code, int S_exp, int Cout, int Cin);
 int pack_conv_weights_bf16(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, hipStream_t st, bool transposed);
@@ -285,7 +293,7 @@ static void set_dw_partials(aprnet_plan* p, size_t off, int code, ConvArgs<T>& a
     a.gw_part_ld = (int64_t)a.Cout * a.Cin * (code == 333 ? 27 : code == 133 ? 9 : 25);
 }
 
-template <typename T> static int try_mfma_bwd(aprnet_plan*, const ConvArgs<T>&, const TileList&, int, int, hipStream_t, bool*) { return 0; }
+template <typename T> static int try_mfma_bwd(aprnet_plan*, const ConvArgs<T>&, const TileList&, int, int, hipStream_t, bool*, void*, int64_t) { return 0; }
 static int fork_side(aprnet_plan* p, hipStream_t st, hipStream_t* side);
 static int join_side(aprnet_plan* p, hipStream_t st, hipStream_t side);
 // Joins the side stream on every way out of a backward call, also the failing ones: the caller's stream must not run
@@ -296,7 +304,8 @@ struct SideJoin {
     int join() { open = false; return join_side(p, st, side); }
     ~SideJoin() { if (open) (void)join_side(p, st, side); }
 };
-template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, const TileList& tl, int code, int d, hipStream_t st, bool* done) {
+template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, const TileList& tl, int code, int d, hipStream_t st, bool* done,
+                                    void* ws, int64_t ws_bytes) {
     if (conv_path() == 1 || !conv_mfma_supported(code)) return 0;
     *done = true;
     // weight gradient on the side stream (when there is an input gradient to run next to)
@@ -311,6 +320,13 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     const bool split_faces = a.gx && bwd_deterministic();
     if (a.gx) if (int rc = get_tiles(p, d, code == 333 ? 2 : 1, code == 333 ? 4 : 8, &near, st, 1)) return rc;
     if (split_faces) if (int rc = get_face_lists(p, d, code, &faces, st)) return rc;
+    ConvArgs<float> e = a;          // input gradient on products of bfloat16 pieces: its lists
+    const size_t need = split_faces && ws ? split_dx_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count) : 0;
+    bool pieces = need > 0 && ws_bytes >= 0 && (size_t)ws_bytes >= need && near.n > 0;
+    if (pieces) {
+        if (int rc = set_conv_dx_lists(p, d, code, near, e, st)) return rc;
+        pieces = e.tile_win != nullptr;
+    }
     const size_t wbytes = a.gx ? (conv_packed_floats(code, a.S_exp, a.Cin, a.Cout, true) * sizeof(float) + 255) / 256 * 256 : 0;
     const size_t pbytes = bwd_deterministic() ? conv_dw_partial_bytes(code, a.Cout, a.Cin, a.S_exp, a.Lc, wl) : 0;
     ScratchLease lease;          // before the join guard below: its hand-over event is recorded after the join
@@ -323,8 +339,24 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     if (a.gx) {
         // input gradient: the forward kernel on the output gradient with the transposed, flipped stencil;
         // every row group within one row of an output takes part
-        if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cin, a.Cout, true, (float*)p->d_scratch, st)) return rc;
+        int* mark = nullptr;
+        if (pieces) {
+            // on products of bfloat16 pieces (conv_split.hip), from a copy of the output gradient in groups of four channels; what
+            // follows then runs only if a sum was not finite, and does all of it again
+            char* image = (char*)ws + split_mark_bytes();
+            float* gi = (float*)(image + (conv_packed_split_bytes(code, a.S_exp, a.Cin, a.Cout) + 255) / 256 * 256);
+            mark = (int*)ws;
+            if (int rc = pack_conv_weights_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, st)) return rc;
+            if (int rc = group4_f32(a.gy, a.ldy, nullptr, 0, a.Cout, a.Cout, a.x_count, gi, st)) return rc;
+            e.tiles = near.d_tiles; e.n_tiles = near.n;
+            e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
+            e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
+            if (int rc = launch_conv_dx_split(code, e, near.n, st)) return rc;
+            if (int rc = split_clear(mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin, st)) return rc;
+        }
+        if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cin, a.Cout, true, (float*)p->d_scratch, st, mark)) return rc;
         ConvArgs<float> b = a;
+        b.redo = mark;
         b.tiles = near.d_tiles; b.n_tiles = near.n;
         b.x = a.gy; b.ldx = a.ldy; b.Cin = a.Cout; b.Cout = a.Cin; b.w = (const float*)p->d_scratch; b.bias = nullptr;
         b.tree_data = nullptr; b.t_count = 0;
@@ -366,8 +398,9 @@ static int join_side(aprnet_plan* p, hipStream_t st, hipStream_t side) {
 template <typename T>
 int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, int64_t ldx, int Cin, const T* w, int S_exp,
              int Cout, const T* gy, int64_t ldy, T* gx, int64_t ldgx, T* gw, T* tree_ws, int64_t ldt, T* gtree_ws,
-             int64_t ldgt, hipStream_t st) {
+             int64_t ldgt, hipStream_t st, void* ws = nullptr, int64_t ws_bytes = 0) {
     aprnet_plan* p = const_cast<aprnet_plan*>(cp);
+    if (ws && ((uintptr_t)ws & 15) != 0) return fail(APRNET_ERR_INVALID_ARGUMENT, "conv_backward: the work space is not aligned to 16 bytes");
     if (int rc = check_level_delta(p, d, "conv_backward")) return rc;
     if (int rc = check_plane_size(p, d, sizeof(*x), "conv_backward")) return rc;
     if (int rc = check_rows(ldx, p->number_parts(d), "conv_backward", "input")) return rc;
@@ -403,7 +436,7 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
         constexpr bool f32 = sizeof(T) == 4;
         int rc = 0;
         bool done = false;
-        if ((rc = try_mfma_bwd<T>(p, a, tl, code, d, st, &done))) return rc;
+        if ((rc = try_mfma_bwd<T>(p, a, tl, code, d, st, &done, ws, ws_bytes))) return rc;
         if (!done) switch (code) {
             case 333: rc = launch_bwd<T, X333, (f32 ? 4 : 2), W333, (f32 ? 8 : 4), (f32 ? 32 : 16)>(a, st); break;
             case 133: rc = launch_bwd<T, X133, (f32 ? 8 : 4), W133, (f32 ? 8 : 4), (f32 ? 32 : 16)>(a, st); break;
@@ -599,6 +632,16 @@ int aprnet_conv_bwd_f32(const aprnet_plan* p, int d, int kz, int kx, int ky, con
                         float* gw, float* tree_ws, int64_t ldt, float* gtree_ws, int64_t ldgt, void* st) {
     return conv_bwd<float>(p, d, kz, kx, ky, x, ldx, Cin, w, S_exp, Cout, gy, ldy, gx, ldgx, gw, tree_ws, ldt, gtree_ws,
                            ldgt, (hipStream_t)st);
+}
+int64_t aprnet_conv_bwd_ws_bytes_f32(const aprnet_plan* p, int d, int kz, int kx, int ky, int Cin, int S_exp, int Cout) {
+    if (!p || d < 0 || d >= p->tree.level_max + 1 || Cin <= 0 || S_exp <= 0 || Cout <= 0 || !bwd_deterministic()) return 0;
+    return (int64_t)split_dx_bytes(kz * 100 + kx * 10 + ky, Cin, S_exp, Cout, p->number_parts(d));
+}
+int aprnet_conv_bwd_ws_f32(const aprnet_plan* p, int d, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
+                           const float* w, int S_exp, int Cout, const float* gy, int64_t ldy, float* gx, int64_t ldgx,
+                           float* gw, float* tree_ws, int64_t ldt, float* gtree_ws, int64_t ldgt, void* ws, int64_t ws_bytes, void* st) {
+    return conv_bwd<float>(p, d, kz, kx, ky, x, ldx, Cin, w, S_exp, Cout, gy, ldy, gx, ldgx, gw, tree_ws, ldt, gtree_ws,
+                           ldgt, (hipStream_t)st, ws, ws_bytes);
 }
 int aprnet_conv_bwd_f64(const aprnet_plan* p, int d, int kz, int kx, int ky, const double* x, int64_t ldx, int Cin,
                         const double* w, int S_exp, int Cout, const double* gy, int64_t ldy, double* gx, int64_t ldgx,

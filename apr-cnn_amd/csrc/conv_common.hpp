@@ -33,7 +33,7 @@ struct ConvArgs {
     const T* x2; int64_t ldx2; int c_split; int relu;
     const typename Num<T>::acc* w; int S_exp; int Cout;     // [S_exp][Cout][Cin][K]; fp32 for bfloat16 features
     const typename Num<T>::acc* w_raw;                      // the weights as the caller gave them (kernels whose `w` is a packed image)
-    int* redo;                                              // conv_split.hip: marks of the tiles to compute again
+    int* redo;                                              // conv_split.hip: marks of the tiles to compute again; null in other launches
     const typename Num<T>::acc* bias;                       // [Cout] or null
     T* y; int64_t ldy;
     const T* tree_data; int64_t ldt;
@@ -422,7 +422,7 @@ __device__ __forceinline__ void scan_window_dx(const ConvArgs<T>& a, int L, int 
     s.apr_y = a.apr.y; s.tree_y = a.tree.y; s.tree_off = (int)a.tree_off; s.yn = a.apr.y_num[L]; s.y0 = y0;
     s.tree_from_x = (L == a.Lc); s.out_tree = out_tree;
     s.z0 = z0; s.x0 = x0; s.zn = a.apr.z_num[L]; s.xn = a.apr.x_num[L]; s.pool = pool; s.group = group;
-    s.skip_faces = pool && a.dx_skip_faces != 0;
+    s.skip_faces = (pool || group) && a.dx_skip_faces != 0;
     scan_window_dx_impl<G>(s, sh);
 }
 

@@ -53,7 +53,8 @@ constexpr int STAGE_PRIO = 3;      // wave priority outside the matrix loops
 // of the stencil of the input gradient, M = input channels, contraction over (flipped tap, output channel).
 // Cm / Ck are the channel counts of the M axis and of the contracted axis.
 __global__ void pack_weights16_kernel(const float* __restrict__ w, int S_exp, int Cm, int Ck, int K, int CIB, int COH,
-                                      int transposed, float* __restrict__ out) {
+                                      int transposed, float* __restrict__ out, const int* __restrict__ when) {
+    if (when && when[0] == 0) return;
     const int Cout = transposed ? Ck : Cm, Cin = transposed ? Cm : Ck;
     const int ncb = (Cm + 16 * COH - 1) / (16 * COH), nq = (Ck + CIB - 1) / CIB;
     // 32-bit index arithmetic (the host checks that the image has fewer than 2^31 elements): 64-bit divisions made
@@ -264,6 +265,7 @@ conv_mfma16_kernel(const ConvArgs<T> a) {
     __shared__ __attribute__((aligned(16))) float Wl[CIB * G::K * 16 * COH];
     __shared__ float bias_l[16 * COH];
 
+    if (MODE == 1 && a.redo && a.redo[0] == 0) return;          // only if the products of pieces gave a sum that is not finite
     const ConvTile tile = a.tiles[blockIdx.x];
     const int L = tile.level, z0 = tile.z0, x0 = tile.x0;
     const int co0 = blockIdx.y * 16 * COH;
@@ -930,12 +932,13 @@ size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed) 
     return (size_t)S_exp * ((Cm + 16 * coh - 1) / (16 * coh)) * ((Ck + cib - 1) / cib) * cib * conv_taps(code) * 16 * coh;
 }
 
-int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st) {
+// when: null, or a word on the device that is 0 if nothing is to be packed
+int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const int* when) {
     const size_t n = conv_packed_floats(code, S_exp, Cm, Ck, transposed);
     if (n >= ((size_t)1 << 31)) return fail(APRNET_ERR_UNSUPPORTED, "packed weight image of 2^31 elements or more");
     dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 2048));
     hipLaunchKernelGGL(pack_weights16_kernel, grid, dim3(256), 0, st, w, S_exp, Cm, Ck, conv_taps(code), transposed ? DX_CIB : FWD_CIB, conv_coh(Cm),
-                       transposed ? 1 : 0, packed);
+                       transposed ? 1 : 0, packed, when);
     APRNET_LAUNCH_CHECK("pack_weights16_kernel");
     return 0;
 }

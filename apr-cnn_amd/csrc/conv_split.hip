@@ -17,16 +17,19 @@
 //
 // Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.5 (12.5) ms, 16 -> 16
 // channels 3.4 (4.1) ms; 320 k particles, 64 -> 64 channels 0.51 (0.78) ms.
+// Input gradient, whole backward pass beside the weight gradient: 23 M particles, 32 -> 32 channels 37.6 (42.5) ms, 16 -> 16 14.1
+// (15.3) ms; the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
 // Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: matrix pipes busy 46 %,
 // vector ALU 15 %, LDS 56 % of the cycles.
 // Error against 64 bits (2-norm, 16 to 128 channels): 0.37 to 0.40 of the fp32 instructions' with N(0, 1) features, 0.44 to 0.49
 // with those after a ReLU.
 //
 // Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
-// NaN), and a value within 2^-9 of the largest fp32 number has an infinite first piece.  A result that comes out infinite
-// or NaN is therefore not stored: the tile is marked, and conv_split_redo_kernel computes the marked tiles again from the fp32
-// values.  (As a call inside this kernel it cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart.)  Values below
-// 2^-110 lose low pieces to the end of the exponent range (an absolute error below 2^-133).
+// NaN), and a value within 2^-9 of the largest fp32 number has an infinite first piece.  Where a result comes out infinite or
+// NaN its tile is marked, and conv_split_redo_kernel computes the marked tiles again from the fp32 values (as a call inside this
+// kernel it cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an input gradient that
+// holds one is made again from the start by the fp32 kernel.  Values below 2^-110 lose low pieces to the end of the exponent
+// range (an absolute error below 2^-133).
 #include "conv_common.hpp"
 
 namespace aprnet {
@@ -77,13 +80,15 @@ constexpr unsigned SPLIT_MARKS = 4096;
 __device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit % (SPLIT_MARKS - 1); }
 
 // packed[s][cb][q][step][piece][h][lane] (16 bytes: two taps of four channels), cb = block of 16 * COH output channels, q = chunk
-// of four input channels.  The marks of the launch are cleared on the way.
+// of four contracted channels.  Cm / Ck: channels on the M axis / contracted; with `transposed` the image is that of the
+// input gradient's stencil (channel axes swapped, taps reversed).  The marks of the launch are cleared on the way.
 template <int K>
-__global__ void pack_weights_split_kernel(const float* __restrict__ w, int S_exp, int Cout, int Cin, int COH, uint4* __restrict__ out,
+__global__ void pack_weights_split_kernel(const float* __restrict__ w, int S_exp, int Cm, int Ck, int COH, int transposed, uint4* __restrict__ out,
                                           int* __restrict__ marks) {
     constexpr int nstep = SplitTaps<K>::STEPS;
+    const int Cout = transposed ? Ck : Cm, Cin = transposed ? Cm : Ck;
     for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < SPLIT_MARKS; i += gridDim.x * blockDim.x) marks[i] = 0;
-    const int ncb = (Cout + 16 * COH - 1) / (16 * COH), nq = (Cin + SP_CIB - 1) / SP_CIB;
+    const int ncb = (Cm + 16 * COH - 1) / (16 * COH), nq = (Ck + SP_CIB - 1) / SP_CIB;
     const unsigned n = (unsigned)S_exp * ncb * nq * nstep * COH * 64;          // (the host checks that it fits)
     for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
         unsigned r = e;
@@ -99,7 +104,8 @@ __global__ void pack_weights_split_kernel(const float* __restrict__ w, int S_exp
         for (int j = 0; j < 8; ++j) {
             const int t = SplitTaps<K>::tap[2 * (4 * step + (lane >> 4)) + (j >> 2)], ck = q * SP_CIB + (j & 3);
             v[j] = 0.f;
-            if (t >= 0 && cm < Cout && ck < Cin) v[j] = w[(((int64_t)s * Cout + cm) * Cin + ck) * K + t];
+            if (t >= 0 && cm < Cm && ck < Ck)
+                v[j] = transposed ? w[(((int64_t)s * Cout + ck) * Cin + cm) * K + (K - 1 - t)] : w[(((int64_t)s * Cout + cm) * Cin + ck) * K + t];
         }
         uint4 p[3];
         split_pair(v[0], v[1], p[0].x, p[1].x, p[2].x);
@@ -193,7 +199,23 @@ __device__ __forceinline__ void store_items_split(const SplitItems<G>& R, int ni
     }
 }
 
-template <class G, int COH, int NB>
+// sum over the columns of a coarser particle (see dx_group), lanes that lie next to each other
+template <int CTRL>
+__device__ __forceinline__ float split_dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+template <class G>
+__device__ __forceinline__ float split_group_sum(float s) {
+    s += split_dpp<0xb1>(s);                                       // lanes 1, 0, 3, 2 of each four
+    s += split_dpp<0x4e>(s);                                       // lanes 2, 3, 0, 1
+    if constexpr (dx_group<G>() == 8) s += split_dpp<0x141>(s);    // the eight mirrored
+    return s;
+}
+
+// MODE 0: forward, results stored (plus bias).  MODE 1: input gradient on the plan's input-gradient lists (items = output
+// gradient): the columns of a coarser particle are summed across lanes and the first one takes the sum along; a place that no
+// other column adds to takes a plain store, the others (one more column at most) an atomic addition.
+template <class G, int COH, int NB, int MODE>
 __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, int nc, int nitem, bool tree_items, int first,
                                              const uint4* __restrict__ wl, const WindowLists& gl, int* __restrict__ mark, SplitShared<G, COH>& sh) {
     constexpr int NSTEP = split_steps<G>(), NBA = NB > 0 ? NB : 1;
@@ -283,37 +305,63 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     }
     if constexpr (NB > 0) {
         const __amdgpu_buffer_rsrc_t rci = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(gl.col_idx), 0, nc * 4, 0x00020000);
-        int ocol[NB];
-#pragma unroll
-        for (int j = 0; j < NB; ++j) ocol[j] = __builtin_amdgcn_raw_buffer_load_b32(rci, (((first + G::NWAVE * j) << 4) + (lane & 15)) * 4, 0, 0);
+        int ocol[NB], cpos[NB];
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             const int col = ((first + G::NWAVE * j) << 4) + (lane & 15);
+            ocol[j] = __builtin_amdgcn_raw_buffer_load_b32(rci, col * 4, 0, 0);
+            cpos[j] = MODE == 1 ? (int)__builtin_amdgcn_raw_buffer_load_b16(rcp, col * 2, 0, 0) : 0;
+        }
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            const int col = ((first + G::NWAVE * j) << 4) + (lane & 15);
+            if constexpr (MODE == 1) {
+                const bool boxed = (cpos[j] & (int)COL_BOX) != 0;
+                if (__ballot(boxed)) {
+#pragma unroll
+                    for (int h = 0; h < COH; ++h)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const float s = split_group_sum<G>(acc[j][h][r]);
+                            acc[j][h][r] = boxed ? s : acc[j][h][r];
+                        }
+                }
+                if (boxed && (lane & (dx_group<G>() - 1)) != 0) continue;
+            }
             if (col >= nc) continue;
             float t = 0.f;              // stays 0 unless one of the sums is infinite or NaN
 #pragma unroll
             for (int h = 0; h < COH; ++h)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) t = fmaf(acc[j][h][r], 0.f, t);
-            if (t != 0.f) mark[0] = mark[split_mark(blockIdx.y * gridDim.x + blockIdx.x)] = 1;
-            float* dst = a.y + ocol[j];
+            if (t != 0.f) {
+                mark[0] = 1;
+                if constexpr (MODE == 0) mark[split_mark(blockIdx.y * gridDim.x + blockIdx.x)] = 1;
+            }
+            const bool to_tree = (cpos[j] & (int)COL_TREE) != 0, sole = (cpos[j] & (int)COL_SOLE) != 0;
+            float* dst = (MODE == 0 ? a.y : to_tree ? a.gtree : a.gx) + ocol[j];
+            const int64_t ld = MODE == 0 ? a.ldy : to_tree ? a.ldgt : a.ldgx;
 #pragma unroll
             for (int h = 0; h < COH; ++h)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int cl = h * 16 + 4 * (lane >> 4) + r;
                     if (co0 + cl >= a.Cout) continue;
-                    float v = acc[j][h][r] + sh.bias[cl];
-                    if (a.relu) v = v < 0.f ? 0.f : v;
-                    dst[(int64_t)(co0 + cl) * a.ldy] = v;
+                    float v = acc[j][h][r];
+                    if constexpr (MODE == 0) {
+                        v += sh.bias[cl];
+                        if (a.relu) v = v < 0.f ? 0.f : v;
+                        dst[(int64_t)(co0 + cl) * ld] = v;
+                    } else if (sole) dst[(int64_t)(co0 + cl) * ld] = v;
+                    else unsafeAtomicAdd(dst + (int64_t)(co0 + cl) * ld, v);
                 }
         }
     }
 }
 
 // three workgroups per CU for at most 16 outputs (80 registers), two for 32
-template <class G, int COH>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(COH == 1 ? 6 : 4, COH == 1 ? 6 : 4)))
+template <class G, int COH, int MODE>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(COH == 1 && MODE == 0 ? 6 : 4, COH == 1 && MODE == 0 ? 6 : 4)))
 conv_split_kernel(const ConvArgs<float> a) {
     constexpr int NBW = 4, NSTEP = split_steps<G>();
     static_assert((G::MAXCOL + 15) / 16 <= G::NWAVE * NBW, "a window must fit the accumulators of the block");
@@ -327,10 +375,10 @@ conv_split_kernel(const ConvArgs<float> a) {
     const uint4* __restrict__ wl = reinterpret_cast<const uint4*>(a.w) +
                                    ((int64_t)s_idx * gridDim.y + blockIdx.y) * nq * (NSTEP * 3 * COH * 64);
     const int wave = threadIdx.x >> 6;
-    const bool tree_items = L < a.Lc;
+    const bool tree_items = MODE == 0 && L < a.Lc;       // the output gradient has no tree part
 
     if (threadIdx.x < 16 * COH)
-        sh.bias[threadIdx.x] = (a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
+        sh.bias[threadIdx.x] = (MODE == 0 && a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
     if (threadIdx.x < NSTEP * 4) {
         int o[2];
 #pragma unroll
@@ -356,11 +404,11 @@ conv_split_kernel(const ConvArgs<float> a) {
         const int first = (wave - (int)blockIdx.x - win) & (G::NWAVE - 1);
         const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
         switch (__builtin_amdgcn_readfirstlane(nb)) {
-            case 0: split_window<G, COH, 0>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            case 1: split_window<G, COH, 1>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            case 2: split_window<G, COH, 2>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            case 3: split_window<G, COH, 3>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            default: split_window<G, COH, 4>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 0: split_window<G, COH, 0, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 1: split_window<G, COH, 1, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 2: split_window<G, COH, 2, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            case 3: split_window<G, COH, 3, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+            default: split_window<G, COH, 4, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
         }
         __syncthreads();        // the next window rewrites the patch
     }
@@ -426,13 +474,14 @@ using S155 = ConvGeom<1, 5, 5, 1, 8, 512, 64, 16>;
 static int split_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
 static int split_nstep(int code) { return code == 333 ? split_steps<S333>() : split_steps<S155>(); }
 
-template <class G>
+template <class G, int MODE>
 static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     const int coh = split_coh(a.Cout), n_cb = (a.Cout + 16 * coh - 1) / (16 * coh);
     dim3 grid((unsigned)n_tiles, (unsigned)n_cb);
-    if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1>), grid, dim3(G::NT), 0, st, a);
-    else hipLaunchKernelGGL((conv_split_kernel<G, 2>), grid, dim3(G::NT), 0, st, a);
+    if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1, MODE>), grid, dim3(G::NT), 0, st, a);
+    else hipLaunchKernelGGL((conv_split_kernel<G, 2, MODE>), grid, dim3(G::NT), 0, st, a);
     APRNET_LAUNCH_CHECK("conv_split_kernel");
+    if (MODE == 1) return 0;
     hipLaunchKernelGGL(conv_split_redo_kernel<G>, dim3((unsigned)std::min(n_tiles * n_cb, 256)), dim3(G::NT), 0, st, a, n_tiles, n_cb, 16 * coh);
     APRNET_LAUNCH_CHECK("conv_split_redo_kernel");
     return 0;
@@ -441,10 +490,32 @@ static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
 // a.xi / a.ti = copies of group4_f32 of what a.x, a.x2 and a.tree_data hold, a.tile_win ... the forward lists of the plan
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     switch (code) {
-        case 333: return launch_split<S333>(a, n_tiles, st);
-        case 155: return launch_split<S155>(a, n_tiles, st);
+        case 333: return launch_split<S333, 0>(a, n_tiles, st);
+        case 155: return launch_split<S155, 0>(a, n_tiles, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
+}
+// Input gradient: a.x / a.xi / a.Cin describe the output gradient, a.Cout the layer's input channels, a.w the transposed image,
+// a.tile_win ... the input-gradient lists of the plan without the particles on far faces.  a.redo[0] is set if a sum is not finite.
+int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+    switch (code) {
+        case 333: return launch_split<S333, 1>(a, n_tiles, st);
+        case 155: return launch_split<S155, 1>(a, n_tiles, st);
+    }
+    return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
+}
+// Rows of zeros in gx and gtree if the mark is set: what was added there is summed again.
+__global__ void split_clear_kernel(const int* __restrict__ mark, float* __restrict__ gx, int64_t ldgx, int64_t n, float* __restrict__ gtree, int64_t ldgt, int64_t nt, int C) {
+    if (mark[0] == 0) return;
+    for (int c = 0; c < C; ++c) {
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) gx[c * ldgx + i] = 0.f;
+        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nt; i += (int64_t)gridDim.x * blockDim.x) gtree[c * ldgt + i] = 0.f;
+    }
+}
+int split_clear(const int* mark, float* gx, int64_t ldgx, int64_t n, float* gtree, int64_t ldgt, int64_t nt, int C, hipStream_t st) {
+    hipLaunchKernelGGL(split_clear_kernel, dim3(256), dim3(256), 0, st, mark, gx, ldgx, n, gtree, ldgt, nt, C);
+    APRNET_LAUNCH_CHECK("split_clear_kernel");
+    return 0;
 }
 // x (and x2 from channel c_split on) -> out[(C + 3) / 4][count][4]
 int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st) {
@@ -455,15 +526,16 @@ int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c
     return 0;
 }
 size_t split_mark_bytes() { return SPLIT_MARKS * sizeof(int); }
-size_t conv_packed_split_bytes(int code, int S_exp, int Cout, int Cin) {
-    const int coh = split_coh(Cout);
-    return (size_t)S_exp * ((Cout + 16 * coh - 1) / (16 * coh)) * ((Cin + SP_CIB - 1) / SP_CIB) * split_nstep(code) * 3 * coh * 64 * sizeof(uint4);
+// Cm: channels on the M axis of the kernel, Ck: contracted channels (forward: Cout, Cin; transposed: Cin, Cout)
+size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck) {
+    const int coh = split_coh(Cm);
+    return (size_t)S_exp * ((Cm + 16 * coh - 1) / (16 * coh)) * ((Ck + SP_CIB - 1) / SP_CIB) * split_nstep(code) * 3 * coh * 64 * sizeof(uint4);
 }
-int pack_conv_weights_split(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, int* marks, hipStream_t st) {
-    const size_t n = conv_packed_split_bytes(code, S_exp, Cout, Cin) / (3 * sizeof(uint4));
+int pack_conv_weights_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, hipStream_t st) {
+    const size_t n = conv_packed_split_bytes(code, S_exp, Cm, Ck) / (3 * sizeof(uint4));
     if (n >= ((size_t)1 << 29)) return fail(APRNET_ERR_UNSUPPORTED, "packed weight image of 2^31 elements or more");
     dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 2048));
-#define APRNET_PACK(K) hipLaunchKernelGGL(pack_weights_split_kernel<K>, grid, dim3(256), 0, st, w, S_exp, Cout, Cin, split_coh(Cout), (uint4*)packed, marks)
+#define APRNET_PACK(K) hipLaunchKernelGGL(pack_weights_split_kernel<K>, grid, dim3(256), 0, st, w, S_exp, Cm, Ck, split_coh(Cm), transposed ? 1 : 0, (uint4*)packed, marks)
     if (code == 333) APRNET_PACK(27); else APRNET_PACK(25);
 #undef APRNET_PACK
     APRNET_LAUNCH_CHECK("pack_weights_split_kernel");

@@ -134,9 +134,10 @@ void free_lists(WinLists& wl) {
 
 // Lists of the forward convolution at `level_delta` for stencil `code` (333, 133, 155); `tl` must be the tile list
 // of the same stencil.  Built on first use (synchronises the stream and allocates), then served from the plan.
-// dx: the lists of the input gradient instead; `tl` is then the tile list with a halo of one row.
-int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, WinLists* out, hipStream_t st, bool dx) {
-    auto key = std::make_pair(level_delta, code + (dx ? 1000 : 0));
+// dx: 1 = the lists of the input gradient instead, `tl` is then the tile list with a halo of one row; 2 = those without the
+// particles that stick out of a far face (faces.hip sums these).
+int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, WinLists* out, hipStream_t st, int dx) {
+    auto key = std::make_pair(level_delta, code + 1000 * dx);
     auto it = p->lists.find(key);
     if (it != p->lists.end()) {
         *out = it->second;
@@ -151,6 +152,7 @@ int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, Win
     if (tl.n > 0) {
         ConvArgs<float> a{};
         a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.Lc = p->lc(level_delta); a.tree_off = p->tree_offset(a.Lc);
+        a.dx_skip_faces = dx == 2 ? 1 : 0;
         int4* d_counts = nullptr; int4* d_offs = nullptr;
         APRNET_HIP_CHECK(hipMalloc((void**)&d_counts, (size_t)tl.n * sizeof(int4)));
         launch_build_code(code, a, tl.n, 0, d_counts, nullptr, wl, dx, st);

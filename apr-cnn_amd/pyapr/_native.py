@@ -135,6 +135,9 @@ def hip():
     lib.aprnet_channel_sum_work_elems.argtypes = [i32]
     lib.aprnet_channel_sum_static_f32.argtypes = [vp, i64, i32, i64, vp, i32, vp]
     lib.aprnet_channel_sum_bf16.argtypes = [vp, i64, i32, i64, vp, i32, vp, vp]
+    lib.aprnet_conv_bwd_ws_bytes_f32.argtypes = [vp, i32, i32, i32, i32, i32, i32, i32]
+    lib.aprnet_conv_bwd_ws_bytes_f32.restype = i64
+    lib.aprnet_conv_bwd_ws_f32.argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, vp, i32, i32, vp, i64, vp, i64, vp, vp, i64, vp, i64, vp, i64, vp]
     lib.aprnet_conv_bwd_bf16.argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, vp, i32, i32, vp, i64, vp, i64, vp,
                                          vp, i64, vp, i64, vp, i64, vp]
     # bfloat16 features grouped by eight channels

@@ -451,11 +451,16 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
             ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
             tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             gtree_ws = None if skip_gx else torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
-            fn = getattr(_lib(), "aprnet_conv_bwd_" + sfx)
+            fn = getattr(_lib(), "aprnet_conv_bwd_" + ("ws_f32" if sfx == "f32" else sfx))
+            extra = ()
+            if sfx == "f32":
+                ws, ws_bytes = _workspace(0 if skip_gx else max(_lib().aprnet_conv_bwd_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
+                                                                for b in range(B)), x.device)
+                extra = (_optr(ws), ws_bytes)
             for b in range(B):
                 rc = fn(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout,
                         _ptr(grad_output[b]), grad_output.size(2), gxp(b), N, _ptr(gw),
-                        _ptr(tree_ws), ld_tree, None if skip_gx else _ptr(gtree_ws), ld_tree, st)
+                        _ptr(tree_ws), ld_tree, None if skip_gx else _ptr(gtree_ws), ld_tree, *extra, st)
                 if rc:
                     _raise(rc, "conv_backward failed")
     return [gx, gw]

@@ -247,6 +247,12 @@ int64_t aprnet_conv_ws_bytes_f32(const aprnet_plan*, int level_delta, int kz, in
 int aprnet_conv_fwd_ws_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
                            const float* w, int S_exp, int Cout, const float* bias, float* y, int64_t ldy, float* tree_ws,
                            int64_t ld_tree, const aprnet_conv_fusion* fusion, void* ws, int64_t ws_bytes, void* stream);
+/* The same of the backward pass: with aprnet_conv_bwd_ws_bytes_f32() bytes the input gradient is made of products of pieces, from window
+ * lists that the plan builds and keeps with the first such call at a level delta; with less, or NULL, it is aprnet_conv_bwd_f32. */
+int64_t aprnet_conv_bwd_ws_bytes_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, int Cin, int S_exp, int Cout);
+int aprnet_conv_bwd_ws_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
+                           const float* w, int S_exp, int Cout, const float* gy, int64_t ldy, float* gx, int64_t ldgx, float* gw,
+                           float* tree_ws, int64_t ld_tree, float* gtree_ws, int64_t ld_gtree, void* ws, int64_t ws_bytes, void* stream);
 
 /* bfloat16 features (uint16_t bit patterns; no counterpart in the reference, which has no 16-bit path).
  * Values are widened to fp32 on load, accumulated in fp32 and rounded to nearest even on store.  Weights

@@ -137,8 +137,46 @@ def test_under_capture(path):
         assert torch.equal(torch.nan_to_num(y), torch.nan_to_num(want)) and torch.equal(y.isnan(), want.isnan())
 
 
+def gradients(path, p, aprs, xd, wd, gy, ld):
+    path(p)
+    return _ops.conv_backward(aprs, xd, wd, gy, ld)
+
+
+@pytest.mark.parametrize("cin,cout", [(1, 16), (16, 18), (17, 19), (33, 32)])
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 5, 5)], ids=["k333", "k155"])
+@pytest.mark.parametrize("bt", [[("3d_s", 0), ("3d_t", 1)], [("3d_a", 0)], [("3d_c", 2)], [("2d_a", 1), ("2d_s", 0)]], ids=["3d", "3d_odd", "3d_coarse", "2d"])
+def test_input_gradient_against_float64(path, bt, ksize, cin, cout):
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, cin, cout, torch.float32)
+    gy = torch.randn(x.size(0), cout, x.size(2), generator=torch.Generator().manual_seed(3))
+    for i, a in enumerate(aprs):
+        gy[i, :, oracle.number_parts(a, int(ld[i])):] = 0
+    xd, wd, gd = x.to(DEV), layer(w_exp), gy.to(DEV)
+    ref = _ops.conv_backward(aprs, xd.double(), wd.double(), gd.double(), ld)[0].cpu()
+    fp32, fp32_w = gradients(path, 19, aprs, xd, wd, gd, ld)
+    got, got_w = gradients(path, 20, aprs, xd, wd, gd, ld)
+    assert not torch.equal(got, fp32) and torch.equal(got_w, fp32_w)
+    close(got, ref.float(), torch.float32)
+    assert error(got, ref) <= error(fp32, ref)
+    # repeats bit for bit, far faces included; a flat stencil in a volume adds three sums to a coarser particle, from two slices and
+    # its own level, in any order (on the fp32 path as well)
+    if ksize[0] == 3 or bt[0][0].startswith("2d"):
+        assert torch.equal(got, gradients(path, 20, aprs, xd, wd, gd, ld)[0])
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+def test_input_gradient_that_is_not_finite(path, value):
+    """Then all of it is the fp32 instructions', bit for bit; 3.4e38 has an infinite first piece but finite results."""
+    x, aprs, ld, w_exp = _conv_case([("3d_a", 0)], (3, 3, 3), 2, 8, 16, torch.float32)
+    gy = torch.randn(1, 16, x.size(2), generator=torch.Generator().manual_seed(3))
+    gy[0, 3, 11] = value
+    xd, wd, gd = x.to(DEV), layer(w_exp) * 1e-3, gy.to(DEV)
+    fp32 = gradients(path, 19, aprs, xd, wd, gd, ld)[0]
+    got = gradients(path, 20, aprs, xd, wd, gd, ld)[0]
+    assert torch.equal(got.nan_to_num(nan=7.0), fp32.nan_to_num(nan=7.0)) and bool(fp32.isfinite().all()) == (value == 3.4e38)
+
+
 def test_recorded_pass_keeps_the_fp32_products(path):
-    """A forward pass that a backward pass may follow is the fp32 instructions', as are its gradients."""
+    """A forward pass that a backward pass may follow is the fp32 instructions', as is the weight gradient."""
     from pyapr import aprnet
     x, aprs, ld, _ = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
     conv, xd = aprnet.cuda.APRConv(16, 32, nstencils=2).to(DEV), x.to(DEV)

@@ -101,13 +101,14 @@ struct NeedLists {
 
 // Particles that stick out of a far face of the next finer level, with the (output, tap) pairs that read them
 // (faces.hip); device arrays owned by the plan.
+constexpr int FACE_PB = 4;                      // particles of a workgroup
 struct FaceLists {
-    int n_part = 0;
-    int* d_part_idx = nullptr;                  // [n_part] index of the particle in the input gradient
+    int n_part = 0;                             // a multiple of FACE_PB; the particles of each level are filled up to one
+    int* d_part_idx = nullptr;                  // [n_part] index of the particle in the input gradient, -1: filled up
     int* d_part_level = nullptr;                // [n_part] level of the outputs that read it (its own level + 1)
-    int* d_pair_begin = nullptr;                // [n_part + 1]
-    int* d_pair_out = nullptr;                  // [pairs] index into the output gradient
-    unsigned char* d_pair_tap = nullptr;        // [pairs]
+    int* d_out_begin = nullptr;                 // [n_part + 1]
+    int* d_out = nullptr;                       // [outs] index into the output gradient
+    unsigned* d_taps = nullptr;                 // [outs] the taps through which that output reads the particle, one bit each
 };
 
 }  // namespace aprnet

@@ -816,6 +816,18 @@ def test_conv_backward_fp32_repeats_bit_for_bit_on_odd_sizes(bt, ksize):
     close(gw_a.permute(2, 0, 1, 3, 4, 5), gw_ref, torch.float32)
 
 
+@pytest.mark.parametrize("cin,cout", [(1, 64), (65, 63), (64, 130), (3, 65)])
+@pytest.mark.parametrize("bt,ksize", [([("3d_t", 0), ("3d_a", 1)], (3, 3, 3)), ([("2d_t", 0)], (1, 3, 3)), ([("2d_s", 1)], (1, 5, 5))],
+                         ids=["333", "133", "155"])
+def test_input_gradient_on_far_faces(bt, ksize, cin, cout):
+    """Channel counts around the 64 of a workgroup of the far-face kernel."""
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, cin, cout, torch.float32)
+    go = torch.randn(x.size(0), cout, x.size(2), generator=torch.Generator().manual_seed(31))
+    ref = oracle.conv_backward(aprs, x, w_exp, go, ld)[0]
+    wd = w_exp.permute(1, 2, 0, 3, 4, 5).contiguous().to(DEV)
+    close(_ops.conv_backward(aprs, x.to(DEV), wd, go.to(DEV), ld)[0], ref, torch.float32)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16], ids=["f32", "f64", "bf16"])
 def test_conv111_backward_repeats_bit_for_bit(dtype):
     """The 1x1x1 weight gradient is summed from per-workgroup partials in a fixed order (each level range adds to its

@@ -240,13 +240,13 @@ static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx
 }
 
 // The same of the input gradient: packed weights and the output gradient in groups of four channels.
-// Next to the weight gradient, which bounds many of these calls, it takes more work to gain by it (whole backward pass, split against
-// fp32: 3x3x3 16 -> 16 channels on 70 k particles 224 and 220 us, on 320 k 384 and 418; 32 -> 32 on 70 k 434 and 435, on 320 k
-// 868 and 976; 64 -> 64 on 14 k 614 and 626; 1x5x5 32 -> 32 on 70 k 409 and 410, 64 -> 64 879 and 937; at 16 input channels
-// the fp32 kernel's staging of the small stencil is the faster one, 320 k 355 and 343).
+// Next to the weight gradient, which bounds many of these calls, it gains less by it (whole backward pass, split against fp32:
+// 3x3x3 16 -> 16 channels on 70 k particles 152 and 159 us, on 320 k 319 and 353; 32 -> 32 on 14 k 144 and 142, on 70 k 242
+// and 266; 64 -> 64 on 14 k 212 and 220; 128 -> 128 on 2 k 218 and 278; 1x5x5 16 -> 16 on 14 k 139 and 119, on 70 k 142
+// and 157, 64 -> 64 on 14 k 209 and 209).
 size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n) {
     if (!g_f32_split || !g_use_lists || g_conv_path == 1 || (code != 333 && code != 155) || Cout < SPLIT_MIN_CIN || n >= (1ll << 28)) return 0;
-    if (g_f32_split == 1 && ((code == 155 && Cin <= 16) || (double)n * Cout * ((Cin + 15) / 16 * 16) < (code == 155 ? 1 << 28 : 1 << 26))) return 0;
+    if (g_f32_split == 1 && (double)n * Cout * ((Cin + 15) / 16 * 16) < 1 << 24) return 0;
     if (conv_packed_split_bytes(code, S_exp, Cin, Cout) / 48 >= (1u << 29)) return 0;
     return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cin, Cout)) + (size_t)(Cout + 3) / 4 * (size_t)n * 16;
 }

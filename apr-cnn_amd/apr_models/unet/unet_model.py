@@ -82,10 +82,10 @@ class APRUNet(nn.Module):
         """Builds the restricted stencils (restrict_kernel) of every stencil convolution once and keeps them on the
         convolution modules, so that the grouped inference path does not recompute them in every forward pass.
         ``levels``: number of APR levels the stencils are expanded to (default: taken from ``aprs``).  The kept
-        stencils are dropped by ``train()``, ``load_state_dict()``, ``.to()`` / ``.float()`` ... and
+        stencils, and the images of them that the bfloat16 kernels read, are dropped by ``train()``, ``load_state_dict()``, ``.to()`` / ``.float()`` ... and
         ``invalidate_inference_cache()``; call the latter after writing weights in a way autograd does not see
         (``weight.data.copy_()``, EMA swaps).  Without this call every forward pass restricts its stencils anew."""
-        from pyapr.aprnet import _ops
+        from pyapr.aprnet import _ops, grouped as g8
         if levels is None:
             if aprs is None:
                 raise ValueError("prepare_inference needs the APRs or the number of levels")
@@ -95,12 +95,14 @@ class APRUNet(nn.Module):
             for m in self.modules():
                 if isinstance(m, aprnet.APRConv) and tuple(m.weight.shape[3:]) != (1, 1, 1) and m.weight.is_cuda:
                     m._inference_stencils = (int(levels), _ops.restrict_kernel_forward(m.weight.detach().float().contiguous(), int(levels)))
+                    m._inference_image = g8.pack_weights(m._inference_stencils[1])
         return self
 
     def invalidate_inference_cache(self):
         for m in self.modules():
-            if hasattr(m, "_inference_stencils"):
-                del m._inference_stencils
+            for kept in ("_inference_stencils", "_inference_image"):
+                if hasattr(m, kept):
+                    delattr(m, kept)
         return self
 
     def train(self, mode=True):
@@ -126,15 +128,16 @@ class APRUNet(nn.Module):
             # otherwise computed here (never cached implicitly: a write through weight.data would go unnoticed)
             kept = getattr(conv_module, "_inference_stencils", None)
             if kept is not None and kept[0] == levels:
-                return kept[1]
-            return _ops.restrict_kernel_forward(conv_module.weight.detach().float().contiguous(), levels)
+                return kept[1], getattr(conv_module, "_inference_image", None)
+            return _ops.restrict_kernel_forward(conv_module.weight.detach().float().contiguous(), levels), None
 
         def conv(bb, inp, second=None, coarse=None):
             w = bb.conv.weight.detach().float()
             bias = None if bb.conv.bias is None else bb.conv.bias.detach()
             if tuple(w.shape[3:]) == (1, 1, 1):
                 return g8.conv111_forward(aprs, inp, w, level_deltas, bias, relu=True)
-            return g8.conv_forward(aprs, inp, restricted(bb.conv), level_deltas, bias, relu=True, x2=second, x2_coarse=coarse)
+            w, packed = restricted(bb.conv)
+            return g8.conv_forward(aprs, inp, w, level_deltas, bias, relu=True, x2=second, x2_coarse=coarse, packed=packed)
 
         def block(cb, inp, second=None):
             for i, bb in enumerate(cb.blocks):
@@ -154,8 +157,9 @@ class APRUNet(nn.Module):
             # the network's last stencil convolution and the 1x1x1 head in one kernel: its 16 channels at full
             # resolution are neither written nor read back
             bias = None if bb.conv.bias is None else bb.conv.bias.detach()
-            return g8.conv_head_forward(aprs, inp, restricted(bb.conv), level_deltas, bias, hw, hb, relu=True, x2=second,
-                                        x2_coarse=coarse)
+            w, packed = restricted(bb.conv)
+            return g8.conv_head_forward(aprs, inp, w, level_deltas, bias, hw, hb, relu=True, x2=second, x2_coarse=coarse,
+                                        packed=packed)
 
         y = skips.pop()
         for si, stage in enumerate(self.decoder):

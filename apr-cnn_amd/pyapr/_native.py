@@ -151,5 +151,12 @@ def hip():
                                                 vp, i64, vp, vp]
     lib.aprnet_conv_fwd_head_bf16g.argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, vp, i32, i32, vp, vp, i64, vp,
                                                vp, i32, i32, vp, vp, i64, vp]
+    lib.aprnet_conv_pack_bf16_bytes.argtypes = [i32, i32, i32, i32, i32, i32]
+    lib.aprnet_conv_pack_bf16_bytes.restype = i64
+    lib.aprnet_conv_pack_bf16.argtypes = [i32, i32, i32, vp, i32, i32, i32, vp, vp]
+    lib.aprnet_conv_fwd_packed_bf16l.argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, i32, vp, vp, i32, i32, vp, vp, i64, i32,
+                                                 vp, i64, vp, vp]
+    lib.aprnet_conv_fwd_head_packed_bf16g.argtypes = [vp, i32, i32, i32, i32, vp, i64, i32, vp, vp, i32, i32, vp, vp, i64, vp,
+                                                      vp, i32, i32, vp, vp, i64, vp]
     _hip = lib
     return lib

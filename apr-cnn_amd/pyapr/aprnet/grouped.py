@@ -79,12 +79,38 @@ def _fusion(x2, b, N, c2, relu, x2_coarse):
     return fu
 
 
-def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, grouped_output=True, x2_coarse=None):
+def pack_weights(weights):
+    """Image of fp32 stencils [S_exp, Cout, Cin, kz, kx, ky] as the kernels of this module read them, for callers that keep it
+    beside weights that stand still; None for layers without one."""
+    s_exp, cout, cin, kz, kx, ky = weights.shape
+    nbytes = _lib().aprnet_conv_pack_bf16_bytes(kz, kx, ky, s_exp, cout, cin)
+    if nbytes == 0 or cin % 8:                 # (a planes input, of 1 to 3 channels, is convolved from the weights themselves)
+        return None
+    _check_input(weights, "weights")
+    out = torch.empty(nbytes, dtype=torch.uint8, device=weights.device)
+    with torch.cuda.device(out.device):
+        rc = _lib().aprnet_conv_pack_bf16(kz, kx, ky, _ptr(weights), s_exp, cout, cin, _ptr(out), _stream())
+        if rc:
+            _raise(rc, "conv_pack failed")
+    return out
+
+
+def _image(packed, weights, device):
+    if packed is None:
+        return None
+    s_exp, cout, cin, kz, kx, ky = weights.shape
+    if packed.device != device or packed.numel() != _lib().aprnet_conv_pack_bf16_bytes(kz, kx, ky, s_exp, cout, cin):
+        raise ValueError("the packed weights do not belong to these weights")
+    return _ptr(packed)
+
+
+def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, grouped_output=True, x2_coarse=None, packed=None):
     """Stencil convolution (3x3x3, 1x3x3, 1x5x5) on the bfloat16 matrix cores.  ``x``: Grouped, or a [B, C <= 3, N]
     bfloat16 plane tensor (the first layer of a network); ``x2``: optional Grouped second input whose channels follow
     those of x (the concatenation of a decoder stage).  weights [S_exp, Cout, Cin, kz, kx, ky] fp32.
     ``x2_coarse``: the Grouped tensor at level_delta + 1 that x2 is the upsample_const_forward of; the mean tree of x2
     is then read off it instead of computed from x2 (same values, an eighth of the reads).
+    ``packed``: pack_weights(weights), kept by the caller.
     -> Grouped, or [B, Cout, N] planes with ``grouped_output=False``."""
     planes_in = not isinstance(x, Grouped)
     xd = x if planes_in else x.data
@@ -117,12 +143,13 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
     ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
     tree_ws = torch.empty((cin if planes_in else cin // 8, ld_tree, 1 if planes_in else 8), dtype=torch.bfloat16, device=xd.device)
     plans = _plans(aprs, xd.device)
+    image = None if planes_in else _image(packed, weights, xd.device)
     with torch.cuda.device(xd.device):
         st = _stream()
         for b in range(B):
             fu = _fusion(x2, b, N, c2, relu, x2_coarse)
-            rc = _lib().aprnet_conv_fwd_fused_bf16l(plans[b], d[b], kz, kx, ky, _ptr(xd[b]), N, c1, 0 if planes_in else 1, _ptr(weights),
-                                                    s_exp, cout, None if bias is None else _ptr(bias), _ptr(out[b]), N,
+            rc = _lib().aprnet_conv_fwd_packed_bf16l(plans[b], d[b], kz, kx, ky, _ptr(xd[b]), N, c1, 0 if planes_in else 1, _ptr(weights),
+                                                     image, s_exp, cout, None if bias is None else _ptr(bias), _ptr(out[b]), N,
                                                     1 if grouped_output else 0, _ptr(tree_ws), ld_tree, C.byref(fu), st)
             if rc:
                 _raise(rc, "conv_forward failed")
@@ -134,10 +161,10 @@ def head_limits_ok(cout, head_weights):
     return cout <= 16 and head_weights.shape[1] <= 4 and tuple(head_weights.shape[3:]) == (1, 1, 1) and head_weights.shape[2] == cout
 
 
-def conv_head_forward(aprs, x, weights, level_delta, bias, head_weights, head_bias=None, relu=True, x2=None, x2_coarse=None):
+def conv_head_forward(aprs, x, weights, level_delta, bias, head_weights, head_bias=None, relu=True, x2=None, x2_coarse=None, packed=None):
     """The last stencil convolution of a network and the 1x1x1 convolution that follows it (unet_model.py:94) in one
     kernel: conv111(relu(conv(x) + bias)) without storing the layer's result.  ``x`` (and ``x2``) Grouped, weights
-    [S_exp, Cout <= 16, Cin, kz, kx, ky], head_weights [S, C <= 4, Cout, 1, 1, 1] (not expanded), fp32
+    [S_exp, Cout <= 16, Cin, kz, kx, ky], head_weights [S, C <= 4, Cout, 1, 1, 1] (not expanded), fp32; ``packed`` as in conv_forward
     -> [B, C, N] bfloat16 planes."""
     _check_input(weights, "weights")
     weights = weights.float()
@@ -165,11 +192,12 @@ def conv_head_forward(aprs, x, weights, level_delta, bias, head_weights, head_bi
     ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
     tree_ws = torch.empty((cin // 8, ld_tree, 8), dtype=torch.bfloat16, device=out.device)
     plans = _plans(aprs, out.device)
+    image = _image(packed, weights, out.device)
     with torch.cuda.device(out.device):
         st = _stream()
         for b in range(B):
             fu = _fusion(x2, b, N, c2, relu, x2_coarse)
-            rc = _lib().aprnet_conv_fwd_head_bf16g(plans[b], d[b], kz, kx, ky, _ptr(x.data[b]), N, c1, _ptr(weights), s_exp, cout,
+            rc = _lib().aprnet_conv_fwd_head_packed_bf16g(plans[b], d[b], kz, kx, ky, _ptr(x.data[b]), N, c1, _ptr(weights), image, s_exp, cout,
                                                    None if bias is None else _ptr(bias), _ptr(tree_ws), ld_tree, C.byref(fu),
                                                    _ptr(hw), hs, hc, None if hb is None else _ptr(hb), _ptr(out[b]), N, st)
             if rc:

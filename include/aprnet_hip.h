@@ -355,6 +355,18 @@ int aprnet_conv_fwd_head_bf16g(const aprnet_plan*, int level_delta, int kz, int 
                                const float* w, int S_exp, int Cout, const float* bias, uint16_t* tree_ws, int64_t ld_tree,
                                const aprnet_conv_fusion* fusion, const float* head_w, int head_S, int head_C,
                                const float* head_bias, uint16_t* out, int64_t ldo, void* stream);
+/* The two with an image of the weights that the caller keeps (a network whose weights stand still): `packed`, 16-byte aligned, was
+ * made by aprnet_conv_pack_bf16 from the same w, S_exp, Cout and Cin (both inputs together), aprnet_conv_pack_bf16_bytes long (0: no such
+ * stencil).  NULL, or a planes input: as without.  `w` is not read where `packed` is. */
+int64_t aprnet_conv_pack_bf16_bytes(int kz, int kx, int ky, int S_exp, int Cout, int Cin);
+int aprnet_conv_pack_bf16(int kz, int kx, int ky, const float* w, int S_exp, int Cout, int Cin, void* packed, void* stream);
+int aprnet_conv_fwd_packed_bf16l(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const uint16_t* x, int64_t ldx, int Cin,
+                                 int x_grouped, const float* w, const void* packed, int S_exp, int Cout, const float* bias, uint16_t* y,
+                                 int64_t ldy, int y_grouped, uint16_t* tree_ws, int64_t ld_tree, const aprnet_conv_fusion* fusion, void* stream);
+int aprnet_conv_fwd_head_packed_bf16g(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const uint16_t* x, int64_t ldx, int Cin,
+                                      const float* w, const void* packed, int S_exp, int Cout, const float* bias, uint16_t* tree_ws,
+                                      int64_t ld_tree, const aprnet_conv_fusion* fusion, const float* head_w, int head_S, int head_C,
+                                      const float* head_bias, uint16_t* out, int64_t ldo, void* stream);
 
 /* Label and coordinate utilities of the StarDist networks (pyapr/aprnet/src/utils.hpp:86-333; CPU loops in the
  * reference, device kernels here).  Particle order = feature order at level_delta.  Images are dense device arrays

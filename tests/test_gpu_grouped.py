@@ -167,6 +167,23 @@ def test_tree_of_an_upsampled_second_input_is_read_off_its_source(fill, ksize):
         g8.conv_forward(aprs, xa, w, ld, bias, relu=True, x2=u, x2_coarse=g8.regroup(z[:, :16].contiguous().to(DEV)))
 
 
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 5, 5)], ids=["333", "155"])
+@pytest.mark.parametrize("c1,c2,cout", [(8, 0, 8), (16, 16, 16), (32, 0, 40)])
+def test_kept_weight_images_give_the_same_bits(c1, c2, cout, ksize):
+    aprs, ld, x, g = _batch(c1 + c2, seed=5)
+    levels = max(a.level_max() - a.level_min() + 1 for a in aprs)
+    w = (torch.randn(levels, cout, c1 + c2, *ksize, generator=g) * 0.1).to(DEV)
+    xa, xb = g8.regroup(x[:, :c1].contiguous()), (g8.regroup(x[:, c1:].contiguous()) if c2 else None)
+    image = g8.pack_weights(w)
+    assert torch.equal(g8.conv_forward(aprs, xa, w, ld, x2=xb, packed=image).data, g8.conv_forward(aprs, xa, w, ld, x2=xb).data)
+    if cout <= 16:
+        hw = torch.randn(1, 3, cout, 1, 1, 1, generator=g).to(DEV)
+        assert torch.equal(g8.conv_head_forward(aprs, xa, w, ld, None, hw, x2=xb, packed=image), g8.conv_head_forward(aprs, xa, w, ld, None, hw, x2=xb))
+    with pytest.raises(ValueError):
+        g8.conv_forward(aprs, xa, w, ld, x2=xb, packed=image[16:])
+    assert g8.pack_weights(torch.zeros(1, 16, 1, *ksize, device=DEV)) is None
+
+
 def test_fused_head_refuses_what_it_does_not_take():
     aprs, ld, x, g = _batch(32, seed=2)
     levels = max(a.level_max() - a.level_min() + 1 for a in aprs)

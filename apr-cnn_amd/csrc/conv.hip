@@ -148,12 +148,12 @@ static std::atomic<int> g_bf16_regroup{1};   // bfloat16 forward: 1 = stage from
 int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx, int C, bf16_t* tree, int64_t ldt, hipStream_t st,
                        const NeedLists* need);
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
-int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const int* when = nullptr);
+int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const RedoClear* redo = nullptr);
 
 size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
-int pack_conv_weights_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, hipStream_t st);
-int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st);
+int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
+                  const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
 
@@ -236,6 +236,7 @@ static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx
     if (!g_f32_split || g_conv_path == 1 || (code != 333 && code != 155) || Cin < SPLIT_MIN_CIN || nx >= (1ll << 28) || nt >= (1ll << 28)) return 0;
     if (g_f32_split == 1 && (double)nx * Cin * ((Cout + 15) / 16 * 16) < (Cout <= 16 ? 1 << 26 : 1 << 23)) return 0;
     if (conv_packed_split_bytes(code, S_exp, Cout, Cin) / 48 >= (1u << 29)) return 0;               // elements the packing kernel counts in 32 bits
+    if ((double)(Cin + 3) / 4 * (nx + nt) >= 1.6e10) return 0;                                   // 2^32 threads of the copies, four elements each
     return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cout, Cin)) + (size_t)(Cin + 3) / 4 * (size_t)(nx + nt) * 16;
 }
 
@@ -248,6 +249,7 @@ size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n) {
     if (!g_f32_split || !g_use_lists || g_conv_path == 1 || (code != 333 && code != 155) || Cout < SPLIT_MIN_CIN || n >= (1ll << 28)) return 0;
     if (g_f32_split == 1 && (double)n * Cout * ((Cin + 15) / 16 * 16) < 1 << 24) return 0;
     if (conv_packed_split_bytes(code, S_exp, Cin, Cout) / 48 >= (1u << 29)) return 0;
+    if ((double)(Cout + 3) / 4 * n >= 1.6e10) return 0;
     return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cin, Cout)) + (size_t)(Cout + 3) / 4 * (size_t)n * 16;
 }
 
@@ -266,9 +268,8 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
         const size_t wbytes = split_align(conv_packed_split_bytes(code, a.S_exp, a.Cout, a.Cin)), ng = (size_t)(a.Cin + 3) / 4;
         char* image = (char*)ws + split_mark_bytes();
         float* xi = (float*)(image + wbytes), *ti = xi + ng * (size_t)a.x_count * 4;
-        if (int rc = pack_conv_weights_split(code, a.w, a.S_exp, a.Cout, a.Cin, false, image, (int*)ws, st)) return rc;
-        if (int rc = group4_f32(a.x, a.ldx, a.x2, a.ldx2, a.c_split, a.Cin, a.x_count, xi, st)) return rc;
-        if (int rc = group4_f32(a.tree_data, a.ldt, nullptr, 0, a.Cin, a.Cin, a.t_count, ti, st)) return rc;
+        if (int rc = prepare_split(code, a.w, a.S_exp, a.Cout, a.Cin, false, image, (int*)ws, a.x, a.ldx, a.x2, a.ldx2, a.c_split, a.x_count, xi,
+                                   a.tree_data, a.ldt, a.t_count, ti, st)) return rc;
         b.w_raw = a.w; b.w = (const float*)image; b.redo = (int*)ws;
         b.xi = xi; b.ti = ti; b.xi_ld = a.x_count; b.ti_ld = a.t_count;
         TimedLaunch timed(st);

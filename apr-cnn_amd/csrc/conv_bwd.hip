@@ -254,7 +254,7 @@ int launch_conv_dx_mfma(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStr
 int launch_conv_dw_mfma(int code, const ConvArgs<bf16_t>& a, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st);
 int fill_tree_for_conv(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx, int C, bf16_t* tree, int64_t ldt, hipStream_t st, const NeedLists* need);
 size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed);
-int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const int* when = nullptr);
+int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const RedoClear* redo = nullptr);
 int conv_path();
 // the tree nodes the forward window lists name, null: fill every node (conv.hip)
 const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& tl, hipStream_t st, NeedLists* store);
@@ -266,10 +266,9 @@ int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvA
 size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n);
 size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
-int pack_conv_weights_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, hipStream_t st);
-int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st);
+int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
+                  const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
 int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
-int split_clear(const int* mark, float* gx, int64_t ldgx, int64_t n, float* gtree, int64_t ldgt, int64_t nt, int C, hipStream_t st);
 int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
 size_t conv_packed_bf16_bytes(int code, int S_exp, int Cout, int Cin);
 int pack_conv_weights_bf16(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, hipStream_t st, bool transposed);
@@ -340,21 +339,22 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
         // input gradient: the forward kernel on the output gradient with the transposed, flipped stencil;
         // every row group within one row of an output takes part
         int* mark = nullptr;
+        RedoClear redo{};
         if (pieces) {
             // on products of bfloat16 pieces (conv_split.hip), from a copy of the output gradient in groups of four channels; what
             // follows then runs only if a sum was not finite, and does all of it again
             char* image = (char*)ws + split_mark_bytes();
             float* gi = (float*)(image + (conv_packed_split_bytes(code, a.S_exp, a.Cin, a.Cout) + 255) / 256 * 256);
             mark = (int*)ws;
-            if (int rc = pack_conv_weights_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, st)) return rc;
-            if (int rc = group4_f32(a.gy, a.ldy, nullptr, 0, a.Cout, a.Cout, a.x_count, gi, st)) return rc;
+            redo = RedoClear{mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin};
+            if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, nullptr, 0, a.Cout, a.x_count, gi,
+                                       nullptr, 0, 0, nullptr, st)) return rc;
             e.tiles = near.d_tiles; e.n_tiles = near.n;
             e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
             e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
             if (int rc = launch_conv_dx_split(code, e, near.n, st)) return rc;
-            if (int rc = split_clear(mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin, st)) return rc;
         }
-        if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cin, a.Cout, true, (float*)p->d_scratch, st, mark)) return rc;
+        if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cin, a.Cout, true, (float*)p->d_scratch, st, &redo)) return rc;
         ConvArgs<float> b = a;
         b.redo = mark;
         b.tiles = near.d_tiles; b.n_tiles = near.n;

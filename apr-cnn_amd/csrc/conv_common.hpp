@@ -432,6 +432,9 @@ __device__ __forceinline__ void close_window(ConvShared<G>& sh) {
     if (threadIdx.x == 0) { sh.ncol = 0; sh.nitem = 0; sh.nbox = 0; }
 }
 
+// An input gradient that is made again if a word on the device is set: what was added so far, cleared first.
+struct RedoClear { const int* mark; float* gx; int64_t ldgx, n; float* gtree; int64_t ldgt, nt; int C; };
+
 // Buffer loads: the channel plane is described by a wave-uniform resource (base, size in bytes), the lane
 // supplies a 32-bit byte offset, and an offset outside the plane returns zero without touching memory.
 // That keeps the address registers to one per item and makes every predicate of the gather (item

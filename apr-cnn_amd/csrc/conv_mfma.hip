@@ -53,8 +53,14 @@ constexpr int STAGE_PRIO = 3;      // wave priority outside the matrix loops
 // of the stencil of the input gradient, M = input channels, contraction over (flipped tap, output channel).
 // Cm / Ck are the channel counts of the M axis and of the contracted axis.
 __global__ void pack_weights16_kernel(const float* __restrict__ w, int S_exp, int Cm, int Ck, int K, int CIB, int COH,
-                                      int transposed, float* __restrict__ out, const int* __restrict__ when) {
-    if (when && when[0] == 0) return;
+                                      int transposed, float* __restrict__ out, const RedoClear redo) {
+    if (redo.mark) {
+        if (redo.mark[0] == 0) return;
+        for (int c = 0; c < redo.C; ++c) {
+            for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < redo.n; i += (int64_t)gridDim.x * blockDim.x) redo.gx[c * redo.ldgx + i] = 0.f;
+            for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < redo.nt; i += (int64_t)gridDim.x * blockDim.x) redo.gtree[c * redo.ldgt + i] = 0.f;
+        }
+    }
     const int Cout = transposed ? Ck : Cm, Cin = transposed ? Cm : Ck;
     const int ncb = (Cm + 16 * COH - 1) / (16 * COH), nq = (Ck + CIB - 1) / CIB;
     // 32-bit index arithmetic (the host checks that the image has fewer than 2^31 elements): 64-bit divisions made
@@ -932,13 +938,13 @@ size_t conv_packed_floats(int code, int S_exp, int Cm, int Ck, bool transposed) 
     return (size_t)S_exp * ((Cm + 16 * coh - 1) / (16 * coh)) * ((Ck + cib - 1) / cib) * cib * conv_taps(code) * 16 * coh;
 }
 
-// when: null, or a word on the device that is 0 if nothing is to be packed
-int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const int* when) {
+// redo: null, or with a word on the device that is 0 if nothing is to be done, and rows to clear otherwise
+int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, float* packed, hipStream_t st, const RedoClear* redo) {
     const size_t n = conv_packed_floats(code, S_exp, Cm, Ck, transposed);
     if (n >= ((size_t)1 << 31)) return fail(APRNET_ERR_UNSUPPORTED, "packed weight image of 2^31 elements or more");
     dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 2048));
     hipLaunchKernelGGL(pack_weights16_kernel, grid, dim3(256), 0, st, w, S_exp, Cm, Ck, conv_taps(code), transposed ? DX_CIB : FWD_CIB, conv_coh(Cm),
-                       transposed ? 1 : 0, packed, when);
+                       transposed ? 1 : 0, packed, redo ? *redo : RedoClear{});
     APRNET_LAUNCH_CHECK("pack_weights16_kernel");
     return 0;
 }

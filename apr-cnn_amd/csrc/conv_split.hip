@@ -76,6 +76,7 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsig
 
 // Marks of a launch: word 0 = any, the others one per tile and block of output channels, several of them to a word where there are more
 // (all of these are then computed again).
+constexpr int PREP_TB = 256;
 constexpr unsigned SPLIT_MARKS = 4096;
 __device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit % (SPLIT_MARKS - 1); }
 
@@ -83,14 +84,14 @@ __device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit 
 // of four contracted channels.  Cm / Ck: channels on the M axis / contracted; with `transposed` the image is that of the
 // input gradient's stencil (channel axes swapped, taps reversed).  The marks of the launch are cleared on the way.
 template <int K>
-__global__ void pack_weights_split_kernel(const float* __restrict__ w, int S_exp, int Cm, int Ck, int COH, int transposed, uint4* __restrict__ out,
-                                          int* __restrict__ marks) {
+__device__ __forceinline__ void pack_weights_split(const float* __restrict__ w, int S_exp, int Cm, int Ck, int COH, int transposed, uint4* __restrict__ out,
+                                                   int* __restrict__ marks, unsigned block, unsigned blocks) {
     constexpr int nstep = SplitTaps<K>::STEPS;
     const int Cout = transposed ? Ck : Cm, Cin = transposed ? Cm : Ck;
-    for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < SPLIT_MARKS; i += gridDim.x * blockDim.x) marks[i] = 0;
+    for (unsigned i = block * PREP_TB + threadIdx.x; i < SPLIT_MARKS; i += blocks * PREP_TB) marks[i] = 0;
     const int ncb = (Cm + 16 * COH - 1) / (16 * COH), nq = (Ck + SP_CIB - 1) / SP_CIB;
     const unsigned n = (unsigned)S_exp * ncb * nq * nstep * COH * 64;          // (the host checks that it fits)
-    for (unsigned e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x) {
+    for (unsigned e = block * PREP_TB + threadIdx.x; e < n; e += blocks * PREP_TB) {
         unsigned r = e;
         const int lane = (int)(r % 64u); r /= 64u;
         const int h = (int)(r % (unsigned)COH); r /= (unsigned)COH;
@@ -121,12 +122,11 @@ __global__ void pack_weights_split_kernel(const float* __restrict__ w, int S_exp
 // ---- input in groups of four channels: [Cin / 4][count][4] ---------------------------------------------------
 // out[q][i][c] = channel 4 q + c of element i; channels from c_split on come from x2 (null: all from x), channels past C
 // are zeros.  A streaming pass (8 bytes per value), four elements per thread, all reads issued before the first is used.
-constexpr int IG_TB = 256, IG_E = 4;
-__global__ void __launch_bounds__(IG_TB)
-group4_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict__ x2, int64_t ldx2, int c_split, int C, int64_t count,
-              float4* __restrict__ out) {
-    const int q = blockIdx.y;
-    const int64_t i0 = (int64_t)blockIdx.x * (IG_TB * IG_E) + threadIdx.x;
+constexpr int IG_E = 4;
+__device__ __forceinline__ void group4(const float* __restrict__ x, int64_t ldx, const float* __restrict__ x2, int64_t ldx2, int c_split, int C, int64_t count,
+                                       float4* __restrict__ out, unsigned block, int q) {
+    constexpr int IG_TB = PREP_TB;
+    const int64_t i0 = (int64_t)block * (IG_TB * IG_E) + threadIdx.x;
     float v[SP_CIB][IG_E];
 #pragma unroll
     for (int c = 0; c < SP_CIB; ++c) {
@@ -145,6 +145,23 @@ group4_kernel(const float* __restrict__ x, int64_t ldx, const float* __restrict_
 #pragma unroll
     for (int e = 0; e < IG_E; ++e)
         if (i0 + e * IG_TB < count) dst[i0 + e * IG_TB] = make_float4(v[0][e], v[1][e], v[2][e], v[3][e]);
+}
+
+// What the convolution reads, in one launch: the first blocks pack the weights and clear the marks, the others copy the features (nbx
+// blocks per group of channels) and the tree (nbt).  (As three launches the copies of small layers cost more than the
+// convolution gained where the host is behind: a group-normed fp32 U-Net on a small crop 2.57 against 2.44 ms without.)
+struct SplitCopy { const float* x; int64_t ldx; const float* x2; int64_t ldx2; int c_split; int64_t count; float4* out; };
+template <int K>
+__global__ void __launch_bounds__(PREP_TB)
+split_prepare_kernel(const float* __restrict__ w, int S_exp, int Cm, int Ck, int COH, int transposed, uint4* __restrict__ image,
+                     int* __restrict__ marks, unsigned nb_pack, const SplitCopy fx, unsigned nbx, const SplitCopy ft, unsigned nbt) {
+    unsigned b = blockIdx.x;
+    if (b < nb_pack) { pack_weights_split<K>(w, S_exp, Cm, Ck, COH, transposed, image, marks, b, nb_pack); return; }
+    b -= nb_pack;
+    const unsigned nq = (unsigned)(Ck + SP_CIB - 1) / SP_CIB;
+    if (b < nbx * nq) { group4(fx.x, fx.ldx, fx.x2, fx.ldx2, fx.c_split, Ck, fx.count, fx.out, b % nbx, (int)(b / nbx)); return; }
+    b -= nbx * nq;
+    group4(ft.x, ft.ldx, nullptr, 0, Ck, Ck, ft.count, ft.out, b % nbt, (int)(b / nbt));
 }
 
 template <class G> struct SplitItems : ItemRegs16<G, (G::MAXITEM + G::NT - 1) / G::NT> {
@@ -486,8 +503,8 @@ static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     APRNET_LAUNCH_CHECK("conv_split_redo_kernel");
     return 0;
 }
-// a.w = image of pack_conv_weights_split, a.w_raw = the weights it was made from, a.redo = the marks that it cleared,
-// a.xi / a.ti = copies of group4_f32 of what a.x, a.x2 and a.tree_data hold, a.tile_win ... the forward lists of the plan
+// a.w, a.redo, a.xi, a.ti: what prepare_split made of the weights a.w_raw and of a.x, a.x2 and a.tree_data; a.tile_win ... the forward
+// lists of the plan
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     switch (code) {
         case 333: return launch_split<S333, 0>(a, n_tiles, st);
@@ -504,41 +521,25 @@ int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStr
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }
-// Rows of zeros in gx and gtree if the mark is set: what was added there is summed again.
-__global__ void split_clear_kernel(const int* __restrict__ mark, float* __restrict__ gx, int64_t ldgx, int64_t n, float* __restrict__ gtree, int64_t ldgt, int64_t nt, int C) {
-    if (mark[0] == 0) return;
-    for (int c = 0; c < C; ++c) {
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) gx[c * ldgx + i] = 0.f;
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nt; i += (int64_t)gridDim.x * blockDim.x) gtree[c * ldgt + i] = 0.f;
-    }
-}
-int split_clear(const int* mark, float* gx, int64_t ldgx, int64_t n, float* gtree, int64_t ldgt, int64_t nt, int C, hipStream_t st) {
-    hipLaunchKernelGGL(split_clear_kernel, dim3(256), dim3(256), 0, st, mark, gx, ldgx, n, gtree, ldgt, nt, C);
-    APRNET_LAUNCH_CHECK("split_clear_kernel");
-    return 0;
-}
-// x (and x2 from channel c_split on) -> out[(C + 3) / 4][count][4]
-int group4_f32(const float* x, int64_t ldx, const float* x2, int64_t ldx2, int c_split, int C, int64_t count, float* out, hipStream_t st) {
-    if (count <= 0 || C <= 0) return 0;
-    dim3 grid((unsigned)((count + IG_TB * IG_E - 1) / (IG_TB * IG_E)), (unsigned)((C + SP_CIB - 1) / SP_CIB));
-    hipLaunchKernelGGL(group4_kernel, grid, dim3(IG_TB), 0, st, x, ldx, x2, ldx2, c_split, C, count, (float4*)out);
-    APRNET_LAUNCH_CHECK("group4_kernel");
-    return 0;
-}
 size_t split_mark_bytes() { return SPLIT_MARKS * sizeof(int); }
 // Cm: channels on the M axis of the kernel, Ck: contracted channels (forward: Cout, Cin; transposed: Cin, Cout)
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck) {
     const int coh = split_coh(Cm);
     return (size_t)S_exp * ((Cm + 16 * coh - 1) / (16 * coh)) * ((Ck + SP_CIB - 1) / SP_CIB) * split_nstep(code) * 3 * coh * 64 * sizeof(uint4);
 }
-int pack_conv_weights_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, hipStream_t st) {
+// Packed weights, cleared marks and copies of x (x2 from channel c_split on) and of the tree in groups of four channels:
+// [(Ck + 3) / 4][count][4] each.  Fewer than 2^28 elements and 2^32 threads (split_fwd_bytes).
+int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
+                  const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st) {
     const size_t n = conv_packed_split_bytes(code, S_exp, Cm, Ck) / (3 * sizeof(uint4));
-    if (n >= ((size_t)1 << 29)) return fail(APRNET_ERR_UNSUPPORTED, "packed weight image of 2^31 elements or more");
-    dim3 grid((unsigned)std::min<size_t>((n + 255) / 256, 2048));
-#define APRNET_PACK(K) hipLaunchKernelGGL(pack_weights_split_kernel<K>, grid, dim3(256), 0, st, w, S_exp, Cm, Ck, split_coh(Cm), transposed ? 1 : 0, (uint4*)packed, marks)
-    if (code == 333) APRNET_PACK(27); else APRNET_PACK(25);
-#undef APRNET_PACK
-    APRNET_LAUNCH_CHECK("pack_weights_split_kernel");
+    const unsigned nb = (unsigned)std::min<size_t>((n + PREP_TB - 1) / PREP_TB, 2048), nq = (unsigned)(Ck + SP_CIB - 1) / SP_CIB;
+    const unsigned nbx = (unsigned)((nx + PREP_TB * IG_E - 1) / (PREP_TB * IG_E)), nbt = (unsigned)((nt + PREP_TB * IG_E - 1) / (PREP_TB * IG_E));
+    const SplitCopy fx{x, ldx, x2, ldx2, c_split, nx, (float4*)xi}, ft{tree, ldt, nullptr, 0, Ck, nt, (float4*)ti};
+#define APRNET_PREP(K) hipLaunchKernelGGL(split_prepare_kernel<K>, dim3(nb + nq * (nbx + nbt)), dim3(PREP_TB), 0, st, w, S_exp, Cm, Ck, split_coh(Cm), \
+                                          transposed ? 1 : 0, (uint4*)packed, marks, nb, fx, nbx, ft, nbt)
+    if (code == 333) APRNET_PREP(27); else APRNET_PREP(25);
+#undef APRNET_PREP
+    APRNET_LAUNCH_CHECK("split_prepare_kernel");
     return 0;
 }
 

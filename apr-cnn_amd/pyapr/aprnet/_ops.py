@@ -137,15 +137,17 @@ class _Fusion(C.Structure):
                 ("x2_coarse", C.c_void_p), ("ld_coarse", C.c_int64)]
 
 
-def _workspace(nbytes, device):
-    """Optional work space of a call: (tensor, bytes), or (None, 0) when none is asked for or there is no memory for it (the
-    call then runs without)."""
-    if nbytes <= 0:
-        return None, 0
-    try:
-        return torch.empty(nbytes, dtype=torch.uint8, device=device), nbytes
-    except torch.cuda.OutOfMemoryError:
-        return None, 0
+def _workspace(nbytes, optional, device):
+    """Work space of a call, ``nbytes`` and behind them (256-byte aligned) ``optional`` more: (tensor, address of the optional part
+    or None, its bytes).  The call runs without the optional part when there is no memory for it."""
+    at = (nbytes + 255) // 256 * 256
+    if optional > 0:
+        try:
+            buf = torch.empty(at + optional, dtype=torch.uint8, device=device)
+            return buf, buf.data_ptr() + at, optional
+        except torch.cuda.OutOfMemoryError:
+            pass
+    return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device), None, 0
 
 
 def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, pieces=True):
@@ -202,12 +204,13 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
         st = _stream()
         if sfx == "f32" and pieces and (kz, kx, ky) != (1, 1, 1):
             ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
-            tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
-            ws, ws_bytes = _workspace(max(_lib().aprnet_conv_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout) for b in range(B)), x.device)
+            lib = _lib()
+            tree_ws, ws, ws_bytes = _workspace(cin * ld_tree * 4, max([lib.aprnet_conv_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
+                                                                       for b in range(B)]), x.device)
             for b in range(B):
-                fu = _Fusion(_ptr(x2[b]) if x2 is not None else None, N, c2, 1 if relu else 0)
-                rc = _lib().aprnet_conv_fwd_ws_f32(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, c1, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N,
-                                                   _ptr(tree_ws), ld_tree, C.byref(fu) if fused else None, _optr(ws), ws_bytes, st)
+                fu = _Fusion(_ptr(x2[b]) if x2 is not None else None, N, c2, 1 if relu else 0) if fused else None
+                rc = lib.aprnet_conv_fwd_ws_f32(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, c1, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N,
+                                                _ptr(tree_ws), ld_tree, C.byref(fu) if fused else None, ws, ws_bytes, st)
                 if rc:
                     _raise(rc, "conv_forward failed")
         elif fused:
@@ -449,14 +452,14 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
                     _raise(rc, "conv111_backward failed")
         else:
             ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
-            tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             gtree_ws = None if skip_gx else torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             fn = getattr(_lib(), "aprnet_conv_bwd_" + ("ws_f32" if sfx == "f32" else sfx))
             extra = ()
             if sfx == "f32":
-                ws, ws_bytes = _workspace(0 if skip_gx else max(_lib().aprnet_conv_bwd_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
-                                                                for b in range(B)), x.device)
-                extra = (_optr(ws), ws_bytes)
+                tree_ws, *extra = _workspace(cin * ld_tree * 4, 0 if skip_gx else max([_lib().aprnet_conv_bwd_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
+                                                                                       for b in range(B)]), x.device)
+            else:
+                tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             for b in range(B):
                 rc = fn(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout,
                         _ptr(grad_output[b]), grad_output.size(2), gxp(b), N, _ptr(gw),

@@ -661,7 +661,7 @@ int aprnet_set_conv_path(int path) {
                                                  "fixed-order partial sums / atomic additions), 12 / 13 (1 to 3 input channels: pipelined kernel / general kernel), "
                                                  "14 / 15 (grouped bfloat16 forward: 32-bit offsets where they suffice / 64-bit addresses always), "
                                                  "16 / 17 (tree fill before a forward convolution: the nodes it reads / every node), "
-                                                 "18 / 19 (fp32 features: products of bfloat16 pieces where a work space is given / fp32 matrix instructions)");
+                                                 "18 / 19 / 20 (fp32 features with a work space: products of bfloat16 pieces where faster / fp32 matrix instructions / pieces at any size)");
     g_conv_path = path;
     return 0;
 }

@@ -1,8 +1,8 @@
 // Input gradient of the particles that stick out of the far faces of a level.
 //
 // A particle one level coarser than a tile fills the 2 x 2 x 2 cells it covers (helpers.hpp:381-399).  The input
-// gradient kernel gives such a particle ONE column that reads the box-summed output gradient (conv_mfma.hip), which
-// needs all eight cells to exist.  Where a level has an odd size, the particles on its far faces cover cells outside
+// gradient kernels give such a particle ONE column that reads the box-summed output gradient (conv_mfma.hip) or add up
+// the columns of its cells (conv_split.hip), which needs all eight cells to exist.  Where a level has an odd size, the particles on its far faces cover cells outside
 // the image; the forward pass never read those cells (zero_boundary, helpers.hpp:481-502), so only the existing
 // cells count.  There are few such particles (a 2-D set), and they are handled here, away from the main kernel,
 // so that every element of the input gradient receives at most two atomic contributions there (same-level term and

@@ -38,11 +38,6 @@ for _p in (ROOT, os.path.join(ROOT, "apr-cnn_amd")):
 PEAK_FP32_MATRIX_TFLOPS = 157.3
 PEAK_BF16_MATRIX_TFLOPS = 2500.0
 PEAK_HBM_GBS = 8000.0
-# HBM-side bytes of one launch of the convolution kernel on the default workload: FETCH_SIZE + WRITE_SIZE of two
-# profiler passes, scaled by what the same counters read for a device-to-device copy of known size
-# (profiles/conv333_fwd_32x32_f32_blobs512_hbm_traffic.txt).  Counters cannot be read from inside this script: the
-# figure is a constant taken from that profile and only reported when the workload is the one it was measured on.
-PROFILED_TRAFFIC_BYTES = {23245996: 27.18e9 + 3.91e9}
 
 
 # ------------------------------------------------------------------------------------------------ workloads
@@ -297,8 +292,8 @@ def run_blobs512(args, dev, lib):
     if flop_pp / (e * (CIN + COUT) + 2) < peak * 1e12 / (PEAK_HBM_GBS * 1e9):      # fewer flops per byte than the machine: HBM bounds it
         out["roofline"] = hbm_roofline(alg_bytes, kernel_ms, "conv_narrow_kernel" if CIN <= 3 else "conv kernel", flop_pp * n)
     else:
-        out["roofline"] = mfma_roofline(flop_pp * n, kernel_ms, peak, "conv_mfma_bf16_kernel" if bf16 else "conv_mfma16_kernel",
-                                        alg_bytes, None if bf16 or (CIN, COUT) != (32, 32) else PROFILED_TRAFFIC_BYTES.get(n))
+        # fp32: priced by the algorithm's flops against the fp32 matrix peak; the kernel forms six bfloat16 products for each
+        out["roofline"] = mfma_roofline(flop_pp * n, kernel_ms, peak, "conv_mfma_bf16_kernel" if bf16 else "conv_split_kernel", alg_bytes)
     if not args.no_extra:                  # (profiler runs pass --no-extra: the convolution step only)
         # second half of the metric: forward latency of the 4-level network (16-32-64-128, norms folded) on this APR
         net = make_unet(dev)
@@ -455,7 +450,8 @@ def run_nuclei2048(args, dev, lib):
                     {"workload": f"tree fill (mean of children) + APRConv 3x3x3 16->16 fp32 forward reading tree parents, batch 1, APR of the "
                                  f"seeded 2048x2048x512 nuclei volume (configs[2]), {what}",
                      "n_particles": n, "tree_nodes": nt, "levels": level_counts(apr), "apr_build_s": round(t_build, 1)})
-    out["roofline"] = mfma_roofline(2 * 27 * C * C * n, kernel_ms, PEAK_FP32_MATRIX_TFLOPS, "conv_mfma16_kernel", (8 * C + 2) * n)
+    out["roofline"] = mfma_roofline(2 * 27 * C * C * n, kernel_ms, PEAK_FP32_MATRIX_TFLOPS,
+                                    "conv_split_kernel" if n < 1 << 28 else "conv_mfma16_kernel", (8 * C + 2) * n)
     fill_bytes = 4 * C * (n + 2 * nt)
     out["extra"] = {"fill_tree_mean_ms": fill_ms, "fill_tree_mean_GBs": fill_bytes / fill_ms / 1e6,
                     "fill_tree_mean_hbm_frac": fill_bytes / fill_ms / 1e6 / PEAK_HBM_GBS,

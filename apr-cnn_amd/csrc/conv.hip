@@ -223,12 +223,12 @@ static int try_narrow(aprnet_plan* p, const ConvArgs<T>& a, int code, int d, con
 // Work space of the forward pass on products of bfloat16 pieces: packed weights, the input and its mean tree in groups of four
 // channels.  0: the layer does not take that path.
 //  - fewer than SPLIT_MIN_CIN input channels: with 8 it is no faster (8 -> 16 channels on 320 k particles 0.080 against 0.078 ms,
-//    copies included), and with 5 the fp32 instructions' short sums have the smaller error (2.07 against 2.28 of 1e-7).
+//    copies included).
 //  - 1x3x3: two steps of eight taps for nine, less than the copies cost (64 -> 64 channels on 70 k particles 107 against 98 us,
 //    on 320 k 346 against 352).
-//  - little work: the copies and launches take 8 us (3x3x3, split against fp32; 16 outputs: 70 k particles 52 and 47 us, 320 k
-//    96 and 107; 32 outputs: 13 k particles x 16 channels 43 and 39, x 32 49 and 55, 2 k x 32 39 and 34; 64 outputs:
-//    2 k x 64 46 and 53 us).
+//  - little work: one more launch than the fp32 kernel's, which also counts where the host is behind the device (3x3x3, split against
+//    fp32; 16 outputs: 70 k particles 45 and 46 us, 320 k 90 and 104; 32 outputs: 14 k particles x 16 channels 34 and 37, x 32 42
+//    and 54, 2 k x 32 30 and 32; 64 outputs: 2 k x 64 39 and 51 us).
 //  - the 16-byte items are reached with 32-bit offsets: fewer than 2^28 particles.
 constexpr int SPLIT_MIN_CIN = 16;
 static size_t split_align(size_t v) { return (v + 255) / 256 * 256; }

@@ -28,8 +28,8 @@
 // NaN), and a value within 2^-9 of the largest fp32 number has an infinite first piece.  Where a result comes out infinite or
 // NaN its tile is marked, and conv_split_redo_kernel computes the marked tiles again from the fp32 values (as a call inside this
 // kernel it cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an input gradient that
-// holds one is made again from the start by the fp32 kernel.  Values below 2^-110 lose low pieces to the end of the exponent
-// range (an absolute error below 2^-133).
+// holds one is made again from the start by the fp32 kernel.  Values and products below 2^-110 lose low pieces to the end of
+// the exponent range (an absolute error below 2^-133).
 #include "conv_common.hpp"
 
 namespace aprnet {

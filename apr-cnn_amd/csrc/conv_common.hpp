@@ -435,6 +435,11 @@ __device__ __forceinline__ void close_window(ConvShared<G>& sh) {
 // An input gradient that is made again if a word on the device is set: what was added so far, cleared first.
 struct RedoClear { const int* mark; float* gx; int64_t ldgx, n; float* gtree; int64_t ldgt, nt; int C; };
 
+// Marks of a forward launch on products of bfloat16 pieces (conv_split.hip), set where a result is not finite: word 0 = any, the others
+// one per tile and block of output channels, several of them to a word where there are more (all of these are then computed again).
+constexpr unsigned SPLIT_MARKS = 4096;
+__device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit % (SPLIT_MARKS - 1); }
+
 // Buffer loads: the channel plane is described by a wave-uniform resource (base, size in bytes), the lane
 // supplies a 32-bit byte offset, and an offset outside the plane returns zero without touching memory.
 // That keeps the address registers to one per item and makes every predicate of the gather (item

@@ -86,7 +86,9 @@ __global__ void pack_weights16_kernel(const float* __restrict__ w, int S_exp, in
 
 // MODE 0: forward, results stored (plus bias).  MODE 1: input gradient, results added atomically to the
 // place each column names (feature gradient, or tree gradient with COL_TREE).
-template <typename T, class G, int CIB, int COH, int NB, int MODE, bool FUSE, class Lists>
+// RAW: `wl` are the weights of the tile's stencil as the caller gave them, [Cout][Cin][K], not a packed image (four reads 4 bytes wide
+// in place of one of 16; for launches that rarely do anything and would have an image made for nothing)
+template <typename T, class G, int CIB, int COH, int NB, int MODE, bool FUSE, bool RAW = false, class Lists>
 __device__ __forceinline__ void mfma16_window(const ConvArgs<T>& a, int co0, int nc, int nitem, bool tree_items, int first,
                                               const float4* __restrict__ wl, const Lists& sh,
                                               float* __restrict__ patch, float* __restrict__ Wl,
@@ -134,13 +136,25 @@ __device__ __forceinline__ void mfma16_window(const ConvArgs<T>& a, int co0, int
     // per-lane branch the compiler waits for every load in flight before it enters the branch, which made each
     // chunk wait for the feature loads issued just before instead of letting them travel during the matrix phase.
     intx4w wr[WPT];
-#define APRNET_LOAD_WEIGHTS(q)                                                                     \
-    {                                                                                              \
-        const __amdgpu_buffer_rsrc_t rw_ = __builtin_amdgcn_make_buffer_rsrc(                      \
-            const_cast<float4*>(wl + (int64_t)(q) * W4), 0, W4 * 16, 0x00020000);                  \
-        _Pragma("unroll") for (int k = 0; k < WPT; ++k)                                            \
-            wr[k] = __builtin_amdgcn_raw_buffer_load_b128(rw_, (int)(threadIdx.x + k * G::NT) * 16, 0, 0); \
-    }
+    auto load_weights = [&](int q) {
+        if constexpr (RAW) {
+            const float* w = reinterpret_cast<const float*>(wl);
+#pragma unroll
+            for (int k = 0; k < WPT; ++k) {
+                const int i = min((int)threadIdx.x + k * G::NT, W4 - 1);              // [t][h][c][16 co] in fours
+                const int ci = q * CIB + (i >> 2) % CIB, h = i / (4 * CIB) % COH, t = i / (4 * CIB * COH), co = co0 + h * 16 + 4 * (i & 3);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float v = w[((int64_t)min(co + r, a.Cout - 1) * a.Cin + min(ci, a.Cin - 1)) * G::K + t];
+                    wr[k][r] = co + r < a.Cout && ci < a.Cin ? __builtin_bit_cast(int, v) : 0;
+                }
+            }
+        } else {
+            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(const_cast<float4*>(wl + (int64_t)q * W4), 0, W4 * 16, 0x00020000);
+#pragma unroll
+            for (int k = 0; k < WPT; ++k) wr[k] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(threadIdx.x + k * G::NT) * 16, 0, 0);
+        }
+    };
 #define APRNET_STORE_WEIGHTS()                                                                     \
     _Pragma("unroll") for (int k = 0; k < WPT; ++k) {                                              \
         const int i = threadIdx.x + k * G::NT;                                                     \
@@ -159,7 +173,7 @@ __device__ __forceinline__ void mfma16_window(const ConvArgs<T>& a, int co0, int
             bbase[j] = (int)(cp & COL_CELL) - G::TAP0 + (lane >> 4) * G::CH_STRIDE + ((MODE == 1 && (cp & COL_BOX)) ? CIB * G::CH_STRIDE : 0);
         }
     }
-    APRNET_LOAD_WEIGHTS(0)
+    load_weights(0);
     for (int i = threadIdx.x; i < CIB * G::CH_STRIDE; i += G::NT) patch[i] = 0.f;     // once per window
     for (int ci0 = 0; ci0 < a.Cin; ci0 += CIB) {
         __syncthreads();
@@ -168,7 +182,7 @@ __device__ __forceinline__ void mfma16_window(const ConvArgs<T>& a, int co0, int
         __syncthreads();
         if (ci0 + CIB < a.Cin) {
             load_values<G, T, CIB>(a, ci0 + CIB, nitem, tree_items, R, 0, std::bool_constant<FUSE>{});
-            APRNET_LOAD_WEIGHTS(ci0 / CIB + 1)
+            load_weights(ci0 / CIB + 1);
         }
         if constexpr (MODE == 1) {
             // Box sums over the cells of a coarser particle, for the pooled columns.  One wave per task
@@ -224,7 +238,6 @@ __device__ __forceinline__ void mfma16_window(const ConvArgs<T>& a, int co0, int
         }
         __builtin_amdgcn_s_setprio(STAGE_PRIO);
     }
-#undef APRNET_LOAD_WEIGHTS
 #undef APRNET_STORE_WEIGHTS
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
@@ -336,6 +349,45 @@ conv_mfma16_kernel(const ConvArgs<T> a) {
         }
     }
 #undef APRNET_WINDOW
+}
+
+// The marked tiles of a forward launch on products of bfloat16 pieces (conv_split.hip), on the fp32 instructions and bit for bit
+// what conv_mfma16_kernel gives.  Persistent workgroups, which end at once where nothing is marked.  With a NaN in every tile: 32 -> 32
+// channels on 320 k particles 0.67 ms in all (finite features 0.22; one thread per column, a channel staged at a time 9.7), on 9.8 M 13.8
+// (4.8; 202).
+template <class G, int COH>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(FWD_WAVES, FWD_WAVES)))
+conv_mfma16_redo_kernel(const ConvArgs<float> a, int n_tiles, int n_cb) {
+    constexpr int CIB = FWD_CIB;
+    __shared__ float patch[CIB * G::CH_STRIDE];
+    __shared__ __attribute__((aligned(16))) float Wl[CIB * G::K * 16 * COH];
+    __shared__ float bias_l[16 * COH];
+    if (a.redo[0] == 0) return;
+    const int wave = threadIdx.x >> 6;
+    for (int u = blockIdx.x; u < n_tiles * n_cb; u += gridDim.x) {              // uniform
+        if (a.redo[split_mark(u)] == 0) continue;
+        const int tile = u % n_tiles, co0 = u / n_tiles * 16 * COH, L = a.tiles[tile].level;
+        const float4* __restrict__ wl = reinterpret_cast<const float4*>(a.w_raw + (int64_t)min(a.S_exp - 1, a.Lc - L) * a.Cout * a.Cin * G::K);
+        const bool tree_items = L < a.Lc;
+        if (threadIdx.x < 16 * COH)                                            // (read behind the barriers of a window)
+            bias_l[threadIdx.x] = (a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
+        const int wb = a.tile_win[tile], we = a.tile_win[tile + 1];
+        for (int w = wb; w < we; ++w) {
+            const int4 hd = a.win[w];
+            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+            const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
+            const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
+            const int nblk = (nc + 15) >> 4, nb = wave < nblk ? (nblk - wave + G::NWAVE - 1) / G::NWAVE : 0;
+            switch (__builtin_amdgcn_readfirstlane(nb)) {
+                case 0: mfma16_window<float, G, CIB, COH, 0, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+                case 1: mfma16_window<float, G, CIB, COH, 1, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+                case 2: mfma16_window<float, G, CIB, COH, 2, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+                case 3: mfma16_window<float, G, CIB, COH, 3, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+                default: mfma16_window<float, G, CIB, COH, 4, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+            }
+            __syncthreads();        // the next window rewrites the patch, the next tile the bias
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -841,6 +893,24 @@ static int launch16_code(int code, const ConvArgs<T>& a, int n_tiles, hipStream_
             else return launch16<T, M333N, MODE>(a, n_tiles, st);
         case 133: return launch16<T, M133N, MODE>(a, n_tiles, st);
         case 155: return launch16<T, M155N, MODE>(a, n_tiles, st);
+    }
+    return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
+}
+
+// The tiles that a.redo marks (a.w_raw: the weights, not packed; forward lists of the plan)
+template <class G>
+static int launch_redo(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+    const int coh = conv_coh(a.Cout), n_cb = (a.Cout + 16 * coh - 1) / (16 * coh);
+    const dim3 grid((unsigned)std::min<int64_t>((int64_t)n_tiles * n_cb, 768));         // three workgroups on each of 256 CUs
+    if (coh == 1) hipLaunchKernelGGL((conv_mfma16_redo_kernel<G, 1>), grid, dim3(G::NT), 0, st, a, n_tiles, n_cb);
+    else hipLaunchKernelGGL((conv_mfma16_redo_kernel<G, 2>), grid, dim3(G::NT), 0, st, a, n_tiles, n_cb);
+    APRNET_LAUNCH_CHECK("conv_mfma16_redo_kernel");
+    return 0;
+}
+int launch_conv_redo(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+    switch (code) {
+        case 333: return launch_redo<M333N>(a, n_tiles, st);
+        case 155: return launch_redo<M155N>(a, n_tiles, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }

@@ -26,9 +26,9 @@
 //
 // Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
 // NaN), and a value within 2^-9 of the largest fp32 number has an infinite first piece.  Where a result comes out infinite or
-// NaN its tile is marked, and conv_split_redo_kernel computes the marked tiles again from the fp32 values (as a call inside this
-// kernel it cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an input gradient that
-// holds one is made again from the start by the fp32 kernel.  Values and products below 2^-110 lose low pieces to the end of
+// NaN its tile is marked, and the fp32 instructions compute the marked tiles again (conv_mfma16_redo_kernel; as a call inside this
+// kernel a second pass cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an input
+// gradient that holds one is made again from the start by the fp32 kernel.  Values and products below 2^-110 lose low pieces to the end of
 // the exponent range (an absolute error below 2^-133).
 #include "conv_common.hpp"
 
@@ -74,11 +74,7 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsig
     p3 = split_round(ra - split_lo(p2), rb - split_hi(p2));
 }
 
-// Marks of a launch: word 0 = any, the others one per tile and block of output channels, several of them to a word where there are more
-// (all of these are then computed again).
 constexpr int PREP_TB = 256;
-constexpr unsigned SPLIT_MARKS = 4096;
-__device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit % (SPLIT_MARKS - 1); }
 
 // packed[s][cb][q][step][piece][h][lane] (16 bytes: two taps of four channels), cb = block of 16 * COH output channels, q = chunk
 // of four contracted channels.  Cm / Ck: channels on the M axis / contracted; with `transposed` the image is that of the
@@ -431,65 +427,13 @@ conv_split_kernel(const ConvArgs<float> a) {
     }
 }
 
-// The marked tiles from the fp32 values: one thread per column, one channel of the input staged at a time.  Rare and slow; a
-// block that finds no mark set ends at once.
-template <class G>
-__global__ void __launch_bounds__(G::NT)
-conv_split_redo_kernel(const ConvArgs<float> a, int n_tiles, int n_cb, int per) {
-    static_assert(G::MAXCOL <= G::NT, "one thread per column");
-    __shared__ float patch[G::CH_STRIDE];
-    if (a.redo[0] == 0) return;
-    for (int u = blockIdx.x; u < n_tiles * n_cb; u += gridDim.x) {          // uniform
-        if (a.redo[split_mark(u)] == 0) continue;
-        const int tile = u % n_tiles, co0 = u / n_tiles * per, co1 = min(co0 + per, a.Cout);
-        const float* __restrict__ w = a.w_raw + (int64_t)min(a.S_exp - 1, a.Lc - a.tiles[tile].level) * a.Cout * a.Cin * G::K;
-        for (int win = a.tile_win[tile]; win < a.tile_win[tile + 1]; ++win) {
-            const int4 hd = a.win[win];
-            const WindowLists l{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z, a.l_col_pos + (unsigned)hd.z};
-            const int col = threadIdx.x, nc = hd.w;
-            const int cell = (col < nc ? (int)(l.col_pos[col] & COL_CELL) : G::TAP0) - G::TAP0;
-#pragma unroll 1
-            for (int m0 = co0; m0 < co1; m0 += 8) {
-                float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-                for (int ci = 0; ci < a.Cin; ++ci) {
-                    __syncthreads();
-                    for (int i = threadIdx.x; i < G::CH_STRIDE; i += G::NT) patch[i] = 0.f;
-                    __syncthreads();
-                    const float* plane = (a.x2 && ci >= a.c_split) ? a.x2 + (int64_t)(ci - a.c_split) * a.ldx2 : a.x + (int64_t)ci * a.ldx;
-                    for (int i = threadIdx.x; i < hd.y; i += G::NT) {
-                        const unsigned pos = l.item_pos[i];
-                        const float v = (pos & ITEM_TREE) ? a.tree_data[(int64_t)ci * a.ldt + l.item_idx[i]] : plane[l.item_idx[i]];
-                        patch[pos & ITEM_CELL] = v;
-                        if (pos & ITEM_PAIR) patch[(pos & ITEM_CELL) + 1] = v;
-                    }
-                    __syncthreads();
-#pragma unroll 1
-                    for (int t = 0; t < G::K; ++t) {
-                        const float v = patch[cell + ((t / (G::KX * G::KY)) * G::RX + (t / G::KY) % G::KX) * G::RS + t % G::KY];
-#pragma unroll
-                        for (int k = 0; k < 8; ++k) acc[k] += w[((int64_t)min(m0 + k, a.Cout - 1) * a.Cin + ci) * G::K + t] * v;
-                    }
-                }
-                if (col >= nc) continue;
-                const int64_t o = l.col_idx[col];
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    if (m0 + k >= co1) continue;
-                    float v = acc[k] + (a.bias ? a.bias[m0 + k] : 0.f);
-                    if (a.relu) v = v < 0.f ? 0.f : v;
-                    a.y[(int64_t)(m0 + k) * a.ldy + o] = v;
-                }
-            }
-        }
-    }
-}
-
 using S333 = ConvGeom<3, 3, 3, 2, 4, 512, 64, 16>;
 using S155 = ConvGeom<1, 5, 5, 1, 8, 512, 64, 16>;
 
 static int split_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
 static int split_nstep(int code) { return code == 333 ? split_steps<S333>() : split_steps<S155>(); }
+
+int launch_conv_redo(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);        // conv_mfma.hip
 
 template <class G, int MODE>
 static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
@@ -498,19 +442,18 @@ static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1, MODE>), grid, dim3(G::NT), 0, st, a);
     else hipLaunchKernelGGL((conv_split_kernel<G, 2, MODE>), grid, dim3(G::NT), 0, st, a);
     APRNET_LAUNCH_CHECK("conv_split_kernel");
-    if (MODE == 1) return 0;
-    hipLaunchKernelGGL(conv_split_redo_kernel<G>, dim3((unsigned)std::min(n_tiles * n_cb, 256)), dim3(G::NT), 0, st, a, n_tiles, n_cb, 16 * coh);
-    APRNET_LAUNCH_CHECK("conv_split_redo_kernel");
     return 0;
 }
 // a.w, a.redo, a.xi, a.ti: what prepare_split made of the weights a.w_raw and of a.x, a.x2 and a.tree_data; a.tile_win ... the forward
 // lists of the plan
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+    int rc;
     switch (code) {
-        case 333: return launch_split<S333, 0>(a, n_tiles, st);
-        case 155: return launch_split<S155, 0>(a, n_tiles, st);
+        case 333: rc = launch_split<S333, 0>(a, n_tiles, st); break;
+        case 155: rc = launch_split<S155, 0>(a, n_tiles, st); break;
+        default: rc = fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
     }
-    return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
+    return rc ? rc : launch_conv_redo(code, a, n_tiles, st);
 }
 // Input gradient: a.x / a.xi / a.Cin describe the output gradient, a.Cout the layer's input channels, a.w the transposed image,
 // a.tile_win ... the input-gradient lists of the plan without the particles on far faces.  a.redo[0] is set if a sum is not finite.

@@ -25,11 +25,11 @@
 // with those after a ReLU.
 //
 // Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
-// NaN), and a value within 2^-9 of the largest fp32 number has an infinite first piece.  Where a result comes out infinite or
-// NaN its tile is marked, and the fp32 instructions compute the marked tiles again (conv_mfma16_redo_kernel; as a call inside this
-// kernel a second pass cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an input
-// gradient that holds one is made again from the start by the fp32 kernel.  Values and products below 2^-110 lose low pieces to the end of
-// the exponent range (an absolute error below 2^-133).
+// NaN), and values of 2^111 and more, or sums of 2^95 and more, are infinite for these kernels (see SPLIT_SCALE).  Where a result comes
+// out infinite or NaN its tile is marked, and the fp32 instructions compute the marked tiles again (conv_mfma16_redo_kernel; as a call
+// inside this kernel a second pass cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an
+// input gradient that holds one is made again from the start by the fp32 kernel.  Small values keep all their bits: features of 1e-37
+// come out with 0.38 of the fp32 instructions' error (split without SPLIT_SCALE, 510 times that error).
 #include "conv_common.hpp"
 
 namespace aprnet {
@@ -65,6 +65,10 @@ __device__ __forceinline__ unsigned split_round(float a, float b) {
 }
 __device__ __forceinline__ float split_lo(unsigned p) { return __builtin_bit_cast(float, p << 16); }
 __device__ __forceinline__ float split_hi(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// What is split lies SPLIT_SCALE times higher than the caller's values (the copies and the packed weights), the results are brought
+// down again: the last bit of any fp32 number, 2^-149 at the least, then is one that a bfloat16 number can hold (2^-133).
+constexpr float SPLIT_SCALE = 65536.f, SPLIT_UNSCALE = 1.f / (SPLIT_SCALE * SPLIT_SCALE);
 
 // two fp32 numbers -> three words with their pieces
 __device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsigned& p2, unsigned& p3) {
@@ -102,7 +106,7 @@ __device__ __forceinline__ void pack_weights_split(const float* __restrict__ w, 
             const int t = SplitTaps<K>::tap[2 * (4 * step + (lane >> 4)) + (j >> 2)], ck = q * SP_CIB + (j & 3);
             v[j] = 0.f;
             if (t >= 0 && cm < Cm && ck < Ck)
-                v[j] = transposed ? w[(((int64_t)s * Cout + ck) * Cin + cm) * K + (K - 1 - t)] : w[(((int64_t)s * Cout + cm) * Cin + ck) * K + t];
+                v[j] = SPLIT_SCALE * (transposed ? w[(((int64_t)s * Cout + ck) * Cin + cm) * K + (K - 1 - t)] : w[(((int64_t)s * Cout + cm) * Cin + ck) * K + t]);
         }
         uint4 p[3];
         split_pair(v[0], v[1], p[0].x, p[1].x, p[2].x);
@@ -116,7 +120,7 @@ __device__ __forceinline__ void pack_weights_split(const float* __restrict__ w, 
 }
 
 // ---- input in groups of four channels: [Cin / 4][count][4] ---------------------------------------------------
-// out[q][i][c] = channel 4 q + c of element i; channels from c_split on come from x2 (null: all from x), channels past C
+// out[q][i][c] = SPLIT_SCALE * channel 4 q + c of element i; channels from c_split on come from x2 (null: all from x), channels past C
 // are zeros.  A streaming pass (8 bytes per value), four elements per thread, all reads issued before the first is used.
 constexpr int IG_E = 4;
 __device__ __forceinline__ void group4(const float* __restrict__ x, int64_t ldx, const float* __restrict__ x2, int64_t ldx2, int c_split, int C, int64_t count,
@@ -140,7 +144,8 @@ __device__ __forceinline__ void group4(const float* __restrict__ x, int64_t ldx,
     float4* dst = out + (int64_t)q * count;
 #pragma unroll
     for (int e = 0; e < IG_E; ++e)
-        if (i0 + e * IG_TB < count) dst[i0 + e * IG_TB] = make_float4(v[0][e], v[1][e], v[2][e], v[3][e]);
+        if (i0 + e * IG_TB < count)
+            dst[i0 + e * IG_TB] = make_float4(SPLIT_SCALE * v[0][e], SPLIT_SCALE * v[1][e], SPLIT_SCALE * v[2][e], SPLIT_SCALE * v[3][e]);
 }
 
 // What the convolution reads, in one launch: the first blocks pack the weights and clear the marks, the others copy the features (nbx
@@ -360,9 +365,9 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
                 for (int r = 0; r < 4; ++r) {
                     const int cl = h * 16 + 4 * (lane >> 4) + r;
                     if (co0 + cl >= a.Cout) continue;
-                    float v = acc[j][h][r];
+                    float v = acc[j][h][r] * SPLIT_UNSCALE;
                     if constexpr (MODE == 0) {
-                        v += sh.bias[cl];
+                        v = fmaf(acc[j][h][r], SPLIT_UNSCALE, sh.bias[cl]);
                         if (a.relu) v = v < 0.f ? 0.f : v;
                         dst[(int64_t)(co0 + cl) * ld] = v;
                     } else if (sole) dst[(int64_t)(co0 + cl) * ld] = v;

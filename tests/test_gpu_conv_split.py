@@ -86,6 +86,23 @@ def test_infinities_and_nan(path, where, cout):
     assert bool(((got.double() - ref).abs() <= 2 * 432 * 2.0 ** -24 * terms)[bounded].all())
 
 
+@pytest.mark.parametrize("x_scale,w_scale", [(1e-33, 1), (1e-36, 1), (1e-38, 1), (1e-41, 1), (1, 1e-35), (1, 1e-38), (1e-36, 1e30), (1e-18, 1e-18), (1e-22, 1e-22)])
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 5, 5)], ids=["k333", "k155"])
+def test_small_operands_keep_their_bits(path, ksize, x_scale, w_scale):
+    """Features, output gradients and weights down to the end of the exponent range: no larger an error than that of the fp32
+    instructions, forward and input gradient.  (The tail of a softmax, or the gradient of a saturated one, lies there.)"""
+    bt = [("3d_s", 0)] if ksize[0] == 3 else [("2d_t", 0)]
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, 16, 16, torch.float32)
+    x, w_exp = x * x_scale, w_exp * w_scale
+    ref = oracle.conv_forward(aprs, x.double(), w_exp.double(), ld)
+    gref = oracle.conv_backward(aprs, x.double(), w_exp.double(), x.double(), ld)[0]
+    xd, wd, err = x.to(DEV), layer(w_exp), {}
+    for p in (19, 20):
+        path(p)
+        err[p] = error(_ops.conv_forward(aprs, xd, wd, ld), ref), error(_ops.conv_backward(aprs, xd, wd, xd, ld)[0], gref)
+    assert err[20][0] <= err[19][0] and err[20][1] <= err[19][1]
+
+
 def nan_places(aprs, ld, x, every):
     x = x.clone()
     for i, a in enumerate(aprs):

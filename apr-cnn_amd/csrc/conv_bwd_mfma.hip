@@ -551,7 +551,7 @@ static int dw_blocks_x(int code, int Cout, int Cin) {
     const int64_t cap = ((int64_t)512 << 20) / (8 * (int64_t)Cout * Cin * dw_taps(code));
     return (int)std::max<int64_t>(16, std::min<int64_t>(std::max(64, 1024 / per), cap));
 }
-// The stencil indices that have windows, and a share of the workgroups for each by its windows.
+// The stencil indices that have windows, and a share of the workgroups for each: one, and of the others by its windows.
 static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists& wl) {
     DwWork k{};
     k.first_coarse = (wl.n_lv > 0 && wl.lv_level[0] == Lc) ? (wl.n_lv > 1 ? wl.lv_first[1] : wl.n_win) : 0;
@@ -561,9 +561,8 @@ static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinL
         if (k.n_s > 0 && k.s_of[k.n_s - 1] == s) { k.nwin[k.n_s - 1] = w1 - k.win0[k.n_s - 1]; continue; }
         k.s_of[k.n_s] = s; k.win0[k.n_s] = w0; k.nwin[k.n_s] = w1 - w0; ++k.n_s;
     }
-    const int64_t bx = dw_blocks_x(code, Cout, Cin);
-    for (int i = 0; i < k.n_s; ++i)                        // (together at most bx + n_s)
-        k.blk0[i + 1] = k.blk0[i] + (int)std::max<int64_t>(1, std::min<int64_t>(k.nwin[i], bx * k.nwin[i] / wl.n_win));
+    const int64_t more = std::max(0, dw_blocks_x(code, Cout, Cin) - k.n_s);
+    for (int i = 0; i < k.n_s; ++i) k.blk0[i + 1] = k.blk0[i] + (int)std::min<int64_t>(k.nwin[i], 1 + more * k.nwin[i] / wl.n_win);
     return k;
 }
 // wl null: the kernels scan

@@ -117,8 +117,8 @@ int aprnet_profile_enable(int on);
  * from the channel planes; and for the weight gradient of the matrix-core
  * kernels: 10 = every workgroup writes the sums of its tiles to its own slots of the plan's scratch buffer and a second
  * kernel adds the slots in a fixed order (default: the gradient repeats bit for bit from call to call on a plan; at most 512 MiB
- * of scratch, for very wide layers 32 times the gradient of one stencil, or the gradient itself where bfloat16 features
- * are staged from grouped copies), 11 = atomic additions; and for forward layers of 1 to 3 input channels (bound by memory, not by the
+ * of scratch, for very wide layers 32 times the gradient of one stencil (or twice the gradient of all, where there are more than
+ * 16), or the gradient itself where bfloat16 features are staged from grouped copies), 11 = atomic additions; and for forward layers of 1 to 3 input channels (bound by memory, not by the
  * contraction): 12 = the pipelined kernel with the (tap, channel) axis flattened (default), 13 = the general kernel;
  * and for the bfloat16 forward kernel on grouped tensors: 14 = 32-bit byte offsets where a group holds fewer than 2^28
  * elements, 64-bit addresses beyond (default), 15 = 64-bit addresses always; and for the tree fill that precedes a

@@ -1,9 +1,11 @@
 """Plan housekeeping around HIP graphs: the scratch buffer of a plan never moves under a captured graph, and what
 would have to allocate during a capture is an error code instead of a failed capture."""
+import numpy as np
 import pytest
 import torch
 
 import apr_cases
+from pyapr import APR
 from pyapr.aprnet import _ops
 
 pytestmark = pytest.mark.gpu
@@ -112,3 +114,25 @@ def test_aprs_built_beside_plans_that_come_and_go(dtype):
             for a, b in zip(apr.get_state()[4:], want[k]):
                 assert (a == b).all()
             del apr
+
+
+def test_partial_sums_of_a_very_wide_layer_stay_within_their_limit():
+    """3x3x3 512 -> 512: the gradient of one stencil is 28 MB, and the weight gradient's partial sums take 32 of them at most, however
+    many stencils (levels) have windows.  Scratch memory is the plan's own, outside torch's allocator."""
+    c, shape = 512, (2, 8, 8192)
+    field = np.zeros((1, 4, 4096), np.uint8)
+    field[:, :, :550] = 13                                           # fine at one end, a few particles on each of eleven coarser levels
+    ld, used = torch.zeros(1, dtype=torch.int32), []
+    for _ in range(2):                                               # (the first turn: torch's own allocations)
+        apr = APR.from_level_field(shape, field)
+        it = apr.iterator()
+        assert sum(it.particles_level_end(lv) > it.particles_level_begin(lv) for lv in range(apr.level_min(), 14)) == 12
+        n = apr.total_number_particles()
+        x, w = torch.randn(1, c, n, device=DEV), torch.randn(apr.level_max() - apr.level_min() + 1, c, c, 3, 3, 3, device=DEV) * 0.01
+        apr.init_cuda()
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        _ops.conv_backward([apr], x, w, x, ld, need_input_grad=False)
+        torch.cuda.synchronize()
+        used.append(free - torch.cuda.mem_get_info()[0])
+    assert used[1] <= 32 * c * c * 27 * 4 + (64 << 20)               # (lists and tables of 18 k particles, in whole pages)

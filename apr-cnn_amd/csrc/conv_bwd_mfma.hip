@@ -15,7 +15,7 @@
 // A block owns 16 input channels (four staged chunks of 4) and 32 output channels.  Wave w takes input
 // channel w%4 of every chunk and half of the columns (w/4), so it holds four accumulators, and keeps them
 // in registers while the (persistent) block walks over many windows of one stencil index (one launch
-// for all of them, see DwWork); its sums go to slots of its own, which sum_slots.hpp adds up in a fixed order.  The patch rows are 67 words
+// for all of them, see DwWork); its sums go to slots of its own (see DW_CHAINS), which sum_slots.hpp adds up in a fixed order.  The patch rows are 67 words
 // apart so that the 27 tap offsets of a B read fall into 27 different LDS banks.
 #include "conv_common.hpp"
 #include "sum_slots.hpp"
@@ -36,14 +36,52 @@ constexpr int DW_KB = 8;          // MFMAs issued back to back between operand p
 constexpr int DW_GLD = 33;         // words per column of gyl (32 output channels + 1 against bank conflicts)
 
 // Work of a launch on the plan's window lists: workgroups blk0[k] .. blk0[k + 1] - 1 (grid.x) take the windows of stencil
-// index s_of[k] in turn.  One launch covers all stencil indices: with a launch and a sum of slots each, most of them left the chip
+// index s_of[k].  One launch covers all stencil indices: with a launch and a sum of slots each, most of them left the chip
 // idle (the coarse levels have a handful of windows), and the weight gradients of a training step of the 16-32-64-128 network on
 // two APRs of 338 k particles took 76 + 102 launches; now 28 + 28, and the step 14.4 instead of 15.8 ms.
 struct DwWork {
     int n_s;
     int s_of[MAX_LEVELS + 1], win0[MAX_LEVELS + 1], nwin[MAX_LEVELS + 1], blk0[MAX_LEVELS + 2];
+    int chain[MAX_LEVELS + 1];     // windows whose products are added up in registers before the sums go to the slots
     int first_coarse;              // windows from here on may stage tree nodes (below the finest level of the call)
 };
+
+// Partial sums of one workgroup and column half, rows of output channels from co0 on: its slot, or (no slots) the result itself.
+struct DwSlot {
+    __amdgpu_buffer_rsrc_t rs;
+    float* p; bool own; int co_n, Cin, K;
+    template <typename T>
+    __device__ __forceinline__ DwSlot(const ConvArgs<T>& a, int co0, int kh, int rows, int K_, int s) : own(a.gw_part != nullptr), co_n(min(rows, a.Cout - co0)), Cin(a.Cin), K(K_) {
+        p = (own ? a.gw_part + (int64_t)(2 * blockIdx.x + kh) * a.gw_part_ld : a.gw + (int64_t)s * a.Cout * Cin * K) + (int64_t)co0 * Cin * K;
+        rs = __builtin_amdgcn_make_buffer_rsrc(p, 0, co_n * Cin * K * 4, 0x00020000);
+    }
+    // first: nothing is in the slot yet.  Later sums come by atomic additions, which are not waited for; the lane that wrote an element is
+    // the only one that adds to it, so they arrive in the order of the program.
+    __device__ __forceinline__ void add(int row, int ci, int t, float v, bool first) const {
+        const bool in = t < K && row < co_n;
+        const int e = (row * Cin + ci) * K + t;
+        if (own && first) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), rs, in ? e * 4 : (int)BUF_OOB, 0, 0);      // (past the end: not written)
+        else if (in && v != 0.f) unsafeAtomicAdd(p + e, v);
+    }
+};
+
+// The windows of this workgroup in turn, window(lists, columns, items, tree items) for each; flush(s, first) after every chain[k] of them
+// and after the last one.
+template <class G, typename T, class Window, class Flush>
+__device__ __forceinline__ void dw_walk(const ConvArgs<T>& a, const DwWork& wk, Window window, Flush flush) {
+    int si = 0;
+    while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
+    const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si], chain = wk.chain[si], s = wk.s_of[si];
+    int left = chain;
+    bool first = true;
+    for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
+        const int4 hd = a.win[w];
+        const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+        const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z, a.l_col_pos + (unsigned)hd.z};
+        window(gl, nc, nitem, w >= wk.first_coarse);
+        if (--left == 0 || w + step >= w_end) { flush(s, first); left = chain; first = false; }
+    }
+}
 
 // Lists of the plan carry patch cells for rows of 64 words; this kernel's rows are RS words apart.
 template <class G> __device__ __forceinline__ unsigned restride(unsigned pos) {
@@ -264,20 +302,25 @@ conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
 #pragma unroll
             for (int r = 0; r < 4; ++r) acc[q][tile][r] = 0.f;
 
-    int s_idx = s_arg;
+    // the sums so far to this workgroup's slot of its column half (first: they start it)
+    auto flush = [&](const int s, const bool first) {
+        int l = lane;
+        asm volatile("" : "+v"(l));         // addresses formed per call, not kept (and spilled) across the window loop
+        const DwSlot slot(a, 0, kh, 16, G::K, s);
+#pragma unroll
+        for (int q = 0; q < NCH; ++q)
+#pragma unroll
+            for (int tile = 0; tile < 2; ++tile)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (cig0 + q * CIB + cil < a.Cin) slot.add(4 * (l >> 4) + r, cig0 + q * CIB + cil, (l & 15) + 16 * tile, acc[q][tile][r], first);
+                    acc[q][tile][r] = 0.f;
+                }
+    };
     if constexpr (LISTS) {
-        int si = 0;
-        while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
-        s_idx = wk.s_of[si];
-        const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si];
-        for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
-            const int4 hd = a.win[w];
-            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-            const bool tree_items = w >= wk.first_coarse;
-            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
-                                 a.l_col_pos + (unsigned)hd.z};
+        dw_walk<G>(a, wk, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
             dw_window16<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, bl, kh, wave, lane, patch, gyl, cpl, acc);
-        }
+        }, flush);
     } else {
         for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
             const ConvTile tile = a.tiles[ti];
@@ -299,21 +342,7 @@ conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
                 __syncthreads();
             }
         }
-    }
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-        const int ci = cig0 + q * CIB + cil;
-#pragma unroll
-        for (int tile = 0; tile < 2; ++tile)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int co = 4 * (lane >> 4) + r, t = (lane & 15) + 16 * tile;
-                if (t < G::K && ci < a.Cin && co < a.Cout) {
-                    const int64_t e = ((int64_t)co * a.Cin + ci) * G::K + t;
-                    if (a.gw_part) a.gw_part[(int64_t)(2 * blockIdx.x + kh) * a.gw_part_ld + e] = acc[q][tile][r];
-                    else if (acc[q][tile][r] != 0.f) unsafeAtomicAdd(a.gw + (int64_t)s_idx * a.Cout * a.Cin * G::K + e, acc[q][tile][r]);
-                }
-            }
+        flush(s_arg, true);
     }
 }
 
@@ -412,20 +441,23 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const DwWork wk, const int s_arg) 
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
 
-    int s_idx = s_arg;
+    // the sums so far to this workgroup's slot of its column half (first: they start it)
+    auto flush = [&](const int s, const bool first) {
+        int l = lane;
+        asm volatile("" : "+v"(l));         // addresses formed per call, not kept (and spilled) across the window loop
+        const DwSlot slot(a, co0, kh, 32, G::K, s);
+#pragma unroll
+        for (int q = 0; q < NCH; ++q)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (cig0 + q * CIB + cil < a.Cin) slot.add(4 * (l >> 5) + 8 * (r >> 2) + (r & 3), cig0 + q * CIB + cil, l & 31, acc[q][r], first);
+                acc[q][r] = 0.f;
+            }
+    };
     if constexpr (LISTS) {
-        int si = 0;
-        while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
-        s_idx = wk.s_of[si];
-        const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si];
-        for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
-            const int4 hd = a.win[w];
-            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-            const bool tree_items = w >= wk.first_coarse;
-            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
-                                 a.l_col_pos + (unsigned)hd.z};
+        dw_walk<G>(a, wk, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
             dw_window_bf16<G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, acc);
-        }
+        }, flush);
     } else {
         for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
             const ConvTile tile = a.tiles[ti];
@@ -447,19 +479,7 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const DwWork wk, const int s_arg) 
                 __syncthreads();
             }
         }
-    }
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-        const int ci = cig0 + q * CIB + cil;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int co = co0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-            if (t < G::K && ci < a.Cin && co < a.Cout) {
-                const int64_t e = ((int64_t)co * a.Cin + ci) * G::K + t;
-                if (a.gw_part) a.gw_part[(int64_t)(2 * blockIdx.x + kh) * a.gw_part_ld + e] = acc[q][r];
-                else if (acc[q][r] != 0.f) unsafeAtomicAdd(a.gw + (int64_t)s_idx * a.Cout * a.Cin * G::K + e, acc[q][r]);
-            }
-        }
+        flush(s_arg, true);
     }
 }
 
@@ -489,20 +509,23 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[q][r] = 0.f;
 
-    int s_idx = s_arg;
+    // the sums so far to this workgroup's slot of its column half (first: they start it)
+    auto flush = [&](const int s, const bool first) {
+        int l = lane;
+        asm volatile("" : "+v"(l));         // addresses formed per call, not kept (and spilled) across the window loop
+        const DwSlot slot(a, co0, kh, 32, G::K, s);
+#pragma unroll
+        for (int q = 0; q < NCH; ++q)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (cig0 + q * CIB + cil < a.Cin) slot.add(4 * (l >> 5) + 8 * (r >> 2) + (r & 3), cig0 + q * CIB + cil, l & 31, acc[q][r], first);
+                acc[q][r] = 0.f;
+            }
+    };
     if constexpr (LISTS) {
-        int si = 0;
-        while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
-        s_idx = wk.s_of[si];
-        const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si];
-        for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
-            const int4 hd = a.win[w];
-            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-            const bool tree_items = w >= wk.first_coarse;
-            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z,
-                                 a.l_col_pos + (unsigned)hd.z};
+        dw_walk<G>(a, wk, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
             dw_window<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, ap, acc);
-        }
+        }, flush);
     } else {
         for (int ti = blockIdx.x; ti < a.n_tiles; ti += gridDim.x) {
             const ConvTile tile = a.tiles[ti];
@@ -524,33 +547,32 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
                 __syncthreads();
             }
         }
-    }
-#pragma unroll
-    for (int q = 0; q < NCH; ++q) {
-        const int ci = cig0 + q * CIB + cil;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int co = co0 + 8 * (r >> 2) + 4 * hi + (r & 3);
-            if (t < G::K && ci < a.Cin && co < a.Cout) {
-                const int64_t e = ((int64_t)co * a.Cin + ci) * G::K + t;
-                if (a.gw_part) a.gw_part[(int64_t)(2 * blockIdx.x + kh) * a.gw_part_ld + e] = acc[q][r];
-                else if (acc[q][r] != 0.f) unsafeAtomicAdd(a.gw + (int64_t)s_idx * a.Cout * a.Cin * G::K + e, acc[q][r]);
-            }
-        }
+        flush(s_arg, true);
     }
 }
 
 static int dw_taps(int code) { return code == 333 ? 27 : code == 133 ? 9 : 25; }
 // a narrow input (the first layer of a network) fits one chunk: no staging and products of empty chunks
 static int dw_chunks(int Cin) { return Cin <= DW_CIB ? 1 : DW_NCH; }
-// Workgroups along grid.x: two rounds of the 512 that the chip holds, fewer for layers with several channel blocks, whose every
-// window is visited once per block, and for very wide layers, so that the partial sums (two slots per workgroup) stay
-// within 512 MiB.
+// Slots for partial sums: two for each of `blocks` workgroups along grid.x, within 512 MiB, but 16 workgroups at least.
+static int dw_slot_cap(int code, int Cout, int Cin, int blocks) {
+    const int64_t cap = ((int64_t)512 << 20) / (8 * (int64_t)Cout * Cin * dw_taps(code));
+    return (int)std::max<int64_t>(16, std::min<int64_t>(blocks, cap));
+}
+// Workgroups along grid.x of a launch on lists: the 512 that the chip holds, two rounds of them for layers of one channel block.
 static int dw_blocks_x(int code, int Cout, int Cin) {
     const int nci = DW_CIB * dw_chunks(Cin), per = ((Cin + nci - 1) / nci) * ((Cout + 31) / 32);
-    const int64_t cap = ((int64_t)512 << 20) / (8 * (int64_t)Cout * Cin * dw_taps(code));
-    return (int)std::max<int64_t>(16, std::min<int64_t>(std::max(64, 1024 / per), cap));
+    return dw_slot_cap(code, Cout, Cin, std::max(512, 1024 / per));
 }
+// Windows whose products a workgroup adds up in registers before the sums go to its slots: the relative error of a sum of n products
+// of either sign grows with the root of the additions that one accumulator sees.  A chain ends after a 512th of the stencil index's
+// windows (of fewer where the slots are, see above), but not before DW_SHORT windows: the few windows of a coarse level in chains of one
+// cost 3 to 10 % for nothing, since their gradient's error is below that of the finest level's all the same.
+// 64 -> 64 channels on 2.8 M particles, error against 64 bits 0.85e-6, 9.7 ms, with 128 workgroups and chains to their end 1.95e-6, 9.9 ms;
+// on 320 k 0.34e-6, 1.54 ms (0.63e-6, 1.38); 128 -> 128 on 320 k 0.52e-6, 4.95 ms (0.87e-6, 4.75); 32 -> 32 on 9.8 M 1.38e-6, 8.95 ms
+// (1.66e-6, 8.75); 16 -> 16 on 9.8 M 1.14e-6, 3.19 ms (1.15e-6, 3.20).  Read back, added and stored instead of added by atomic
+// operations that nobody waits for, 64 -> 64 took 11.5 and 1.73 ms.
+constexpr int DW_CHAINS = 512, DW_SHORT = 4;
 // The stencil indices that have windows, and a share of the workgroups for each: one, and of the others by its windows.
 static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists& wl) {
     DwWork k{};
@@ -561,13 +583,17 @@ static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinL
         if (k.n_s > 0 && k.s_of[k.n_s - 1] == s) { k.nwin[k.n_s - 1] = w1 - k.win0[k.n_s - 1]; continue; }
         k.s_of[k.n_s] = s; k.win0[k.n_s] = w0; k.nwin[k.n_s] = w1 - w0; ++k.n_s;
     }
-    const int64_t more = std::max(0, dw_blocks_x(code, Cout, Cin) - k.n_s);
-    for (int i = 0; i < k.n_s; ++i) k.blk0[i + 1] = k.blk0[i] + (int)std::min<int64_t>(k.nwin[i], 1 + more * k.nwin[i] / wl.n_win);
+    const int chains = dw_slot_cap(code, Cout, Cin, DW_CHAINS), most = *std::max_element(k.nwin, k.nwin + k.n_s), longest = (most + chains - 1) / chains;
+    const int64_t more = std::max(0, dw_slot_cap(code, Cout, Cin, dw_blocks_x(code, Cout, Cin)) - k.n_s);
+    for (int i = 0; i < k.n_s; ++i) {
+        k.blk0[i + 1] = k.blk0[i] + (int)std::min<int64_t>(k.nwin[i], 1 + more * k.nwin[i] / wl.n_win);
+        k.chain[i] = std::max((k.nwin[i] + chains - 1) / chains, std::min(DW_SHORT, longest));
+    }
     return k;
 }
 // wl null: the kernels scan
 size_t conv_dw_partial_bytes(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists* wl) {
-    const int blocks = wl ? [&] { const DwWork k = dw_work(code, Cout, Cin, S_exp, Lc, *wl); return k.blk0[k.n_s]; }() : dw_blocks_x(code, Cout, Cin);
+    const int blocks = wl ? [&] { const DwWork k = dw_work(code, Cout, Cin, S_exp, Lc, *wl); return k.blk0[k.n_s]; }() : dw_slot_cap(code, Cout, Cin, DW_CHAINS);
     return (size_t)(2 * blocks) * Cout * Cin * dw_taps(code) * sizeof(float);
 }
 
@@ -622,7 +648,7 @@ static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, const WinLists* 
         if (n == 0) continue;
         ConvArgs<T> a = a0;
         a.tiles = tl.d_tiles + tl.level_begin[l_hi]; a.n_tiles = n;
-        const int blocks = std::min(n, a.gw_part ? dw_blocks_x(code, a.Cout, a.Cin) : 512);
+        const int blocks = std::min(n, a.gw_part ? dw_slot_cap(code, a.Cout, a.Cin, DW_CHAINS) : DW_CHAINS);
         if (int rc = launch_dw_kernel<T, G, false>(a, DwWork{}, s, blocks, st)) return rc;
         if (a.gw_part)
             if (int rc = launch_sum_slots((const float*)a.gw_part, a.gw_part_ld, 2 * blocks, n_el, (float*)a.gw + (int64_t)s * n_el, st)) return rc;

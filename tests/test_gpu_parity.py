@@ -9,7 +9,7 @@ import torch
 
 import apr_cases
 from oracle import oracle
-from pyapr import _native
+from pyapr import APR, _native
 from pyapr.aprnet import _ops
 
 pytestmark = pytest.mark.gpu
@@ -1108,3 +1108,27 @@ def test_conv_backward_bf16_groups_of_coarser_particles(shape, ksize, cin, cout)
     if all(s % 2 == 0 for s in shape[1:]) and all(v % 2 == 0 or v == 1 for lv in range(apr.level_min() + 1, apr.level_max() + 1)
                                                  for v in (apr.iterator().z_num(lv), apr.iterator().x_num(lv), apr.iterator().y_num(lv))):
         assert all(torch.equal(gx, run()) for _ in range(3))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16_planes"])
+def test_weight_gradient_error_of_a_wide_layer(dtype):
+    """64 -> 64 channels on 1.8 M particles of one level: 4608 windows of at most 384 columns, so no accumulator sees more than nine of
+    them, half of the columns each: 1728 additions.  A sum of n rounded additions of products of either sign is off by sqrt(n / 2) of a
+    rounding error in the root mean square, 0.41 * 2^-24 of the sum each (uniform within half a unit, averaged over a binade)."""
+    shape, c = (96, 96, 192), 64
+    apr = APR.from_level_field(shape, np.full((48, 48, 96), 8, np.uint8))
+    n, ld = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32)
+    assert n == 96 * 96 * 192
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    x = torch.randn(1, c, n, device=DEV, generator=gen).to(dtype)
+    gy = (0.5 + torch.rand(1, c, n, device=DEV, generator=gen)).to(dtype)
+    w = torch.zeros(apr.level_max() - apr.level_min() + 1, c, c, 3, 3, 3, device=DEV)
+    lib = _native.hip()
+    lib.aprnet_set_conv_path(9)                      # (bfloat16: the kernel on channel planes, the one that shares its work list with fp32)
+    try:
+        got = _ops.conv_backward([apr], x, w, gy, ld, need_input_grad=False)[1][0].double()
+    finally:
+        lib.aprnet_set_conv_path(8)
+    ref = _ops.conv_backward([apr], x.double(), w.double(), gy.double(), ld, need_input_grad=False)[1][0]
+    error = float((got - ref).norm() / ref.norm())
+    assert error <= 1.5 * 0.41 * 2.0 ** -24 * (1728 / 2) ** 0.5

@@ -88,6 +88,7 @@ struct WinLists {
     bool unavailable = false;                   // building them failed once (no memory, too many entries): do not retry
     // the levels that have windows, in window order (finest first): first window and level of each
     int n_lv = 0; int lv_first[MAX_LEVELS] = {}; int lv_level[MAX_LEVELS] = {};
+    int64_t lv_cols[MAX_LEVELS] = {};           // columns of each
 };
 
 // Tree nodes whose mean a convolution reads (need.hip): per tree level an ascending list of node indices in `d_nodes`.

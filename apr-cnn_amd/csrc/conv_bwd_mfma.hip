@@ -42,6 +42,8 @@ constexpr int DW_GLD = 33;         // words per column of gyl (32 output channel
 struct DwWork {
     int n_s;
     int s_of[MAX_LEVELS + 1], win0[MAX_LEVELS + 1], nwin[MAX_LEVELS + 1], blk0[MAX_LEVELS + 2];
+    // The windows of an index are cut into n_run runs of len or (the first `rem`) len + 1 neighbours, which its workgroups take in turn.
+    int n_run[MAX_LEVELS + 1], len[MAX_LEVELS + 1], rem[MAX_LEVELS + 1];
     int chain[MAX_LEVELS + 1];     // windows whose products are added up in registers before the sums go to the slots
     int first_coarse;              // windows from here on may stage tree nodes (below the finest level of the call)
 };
@@ -71,15 +73,19 @@ template <class G, typename T, class Window, class Flush>
 __device__ __forceinline__ void dw_walk(const ConvArgs<T>& a, const DwWork& wk, Window window, Flush flush) {
     int si = 0;
     while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
-    const int w_end = wk.win0[si] + wk.nwin[si], step = wk.blk0[si + 1] - wk.blk0[si], chain = wk.chain[si], s = wk.s_of[si];
+    const int n_run = wk.n_run[si], len = wk.len[si], rem = wk.rem[si], win0 = wk.win0[si], step = wk.blk0[si + 1] - wk.blk0[si];
+    const int chain = wk.chain[si], s = wk.s_of[si];
     int left = chain;
     bool first = true;
-    for (int w = wk.win0[si] + (int)blockIdx.x - wk.blk0[si]; w < w_end; w += step) {
-        const int4 hd = a.win[w];
-        const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-        const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z, a.l_col_pos + (unsigned)hd.z};
-        window(gl, nc, nitem, w >= wk.first_coarse);
-        if (--left == 0 || w + step >= w_end) { flush(s, first); left = chain; first = false; }
+    for (int run = (int)blockIdx.x - wk.blk0[si]; run < n_run; run += step) {
+        const int w0 = win0 + run * len + min(run, rem), w1 = w0 + len + (run < rem ? 1 : 0);
+        for (int w = w0; w < w1; ++w) {
+            const int4 hd = a.win[w];
+            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+            const WindowLists gl{a.l_item_idx + (unsigned)hd.x, a.l_item_pos + (unsigned)hd.x, a.l_col_idx + (unsigned)hd.z, a.l_col_pos + (unsigned)hd.z};
+            window(gl, nc, nitem, w >= wk.first_coarse);
+            if (--left == 0 || (w + 1 == w1 && run + step >= n_run)) { flush(s, first); left = chain; first = false; }
+        }
     }
 }
 
@@ -573,20 +579,33 @@ static int dw_blocks_x(int code, int Cout, int Cin) {
 // (1.66e-6, 8.75); 16 -> 16 on 9.8 M 1.14e-6, 3.19 ms (1.15e-6, 3.20).  Read back, added and stored instead of added by atomic
 // operations that nobody waits for, 64 -> 64 took 11.5 and 1.73 ms.
 constexpr int DW_CHAINS = 512, DW_SHORT = 4;
-// The stencil indices that have windows, and a share of the workgroups for each: one, and of the others by its windows.
+// Neighbouring windows of a run, where there are that many per workgroup: they read the same lines along y.  64 -> 64 channels on 320 k
+// particles 1.54 -> 1.47 ms, 32 -> 32 0.47 -> 0.45 ms; runs of 16, whose windows are dense or sparse together, 32 -> 32 on 9.8 M 9.0 -> 9.7 ms.
+constexpr int DW_RUN = 4;
+// A window without a column costs a workgroup about what 256 columns cost it.  By windows alone the finest level's workgroups, whose windows
+// are fuller, were the last to end: backward pass of 1x5x5 64 -> 64 on bfloat16
+// planes, 15.4 M particles, 29.0 -> 28.3 ms (32.3 with 128 workgroups), 32 -> 32 on 2.8 M 2.83 -> 2.72 ms.
+constexpr int DW_WINDOW_COST = 256;
+// The stencil indices that have windows, and a share of the workgroups for each: one, and of the others by the cost of its windows.
 static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists& wl) {
     DwWork k{};
     k.first_coarse = (wl.n_lv > 0 && wl.lv_level[0] == Lc) ? (wl.n_lv > 1 ? wl.lv_first[1] : wl.n_win) : 0;
+    int64_t cost[MAX_LEVELS + 1] = {}, total = 0;
     for (int i = 0; i < wl.n_lv; ++i) {                    // finest level first: stencil indices ascend
         const int s = std::min(S_exp - 1, Lc - wl.lv_level[i]);
         const int w0 = wl.lv_first[i], w1 = i + 1 < wl.n_lv ? wl.lv_first[i + 1] : wl.n_win;
-        if (k.n_s > 0 && k.s_of[k.n_s - 1] == s) { k.nwin[k.n_s - 1] = w1 - k.win0[k.n_s - 1]; continue; }
-        k.s_of[k.n_s] = s; k.win0[k.n_s] = w0; k.nwin[k.n_s] = w1 - w0; ++k.n_s;
+        if (k.n_s == 0 || k.s_of[k.n_s - 1] != s) { k.s_of[k.n_s] = s; k.win0[k.n_s] = w0; ++k.n_s; }
+        k.nwin[k.n_s - 1] = w1 - k.win0[k.n_s - 1];
+        const int64_t c = wl.lv_cols[i] + (int64_t)DW_WINDOW_COST * (w1 - w0);
+        cost[k.n_s - 1] += c; total += c;
     }
-    const int chains = dw_slot_cap(code, Cout, Cin, DW_CHAINS), most = *std::max_element(k.nwin, k.nwin + k.n_s), longest = (most + chains - 1) / chains;
-    const int64_t more = std::max(0, dw_slot_cap(code, Cout, Cin, dw_blocks_x(code, Cout, Cin)) - k.n_s);
+    const int chains = dw_slot_cap(code, Cout, Cin, DW_CHAINS), longest = (*std::max_element(k.nwin, k.nwin + k.n_s) + chains - 1) / chains;
+    const int64_t more = std::max(0, dw_blocks_x(code, Cout, Cin) - k.n_s);
     for (int i = 0; i < k.n_s; ++i) {
-        k.blk0[i + 1] = k.blk0[i] + (int)std::min<int64_t>(k.nwin[i], 1 + more * k.nwin[i] / wl.n_win);
+        const int nb = (int)std::min<int64_t>(k.nwin[i], 1 + more * cost[i] / total);
+        k.blk0[i + 1] = k.blk0[i] + nb;
+        k.n_run[i] = nb * std::max(1, k.nwin[i] / (nb * DW_RUN));              // at most nwin: no run is empty
+        k.len[i] = k.nwin[i] / k.n_run[i]; k.rem[i] = k.nwin[i] % k.n_run[i];
         k.chain[i] = std::max((k.nwin[i] + chains - 1) / chains, std::min(DW_SHORT, longest));
     }
     return k;

@@ -176,7 +176,10 @@ int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, Win
         for (int l = MAX_LEVELS; l >= 0; --l) {        // tiles are sorted finest level first
             if (tl.level_count[l] <= 0) continue;
             const int fw = tile_win[tl.level_begin[l]], lw = tile_win[tl.level_begin[l] + tl.level_count[l]];
-            if (lw > fw) { wl.lv_first[wl.n_lv] = fw; wl.lv_level[wl.n_lv] = l; ++wl.n_lv; }
+            if (lw <= fw) continue;
+            wl.lv_first[wl.n_lv] = fw; wl.lv_level[wl.n_lv] = l;
+            for (int t = 0; t < tl.level_count[l]; ++t) wl.lv_cols[wl.n_lv] += counts[tl.level_begin[l] + t].z;
+            ++wl.n_lv;
         }
         auto alloc = [&](void** q, size_t bytes) -> int { APRNET_HIP_CHECK(hipMalloc(q, std::max<size_t>(bytes, 16))); return 0; };
         int rc = alloc((void**)&d_offs, (size_t)tl.n * sizeof(int4));

@@ -21,15 +21,15 @@
 // (15.3) ms; the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
 // Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: matrix pipes busy 46 %,
 // vector ALU 15 %, LDS 56 % of the cycles.
-// Error against 64 bits (2-norm, 16 to 128 channels): 0.37 to 0.40 of the fp32 instructions' with N(0, 1) features, 0.44 to 0.49
-// with those after a ReLU.
+// Error against 64 bits (2-norm): 0.31 to 0.33 of the fp32 instructions' with N(0, 1) features, 0.31 to 0.35 with those after a ReLU, below theirs
+// also where few products are not zero, but for a single one (1.02; see split_window).
 //
 // Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
 // NaN), and values of 2^111 and more, or sums of 2^95 and more, are infinite for these kernels (see SPLIT_SCALE).  Where a result comes
 // out infinite or NaN its tile is marked, and the fp32 instructions compute the marked tiles again (conv_mfma16_redo_kernel; as a call
-// inside this kernel a second pass cost registers: 16 -> 16 channels 3.47 instead of 3.26 ms before the products were summed apart); an
+// inside this kernel a second pass cost registers: 16 -> 16 channels on 23 M particles 3.47 instead of 3.26 ms); an
 // input gradient that holds one is made again from the start by the fp32 kernel.  Small values keep all their bits: features of 1e-37
-// come out with 0.38 of the fp32 instructions' error (split without SPLIT_SCALE, 510 times that error).
+// come out with 0.4 of the fp32 instructions' error (split without SPLIT_SCALE, 510 times that error).
 #include "conv_common.hpp"
 
 namespace aprnet {
@@ -243,11 +243,16 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     const __amdgpu_buffer_rsrc_t rcp = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(gl.col_pos), 0, nc * 2, 0x00020000);
 #pragma unroll
     for (int j = 0; j < NB; ++j) cell[j] = (int)__builtin_amdgcn_raw_buffer_load_b16(rcp, (((first + G::NWAVE * j) << 4) + (lane & 15)) * 2, 0, 0);
-    floatx4s acc[NBA][COH];
+    // Sums of x1 w1, and of the five products below 2^-8 of it: the large ones are rounded once per step, like a chain of fp32
+    // multiply-adds or less often.  (Error against 64 bits relative to the fp32 instructions', 3x3x3, 32 channels: 0.32 dense, 0.35 after a ReLU;
+    // where weights are zero but 2, 9 or 27 of them 0.85, 0.54, 0.45; a single product 1.02, what is left out.  With the five summed per step and
+    // added to the sum so far, a second rounding: 0.38, 0.44; 1.30, 1.20, 1.01.  32 -> 32 channels on 23 M particles 11.8 and 11.7 ms, 16 -> 16
+    // on 43 M 9.35 and 9.13, 64 -> 64 on 8 M 19.6 and 19.4, 1x5x5 16 -> 16 on 2 M 0.63 and 0.95.)
+    floatx4s acc[NBA][COH], low[NBA][COH];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
-        for (int h = 0; h < COH; ++h) acc[j][h] = floatx4s{0.f, 0.f, 0.f, 0.f};
+        for (int h = 0; h < COH; ++h) acc[j][h] = low[j][h] = floatx4s{0.f, 0.f, 0.f, 0.f};
 
     constexpr int W16 = NSTEP * 3 * COH * 64;                    // 16-byte elements of a weight chunk
     constexpr int WPT = (W16 + G::NT - 1) / G::NT;
@@ -265,9 +270,14 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
         cell[j] = col < nc ? ((cell[j] & (int)COL_CELL) - G::TAP0) * 8 : 0;
     }
     load_values_split<G>(a, 0, nitem, tree_items, R);
-    load_weights(0);
+    // With 32 outputs the weights of a chunk are asked for in front of the barrier that ends the chunk before it, whose operands no longer
+    // need registers then (next to that chunk's products: 88 instead of 34 registers spilled, 32 -> 32 on 23 M particles 12.05 instead of
+    // 11.8 ms).  With 16 outputs they travel with the values (16 -> 16 on 43 M 9.35 ms, in front of the barrier 10.3).
+    constexpr bool LATE = COH == 2;
+    if constexpr (!LATE) load_weights(0);
     for (int i = threadIdx.x; i < 3 * G::CH_STRIDE / 2; i += G::NT) reinterpret_cast<uint4*>(sh.patch)[i] = make_uint4(0u, 0u, 0u, 0u);
     for (int ci0 = 0; ci0 < a.Cin; ci0 += SP_CIB) {
+        if constexpr (LATE) load_weights(ci0 / SP_CIB);
         __syncthreads();
         store_items_split<G, COH>(R, nitem, sh);
 #pragma unroll
@@ -278,7 +288,7 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
         __syncthreads();
         if (ci0 + SP_CIB < a.Cin) {
             load_values_split<G>(a, ci0 / SP_CIB + 1, nitem, tree_items, R);
-            load_weights(ci0 / SP_CIB + 1);
+            if constexpr (!LATE) load_weights(ci0 / SP_CIB + 1);
         }
         if constexpr (NB > 0) {
             const uintx4s* wa = reinterpret_cast<const uintx4s*>(sh.w) + lane;
@@ -307,21 +317,19 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
                         const uintx2s u = *reinterpret_cast<const uintx2s*>(qa + i * PL), v = *reinterpret_cast<const uintx2s*>(qb + i * PL);
                         b[i] = __builtin_bit_cast(bf16x8s, uintx4s{u.x, u.y, v.x, v.y});
                     }
-                    // the five products below 2^-8 of the first among themselves: the sum so far is rounded twice per step and not six
-                    // times (error 0.45 instead of 1.15 of the fp32 instructions' with ReLU's zeros among the features; 32 -> 32
-                    // channels on 23 M particles 9.5 instead of 9.2 ms).  All six apart: 0.32 and 9.9 ms.
-                    floatx4s t[COH];
-#define APRNET_PRODUCT(C, A, B) _Pragma("unroll") for (int h = 0; h < COH; ++h) t[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[h], B, C, 0, 0, 0);
-                    APRNET_PRODUCT((floatx4s{0.f, 0.f, 0.f, 0.f}), a3, b[0]) APRNET_PRODUCT(t[h], a1, b[2]) APRNET_PRODUCT(t[h], a2, b[1])
-                    APRNET_PRODUCT(t[h], a2, b[0]) APRNET_PRODUCT(t[h], a1, b[1])
-#pragma unroll
-                    for (int h = 0; h < COH; ++h) acc[j][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[h], b[0], acc[j][h], 0, 0, 0) + t[h];
+#define APRNET_PRODUCT(C, A, B) _Pragma("unroll") for (int h = 0; h < COH; ++h) C[j][h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[h], B, C[j][h], 0, 0, 0);
+                    APRNET_PRODUCT(low, a3, b[0]) APRNET_PRODUCT(low, a1, b[2]) APRNET_PRODUCT(low, a2, b[1])
+                    APRNET_PRODUCT(low, a2, b[0]) APRNET_PRODUCT(low, a1, b[1]) APRNET_PRODUCT(acc, a1, b[0])
 #undef APRNET_PRODUCT
                 }
             }
         }
     }
     if constexpr (NB > 0) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int h = 0; h < COH; ++h) acc[j][h] += low[j][h];
         const __amdgpu_buffer_rsrc_t rci = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(gl.col_idx), 0, nc * 4, 0x00020000);
         int ocol[NB], cpos[NB];
 #pragma unroll
@@ -377,9 +385,10 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     }
 }
 
-// three workgroups per CU for at most 16 outputs (80 registers), two for 32
+// Two workgroups per CU.  Three (80 registers) spill with the second set of sums: 16 -> 16 channels on 43 M particles 10.4 instead of 9.35 ms,
+// 32 -> 16 on 8 M 4.46 instead of 3.81, 1x5x5 16 -> 16 on 2 M 0.86 instead of 0.63 ms.
 template <class G, int COH, int MODE>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(COH == 1 && MODE == 0 ? 6 : 4, COH == 1 && MODE == 0 ? 6 : 4)))
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 conv_split_kernel(const ConvArgs<float> a) {
     constexpr int NBW = 4, NSTEP = split_steps<G>();
     static_assert((G::MAXCOL + 15) / 16 <= G::NWAVE * NBW, "a window must fit the accumulators of the block");

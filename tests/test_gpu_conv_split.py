@@ -275,3 +275,34 @@ def test_recorded_pass_keeps_the_fp32_products(path):
     assert torch.equal(out[19, "training"], out[20, "training"]) and torch.equal(out[19, "inference"], out[19, "training"])
     assert all(torch.equal(a, b) for a, b in zip(out[19, "grads"], out[20, "grads"]))
     assert not torch.equal(out[20, "inference"], out[20, "training"])
+
+
+@pytest.mark.parametrize("products", [1, 2, 3, 9, 27])
+@pytest.mark.parametrize("zeros", ["weights", "features"])
+@pytest.mark.parametrize("ksize,cout", [((3, 3, 3), 16), ((3, 3, 3), 32), ((1, 5, 5), 16), ((1, 5, 5), 32)], ids=["k333_16", "k333_32", "k155_16", "k155_32"])
+def test_few_products(path, ksize, cout, zeros, products):
+    """Stencils or features with hardly a value that is not zero: a chain of fp32 multiply-adds is then rounded only a few times, and the
+    error of the pieces is no larger.  (But for one product: what is left out of it, at most 2^-26 of it twice, has a quarter of
+    the spread of one rounding at the most, so the error is at most sqrt(1 + 1/16) = 1.03 of one rounding's; 0.03 for the sample.)"""
+    apr = apr_cases.random_apr((48, 64, 64), 43, 0.4)
+    apr.init_cuda()
+    n, ld, S, cin = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32), apr.level_max() - apr.level_min() + 1, 16
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(1, cin, n, generator=g), torch.randn(S, cout, cin, *ksize, generator=g)
+    taps = cin * w[0, 0, 0].numel()
+    if zeros == "weights":
+        flat = w.view(S, cout, taps)
+        flat *= torch.zeros_like(flat).scatter_(2, torch.rand(flat.shape, generator=g).topk(products, 2)[1], 1.0)
+    else:
+        x *= torch.rand(x.shape, generator=g) < products / taps
+    xd, wd, err = x.to(DEV), w.to(DEV), {}
+    gd = torch.randn(1, cout, n, generator=g).to(DEV)
+    if zeros == "features":
+        gd *= (torch.rand(gd.shape, generator=g) < products / (taps * cout // cin)).to(DEV)
+    ref, gref = (t.cpu() for t in (_ops.conv_forward([apr], xd.double(), wd.double(), ld), _ops.conv_backward([apr], xd.double(), wd.double(), gd.double(), ld)[0]))
+    for p in (19, 20):
+        path(p)
+        err[p] = error(_ops.conv_forward([apr], xd, wd, ld), ref), error(_ops.conv_backward([apr], xd, wd, gd, ld)[0], gref)
+    most = 1.06 if products == 1 else 1.0
+    assert err[20][0] <= most * err[19][0]
+    assert err[20][1] <= most * err[19][1]

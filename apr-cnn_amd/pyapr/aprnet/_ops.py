@@ -9,6 +9,7 @@ kernels consume; the CPU-flavour names (``convolve333_forward`` ...) take [Cin, 
 (conv.py:164) and are permuted on the way in and out.
 """
 import ctypes as C
+import warnings
 
 import torch
 
@@ -139,14 +140,15 @@ class _Fusion(C.Structure):
 
 def _workspace(nbytes, optional, device):
     """Work space of a call, ``nbytes`` and behind them (256-byte aligned) ``optional`` more: (tensor, address of the optional part
-    or None, its bytes).  The call runs without the optional part when there is no memory for it."""
+    or None, its bytes).  The call runs without the optional part when there is no memory for it, and says so: its sums are then in
+    the order of the fp32 instructions."""
     at = (nbytes + 255) // 256 * 256
     if optional > 0:
         try:
             buf = torch.empty(at + optional, dtype=torch.uint8, device=device)
             return buf, buf.data_ptr() + at, optional
         except torch.cuda.OutOfMemoryError:
-            pass
+            warnings.warn("no memory for the work space of a convolution on bfloat16 pieces: fp32 products, with another order of the sums", RuntimeWarning)
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device), None, 0
 
 

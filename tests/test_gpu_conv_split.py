@@ -306,3 +306,26 @@ def test_few_products(path, ksize, cout, zeros, products):
     most = 1.06 if products == 1 else 1.0
     assert err[20][0] <= most * err[19][0]
     assert err[20][1] <= most * err[19][1]
+
+
+def test_no_memory_for_the_work_space(path, monkeypatch):
+    """The call runs on the fp32 instructions then, and says so."""
+    x, aprs, ld, w_exp = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
+    xd, wd = x.to(DEV), layer(w_exp)
+    gd = torch.randn(1, 32, x.size(2), generator=torch.Generator().manual_seed(3)).to(DEV)
+    path(19)
+    fp32, fp32_g = _ops.conv_forward(aprs, xd, wd, ld), _ops.conv_backward(aprs, xd, wd, gd, ld)[0]
+    path(20)
+    empty, refused = torch.empty, []
+
+    def full(*size, **kw):
+        if kw.get("dtype") is torch.uint8 and not refused:
+            refused.append(size)
+            raise torch.cuda.OutOfMemoryError("full")
+        return empty(*size, **kw)
+    for call, want in ((lambda: _ops.conv_forward(aprs, xd, wd, ld), fp32), (lambda: _ops.conv_backward(aprs, xd, wd, gd, ld)[0], fp32_g)):
+        refused.clear()
+        with monkeypatch.context() as m, pytest.warns(RuntimeWarning, match="work space"):
+            m.setattr(torch, "empty", full)
+            got = call()
+        assert refused and torch.equal(got, want)

@@ -47,7 +47,8 @@ class APRConv(nn.Module):
             init.uniform_(self.bias, -bound, bound)
 
     def forward(self, input_features, aprs, level_deltas):
-        return ConvFunction.apply(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout, torch.is_grad_enabled())
+        recorded = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (input_features, self.weight, self.bias))
+        return ConvFunction.apply(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout, recorded)
 
     def forward_fused(self, input_features, aprs, level_deltas, relu=False, second_input=None):
         """Inference-only forward (no autograd record): optionally clamps the result at zero inside the kernel and

@@ -329,3 +329,17 @@ def test_no_memory_for_the_work_space(path, monkeypatch):
             m.setattr(torch, "empty", full)
             got = call()
         assert refused and torch.equal(got, want)
+
+
+def test_what_counts_as_recorded(path):
+    """Grad mode on with nothing that requires a gradient: no backward pass can follow, so the pass is inference's."""
+    from pyapr import aprnet
+    x, aprs, ld, _ = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
+    conv, xd = aprnet.cuda.APRConv(16, 32, nstencils=2).to(DEV), x.to(DEV)
+    path(20)
+    recorded = conv(xd, aprs, ld).detach()
+    with torch.no_grad():
+        inference = conv(xd, aprs, ld)
+    conv.requires_grad_(False)
+    assert torch.equal(conv(xd, aprs, ld), inference) and not torch.equal(inference, recorded)
+    assert torch.equal(conv(xd.clone().requires_grad_(True), aprs, ld).detach(), recorded)

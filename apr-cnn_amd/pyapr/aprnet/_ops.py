@@ -396,9 +396,10 @@ def norm_backward_apply(gy, x, y, mean, rstd, a, b, c):
     return gx
 
 
-def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=True):
+def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=True, pieces=True):
     """conv333_backward / conv111_backward (wrap_conv_gpu.hpp:87-133, 216-246) -> [grad_input, grad_weights].
-    ``need_input_grad=False`` (stencil convolutions): the input gradient is not computed, grad_input is None."""
+    ``need_input_grad=False`` (stencil convolutions): the input gradient is not computed, grad_input is None.
+    ``pieces``: the input gradient of fp32 features may be made of products of bfloat16 pieces (see conv_forward)."""
     _check_input(x, "input")
     _check_input(weights, "weights")
     _check_input(grad_output, "grad_output")
@@ -458,8 +459,8 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
             fn = getattr(_lib(), "aprnet_conv_bwd_" + ("ws_f32" if sfx == "f32" else sfx))
             extra = ()
             if sfx == "f32":
-                tree_ws, *extra = _workspace(cin * ld_tree * 4, 0 if skip_gx else max([_lib().aprnet_conv_bwd_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
-                                                                                       for b in range(B)]), x.device)
+                tree_ws, *extra = _workspace(cin * ld_tree * 4, 0 if skip_gx or not pieces else max([_lib().aprnet_conv_bwd_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
+                                                                                                     for b in range(B)]), x.device)
             else:
                 tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             for b in range(B):

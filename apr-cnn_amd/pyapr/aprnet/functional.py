@@ -33,9 +33,10 @@ def _from_device_layout(w, layout):
 
 class ConvFunction(Function):
     @staticmethod
-    def forward(ctx, inputs, weights, bias, aprs, level_deltas, layout, recorded=True):
+    def forward(ctx, inputs, weights, bias, aprs, level_deltas, layout, recorded=True, pieces=True):
         ctx.aprs = aprs
         ctx.layout = layout
+        ctx.pieces = pieces
         ctx.param_dtypes = (weights.dtype, None if bias is None else bias.dtype)
         w = _to_device_layout(weights, layout).contiguous()
         if inputs.dtype == torch.bfloat16:
@@ -51,24 +52,24 @@ class ConvFunction(Function):
         inputs = inputs.contiguous()
         ctx.save_for_backward(inputs, w, bias, level_deltas.clone())
         # the bias add of conv.py:101 is fused into the kernel's store
-        return _ops.conv_forward(aprs, inputs, w, level_deltas, None if bias is None else bias.contiguous(), pieces=not recorded)
+        return _ops.conv_forward(aprs, inputs, w, level_deltas, None if bias is None else bias.contiguous(), pieces=pieces and not recorded)
 
     @staticmethod
     def backward(ctx, grad_output):
         inputs, w_exp, bias, level_deltas = ctx.saved_tensors
         grad_output = grad_output.contiguous()
         grad_input, grad_w = _ops.conv_backward(ctx.aprs, inputs, w_exp, grad_output, level_deltas,
-                                                need_input_grad=ctx.needs_input_grad[0])
+                                                need_input_grad=ctx.needs_input_grad[0], pieces=ctx.pieces)
         grad_bias = None if bias is None else _ops.channel_sum(grad_output)
         if ctx.expand:
             grad_w = _ops.restrict_kernel_backward(grad_w, ctx.num_stencils)
         grad_w = _from_device_layout(grad_w, ctx.layout).to(ctx.param_dtypes[0])     # fp32 sums for bfloat16 features
         if grad_bias is not None:
             grad_bias = grad_bias.to(ctx.param_dtypes[1])
-        return grad_input, grad_w, grad_bias, None, None, None, None
+        return grad_input, grad_w, grad_bias, None, None, None, None, None
 
 
-def conv_inference(inputs, weights, bias, aprs, level_deltas, layout, relu=False, inputs2=None, kept_stencils=None):
+def conv_inference(inputs, weights, bias, aprs, level_deltas, layout, relu=False, inputs2=None, kept_stencils=None, pieces=True):
     """ConvFunction.forward without the autograd record, with the two fusions the kernel offers: the ReLU that
     follows the convolution in BasicBlock (unet_parts.py:17-26, norm folded away) and a second input tensor in
     place of torch.cat([inputs, inputs2], dim=1) (unet_parts.py:82).  For inference under torch.no_grad().
@@ -79,7 +80,7 @@ def conv_inference(inputs, weights, bias, aprs, level_deltas, layout, relu=False
             and kept_stencils[1].device == inputs.device):
         return _ops.conv_forward(aprs, inputs.contiguous(), kept_stencils[1], level_deltas,
                                  None if bias is None else bias.detach().contiguous(),
-                                 relu=relu, x2=None if inputs2 is None else inputs2.contiguous())
+                                 relu=relu, x2=None if inputs2 is None else inputs2.contiguous(), pieces=pieces)
     w = _to_device_layout(weights.detach(), layout).contiguous()
     if inputs.dtype == torch.bfloat16:
         w = w.float()
@@ -89,7 +90,7 @@ def conv_inference(inputs, weights, bias, aprs, level_deltas, layout, relu=False
     if ksize != (1, 1, 1):
         w = _ops.restrict_kernel_forward(w, levels)
     return _ops.conv_forward(aprs, inputs.contiguous(), w, level_deltas, None if bias is None else bias.detach().contiguous(),
-                             relu=relu, x2=None if inputs2 is None else inputs2.contiguous())
+                             relu=relu, x2=None if inputs2 is None else inputs2.contiguous(), pieces=pieces)
 
 
 class NormFunction(Function):

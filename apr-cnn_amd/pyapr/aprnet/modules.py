@@ -18,6 +18,11 @@ from .functional import (ConvFunction, conv_inference, MaxPoolFunction, UpSample
 class APRConv(nn.Module):
     weight_layout = CPU_LAYOUT
     allowed_kernels = SUPPORTED_KERNELS
+    # fp32 features may be multiplied as bfloat16 pieces (_ops.conv_forward): in forward passes that no backward pass follows and for
+    # the input gradient.  False on a module keeps all its passes on the fp32 instructions, so that a pass without and one with a
+    # record give the same bits: re-entrant activation checkpointing (torch.utils.checkpoint with use_reentrant=True) runs its first
+    # forward pass without a record and repeats it with one.  (With use_reentrant=False both are recorded.)
+    pieces = True
 
     def __init__(self, in_channels, out_channels, nstencils=1, kernel_size=(3, 3, 3), bias=True):
         super().__init__()
@@ -48,7 +53,7 @@ class APRConv(nn.Module):
 
     def forward(self, input_features, aprs, level_deltas):
         recorded = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (input_features, self.weight, self.bias))
-        return ConvFunction.apply(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout, recorded)
+        return ConvFunction.apply(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout, recorded, self.pieces)
 
     def forward_fused(self, input_features, aprs, level_deltas, relu=False, second_input=None):
         """Inference-only forward (no autograd record): optionally clamps the result at zero inside the kernel and
@@ -58,7 +63,7 @@ class APRConv(nn.Module):
         # would be restricted to the same values here
         kept = getattr(self, "_inference_stencils", None) if self.weight.dtype == torch.float32 else None
         return conv_inference(input_features, self.weight, self.bias, aprs, level_deltas, self.weight_layout,
-                              relu=relu, inputs2=second_input, kept_stencils=kept)
+                              relu=relu, inputs2=second_input, kept_stencils=kept, pieces=self.pieces)
 
 
 class MaxPool(nn.Module):

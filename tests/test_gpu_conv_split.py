@@ -343,3 +343,40 @@ def test_what_counts_as_recorded(path):
     conv.requires_grad_(False)
     assert torch.equal(conv(xd, aprs, ld), inference) and not torch.equal(inference, recorded)
     assert torch.equal(conv(xd.clone().requires_grad_(True), aprs, ld).detach(), recorded)
+
+
+def test_pieces_switched_off_on_modules(path):
+    """Re-entrant checkpointing runs its first forward pass without a record and repeats it with one: with ``pieces = False`` both
+    give the same bits, those of the fp32 instructions, and so does the input gradient."""
+    from pyapr import aprnet
+    from torch.utils.checkpoint import checkpoint
+    x, aprs, ld, _ = _conv_case([("3d_s", 0)], (3, 3, 3), 2, 16, 32, torch.float32)
+    net = torch.nn.ModuleList([aprnet.cuda.APRConv(16, 32, nstencils=2), aprnet.cuda.APRConv(32, 16, nstencils=2)]).to(DEV)
+    seen = []
+
+    def region(t):
+        for conv in net:
+            t = conv(t, aprs, ld)
+            seen.append(t.detach().clone())
+        return t
+
+    def step(p):
+        path(p)
+        seen.clear()
+        xg = x.to(DEV).requires_grad_(True)
+        y = checkpoint(region, xg, use_reentrant=True)
+        net.zero_grad()
+        y.square().sum().backward()
+        return [xg.grad, *(w.grad.clone() for w in net.parameters())]
+    with_pieces = step(20)
+    assert len(seen) == 4 and not torch.equal(seen[0], seen[2])
+    for conv in net:
+        conv.pieces = False
+    want = step(19)
+    got = step(20)
+    assert torch.equal(seen[0], seen[2]) and torch.equal(seen[1], seen[3])
+    assert all(torch.equal(a, b) for a, b in zip(got, want)) and not torch.equal(got[0], with_pieces[0])
+    with torch.no_grad():                                                # the fused form of inference
+        fused = net[0].forward_fused(x.to(DEV), aprs, ld, relu=True)
+        path(19)
+        assert torch.equal(fused, net[0].forward_fused(x.to(DEV), aprs, ld, relu=True))

@@ -280,6 +280,18 @@ constexpr unsigned COL_TREE = 0x8000u;
 // takes the sum to the particle.  They come first in a window's columns.  (A scan leaves them at the front of the column
 // arrays, nbox particles, and the other columns, ncol of them, at the back in reverse.)
 template <class G> __host__ __device__ constexpr int dx_group() { return G::TZ >= 2 ? 8 : 4; }
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
+// the sum over such a group of lanes, in each of them
+template <class G>
+__device__ __forceinline__ float dx_group_sum(float s) {
+    s += dpp_f32<0xb1>(s);                                       // lanes 1, 0, 3, 2 of each four
+    s += dpp_f32<0x4e>(s);                                       // lanes 2, 3, 0, 1
+    if constexpr (dx_group<G>() == 8) s += dpp_f32<0x141>(s);    // the eight mirrored
+    return s;
+}
 
 template <class G>
 __device__ __attribute__((noinline)) void scan_window_dx_impl(const ScanArgs a, ConvShared<G>& sh) {

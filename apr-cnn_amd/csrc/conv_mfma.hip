@@ -556,11 +556,6 @@ interleave8_kernel(const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __re
         if (b0 + e * IL_TB + threadIdx.x < count) dst[e * IL_TB + threadIdx.x] = buf[e * IL_TB + threadIdx.x];
 }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
-
 // MODE 0: forward.  MODE 1: input gradient (items = output gradient, results added in fp32 onto the place each column
 // names; the columns of a coarser particle summed across lanes first).
 // IL: the input comes regrouped (a.xi, a.ti), see above
@@ -703,10 +698,7 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
                 for (int h = 0; h < COH; ++h)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
-                        float s = acc[j][h][r];
-                        s += dpp_f32<0xb1>(s);                                       // lanes 1, 0, 3, 2 of each four
-                        s += dpp_f32<0x4e>(s);                                       // lanes 2, 3, 0, 1
-                        if constexpr (dx_group<G>() == 8) s += dpp_f32<0x141>(s);    // the eight mirrored
+                        const float s = dx_group_sum<G>(acc[j][h][r]);
                         acc[j][h][r] = boxed ? s : acc[j][h][r];
                     }
             }

@@ -217,19 +217,6 @@ __device__ __forceinline__ void store_items_split(const SplitItems<G>& R, int ni
     }
 }
 
-// sum over the columns of a coarser particle (see dx_group), lanes that lie next to each other
-template <int CTRL>
-__device__ __forceinline__ float split_dpp(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
-}
-template <class G>
-__device__ __forceinline__ float split_group_sum(float s) {
-    s += split_dpp<0xb1>(s);                                       // lanes 1, 0, 3, 2 of each four
-    s += split_dpp<0x4e>(s);                                       // lanes 2, 3, 0, 1
-    if constexpr (dx_group<G>() == 8) s += split_dpp<0x141>(s);    // the eight mirrored
-    return s;
-}
-
 // MODE 0: forward, results stored (plus bias).  MODE 1: input gradient on the plan's input-gradient lists (items = output
 // gradient): the columns of a coarser particle are summed across lanes and the first one takes the sum along; a place that no
 // other column adds to takes a plain store, the others (one more column at most) an atomic addition.
@@ -348,7 +335,7 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
                     for (int h = 0; h < COH; ++h)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            const float s = split_group_sum<G>(acc[j][h][r]);
+                            const float s = dx_group_sum<G>(acc[j][h][r]);
                             acc[j][h][r] = boxed ? s : acc[j][h][r];
                         }
                 }

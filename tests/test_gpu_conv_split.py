@@ -43,8 +43,8 @@ def test_against_float64(path, bt, ksize, cin, cout):
     got = _ops.conv_forward(aprs, xd, wd, ld)
     assert not torch.equal(got, fp32)                                    # the other kernel ran
     close(got, ref.float(), torch.float32)
-    # six products of pieces leave out less than 2^-25 of |x w| and a sum is rounded twice per 32 products, not once per product: no
-    # larger an error than that of the fp32 products
+    # six products of pieces leave out less than 2^-25 of |x w| and the large sum is rounded once per 32 products, not once per
+    # product: no larger an error than that of the fp32 products
     assert error(got, ref) <= error(fp32, ref)
     assert torch.equal(got, _ops.conv_forward(aprs, xd, wd, ld))         # no atomics
     # the input in two tensors, bias and ReLU
@@ -257,6 +257,25 @@ def test_input_gradient_that_is_not_finite(path, value):
     fp32 = gradients(path, 19, aprs, xd, wd, gd, ld)[0]
     got = gradients(path, 20, aprs, xd, wd, gd, ld)[0]
     assert torch.equal(got.nan_to_num(nan=7.0), fp32.nan_to_num(nan=7.0)) and bool(fp32.isfinite().all()) == (value == 3.4e38)
+
+@pytest.mark.parametrize("cin,cout", [(8, 18), (33, 16), (17, 64)])
+@pytest.mark.parametrize("bt,ksize", [([("3d_c", 2)], (3, 3, 3)), ([("3d_s", 0), ("3d_a", 0)], (3, 3, 3)), ([("2d_a", 1), ("2d_s", 0)], (1, 5, 5))], ids=["333_coarse", "333_two", "155"])
+def test_input_gradient_made_again(path, bt, ksize, cin, cout):
+    """As above for other stencils, level deltas, blocks of channels and batches of which one item is finite: the item with a NaN is
+    the fp32 instructions', the other one the pieces'."""
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, cin, cout, torch.float32)
+    gy = torch.randn(x.size(0), cout, x.size(2), generator=torch.Generator().manual_seed(3))
+    for i, a in enumerate(aprs):
+        gy[i, :, oracle.number_parts(a, int(ld[i])):] = 0
+    xd, wd = x.to(DEV), layer(w_exp)
+    pieces = gradients(path, 20, aprs, xd, wd, gy.to(DEV), ld)[0]
+    gy[0, cout // 2, oracle.number_parts(aprs[0], int(ld[0])) // 2] = float("nan")
+    fp32 = gradients(path, 19, aprs, xd, wd, gy.to(DEV), ld)[0]
+    got = gradients(path, 20, aprs, xd, wd, gy.to(DEV), ld)[0]
+    assert bool(fp32[0].isnan().any()) and torch.equal(got[0].isnan(), fp32[0].isnan())
+    assert torch.equal(got[0].nan_to_num(nan=7.0), fp32[0].nan_to_num(nan=7.0))
+    assert torch.equal(got[1:], pieces[1:])
+
 
 
 def test_recorded_pass_keeps_the_fp32_products(path):

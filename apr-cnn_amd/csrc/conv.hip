@@ -229,6 +229,8 @@ static int try_narrow(aprnet_plan* p, const ConvArgs<T>& a, int code, int d, con
 //  - little work: one more launch than the fp32 kernel's, which also counts where the host is behind the device (3x3x3, split against
 //    fp32; 16 outputs: 70 k particles 45 and 46 us, 320 k 90 and 104; 32 outputs: 14 k particles x 16 channels 34 and 37, x 32 42
 //    and 54, 2 k x 32 30 and 32; 64 outputs: 2 k x 64 39 and 51 us).
+//    1x5x5 gains from less work on, but takes the same line: 4 k particles 16 -> 16 channels 35 and 42 us, 64 -> 64 115 and 163; 99 k 89 and
+//    114, 406 and 614; 2 M 423 and 497 us, 3.54 and 4.94 ms.
 //  - the 16-byte items are reached with 32-bit offsets: fewer than 2^28 particles.
 constexpr int SPLIT_MIN_CIN = 16;
 static size_t split_align(size_t v) { return (v + 255) / 256 * 256; }
@@ -245,6 +247,9 @@ static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx
 // 3x3x3 16 -> 16 channels on 70 k particles 152 and 159 us, on 320 k 319 and 353; 32 -> 32 on 14 k 144 and 142, on 70 k 242
 // and 266; 64 -> 64 on 14 k 212 and 220; 128 -> 128 on 2 k 218 and 278; 1x5x5 16 -> 16 on 14 k 139 and 119, on 70 k 142
 // and 157, 64 -> 64 on 14 k 209 and 209).
+// The first such pass of a plan also builds its window lists, 0.1 to 0.5 ms once per level delta: 16 -> 16 channels on 0.7 M particles 1.04
+// and 0.79 ms (later passes 0.53 and 0.63), on 14 M 10.6 and 10.1 (8.6 and 9.1); 32 -> 32 on 0.7 M 1.83 and 1.85, on 14 M 24.5 and 25.8; 64 -> 64
+// on 0.7 M 5.5 and 5.9.  Whether the lists are there decides nothing: the first pass and the later ones have the same bits.
 size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n) {
     if (!g_f32_split || !g_use_lists || g_conv_path == 1 || (code != 333 && code != 155) || Cout < SPLIT_MIN_CIN || n >= (1ll << 28)) return 0;
     if (g_f32_split == 1 && (double)n * Cout * ((Cin + 15) / 16 * 16) < 1 << 24) return 0;

@@ -14,8 +14,9 @@ __device__ __forceinline__ float overlap1(int o, int i, int k, int step) {
     return (float)max(v, 0);
 }
 
-// Weight of source tap i for output tap o of a stencil of compile-time size, with the 1 / step^ndim in it: all factors are
-// small integers or powers of two, so the products are exact whatever their order.
+// Weight of source tap i for output tap o of a stencil of compile-time size, with the 1 / step^ndim in it: integers of at most `step`
+// and a power of two.  Exact up to a step of 2^8; from 2^9 on the product of the integers is rounded
+// to 24 bits, in the order x, y, z for every size of stencil.
 template <int KZ, int KX, int KY>
 __device__ __forceinline__ float overlap3(int zo, int xo, int yo, int zi, int xi, int yi, int step, float scale) {
     return overlap1(xo, xi, KX, step) * overlap1(yo, yi, KY, step) * overlap1(zo, zi, KZ, step) * scale;

@@ -590,8 +590,8 @@ int fill_tree_mean_needed(const aprnet_plan* p, int d, const NeedLists& need, co
         }
     }
     // The coarse levels (a few thousand nodes together) are filled whole, in one launch, down to the coarsest one that is
-    // read: levels without particles are never read, and on most APRs those are all of them (a launch of 14 to 20 us, for
-    // one workgroup per four channels walks the levels one after the other, in front of every convolution).
+    // read: levels without particles are never read, and on most APRs those are all of them (a launch of about 11 us, for
+    // one workgroup per COARSE_C channels walks the levels one after the other, in front of every convolution).
     int l_read = l_coarse + 1;
     for (int l = p->tree.level_min; l <= l_coarse; ++l)
         if (need.cnt[l] > 0) { l_read = l; break; }

@@ -159,7 +159,8 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
     relu: the result is clamped at zero in the kernel (the ReLU of BasicBlock, unet_parts.py:17-26).
     x2 ([B, C2, N], optional): the kernel reads its channels after those of x, which stands for
     conv(torch.cat([x, x2], dim=1)) (unet_parts.py:82) without writing the concatenated tensor.
-    pieces: fp32 features may be multiplied as bfloat16 pieces (smaller error, another order of the sums).  A forward pass that is
+    pieces: fp32 features may be multiplied as bfloat16 pieces (an error of a third of the fp32 instructions' on dense features, at most
+    1.03 times theirs where a result is a single product; another order of the sums).  A forward pass that is
     recorded for a backward one does without: a sign or pooled maximum that tips over moves whole gradients, and the sums of
     training runs stay those of the fp32 instructions bit for bit (a training step of a U-Net gains 2 % from it, its inference 25 %)."""
     _check_input(x, "input")

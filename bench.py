@@ -203,6 +203,14 @@ def mfma_roofline(flop, kernel_ms, peak, kernel, hbm_bytes, traffic=None):
             "kernel": kernel, "kernel_ms": kernel_ms, "hbm_achieved_GBs": gbs, "hbm_frac": gbs / PEAK_HBM_GBS}
 
 
+def pieces_roofline(flop, kernel_ms, hbm_bytes):
+    """fp32 features on bfloat16 pieces: six bfloat16 products for each multiply-add of the algorithm."""
+    out = mfma_roofline(flop, kernel_ms, PEAK_BF16_MATRIX_TFLOPS / 6, "conv_split_kernel", hbm_bytes)
+    out["peak_source"] = "bfloat16 matrix peak / 6 products per fp32 product"
+    out["frac_of_fp32_matrix_peak"] = out["achieved"] / PEAK_FP32_MATRIX_TFLOPS
+    return out
+
+
 def hbm_roofline(nbytes, kernel_ms, kernel, flop=None):
     gbs = nbytes / (kernel_ms * 1e-3) / 1e9
     out = {"bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_GBS, "unit": "GB/s", "frac": gbs / PEAK_HBM_GBS, "traffic": None,
@@ -292,8 +300,8 @@ def run_blobs512(args, dev, lib):
     if flop_pp / (e * (CIN + COUT) + 2) < peak * 1e12 / (PEAK_HBM_GBS * 1e9):      # fewer flops per byte than the machine: HBM bounds it
         out["roofline"] = hbm_roofline(alg_bytes, kernel_ms, "conv_narrow_kernel" if CIN <= 3 else "conv kernel", flop_pp * n)
     else:
-        # fp32: priced by the algorithm's flops against the fp32 matrix peak; the kernel forms six bfloat16 products for each
-        out["roofline"] = mfma_roofline(flop_pp * n, kernel_ms, peak, "conv_mfma_bf16_kernel" if bf16 else "conv_split_kernel", alg_bytes)
+        out["roofline"] = (mfma_roofline(flop_pp * n, kernel_ms, peak, "conv_mfma_bf16_kernel", alg_bytes) if bf16 else
+                           pieces_roofline(flop_pp * n, kernel_ms, alg_bytes))
     if not args.no_extra:                  # (profiler runs pass --no-extra: the convolution step only)
         # second half of the metric: forward latency of the 4-level network (16-32-64-128, norms folded) on this APR
         net = make_unet(dev)
@@ -450,8 +458,8 @@ def run_nuclei2048(args, dev, lib):
                     {"workload": f"tree fill (mean of children) + APRConv 3x3x3 16->16 fp32 forward reading tree parents, batch 1, APR of the "
                                  f"seeded 2048x2048x512 nuclei volume (configs[2]), {what}",
                      "n_particles": n, "tree_nodes": nt, "levels": level_counts(apr), "apr_build_s": round(t_build, 1)})
-    out["roofline"] = mfma_roofline(2 * 27 * C * C * n, kernel_ms, PEAK_FP32_MATRIX_TFLOPS,
-                                    "conv_split_kernel" if n < 1 << 28 else "conv_mfma16_kernel", (8 * C + 2) * n)
+    out["roofline"] = (pieces_roofline(2 * 27 * C * C * n, kernel_ms, (8 * C + 2) * n) if n < 1 << 28 else
+                       mfma_roofline(2 * 27 * C * C * n, kernel_ms, PEAK_FP32_MATRIX_TFLOPS, "conv_mfma16_kernel", (8 * C + 2) * n))
     fill_bytes = 4 * C * (n + 2 * nt)
     out["extra"] = {"fill_tree_mean_ms": fill_ms, "fill_tree_mean_GBs": fill_bytes / fill_ms / 1e6,
                     "fill_tree_mean_hbm_frac": fill_bytes / fill_ms / 1e6 / PEAK_HBM_GBS,
@@ -690,7 +698,7 @@ def other_ops(apr, x, dev):
     ms = _time(lambda: torch.autograd.grad(y, (xg, conv.weight), go, retain_graph=True), iters=3, warmup=1)
     fl = 2 * 2 * 27 * C * C * n0
     res.append({"op": "conv333_bwd", "ms": ms, "particles_per_s": n0 / ms * 1e3, "TFLOPs": fl / ms / 1e9,
-                "mfma_frac": fl / ms / 1e9 / PEAK_FP32_MATRIX_TFLOPS, "note": f"{C}->{C} grad_input + grad_weight"})
+                "mfma_frac": fl / ms / 1e9 / PEAK_FP32_MATRIX_TFLOPS, "note": f"{C}->{C} grad_input (bfloat16 pieces) + grad_weight; frac of the fp32 matrix peak"})
     del y, go, xg
     torch.manual_seed(0)
     net = fold_norms(APRUNet(1, 3, depth=3, n_filters_base=16, n_stencils=2, norm="batch").eval()).to(dev)
@@ -768,7 +776,7 @@ def other_ops(apr, x, dev):
         ms = _time(lambda: conv5(x64, [apr], ld0), iters=3, warmup=1)
     fl = 2 * 25 * 64 * 64 * n0
     res.append({"op": "conv155_fwd", "ms": ms, "particles_per_s": n0 / ms * 1e3, "TFLOPs": fl / ms / 1e9,
-                "mfma_frac": fl / ms / 1e9 / PEAK_FP32_MATRIX_TFLOPS, "note": "1x5x5 64->64 fp32, whole APRConv.forward"})
+                "mfma_frac": fl / ms / 1e9 / PEAK_FP32_MATRIX_TFLOPS, "note": "1x5x5 64->64 fp32 on bfloat16 pieces, whole APRConv.forward; frac of the fp32 matrix peak"})
     x64.requires_grad_(True)
     y5 = conv5(x64, [apr], ld0)
     go5 = torch.randn_like(y5)

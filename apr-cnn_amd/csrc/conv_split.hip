@@ -15,12 +15,12 @@
 // on 23 M particles.)  Values come from copies in groups of four channels, one 16-byte load per item; a value is split when it is
 // written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
 //
-// Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.5 (12.5) ms, 16 -> 16
+// Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.6 (12.5) ms, 16 -> 16
 // channels 3.4 (4.1) ms; 320 k particles, 64 -> 64 channels 0.51 (0.78) ms.
-// Input gradient, whole backward pass beside the weight gradient: 23 M particles, 32 -> 32 channels 37.6 (42.5) ms, 16 -> 16 14.1
+// Input gradient, whole backward pass beside the weight gradient: 23 M particles, 32 -> 32 channels 38.3 (43.5) ms, 16 -> 16 14.1
 // (15.3) ms; the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
-// Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: matrix pipes busy 46 %,
-// vector ALU 15 %, LDS 56 % of the cycles.
+// Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: 32 -> 32 channels, matrix pipes busy
+// 43 % of the launch, waves waiting for memory, LDS or a barrier 53 % of their cycles.
 // Error against 64 bits (2-norm): 0.31 to 0.33 of the fp32 instructions' with N(0, 1) features, 0.31 to 0.35 with those after a ReLU, below theirs
 // also where few products are not zero, but for a single one (1.02; see split_window).
 //

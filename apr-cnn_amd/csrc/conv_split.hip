@@ -233,8 +233,8 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     // Sums of x1 w1, and of the five products below 2^-8 of it: the large ones are rounded once per step, like a chain of fp32
     // multiply-adds or less often.  (Error against 64 bits relative to the fp32 instructions', 3x3x3, 32 channels: 0.32 dense, 0.35 after a ReLU;
     // where weights are zero but 2, 9 or 27 of them 0.85, 0.54, 0.45; a single product 1.02, what is left out.  With the five summed per step and
-    // added to the sum so far, a second rounding: 0.38, 0.44; 1.30, 1.20, 1.01.  32 -> 32 channels on 23 M particles 11.8 and 11.7 ms, 16 -> 16
-    // on 43 M 9.35 and 9.13, 64 -> 64 on 8 M 19.6 and 19.4, 1x5x5 16 -> 16 on 2 M 0.63 and 0.95.)
+    // added to the sum so far, a second rounding: 0.38, 0.44; 1.30, 1.20, 1.01.  32 -> 32 channels on 23 M particles 11.3 and 11.3 ms, 16 -> 16
+    // on 43 M 9.35 and 9.13, 64 -> 64 on 8 M 18.9 and 18.9, 24 -> 32 on 4.9 M in sparse windows 1.98 and 1.94, 1x5x5 16 -> 16 on 2 M 0.63 and 0.95.)
     floatx4s acc[NBA][COH], low[NBA][COH];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
@@ -257,10 +257,12 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
         cell[j] = col < nc ? ((cell[j] & (int)COL_CELL) - G::TAP0) * 8 : 0;
     }
     load_values_split<G>(a, 0, nitem, tree_items, R);
-    // With 32 outputs the weights of a chunk are asked for in front of the barrier that ends the chunk before it, whose operands no longer
-    // need registers then (next to that chunk's products: 88 instead of 34 registers spilled, 32 -> 32 on 23 M particles 12.05 instead of
-    // 11.8 ms).  With 16 outputs they travel with the values (16 -> 16 on 43 M 9.35 ms, in front of the barrier 10.3).
-    constexpr bool LATE = COH == 2;
+    // With 32 outputs a wave that holds two and more blocks of columns asks for the weights of a chunk in front of the barrier that ends the
+    // chunk before it, whose operands no longer need registers then; a wave with one block, as in sparse windows, has them to spare and asks
+    // together with the values.  32 -> 32 channels on 23 M particles 11.3 ms (always in front of the barrier 11.5, always with the values
+    // 11.8), 24 -> 32 on 4.9 M in sparse windows 1.98 (2.08, 2.11), 64 -> 64 on 8 M 18.9 (19.1, 20.0).  With 16 outputs they travel with the
+    // values (16 -> 16 on 43 M 9.35 ms, in front of the barrier 10.3).
+    constexpr bool LATE = COH == 2 && NB >= 2;
     if constexpr (!LATE) load_weights(0);
     for (int i = threadIdx.x; i < 3 * G::CH_STRIDE / 2; i += G::NT) reinterpret_cast<uint4*>(sh.patch)[i] = make_uint4(0u, 0u, 0u, 0u);
     for (int ci0 = 0; ci0 < a.Cin; ci0 += SP_CIB) {

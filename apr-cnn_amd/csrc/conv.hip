@@ -154,7 +154,7 @@ size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
 int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
                   const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
-int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, const WinLists& wl, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
 
 bool conv_narrow_supported(int code, int Cin);
@@ -267,7 +267,8 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
     *done = true;
     ConvArgs<float> b = a;
     if (int rc = set_lists(p, d, code, tl, b, st)) return rc;
-    const size_t need = b.tile_win ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
+    WinLists wl;
+    const size_t need = b.tile_win && get_lists(p, d, code, tl, &wl, st) == 0 ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
     if (need > 0 && ws && ws_bytes >= 0 && (size_t)ws_bytes >= need) {
         // products of bfloat16 pieces on copies in groups of four channels, all in the caller's work space
         const size_t wbytes = split_align(conv_packed_split_bytes(code, a.S_exp, a.Cout, a.Cin)), ng = (size_t)(a.Cin + 3) / 4;
@@ -278,7 +279,7 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
         b.w_raw = a.w; b.w = (const float*)image; b.redo = (int*)ws;
         b.xi = xi; b.ti = ti; b.xi_ld = a.x_count; b.ti_ld = a.t_count;
         TimedLaunch timed(st);
-        return launch_conv_split(code, b, n_tiles, st);
+        return launch_conv_split(code, b, n_tiles, wl, st);
     }
     // plan-owned scratch for the re-laid-out weights, grown on demand
     ScratchLease lease;

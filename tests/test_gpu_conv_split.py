@@ -399,3 +399,28 @@ def test_pieces_switched_off_on_modules(path):
         fused = net[0].forward_fused(x.to(DEV), aprs, ld, relu=True)
         path(19)
         assert torch.equal(fused, net[0].forward_fused(x.to(DEV), aprs, ld, relu=True))
+
+
+@pytest.mark.parametrize("cout", [3, 16])
+@pytest.mark.parametrize("density,drop", [(0.01, 1), (0.95, 0)], ids=["sparse", "dense"])
+def test_sparse_and_dense_windows(path, density, drop, cout):
+    """At most 16 outputs run three workgroups per CU where windows hold few columns and two where they hold many: against 64 bits, and
+    the tiles of a NaN are the fp32 instructions' either way."""
+    apr = apr_cases.random_apr((40, 48, 100), 47, density, drop)
+    apr.init_cuda()
+    n, ld, S, cin = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32), apr.level_max() - apr.level_min() + 1, 18
+    g = torch.Generator().manual_seed(6)
+    x, w, b = torch.randn(1, cin, n, generator=g).to(DEV), torch.randn(S, cout, cin, 3, 3, 3, generator=g).to(DEV), torch.linspace(-1, 1, cout).to(DEV)
+    ref = (_ops.conv_forward([apr], x.double(), w.double(), ld) + b.double()[:, None]).cpu()
+    out = {}
+    for p in (19, 20):
+        path(p)
+        out[p] = _ops.conv_forward([apr], x, w, ld, b)
+    assert not torch.equal(out[20], out[19]) and error(out[20], ref) <= error(out[19], ref)
+    assert torch.equal(out[20], _ops.conv_forward([apr], x[:, :7].contiguous(), w, ld, b, x2=x[:, 7:].contiguous()))
+    x[0, 3, n // 2] = float("nan")
+    got = _ops.conv_forward([apr], x, w, ld, b)
+    path(19)
+    fp32 = _ops.conv_forward([apr], x, w, ld, b)
+    assert bool(fp32.isnan().any()) and torch.equal(got.isnan(), fp32.isnan())
+    assert bool(((got == fp32) | (got == out[20]) | fp32.isnan()).all())

@@ -15,12 +15,12 @@
 // on 23 M particles.)  Values come from copies in groups of four channels, one 16-byte load per item; a value is split when it is
 // written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
 //
-// Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.6 (12.5) ms, 16 -> 16
+// Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.5 (12.5) ms, 16 -> 16
 // channels 3.4 (4.1) ms; 320 k particles, 64 -> 64 channels 0.51 (0.78) ms.
 // Input gradient, whole backward pass beside the weight gradient: 23 M particles, 32 -> 32 channels 38.3 (43.5) ms, 16 -> 16 14.1
 // (15.3) ms; the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
 // Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: 32 -> 32 channels, matrix pipes busy
-// 43 % of the launch, waves waiting for memory, LDS or a barrier 53 % of their cycles.
+// 44 % of the launch, waves waiting for memory, LDS or a barrier 51 % of their cycles.
 // Error against 64 bits (2-norm): 0.31 to 0.33 of the fp32 instructions' with N(0, 1) features, 0.31 to 0.35 with those after a ReLU, below theirs
 // also where few products are not zero, but for a single one (1.02; see split_window).
 //
@@ -234,7 +234,7 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     // multiply-adds or less often.  (Error against 64 bits relative to the fp32 instructions', 3x3x3, 32 channels: 0.32 dense, 0.35 after a ReLU;
     // where weights are zero but 2, 9 or 27 of them 0.85, 0.54, 0.45; a single product 1.02, what is left out.  With the five summed per step and
     // added to the sum so far, a second rounding: 0.38, 0.44; 1.30, 1.20, 1.01.  32 -> 32 channels on 23 M particles 11.3 and 11.3 ms, 16 -> 16
-    // on 43 M 9.35 and 9.13, 64 -> 64 on 8 M 18.9 and 18.9, 24 -> 32 on 4.9 M in sparse windows 1.98 and 1.94, 1x5x5 16 -> 16 on 2 M 0.63 and 0.95.)
+    // on 43 M 9.1 and 9.1, 64 -> 64 on 8 M 18.9 and 18.9, 24 -> 32 on 4.9 M in sparse windows 1.98 and 1.94, 1x5x5 16 -> 16 on 2 M 0.63 and 0.95.)
     floatx4s acc[NBA][COH], low[NBA][COH];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
@@ -260,8 +260,9 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     // With 32 outputs a wave that holds two and more blocks of columns asks for the weights of a chunk in front of the barrier that ends the
     // chunk before it, whose operands no longer need registers then; a wave with one block, as in sparse windows, has them to spare and asks
     // together with the values.  32 -> 32 channels on 23 M particles 11.3 ms (always in front of the barrier 11.5, always with the values
-    // 11.8), 24 -> 32 on 4.9 M in sparse windows 1.98 (2.08, 2.11), 64 -> 64 on 8 M 18.9 (19.1, 20.0).  With 16 outputs they travel with the
-    // values (16 -> 16 on 43 M 9.35 ms, in front of the barrier 10.3).
+    // 11.8), 24 -> 32 on 4.9 M in sparse windows 1.98 (2.08, 2.11), 64 -> 64 on 8 M 18.9 (19.1, 20.0).  With 16 outputs and two workgroups
+    // per CU they travel with the values (16 -> 16 on 43 M 9.35 ms, in front of the barrier 9.65); with three (TIGHT) as with 32 outputs (9.1, always with
+    // the values 10.4).
     constexpr bool LATE = (COH == 2 || TIGHT) && NB >= 2;
     if constexpr (!LATE) load_weights(0);
     for (int i = threadIdx.x; i < 3 * G::CH_STRIDE / 2; i += G::NT) reinterpret_cast<uint4*>(sh.patch)[i] = make_uint4(0u, 0u, 0u, 0u);

@@ -156,6 +156,7 @@ int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool tran
                   const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, const WinLists& wl, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
+static std::atomic<int> g_dw_split{1};       // and their weight gradient (conv_dw_split.hip), likewise
 
 bool conv_narrow_supported(int code, int Cin);
 size_t conv_narrow_packed_floats(int code, int S_exp, int Cout, int Cin, bool bf16m);
@@ -256,6 +257,16 @@ size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n) {
     if (conv_packed_split_bytes(code, S_exp, Cin, Cout) / 48 >= (1u << 29)) return 0;
     if ((double)(Cout + 3) / 4 * n >= 1.6e10) return 0;
     return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cin, Cout)) + (size_t)(Cout + 3) / 4 * (size_t)n * 16;
+}
+
+// The weight gradient is made of pieces too where the input gradient is (and reads its copy of the output gradient): faster from the
+// smallest sizes on (backward pass, fp32 instructions against pieces: 3x3x3 64 -> 64 channels on 5 k particles 177 and 162 us, 128 -> 128
+// on 5 k 470 and 383, 32 -> 32 on 42 k 200 and 168, 16 -> 16 on 90 k 173 and 153; 1x5x5 32 -> 32 on 20 k 209 and 184; large
+// ones in conv_dw_split.hip).  "At any size" of the input gradient's switch leaves it where it is.  Eight planes of the features and of the tree are
+// reached with 32-bit byte offsets: rows of fewer than 2^27 values.
+bool split_dw(int Cin, int Cout, int64_t n, int64_t ldx, int64_t ldt) {
+    if (!g_dw_split || ldx >= (1ll << 27) || ldt >= (1ll << 27)) return false;
+    return g_dw_split == 2 || (double)n * Cout * ((Cin + 15) / 16 * 16) >= 1 << 24;
 }
 
 template <typename T> static int try_mfma(aprnet_plan*, const ConvArgs<T>&, int, int, const TileList&, int, hipStream_t, bool*, void*, int64_t) { return 0; }
@@ -659,6 +670,7 @@ int aprnet_set_conv_path(int path) {
     if (path == 12 || path == 13) { g_narrow = path == 12; return 0; }
     if (path == 14 || path == 15) { g_big_addr = path == 15; return 0; }
     if (path == 16 || path == 17) { g_need_fill = path == 16; return 0; }
+    if (path >= 21 && path <= 23) { g_dw_split = path == 21 ? 1 : path == 22 ? 0 : 2; return 0; }
     if (path >= 18 && path <= 20) { g_f32_split = path == 18 ? 1 : path == 19 ? 0 : 2; return 0; }
     if (path != 0 && path != 1)
         return fail(APRNET_ERR_INVALID_ARGUMENT, "set_conv_path: 0 (auto), 1 (VALU only), 2 / 3 (bfloat16 features: bfloat16 / fp32 "
@@ -667,7 +679,8 @@ int aprnet_set_conv_path(int path) {
                                                  "fixed-order partial sums / atomic additions), 12 / 13 (1 to 3 input channels: pipelined kernel / general kernel), "
                                                  "14 / 15 (grouped bfloat16 forward: 32-bit offsets where they suffice / 64-bit addresses always), "
                                                  "16 / 17 (tree fill before a forward convolution: the nodes it reads / every node), "
-                                                 "18 / 19 / 20 (fp32 features with a work space: products of bfloat16 pieces where faster / fp32 matrix instructions / pieces at any size)");
+                                                 "18 / 19 / 20 (fp32 features with a work space: products of bfloat16 pieces where faster / fp32 matrix instructions / pieces at any size), "
+                                                 "21 / 22 / 23 (the same for the weight gradient beside an input gradient on pieces)");
     g_conv_path = path;
     return 0;
 }

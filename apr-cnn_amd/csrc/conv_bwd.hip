@@ -13,7 +13,7 @@
 // (co, ci) pair and keeps its K sums in registers while the (persistent) block walks over many
 // tiles; dO and the patch are staged in LDS.  Sums are flushed with one atomic per element when the
 // stencil index changes and at the end.
-#include "conv_common.hpp"
+#include "dw_work.hpp"
 
 namespace aprnet {
 
@@ -264,11 +264,13 @@ int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs
 int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st);
 int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st);
 size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n);
+bool split_dw(int Cin, int Cout, int64_t n, int64_t ldx, int64_t ldt);
 size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
 int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
                   const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
 int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
+int launch_conv_dw_split(int code, const ConvArgs<float>& a, const DwWork& k, int* mark, hipStream_t st);
 int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
 size_t conv_packed_bf16_bytes(int code, int S_exp, int Cout, int Cin);
 int pack_conv_weights_bf16(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, hipStream_t st, bool transposed);
@@ -331,29 +333,33 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     ScratchLease lease;          // before the join guard below: its hand-over event is recorded after the join
     if (wbytes + pbytes) if (int rc = lease.acquire(p, wbytes + pbytes, st)) return rc;
     if (pbytes) set_dw_partials(p, wbytes, code, c);
+    // On products of bfloat16 pieces both halves read one copy of the output gradient in groups of four channels, and fp32 kernels
+    // follow that do all of it again if a sum was not finite (conv_split.hip, conv_dw_split.hip).
+    int* mark = nullptr;
+    RedoClear redo{};
+    if (pieces) {
+        char* image = (char*)ws + split_mark_bytes();
+        float* gi = (float*)(image + (conv_packed_split_bytes(code, a.S_exp, a.Cin, a.Cout) + 255) / 256 * 256);
+        mark = (int*)ws;
+        redo = RedoClear{mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin};
+        if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, nullptr, 0, a.Cout, a.x_count, gi,
+                                   nullptr, 0, 0, nullptr, st)) return rc;
+        e.tiles = near.d_tiles; e.n_tiles = near.n;
+        e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
+        e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
+    }
     hipStream_t side = st;
     if (a.gx) if (int rc = fork_side(p, st, &side)) return rc;
     SideJoin guard(p, st, side);
+    if (pieces && wl && wl->n_win > 0 && split_dw(a.Cin, a.Cout, a.x_count, a.ldx, a.ldt)) {
+        c.xi = e.xi; c.xi_ld = e.xi_ld; c.redo = mark + 1;
+        if (int rc = launch_conv_dw_split(code, c, dw_work(code, a.Cout, a.Cin, a.S_exp, a.Lc, *wl), mark + 1, side)) return rc;
+    }
     if (int rc = launch_conv_dw_mfma(code, c, tl, wl, p->apr.level_min, side)) return rc;
     if (a.gx) {
         // input gradient: the forward kernel on the output gradient with the transposed, flipped stencil;
         // every row group within one row of an output takes part
-        int* mark = nullptr;
-        RedoClear redo{};
-        if (pieces) {
-            // on products of bfloat16 pieces (conv_split.hip), from a copy of the output gradient in groups of four channels; what
-            // follows then runs only if a sum was not finite, and does all of it again
-            char* image = (char*)ws + split_mark_bytes();
-            float* gi = (float*)(image + (conv_packed_split_bytes(code, a.S_exp, a.Cin, a.Cout) + 255) / 256 * 256);
-            mark = (int*)ws;
-            redo = RedoClear{mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin};
-            if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, nullptr, 0, a.Cout, a.x_count, gi,
-                                       nullptr, 0, 0, nullptr, st)) return rc;
-            e.tiles = near.d_tiles; e.n_tiles = near.n;
-            e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
-            e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
-            if (int rc = launch_conv_dx_split(code, e, near.n, st)) return rc;
-        }
+        if (pieces) if (int rc = launch_conv_dx_split(code, e, near.n, st)) return rc;
         if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cin, a.Cout, true, (float*)p->d_scratch, st, &redo)) return rc;
         ConvArgs<float> b = a;
         b.redo = mark;

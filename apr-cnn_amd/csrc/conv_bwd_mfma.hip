@@ -18,6 +18,7 @@
 // for all of them, see DwWork); its sums go to slots of its own (see DW_CHAINS), which sum_slots.hpp adds up in a fixed order.  The patch rows are 67 words
 // apart so that the 27 tap offsets of a B read fall into 27 different LDS banks.
 #include "conv_common.hpp"
+#include "dw_work.hpp"
 #include "sum_slots.hpp"
 
 namespace aprnet {
@@ -35,49 +36,17 @@ constexpr int DW_GB = 256;         // columns of gY staged at a time
 constexpr int DW_KB = 8;          // MFMAs issued back to back between operand phases (16 would spill registers)
 constexpr int DW_GLD = 33;         // words per column of gyl (32 output channels + 1 against bank conflicts)
 
-// Work of a launch on the plan's window lists: workgroups blk0[k] .. blk0[k + 1] - 1 (grid.x) take the windows of stencil
-// index s_of[k].  One launch covers all stencil indices: with a launch and a sum of slots each, most of them left the chip
-// idle (the coarse levels have a handful of windows), and the weight gradients of a training step of the 16-32-64-128 network on
-// two APRs of 338 k particles took 76 + 102 launches; now 28 + 28, and the step 14.4 instead of 15.8 ms.
-struct DwWork {
-    int n_s;
-    int s_of[MAX_LEVELS + 1], win0[MAX_LEVELS + 1], nwin[MAX_LEVELS + 1], blk0[MAX_LEVELS + 2];
-    // The windows of an index are cut into n_run runs of len or (the first `rem`) len + 1 neighbours, which its workgroups take in turn.
-    int n_run[MAX_LEVELS + 1], len[MAX_LEVELS + 1], rem[MAX_LEVELS + 1];
-    int chain[MAX_LEVELS + 1];     // windows whose products are added up in registers before the sums go to the slots
-    int first_coarse;              // windows from here on may stage tree nodes (below the finest level of the call)
-};
-
-// Partial sums of one workgroup and column half, rows of output channels from co0 on: its slot, or (no slots) the result itself.
-struct DwSlot {
-    __amdgpu_buffer_rsrc_t rs;
-    float* p; bool own; int co_n, Cin, K;
-    template <typename T>
-    __device__ __forceinline__ DwSlot(const ConvArgs<T>& a, int co0, int kh, int rows, int K_, int s) : own(a.gw_part != nullptr), co_n(min(rows, a.Cout - co0)), Cin(a.Cin), K(K_) {
-        p = (own ? a.gw_part + (int64_t)(2 * blockIdx.x + kh) * a.gw_part_ld : a.gw + (int64_t)s * a.Cout * Cin * K) + (int64_t)co0 * Cin * K;
-        rs = __builtin_amdgcn_make_buffer_rsrc(p, 0, co_n * Cin * K * 4, 0x00020000);
-    }
-    // first: nothing is in the slot yet.  Later sums come by atomic additions, which are not waited for; the lane that wrote an element is
-    // the only one that adds to it, so they arrive in the order of the program.
-    __device__ __forceinline__ void add(int row, int ci, int t, float v, bool first) const {
-        const bool in = t < K && row < co_n;
-        const int e = (row * Cin + ci) * K + t;
-        if (own && first) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), rs, in ? e * 4 : (int)BUF_OOB, 0, 0);      // (past the end: not written)
-        else if (in && v != 0.f) unsafeAtomicAdd(p + e, v);
-    }
-};
-
 // The windows of this workgroup in turn, window(lists, columns, items, tree items) for each; flush(s, first) after every chain[k] of them
 // and after the last one.
 template <class G, typename T, class Window, class Flush>
-__device__ __forceinline__ void dw_walk(const ConvArgs<T>& a, const DwWork& wk, Window window, Flush flush) {
+__device__ __forceinline__ void dw_walk(const ConvArgs<T>& a, const DwWork& wk, const int bx, Window window, Flush flush) {
     int si = 0;
-    while (si + 1 < wk.n_s && (int)blockIdx.x >= wk.blk0[si + 1]) ++si;
+    while (si + 1 < wk.n_s && bx >= wk.blk0[si + 1]) ++si;
     const int n_run = wk.n_run[si], len = wk.len[si], rem = wk.rem[si], win0 = wk.win0[si], step = wk.blk0[si + 1] - wk.blk0[si];
     const int chain = wk.chain[si], s = wk.s_of[si];
     int left = chain;
     bool first = true;
-    for (int run = (int)blockIdx.x - wk.blk0[si]; run < n_run; run += step) {
+    for (int run = bx - wk.blk0[si]; run < n_run; run += step) {
         const int w0 = win0 + run * len + min(run, rem), w1 = w0 + len + (run < rem ? 1 : 0);
         for (int w = w0; w < w1; ++w) {
             const int4 hd = a.win[w];
@@ -281,14 +250,13 @@ __device__ __forceinline__ void dw_window16(const ConvArgs<T>& a, const Lists& s
 }
 
 template <typename T, class G, int CIB, int NCH, bool LISTS>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
-conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
+__device__ __forceinline__ void dw16_block(const ConvArgs<T>& a, const DwWork& wk, const int s_arg, const int bx, const int by) {
     static_assert(G::NWAVE == 8 && CIB == 4, "wave w owns input channel w%4 and column half w/4");
     __shared__ float patch[CIB * G::CH_STRIDE];
     __shared__ float gyl[DW_GB * DW_GLD16];
     __shared__ int cpl[DW_GB];
 
-    const int cig0 = blockIdx.y * (CIB * NCH);
+    const int cig0 = by * (CIB * NCH);
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cil = wave & 3, kh = wave >> 2;
@@ -312,7 +280,7 @@ conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
     auto flush = [&](const int s, const bool first) {
         int l = lane;
         asm volatile("" : "+v"(l));         // addresses formed per call, not kept (and spilled) across the window loop
-        const DwSlot slot(a, 0, kh, 16, G::K, s);
+        const DwSlot slot(a, bx, 0, kh, 16, G::K, s);
 #pragma unroll
         for (int q = 0; q < NCH; ++q)
 #pragma unroll
@@ -324,7 +292,7 @@ conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
                 }
     };
     if constexpr (LISTS) {
-        dw_walk<G>(a, wk, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
+        dw_walk<G>(a, wk, bx, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
             dw_window16<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, bl, kh, wave, lane, patch, gyl, cpl, acc);
         }, flush);
     } else {
@@ -451,7 +419,7 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const DwWork wk, const int s_arg) 
     auto flush = [&](const int s, const bool first) {
         int l = lane;
         asm volatile("" : "+v"(l));         // addresses formed per call, not kept (and spilled) across the window loop
-        const DwSlot slot(a, co0, kh, 32, G::K, s);
+        const DwSlot slot(a, blockIdx.x, co0, kh, 32, G::K, s);
 #pragma unroll
         for (int q = 0; q < NCH; ++q)
 #pragma unroll
@@ -461,7 +429,7 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const DwWork wk, const int s_arg) 
             }
     };
     if constexpr (LISTS) {
-        dw_walk<G>(a, wk, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
+        dw_walk<G>(a, wk, blockIdx.x, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
             dw_window_bf16<G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, acc);
         }, flush);
     } else {
@@ -492,14 +460,13 @@ conv_dw_bf16_kernel(const ConvArgs<bf16_t> a, const DwWork wk, const int s_arg) 
 // T: storage type of the features and of the output gradient (float, or bfloat16 widened to fp32 on load).
 // LISTS: the windows come from the plan's lists; otherwise the block scans the access arrays.
 template <typename T, class G, int CIB, int NCH, bool LISTS>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
-conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
+__device__ __forceinline__ void dw_block(const ConvArgs<T>& a, const DwWork& wk, const int s_arg, const int bx, const int by, const int bz) {
     static_assert(G::NWAVE == 8 && CIB == 4, "wave w owns input channel w%4 and column half w/4");
     __shared__ float patch[CIB * G::CH_STRIDE];
     __shared__ float gyl[DW_GB * DW_GLD];
     __shared__ int cpl[DW_GB];
 
-    const int cig0 = blockIdx.y * (CIB * NCH), co0 = blockIdx.z * 32;
+    const int cig0 = by * (CIB * NCH), co0 = bz * 32;
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int cil = wave & 3, kh = wave >> 2;
@@ -519,7 +486,7 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
     auto flush = [&](const int s, const bool first) {
         int l = lane;
         asm volatile("" : "+v"(l));         // addresses formed per call, not kept (and spilled) across the window loop
-        const DwSlot slot(a, co0, kh, 32, G::K, s);
+        const DwSlot slot(a, bx, co0, kh, 32, G::K, s);
 #pragma unroll
         for (int q = 0; q < NCH; ++q)
 #pragma unroll
@@ -529,7 +496,7 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
             }
     };
     if constexpr (LISTS) {
-        dw_walk<G>(a, wk, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
+        dw_walk<G>(a, wk, bx, [&](const WindowLists& gl, int nc, int nitem, bool tree_items) {
             dw_window<T, G, CIB, NCH, true>(a, gl, nc, nitem, tree_items, cig0, co0, bl, kh, hi, wave, lane, patch, gyl, cpl, ap, acc);
         }, flush);
     } else {
@@ -554,6 +521,30 @@ conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
             }
         }
         flush(s_arg, true);
+    }
+}
+
+template <typename T, class G, int CIB, int NCH, bool LISTS>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
+conv_dw16_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
+    dw16_block<T, G, CIB, NCH, LISTS>(a, wk, s_arg, blockIdx.x, blockIdx.y);
+}
+template <typename T, class G, int CIB, int NCH, bool LISTS>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
+conv_dw_mfma_kernel(const ConvArgs<T> a, const DwWork wk, const int s_arg) {
+    dw_block<T, G, CIB, NCH, LISTS>(a, wk, s_arg, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+// The blocks (nx, ny, nz) of one of the two again, where the products of bfloat16 pieces did not come out finite (*a.redo,
+// conv_dw_split.hip).  Few workgroups, which end at once otherwise: as many as there are blocks, up to 16,000 with 128 channels each way,
+// they took longer to launch than the pieces gained.
+template <class G, int CIB, int NCH, bool M16>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
+conv_dw_redo_kernel(const ConvArgs<float> a, const DwWork wk, const int nx, const int ny, const int nz) {
+    if (*a.redo == 0) return;
+    for (int u = blockIdx.x; u < nx * ny * nz; u += gridDim.x) {          // uniform
+        if constexpr (M16) dw16_block<float, G, CIB, NCH, true>(a, wk, 0, u % nx, u / nx);
+        else dw_block<float, G, CIB, NCH, true>(a, wk, 0, u % nx, u / nx % ny, u / nx / ny);
+        __syncthreads();
     }
 }
 
@@ -587,7 +578,7 @@ constexpr int DW_RUN = 4;
 // planes, 15.4 M particles, 29.0 -> 28.3 ms (32.3 with 128 workgroups), 32 -> 32 on 2.8 M 2.83 -> 2.72 ms.
 constexpr int DW_WINDOW_COST = 256;
 // The stencil indices that have windows, and a share of the workgroups for each: one, and of the others by the cost of its windows.
-static DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists& wl) {
+DwWork dw_work(int code, int Cout, int Cin, int S_exp, int Lc, const WinLists& wl) {
     DwWork k{};
     k.first_coarse = (wl.n_lv > 0 && wl.lv_level[0] == Lc) ? (wl.n_lv > 1 ? wl.lv_first[1] : wl.n_win) : 0;
     int64_t cost[MAX_LEVELS + 1] = {}, total = 0;
@@ -620,6 +611,18 @@ template <typename T, class G, bool LISTS>
 static int launch_dw_kernel(const ConvArgs<T>& a, const DwWork& k, int s, int blocks, hipStream_t st) {
     const int nch = dw_chunks(a.Cin);
     dim3 grid((unsigned)blocks, (unsigned)((a.Cin + DW_CIB * nch - 1) / (DW_CIB * nch)), (unsigned)((a.Cout + 31) / 32));
+    if constexpr (std::is_same<T, float>::value && LISTS && G::K != 9) {
+        if (a.redo) {
+            const int nx = (int)grid.x, ny = (int)grid.y, nz = (int)grid.z;
+            const dim3 few((unsigned)std::min<int64_t>((int64_t)nx * ny * nz, 512));
+#define APRNET_REDO(N, M16) hipLaunchKernelGGL((conv_dw_redo_kernel<G, DW_CIB, N, M16>), few, dim3(G::NT), 0, st, a, k, nx, ny, nz)
+            if (a.Cout <= 16) { if (nch == 1) APRNET_REDO(1, true); else APRNET_REDO(DW_NCH, true); }
+            else { if (nch == 1) APRNET_REDO(1, false); else APRNET_REDO(DW_NCH, false); }
+#undef APRNET_REDO
+            APRNET_LAUNCH_CHECK("conv_dw_redo_kernel");
+            return 0;
+        }
+    }
     if constexpr (std::is_same<T, bf16_t>::value) {
         if (bf16_math()) {      // bfloat16 matrix instructions; the fp32 ones below when those are asked for
             if (nch == 1) hipLaunchKernelGGL((conv_dw_bf16_kernel<G, DW_CIB, 1, LISTS>), grid, dim3(G::NT), 0, st, a, k, s);
@@ -655,7 +658,7 @@ static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, const WinLists* 
         g.n = k.n_s;
         for (int i = 0; i < k.n_s; ++i) { g.first[i] = 2 * k.blk0[i]; g.out[i] = k.s_of[i]; }
         g.first[k.n_s] = 2 * k.blk0[k.n_s];
-        return launch_sum_slot_groups((const float*)a0.gw_part, a0.gw_part_ld, g, n_el, (float*)a0.gw, st);
+        return launch_sum_slot_groups((const float*)a0.gw_part, a0.gw_part_ld, g, n_el, (float*)a0.gw, st, a0.redo);
     }
     // scanning kernels: one launch per stencil index, level Lc - s for s < S_exp - 1, every coarser level for the last one
     // (adjacent in the tile list, which is sorted finest level first)

@@ -30,18 +30,12 @@
 // inside this kernel a second pass cost registers: 16 -> 16 channels on 23 M particles 3.47 instead of 3.26 ms); an
 // input gradient that holds one is made again from the start by the fp32 kernel.  Small values keep all their bits: features of 1e-37
 // come out with 0.4 of the fp32 instructions' error (split without SPLIT_SCALE, 510 times that error).
-#include "conv_common.hpp"
+#include "pieces.hpp"
 
 namespace aprnet {
 
 typedef float floatx4s __attribute__((ext_vector_type(4)));
 typedef int intx4s __attribute__((ext_vector_type(4)));
-typedef unsigned uintx2s __attribute__((ext_vector_type(2)));
-typedef unsigned uintx4s __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2s __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8s __attribute__((ext_vector_type(8)));
-
-constexpr int SP_CIB = 4;                      // input channels of a staged chunk
 // The 32 k of an instruction are 4 pairs of taps x 4 channels: lane group g = lane / 16 supplies pair 4 step + g.  Pairs are
 // neighbours along y where the stencil's rows have them (dy 0 and 1, dy 2 and 3), the last taps of the rows among themselves.
 // An LDS read of 8 bytes per lane goes out for two lane groups at a time, sixteen neighbouring cells each (256 bytes, every bank
@@ -57,26 +51,6 @@ template <> struct SplitTaps<25> {
     static constexpr signed char tap[32] = {-1, -1, 7, 8, 0, 1, 2, 3, 17, 18, 15, 16, 12, 13, 10, 11, 22, 23, 20, 21, 14, 19, 4, -1, 24, 9, -1, -1, -1, -1, 5, 6};
 };
 template <class G> constexpr int split_steps() { return SplitTaps<G::K>::STEPS; }
-
-// two fp32 numbers -> their bfloat16 roundings, the first in the low half (v_cvt_pk_bf16_f32)
-__device__ __forceinline__ unsigned split_round(float a, float b) {
-    const bf16x2s h = {(__bf16)a, (__bf16)b};
-    return __builtin_bit_cast(unsigned, h);
-}
-__device__ __forceinline__ float split_lo(unsigned p) { return __builtin_bit_cast(float, p << 16); }
-__device__ __forceinline__ float split_hi(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
-
-// What is split lies SPLIT_SCALE times higher than the caller's values (the copies and the packed weights), the results are brought
-// down again: the last bit of any fp32 number, 2^-149 at the least, then is one that a bfloat16 number can hold (2^-133).
-constexpr float SPLIT_SCALE = 65536.f, SPLIT_UNSCALE = 1.f / (SPLIT_SCALE * SPLIT_SCALE);
-
-// two fp32 numbers -> three words with their pieces
-__device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsigned& p2, unsigned& p3) {
-    p1 = split_round(a, b);
-    const float ra = a - split_lo(p1), rb = b - split_hi(p1);
-    p2 = split_round(ra, rb);
-    p3 = split_round(ra - split_lo(p2), rb - split_hi(p2));
-}
 
 constexpr int PREP_TB = 256;
 

@@ -42,15 +42,17 @@ __global__ void __launch_bounds__(64 * W) sum_slots_kernel(const A* __restrict__
 
 // Several sums in one launch: slots first[k] .. first[k + 1] - 1 are added to out + out[k] * n.
 struct SlotGroups { int n; int first[MAX_LEVELS + 2], out[MAX_LEVELS + 1]; };
+// all: null, or a word that is 0 if only the first slot of every pair holds something.
 template <typename A>
-__global__ void __launch_bounds__(1024) sum_slot_groups_kernel(const A* __restrict__ part, int64_t ld, const SlotGroups g, int64_t n, A* __restrict__ out) {
-    const int k = blockIdx.y;
-    sum_slots_body<A, 16>(part + (int64_t)g.first[k] * ld, ld, g.first[k + 1] - g.first[k], n, out + (int64_t)g.out[k] * n);
+__global__ void __launch_bounds__(1024) sum_slot_groups_kernel(const A* __restrict__ part, int64_t ld, const SlotGroups g, int64_t n, A* __restrict__ out,
+                                                               const int* __restrict__ all) {
+    const int k = blockIdx.y, step = all && *all == 0 ? 2 : 1;
+    sum_slots_body<A, 16>(part + (int64_t)g.first[k] * ld, step * ld, (g.first[k + 1] - g.first[k]) / step, n, out + (int64_t)g.out[k] * n);
 }
 template <typename A>
-int launch_sum_slot_groups(const A* part, int64_t ld, const SlotGroups& g, int64_t n, A* out, hipStream_t st) {
+int launch_sum_slot_groups(const A* part, int64_t ld, const SlotGroups& g, int64_t n, A* out, hipStream_t st, const int* all = nullptr) {
     if (n <= 0 || g.n <= 0) return 0;
-    hipLaunchKernelGGL(sum_slot_groups_kernel<A>, dim3((unsigned)((n + 63) / 64), (unsigned)g.n), dim3(1024), 0, st, part, ld, g, n, out);
+    hipLaunchKernelGGL(sum_slot_groups_kernel<A>, dim3((unsigned)((n + 63) / 64), (unsigned)g.n), dim3(1024), 0, st, part, ld, g, n, out, all);
     APRNET_LAUNCH_CHECK("sum_slot_groups_kernel");
     return 0;
 }

@@ -400,7 +400,8 @@ def norm_backward_apply(gy, x, y, mean, rstd, a, b, c):
 def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=True, pieces=True):
     """conv333_backward / conv111_backward (wrap_conv_gpu.hpp:87-133, 216-246) -> [grad_input, grad_weights].
     ``need_input_grad=False`` (stencil convolutions): the input gradient is not computed, grad_input is None.
-    ``pieces``: the input gradient of fp32 features may be made of products of bfloat16 pieces (see conv_forward)."""
+    ``pieces``: the gradients of fp32 features and weights may be made of products of bfloat16 pieces (see conv_forward), the weight
+    gradient where the input gradient is asked for and made of them."""
     _check_input(x, "input")
     _check_input(weights, "weights")
     _check_input(grad_output, "grad_output")

@@ -19,7 +19,7 @@ class APRConv(nn.Module):
     weight_layout = CPU_LAYOUT
     allowed_kernels = SUPPORTED_KERNELS
     # fp32 features may be multiplied as bfloat16 pieces (_ops.conv_forward): in forward passes that no backward pass follows and for
-    # the input gradient.  False on a module keeps all its passes on the fp32 instructions, so that a pass without and one with a
+    # both gradients.  False on a module keeps all its passes on the fp32 instructions, so that a pass without and one with a
     # record give the same bits: re-entrant activation checkpointing (torch.utils.checkpoint with use_reentrant=True) runs its first
     # forward pass without a record and repeats it with one.  (With use_reentrant=False both are recorded.)
     pieces = True

@@ -126,7 +126,8 @@ int aprnet_profile_enable(int on);
  * nodes that the forward kernel's window lists read, and their descendants (default; the node lists are built with the
  * window lists and kept in the plan, 4 bytes per needed node), 17 = every node.
  * And for fp32 features where the caller gives a work space (aprnet_conv_fwd_ws_f32): 18 = products of bfloat16 pieces
- * where that is faster (default), 19 = fp32 matrix instructions, 20 = products of pieces at any size.
+ * where that is faster (default), 19 = fp32 matrix instructions, 20 = products of pieces at any size; 21, 22 and 23 = the same for
+ * the weight gradient of a backward pass whose input gradient is made of pieces (aprnet_conv_bwd_ws_f32).
  * All are HIP kernels; the switch
  * exists so that tests can cover them and memory-bound callers can do without the lists. */
 int aprnet_set_conv_path(int path);
@@ -248,8 +249,8 @@ int64_t aprnet_conv_ws_bytes_f32(const aprnet_plan*, int level_delta, int kz, in
 int aprnet_conv_fwd_ws_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
                            const float* w, int S_exp, int Cout, const float* bias, float* y, int64_t ldy, float* tree_ws,
                            int64_t ld_tree, const aprnet_conv_fusion* fusion, void* ws, int64_t ws_bytes, void* stream);
-/* The same of the backward pass: with aprnet_conv_bwd_ws_bytes_f32() bytes the input gradient is made of products of pieces, from window
- * lists that the plan builds and keeps with the first such call at a level delta; with less, or NULL, it is aprnet_conv_bwd_f32. */
+/* The same of the backward pass: with aprnet_conv_bwd_ws_bytes_f32() bytes the input gradient, and from some work on the weight gradient beside it, is
+ * made of products of pieces, from window lists that the plan builds and keeps with the first such call at a level delta; with less, or NULL, it is aprnet_conv_bwd_f32. */
 int64_t aprnet_conv_bwd_ws_bytes_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, int Cin, int S_exp, int Cout);
 int aprnet_conv_bwd_ws_f32(const aprnet_plan*, int level_delta, int kz, int kx, int ky, const float* x, int64_t ldx, int Cin,
                            const float* w, int S_exp, int Cout, const float* gy, int64_t ldy, float* gx, int64_t ldgx, float* gw,

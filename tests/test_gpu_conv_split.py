@@ -424,3 +424,110 @@ def test_sparse_and_dense_windows(path, density, drop, cout):
     fp32 = _ops.conv_forward([apr], x, w, ld, b)
     assert bool(fp32.isnan().any()) and torch.equal(got.isnan(), fp32.isnan())
     assert bool(((got == fp32) | (got == out[20]) | fp32.isnan()).all())
+
+
+# ---- weight gradient
+@pytest.fixture
+def dw_path():
+    lib = _native.hip()
+    lib.aprnet_set_conv_path(20)
+    yield lambda p: lib.aprnet_set_conv_path(p)
+    for p in (18, 21, 0):
+        lib.aprnet_set_conv_path(p)
+
+
+def weight_gradients(dw_path, p, aprs, xd, wd, gy, ld):
+    dw_path(p)
+    return _ops.conv_backward(aprs, xd, wd, gy, ld)[1]
+
+
+def _dw_case(bt, ksize, cin, cout):
+    x, aprs, ld, w_exp = _conv_case(bt, ksize, 2, cin, cout, torch.float32)
+    gy = torch.randn(x.size(0), cout, x.size(2), generator=torch.Generator().manual_seed(3))
+    for i, a in enumerate(aprs):
+        gy[i, :, oracle.number_parts(a, int(ld[i])):] = 0
+    return x, aprs, ld, w_exp, gy
+
+
+# one and several blocks of eight input and of 16 or 32 output channels, incomplete groups of four on either side; windows of one to
+# several groups of columns
+@pytest.mark.parametrize("cin,cout", [(1, 16), (7, 17), (8, 32), (9, 33), (18, 16), (30, 70)])
+@pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 5, 5)], ids=["k333", "k155"])
+@pytest.mark.parametrize("bt", [[("3d_s", 0), ("3d_t", 1)], [("3d_a", 0)], [("3d_c", 2)], [("2d_a", 1), ("2d_s", 0)]], ids=["3d", "3d_odd", "3d_coarse", "2d"])
+def test_weight_gradient_against_float64(dw_path, bt, ksize, cin, cout):
+    x, aprs, ld, w_exp, gy = _dw_case(bt, ksize, cin, cout)
+    xd, wd, gd = x.to(DEV), layer(w_exp), gy.to(DEV)
+    ref = _ops.conv_backward(aprs, xd.double(), wd.double(), gd.double(), ld)[1].cpu()
+    fp32 = weight_gradients(dw_path, 22, aprs, xd, wd, gd, ld)
+    got = weight_gradients(dw_path, 23, aprs, xd, wd, gd, ld)
+    assert not torch.equal(got, fp32)
+    close(got, ref.float(), torch.float32)
+    # sums of a handful of products are rounded too few times for the mean to tell: no larger an error over the sample, one per cent of play
+    assert error(got, ref) <= 1.01 * error(fp32, ref)
+    assert torch.equal(got, weight_gradients(dw_path, 23, aprs, xd, wd, gd, ld))
+
+
+@pytest.mark.parametrize("where", ["features", "gradient"])
+@pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("cin,cout", [(16, 16), (9, 40)])
+def test_weight_gradient_that_is_not_finite(dw_path, cin, cout, value, where):
+    """Then all of it is the fp32 instructions', bit for bit, of the batch item that holds the value (3.4e38 has an infinite first
+    piece, the sums are finite)."""
+    x, aprs, ld, w_exp, gy = _dw_case([("3d_s", 0), ("3d_a", 0)], (3, 3, 3), cin, cout)
+    (x if where == "features" else gy)[0, 3, 11] = value
+    (gy if where == "features" else x).mul_(1e-3)
+    xd, wd, gd = x.to(DEV), layer(w_exp), gy.to(DEV)
+    fp32 = weight_gradients(dw_path, 22, aprs[:1], xd[:1], wd, gd[:1], ld[:1])
+    got = weight_gradients(dw_path, 23, aprs[:1], xd[:1], wd, gd[:1], ld[:1])
+    assert torch.equal(got.nan_to_num(nan=7.0), fp32.nan_to_num(nan=7.0)) and bool(fp32.isfinite().all()) == (value == 3.4e38)
+    both, item = (weight_gradients(dw_path, 23, aprs[k:], xd[k:], wd, gd[k:], ld[k:]) for k in (0, 1))
+    assert torch.equal(both.isnan(), fp32.isnan()) and bool(item.isfinite().all())
+    fin = fp32.isfinite() & (fp32.abs() < 1e30)
+    assert torch.equal(both[fin], (got + item)[fin]) or error(both[fin], (got + item)[fin].cpu().double()) < 1e-6
+
+
+@pytest.mark.parametrize("x_scale,g_scale", [(1e-36, 1), (1e-41, 1), (1, 1e-38), (1e-36, 1e30), (1e-18, 1e-18)])
+def test_weight_gradient_of_small_operands(dw_path, x_scale, g_scale):
+    x, aprs, ld, w_exp, gy = _dw_case([("3d_s", 0)], (3, 3, 3), 16, 16)
+    xd, wd, gd = (x * x_scale).to(DEV), layer(w_exp), (gy * g_scale).to(DEV)
+    ref = _ops.conv_backward(aprs, xd.double(), wd.double(), gd.double(), ld)[1].cpu()
+    err = [error(weight_gradients(dw_path, p, aprs, xd, wd, gd, ld), ref) for p in (22, 23)]
+    assert err[1] <= err[0]
+
+
+@pytest.mark.parametrize("products", [1, 2, 3, 9, 27])
+def test_weight_gradient_of_few_products(dw_path, products):
+    """An output gradient that is zero but at a few places.  They lie in different windows, whose products go to sums of their own: each of
+    these is a single product, whose error is at most 1.03 of one rounding's (see test_few_products), and adding them up rounds
+    alike; 0.03 for the sample."""
+    apr = apr_cases.random_apr((48, 64, 64), 43, 0.4)
+    apr.init_cuda()
+    n, ld, S = apr.total_number_particles(), torch.zeros(1, dtype=torch.int32), apr.level_max() - apr.level_min() + 1
+    g = torch.Generator().manual_seed(5)
+    x, w = torch.randn(1, 32, n, generator=g).to(DEV), torch.randn(S, 32, 32, 3, 3, 3, generator=g).to(DEV)
+    gd = torch.zeros(1, 32, n)
+    at = torch.randint(n // 2, n, (32, products), generator=g)
+    gd[0].scatter_(1, at, torch.randn(32, products, generator=g))
+    gd = gd.to(DEV)
+    ref = _ops.conv_backward([apr], x.double(), w.double(), gd.double(), ld)[1].cpu()
+    err = [error(weight_gradients(dw_path, p, [apr], x, w, gd, ld), ref) for p in (22, 23)]
+    assert err[1] <= 1.06 * err[0]
+
+
+def test_weight_gradient_under_capture(dw_path):
+    """Recorded into a graph and replayed on new features, finite ones and others, with eager calls in between."""
+    x, aprs, ld, w_exp, gy = _dw_case([("3d_s", 0)], (3, 3, 3), 16, 32)
+    xs, wd, gd = x.to(DEV), layer(w_exp), gy.to(DEV)
+    weight_gradients(dw_path, 23, aprs, xs, wd, gd, ld)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = _ops.conv_backward(aprs, xs, wd, gd, ld)[1]
+    for i in range(4):
+        xs.copy_(x.to(DEV) * (i + 1))
+        if i == 2:
+            xs[0, 0, 5] = float("nan")
+        want = _ops.conv_backward(aprs, xs, wd, gd, ld)[1]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.nan_to_num(), want.nan_to_num()) and torch.equal(out.isnan(), want.isnan())

@@ -121,6 +121,8 @@ struct aprnet_plan {
     void* d_apr_xz = nullptr; void* d_apr_y = nullptr; void* d_tree_xz = nullptr; void* d_tree_y = nullptr;
     int32_t* d_children = nullptr;      // [8][n_tree], slot-major
     int64_t n_tree = 0, n_apr = 0;
+    uint32_t* d_parents = nullptr;      // [n_apr + n_tree] parents of the particles and of the tree nodes (grad_groups.hip), null: not built yet
+    bool parents_unavailable = false;   // building it failed once: do not retry
     std::map<std::tuple<int, int, int, int>, aprnet::TileList> tiles;   // (level_delta, TZ, TX, halo) -> row groups
     void* d_scratch = nullptr; size_t scratch_bytes = 0;          // re-laid-out weights of the call in flight
     size_t scratch_refused = 0;                                   // a size that could not be allocated (0: none)

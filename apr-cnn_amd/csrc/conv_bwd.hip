@@ -15,6 +15,8 @@
 // stencil index changes and at the end.
 #include "dw_work.hpp"
 
+#include <functional>
+
 namespace aprnet {
 
 // Streaming passes over the rows of the work space: a thread handles STREAM_V consecutive values with 16-byte accesses
@@ -276,6 +278,9 @@ size_t conv_packed_bf16_bytes(int code, int S_exp, int Cout, int Cin);
 int pack_conv_weights_bf16(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, hipStream_t st, bool transposed);
 int interleave8_bf16(const bf16_t* x, int64_t ldx, const bf16_t* x2, int64_t ldx2, int c_split, int C, int64_t count, bf16_t* out,
                      hipStream_t st);
+int get_parents(aprnet_plan* p, hipStream_t st);
+int finish_grouped_gradient(const aprnet_plan* p, int d, const float* gx4, int64_t ldx, int C, float* gt4, int64_t ldt, bf16_t* gx, int64_t ldgx,
+                            const NeedLists* need, hipStream_t st);
 int bf16_regroup();
 int bf16_math();
 int bwd_deterministic();
@@ -294,7 +299,9 @@ static void set_dw_partials(aprnet_plan* p, size_t off, int code, ConvArgs<T>& a
     a.gw_part_ld = (int64_t)a.Cout * a.Cin * (code == 333 ? 27 : code == 133 ? 9 : 25);
 }
 
-template <typename T> static int try_mfma_bwd(aprnet_plan*, const ConvArgs<T>&, const TileList&, int, int, hipStream_t, bool*, void*, int64_t) { return 0; }
+// clear(finest): clears the input gradient and the tree's, with or without the places on the finest level
+typedef std::function<void(bool)> ClearGradient;
+template <typename T> static int try_mfma_bwd(aprnet_plan*, const ConvArgs<T>&, const TileList&, int, int, hipStream_t, bool*, void*, int64_t, const ClearGradient&) { return 0; }
 static int fork_side(aprnet_plan* p, hipStream_t st, hipStream_t* side);
 static int join_side(aprnet_plan* p, hipStream_t st, hipStream_t side);
 // Joins the side stream on every way out of a backward call, also the failing ones: the caller's stream must not run
@@ -306,7 +313,7 @@ struct SideJoin {
     ~SideJoin() { if (open) (void)join_side(p, st, side); }
 };
 template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, const TileList& tl, int code, int d, hipStream_t st, bool* done,
-                                    void* ws, int64_t ws_bytes) {
+                                    void* ws, int64_t ws_bytes, const ClearGradient& clear) {
     if (conv_path() == 1 || !conv_mfma_supported(code)) return 0;
     *done = true;
     // weight gradient on the side stream (when there is an input gradient to run next to)
@@ -333,6 +340,7 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     ScratchLease lease;          // before the join guard below: its hand-over event is recorded after the join
     if (wbytes + pbytes) if (int rc = lease.acquire(p, wbytes + pbytes, st)) return rc;
     if (pbytes) set_dw_partials(p, wbytes, code, c);
+    clear(!pieces);
     // On products of bfloat16 pieces both halves read one copy of the output gradient in groups of four channels, and fp32 kernels
     // follow that do all of it again if a sum was not finite (conv_split.hip, conv_dw_split.hip).
     int* mark = nullptr;
@@ -428,10 +436,12 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
     NeedLists need_store;
     const NeedLists* need = sizeof(T) == 4 ? needed_nodes(p, d, code, tl, st, &need_store) : nullptr;
     if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, need)) return rc;
-    if (gx) {
-        fill2d<T>(gx, ldgx, p->number_parts(d), Cin, (T)0, st);
+    // (products of pieces write every place on the finest level, the last ones of a plane: see conv_bwd_bf16)
+    auto clear = [&](bool finest) {
+        if (!gx) return;
+        fill2d<T>(gx, ldgx, finest ? p->number_parts(d) : p->apr.level_begin(p->lc(d)), Cin, (T)0, st);
         fill2d<T>(gtree_ws, ldgt, nt, Cin, (T)0, st);
-    }
+    };
     if (tl.n > 0) {
         ConvArgs<T> a{};
         a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.n_tiles = tl.n;
@@ -442,7 +452,8 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
         constexpr bool f32 = sizeof(T) == 4;
         int rc = 0;
         bool done = false;
-        if ((rc = try_mfma_bwd<T>(p, a, tl, code, d, st, &done, ws, ws_bytes))) return rc;
+        if ((rc = try_mfma_bwd<T>(p, a, tl, code, d, st, &done, ws, ws_bytes, clear))) return rc;
+        if (!done) clear(true);
         if (!done) switch (code) {
             case 333: rc = launch_bwd<T, X333, (f32 ? 4 : 2), W333, (f32 ? 8 : 4), (f32 ? 32 : 16)>(a, st); break;
             case 133: rc = launch_bwd<T, X133, (f32 ? 8 : 4), W133, (f32 ? 8 : 4), (f32 ? 32 : 16)>(a, st); break;
@@ -450,7 +461,7 @@ int conv_bwd(const aprnet_plan* cp, int d, int kz, int kx, int ky, const T* x, i
             case 555: rc = launch_bwd<T, X555, 1, W555, (f32 ? 4 : 2), (f32 ? 32 : 16)>(a, st); break;
         }
         if (rc) return rc;
-    }
+    } else clear(true);
     return gx ? fill_tree_bwd_for_conv(p, d, gx, ldgx, Cin, gtree_ws, ldgt, st, need) : 0;
 }
 
@@ -523,11 +534,8 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
     NeedLists need_store;            // (a regrouped copy carries the unfilled nodes along unread)
     const NeedLists* nodes = needed_nodes(p, d, code, tl, st, &need_store);
     if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, nodes)) return rc;
-    if (gx) {
-        fill2d<float>(gx32_ws, ldgx32, np, Cin, 0.f, st);
-        fill2d<float>(gtree_ws, ldgt, nt, Cin, 0.f, st);
-    }
     if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &near, st, 1)) return rc;
+    bool g4 = false;                 // the work spaces hold groups of four channels (grad_groups.hip)
     if (tl.n > 0) {
         ConvArgs<bf16_t> a{};
         a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.n_tiles = tl.n;
@@ -547,6 +555,14 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         // everything that can allocate or fail on the host comes before the fork
         if (near.n > 0 && bf16_math())
             if (int rc = set_conv_dx_lists(p, d, code, near, b, st)) return rc;
+        // (the kernels with lists; other channel counts, tables that cannot be built: planes)
+        g4 = near.n > 0 && b.tile_win && Cin % 4 == 0 && (((uintptr_t)gx32_ws | (uintptr_t)gtree_ws) & 15) == 0 && get_parents(p, st) == 0;
+        if (g4) {
+            b.gx_g4 = 1; b.ldgx = np; b.ldgt = nt;
+            // Places on the finest level, the last ones, are written by the one column they have (COL_SOLE): cleared are the others.
+            fill2d<float>(gx32_ws, 4 * np, 4 * p->apr.level_begin(p->lc(d)), Cin / 4, 0.f, st);
+            fill2d<float>(gtree_ws, 4 * nt, 4 * nt, Cin / 4, 0.f, st);
+        }
         // Both halves stage from copies grouped by eight channels behind the packed weights in the scratch buffer: the output
         // gradient (read by both), the features and their tree (weight gradient).
         auto align = [](size_t v) { return (v + 255) / 256 * 256; };
@@ -583,6 +599,10 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
             if (rc) return rc;
         }
         if (pbytes && !dw_g8) set_dw_partials(p, need, code, a);
+        if (gx && !g4) {
+            fill2d<float>(gx32_ws, ldgx32, np, Cin, 0.f, st);
+            fill2d<float>(gtree_ws, ldgt, nt, Cin, 0.f, st);
+        }
         bf16_t* gyi = (bf16_t*)((char*)p->d_scratch + wbytes);
         if (dw_g8 || dx_g8) if (int rc = interleave8_bf16(gy, ldy, nullptr, 0, Cout, Cout, np, gyi, st)) return rc;
         hipStream_t side = st;
@@ -611,8 +631,12 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
             if (int rc = launch_conv_dx_mfma(code, b, near.n, st)) return rc;
         }
         if (int rc = guard.join()) return rc;
+    } else if (gx) {
+        fill2d<float>(gx32_ws, ldgx32, np, Cin, 0.f, st);
+        fill2d<float>(gtree_ws, ldgt, nt, Cin, 0.f, st);
     }
     if (!gx) return 0;
+    if (g4) return finish_grouped_gradient(p, d, gx32_ws, np, Cin, gtree_ws, nt, gx, ldgx, nodes, st);
     if (int rc = fill_tree_bwd_for_conv(p, d, gx32_ws, ldgx32, Cin, gtree_ws, ldgt, st, nodes)) return rc;
     if (np > 0) {
         dim3 grid((unsigned)((np + STREAM_BLOCK - 1) / STREAM_BLOCK), (unsigned)Cin);

@@ -54,6 +54,7 @@ struct ConvArgs {
     // backward only
     // gradients are accumulated in the computation type (fp32 for bfloat16 features)
     const T* gy; typename Num<T>::acc* gx; int64_t ldgx; typename Num<T>::acc* gtree; int64_t ldgt;
+    int gx_g4;                                 // bfloat16 features: gx and gtree hold groups of four channels, [Cin / 4][ld][4] (grad_groups.hip)
     typename Num<T>::acc* gw; int n_tiles;
     // Weight gradient without atomics: every persistent workgroup writes the sums of its tiles to two slots (one per
     // half of the columns) of gw_part [2 * workgroups][gw_part_ld], which a second kernel adds up in slot order and

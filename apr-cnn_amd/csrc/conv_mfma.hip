@@ -736,14 +736,27 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
                     if (co0 + cl < a.Cout) a.y[(int64_t)(co0 + cl) * a.ldy + o] = float_to_bf16(v);
                 }
         } else {
-            // A place that no other column adds to (COL_SOLE) takes a plain store onto the cleared buffer, the same value; the
+            // A place that no other column adds to (COL_SOLE) takes a plain store; the
             // others are added atomically.  With every column added atomically the additions bounded the kernel:
             // training step on 5.5 M particles 24.7 -> 21.4 ms, 1x5x5 64 -> 64 forward and backward on 15.4 M 27.8 -> 25.9 ms.
             // (In the fp32 kernel, bound by its matrix phases, the same changed nothing: 27.22 and 27.32 ms for a chain.)
             const unsigned cp = sh.col_pos[col];
             const bool to_tree = (cp & COL_TREE) != 0;
-            float* dst = (to_tree ? a.gtree : a.gx) + o;
             const int64_t ld = to_tree ? a.ldgt : a.ldgx;
+            if (a.gx_g4) {                      // uniform; the lane's four channels of a part are one group
+#pragma unroll
+                for (int h = 0; h < COH; ++h) {
+                    const int c4 = co0 + h * 16 + 4 * (lane >> 4);
+                    if (c4 >= a.Cout) continue;
+                    float* g = (to_tree ? a.gtree : a.gx) + (((int64_t)(c4 >> 2) * ld + o) << 2);
+                    if (cp & COL_SOLE) *reinterpret_cast<floatx4*>(g) = acc[j][h];
+                    else
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) unsafeAtomicAdd(g + r, acc[j][h][r]);
+                }
+                continue;
+            }
+            float* dst = (to_tree ? a.gtree : a.gx) + o;
             if (cp & COL_SOLE) {
 #pragma unroll
                 for (int h = 0; h < COH; ++h)

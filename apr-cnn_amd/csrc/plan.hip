@@ -319,7 +319,7 @@ int aprnet_plan_create(const aprnet_access_desc* apr, const aprnet_access_desc* 
 void aprnet_plan_destroy(aprnet_plan* p) {
     if (!p) return;
     (void)hipSetDevice(p->device);
-    for (void* q : {p->d_apr_xz, p->d_apr_y, p->d_tree_xz, p->d_tree_y, (void*)p->d_children})
+    for (void* q : {p->d_apr_xz, p->d_apr_y, p->d_tree_xz, p->d_tree_y, (void*)p->d_children, (void*)p->d_parents})
         if (q) (void)hipFree(q);
     for (auto& kv : p->tiles) if (kv.second.d_tiles) (void)hipFree(kv.second.d_tiles);
     if (p->d_scratch) (void)hipFree(p->d_scratch);

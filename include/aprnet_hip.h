@@ -300,7 +300,8 @@ int aprnet_sample_particles_bwd_bf16(const aprnet_plan*, int level_delta, const 
                                      int64_t ld_img, void* stream);
 /* Backward of the stencil convolution with bfloat16 features and output gradient: fp32 weights, fp32 weight
  * gradient (accumulated into gw), fp32 accumulation everywhere; the input gradient is collected in the fp32 work
- * space gx32_ws [Cin][ld_gx32] (ld_gx32 >= aprnet_number_parts) and rounded to bfloat16 into gx at the end.
+ * space gx32_ws [Cin][ld_gx32] (ld_gx32 >= aprnet_number_parts) and rounded to bfloat16 into gx at the end (what the work spaces hold
+ * then, and in which layout, is not defined: groups of four channels where Cin is a multiple of four and both are 16-byte aligned).
  * gtree_ws: fp32 [Cin][ld_gtree].  The input gradient multiplies on the bfloat16 matrix cores (weights rounded to
  * bfloat16) from input-gradient lists that the plan builds on first use; with aprnet_set_conv_path(3) or (5) it
  * runs with fp32 products and scans per call.  The weight gradient multiplies on the bfloat16 matrix cores as well

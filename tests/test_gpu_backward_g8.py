@@ -98,6 +98,34 @@ def test_tree_gradient_of_the_nodes_with_outputs(shape, drop, ksize, deltas, dty
             assert float((got[1] - ref[1]).abs().max()) <= 1e-5 * float(ref[1].abs().max())
 
 
+@pytest.mark.parametrize("cin", [4, 8, 20, 36])
+@pytest.mark.parametrize("shape,drop,ksize,deltas", [((70, 90, 110), 4, (3, 3, 3), (0, 2)), ((1, 500, 611), 6, (1, 5, 5), (0, 1)), ((31, 33, 35), 3, (1, 3, 3), (0, 1)),
+                                                     ((9, 12, 1), 2, (1, 3, 3), (0,)), ((128, 128, 130), 6, (3, 3, 3), (0,))])
+def test_input_gradient_in_groups_of_four_channels(monkeypatch, shape, drop, ksize, deltas, cin):
+    """Work spaces in groups of four channels (whole groups only), cleared where something is added and finished by one pass, against
+    the kernels that scan, on planes that are cleared whole; work spaces hold NaN before the call.  Small whole numbers, as above:
+    bit-identical.  One to several groups per thread, levels of the tree walked in one launch, from a list and whole."""
+    apr = apr_cases.random_apr(shape, 5, 0.01 if drop > 2 else 0.1, drop)
+    gen = torch.Generator().manual_seed(3)
+    lib, empty = _native.hip(), torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: (lambda t: t.fill_(float("nan")) if t.is_floating_point() else t)(empty(*a, **k)))
+    for delta in deltas:
+        n = utils.number_particles(apr, delta)
+        ld = torch.tensor([delta], dtype=torch.int32)
+        x = torch.randint(-3, 4, (1, cin, n), generator=gen).to(torch.bfloat16).to(DEV)
+        gy = torch.randint(-3, 4, (1, 18, n), generator=gen).to(torch.bfloat16).to(DEV)
+        w = torch.randint(-2, 3, (apr.level_max() - apr.level_min() + 1, 18, cin) + ksize, generator=gen).float().to(DEV)
+        got = _ops.conv_backward([apr], x, w, gy, ld)[0]
+        for off, on in ((17, 16), (5, 4)):
+            assert lib.aprnet_set_conv_path(off) == 0
+            try:
+                ref = _ops.conv_backward([apr], x, w, gy, ld)[0]
+            finally:
+                lib.aprnet_set_conv_path(on)
+            assert float(ref.float().abs().max()) > 0
+            assert torch.equal(got, ref)
+
+
 def test_weight_gradient_without_room_for_the_copies():
     """A capture must not grow the plan's scratch buffer: when the copies do not fit what is there, the kernel on channel planes
     runs as it did for the eager call that sized the buffer (same kernel, same order of summation: bit-identical)."""

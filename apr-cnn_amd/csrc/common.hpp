@@ -80,7 +80,8 @@ struct TileList {
 
 // Precomputed window lists of the forward convolution (lists.hip), device arrays owned by the plan.
 struct WinLists {
-    int* d_tile_win = nullptr;                  // [n_tiles + 1]
+    void* d_block = nullptr;                    // one allocation, the arrays below lie in it
+    int* d_level = nullptr;                     // [n_win] level of a window
     int4* d_win = nullptr;                      // [n_win] {first item, items, first column, columns}
     int* d_item_idx = nullptr; unsigned short* d_item_pos = nullptr;
     int* d_col_idx = nullptr; unsigned short* d_col_pos = nullptr;

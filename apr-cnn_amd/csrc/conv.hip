@@ -154,7 +154,7 @@ size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
 int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
                   const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
-int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, const WinLists& wl, hipStream_t st);
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
 static std::atomic<int> g_dw_split{1};       // and their weight gradient (conv_dw_split.hip), likewise
 
@@ -179,15 +179,17 @@ int backward_overlap() { return g_bwd_overlap; }
 static std::atomic<int> g_bwd_deterministic{1};   // backward: weight gradient summed in a fixed order (partial sums per workgroup) instead of atomics
 int bwd_deterministic() { return g_bwd_deterministic; }
 
-// Points the kernel at the plan's window lists.  When the lists are switched off, or cannot be built (no device
-// memory for them, too many entries), a.tile_win stays null and the kernel scans the access arrays itself.
+// Points the kernel at the plan's window lists (a.n_tiles: how many there are).  When the lists are switched off, or cannot be built (no device
+// memory for them, too many entries), a.win_level stays null and the kernel scans the access arrays itself.
 template <typename T>
 static int set_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<T>& a, hipStream_t st, int dx = 0) {
-    a.tile_win = nullptr;
+    a.win_level = nullptr;
     if (!g_use_lists) return 0;
     WinLists wl;
     if (get_lists(p, d, code, tl, &wl, st, dx) != 0) { (void)hipGetLastError(); return 0; }
-    a.tile_win = wl.d_tile_win; a.win = wl.d_win;
+    if (wl.n_win == 0) return 0;
+    a.n_tiles = wl.n_win;
+    a.win_level = wl.d_level; a.win = wl.d_win;
     a.l_item_idx = wl.d_item_idx; a.l_item_pos = wl.d_item_pos; a.l_col_idx = wl.d_col_idx; a.l_col_pos = wl.d_col_pos;
     return 0;
 }
@@ -215,7 +217,7 @@ static int try_narrow(aprnet_plan* p, const ConvArgs<T>& a, int code, int d, con
     if (int rc = pack_conv_weights_narrow(code, (const float*)a.w, a.S_exp, a.Cout, a.Cin, (float*)p->d_scratch, st, bf16m)) return rc;
     ConvArgs<T> b = a;
     b.w = (const float*)p->d_scratch;
-    b.tile_win = wl.d_tile_win; b.win = wl.d_win;
+    b.win_level = wl.d_level; b.win = wl.d_win;
     b.l_item_idx = wl.d_item_idx; b.l_item_pos = wl.d_item_pos; b.l_col_idx = wl.d_col_idx; b.l_col_pos = wl.d_col_pos;
     TimedLaunch timed(st);
     return launch_conv_narrow(code, b, wl, st);
@@ -279,7 +281,7 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
     ConvArgs<float> b = a;
     if (int rc = set_lists(p, d, code, tl, b, st)) return rc;
     WinLists wl;
-    const size_t need = b.tile_win && get_lists(p, d, code, tl, &wl, st) == 0 ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
+    const size_t need = b.win_level && get_lists(p, d, code, tl, &wl, st) == 0 ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
     if (need > 0 && ws && ws_bytes >= 0 && (size_t)ws_bytes >= need) {
         // products of bfloat16 pieces on copies in groups of four channels, all in the caller's work space
         const size_t wbytes = split_align(conv_packed_split_bytes(code, a.S_exp, a.Cout, a.Cin)), ng = (size_t)(a.Cin + 3) / 4;
@@ -290,7 +292,7 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
         b.w_raw = a.w; b.w = (const float*)image; b.redo = (int*)ws;
         b.xi = xi; b.ti = ti; b.xi_ld = a.x_count; b.ti_ld = a.t_count;
         TimedLaunch timed(st);
-        return launch_conv_split(code, b, n_tiles, wl, st);
+        return launch_conv_split(code, b, b.n_tiles, st);
     }
     // plan-owned scratch for the re-laid-out weights, grown on demand
     ScratchLease lease;
@@ -298,7 +300,7 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
     if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cout, a.Cin, false, (float*)p->d_scratch, st)) return rc;
     b.w = (const float*)p->d_scratch;
     TimedLaunch timed(st);
-    return launch_conv_mfma(code, b, n_tiles, st);
+    return launch_conv_mfma(code, b, b.win_level ? b.n_tiles : n_tiles, st);
 }
 
 int fill_tree_for_conv(const aprnet_plan* p, int d, const float* x, int64_t ldx, int C, float* tree, int64_t ldt, hipStream_t st,
@@ -432,7 +434,7 @@ int conv_fwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         if (done) return 0;
     }
     if (int rc = set_lists(p, d, code, tl, a, st)) return rc;
-    const bool bf16_math = g_bf16_math && a.tile_win;      // the bfloat16 contraction exists with window lists only
+    const bool bf16_math = g_bf16_math && a.win_level;      // the bfloat16 contraction exists with window lists only
     const int64_t n_x = p->number_parts(d), n_t = p->tree_parts(d);
     ScratchLease lease;
     if (bf16_math) {
@@ -454,13 +456,14 @@ int conv_fwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         if (int rc = lease.acquire(p, conv_packed_floats(code, S_exp, Cout, Cin, false) * sizeof(float), st)) return rc;
         if (int rc = pack_conv_weights(code, w, S_exp, Cout, Cin, false, (float*)p->d_scratch, st)) return rc;
     }
+    if (!a.win_level) a.n_tiles = tl.n;
     a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles;
     a.x = x; a.ldx = ldx; a.Cin = Cin; a.w = (const float*)p->d_scratch; a.S_exp = S_exp; a.Cout = Cout; a.bias = bias;
     a.x2 = fu.x2; a.ldx2 = fu.ldx2; a.c_split = C1; a.relu = fu.relu;
     a.y = y; a.ldy = ldy; a.tree_data = tree_ws; a.ldt = ldt; a.Lc = p->lc(d); a.tree_off = p->tree_offset(a.Lc);
     a.x_count = p->number_parts(d); a.t_count = p->tree_parts(d);
     TimedLaunch timed(st);
-    return bf16_math ? launch_conv_mfma_bf16(code, a, tl.n, st) : launch_conv_mfma(code, a, tl.n, st);
+    return bf16_math ? launch_conv_mfma_bf16(code, a, a.n_tiles, st) : launch_conv_mfma(code, a, a.n_tiles, st);
 }
 
 // bfloat16 features with a layout per tensor: planes [C][ld] or groups of eight channels [C / 8][ld][8] (grouped.hip).
@@ -531,7 +534,7 @@ int conv_fwd_bf16_layout(const aprnet_plan* cp, int d, int kz, int kx, int ky, c
     }
     if (tl.n == 0) return 0;
     if (int rc = set_lists(p, d, code, tl, a, st)) return rc;
-    if (!a.tile_win) return fail(APRNET_ERR_UNSUPPORTED, "conv_forward: the window lists of the plan are not available");
+    if (!a.win_level) return fail(APRNET_ERR_UNSUPPORTED, "conv_forward: the window lists of the plan are not available");
     // An image of the weights that the caller keeps spares a launch of 6 to 13 us per layer (28 to 1792 small blocks, bound by their
     // start and by reads 27 floats apart), which is what 13 layers of a U-Net on 0.6 M particles spend 7 % of their time on.
     ScratchLease lease;
@@ -545,7 +548,7 @@ int conv_fwd_bf16_layout(const aprnet_plan* cp, int d, int kz, int kx, int ky, c
     // 16-byte items: 32-bit byte offsets reach 2^28 elements of a group; beyond, the kernel takes 64-bit addresses
     a.big = g_big_addr || a.x_count >= (1ll << 28) || a.t_count >= (1ll << 28);
     TimedLaunch timed(st);
-    return launch_conv_mfma_bf16(code, a, tl.n, st);
+    return launch_conv_mfma_bf16(code, a, a.n_tiles, st);
 }
 
 int conv111_fwd_relu(const aprnet_plan*, int, const float*, int64_t, int, const float*, int, int, const float*, float*, int64_t, hipStream_t, int);

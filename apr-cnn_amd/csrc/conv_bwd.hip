@@ -260,7 +260,7 @@ int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool 
 int conv_path();
 // the tree nodes the forward window lists name, null: fill every node (conv.hip)
 const NeedLists* needed_nodes(aprnet_plan* p, int d, int code, const TileList& tl, hipStream_t st, NeedLists* store);
-// points a at the plan's window lists (conv.hip); leaves a.tile_win null when they are off or unavailable
+// points a at the plan's window lists (conv.hip); leaves a.win_level null when they are off or unavailable
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<float>& a, hipStream_t st);
 int set_conv_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st);
 int set_conv_dx_lists(aprnet_plan* p, int d, int code, const TileList& tl, ConvArgs<bf16_t>& a, hipStream_t st);
@@ -320,8 +320,8 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     ConvArgs<float> c = a;
     if (int rc = set_conv_lists(p, d, code, tl, c, st)) return rc;
     WinLists lists;
-    const WinLists* wl = c.tile_win && get_lists(p, d, code, tl, &lists, st) == 0 ? &lists : nullptr;
-    if (!wl) c.tile_win = nullptr;
+    const WinLists* wl = c.win_level && get_lists(p, d, code, tl, &lists, st) == 0 ? &lists : nullptr;
+    if (!wl) c.win_level = nullptr;
     // everything that can allocate or fail on the host comes before the fork
     TileList near;
     FaceLists faces;
@@ -333,7 +333,7 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     bool pieces = need > 0 && ws_bytes >= 0 && (size_t)ws_bytes >= need && near.n > 0;
     if (pieces) {
         if (int rc = set_conv_dx_lists(p, d, code, near, e, st)) return rc;
-        pieces = e.tile_win != nullptr;
+        pieces = e.win_level != nullptr;
     }
     const size_t wbytes = a.gx ? (conv_packed_floats(code, a.S_exp, a.Cin, a.Cout, true) * sizeof(float) + 255) / 256 * 256 : 0;
     const size_t pbytes = bwd_deterministic() ? conv_dw_partial_bytes(code, a.Cout, a.Cin, a.S_exp, a.Lc, wl) : 0;
@@ -352,7 +352,6 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
         redo = RedoClear{mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin};
         if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, nullptr, 0, a.Cout, a.x_count, gi,
                                    nullptr, 0, 0, nullptr, st)) return rc;
-        e.tiles = near.d_tiles; e.n_tiles = near.n;
         e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
         e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
     }
@@ -367,7 +366,7 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
     if (a.gx) {
         // input gradient: the forward kernel on the output gradient with the transposed, flipped stencil;
         // every row group within one row of an output takes part
-        if (pieces) if (int rc = launch_conv_dx_split(code, e, near.n, st)) return rc;
+        if (pieces) if (int rc = launch_conv_dx_split(code, e, e.n_tiles, st)) return rc;
         if (int rc = pack_conv_weights(code, a.w, a.S_exp, a.Cin, a.Cout, true, (float*)p->d_scratch, st, &redo)) return rc;
         ConvArgs<float> b = a;
         b.redo = mark;
@@ -556,7 +555,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         if (near.n > 0 && bf16_math())
             if (int rc = set_conv_dx_lists(p, d, code, near, b, st)) return rc;
         // (the kernels with lists; other channel counts, tables that cannot be built: planes)
-        g4 = near.n > 0 && b.tile_win && Cin % 4 == 0 && (((uintptr_t)gx32_ws | (uintptr_t)gtree_ws) & 15) == 0 && get_parents(p, st) == 0;
+        g4 = near.n > 0 && b.win_level && Cin % 4 == 0 && (((uintptr_t)gx32_ws | (uintptr_t)gtree_ws) & 15) == 0 && get_parents(p, st) == 0;
         if (g4) {
             b.gx_g4 = 1; b.ldgx = np; b.ldgt = nt;
             // Places on the finest level, the last ones, are written by the one column they have (COL_SOLE): cleared are the others.
@@ -568,7 +567,7 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         auto align = [](size_t v) { return (v + 255) / 256 * 256; };
         const size_t ngo = (size_t)(Cout + 7) / 8, ngi = (size_t)(Cin + 7) / 8;
         // the image of the weights that the input gradient below packs: fp32 ones where it has no lists (twice the bfloat16 size)
-        const size_t wbytes = near.n == 0 ? 0 : align(b.tile_win ? conv_packed_bf16_bytes(code, S_exp, Cin, Cout)
+        const size_t wbytes = near.n == 0 ? 0 : align(b.win_level ? conv_packed_bf16_bytes(code, S_exp, Cin, Cout)
                                                                  : conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
         const size_t gybytes = align(ngo * (size_t)np * 16);
         const int chunk = gx ? dw_copy_channels(Cin, np, nt, gybytes) : (Cin + 15) / 16 * 16;
@@ -576,10 +575,10 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
         const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
         WinLists wl;
-        const bool listed = a.tile_win && get_lists(p, d, code, tl, &wl, st, false) == 0;
-        if (!listed) a.tile_win = nullptr;
+        const bool listed = a.win_level && get_lists(p, d, code, tl, &wl, st, false) == 0;
+        if (!listed) a.win_level = nullptr;
         bool dw_g8 = regroup_gy && bwd_deterministic() && listed && gybytes + ngi * (size_t)(np + nt) * 16 <= ((size_t)48 << 30);
-        const bool dx_g8 = near.n > 0 && b.tile_win && regroup_gy;
+        const bool dx_g8 = near.n > 0 && b.win_level && regroup_gy;
         size_t need = 0, pbytes = 0;
         auto layout = [&]() {
             need = wbytes + (dw_g8 || dx_g8 ? gybytes : 0) + (dw_g8 ? xbytes + tbytes : 0);
@@ -619,15 +618,15 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
                                                (float*)((char*)p->d_scratch + need), pbytes, gw, side)) return rc;
             }
         } else if (int rc = launch_conv_dw_mfma(code, a, tl, listed ? &wl : nullptr, p->apr.level_min, side)) return rc;
-        if (near.n > 0 && b.tile_win) {
+        if (near.n > 0 && b.win_level) {
             if (int rc = pack_conv_weights_bf16(code, w, S_exp, Cin, Cout, p->d_scratch, st, true)) return rc;
             if (dx_g8) { b.xi = gyi; b.ti = nullptr; b.xi_ld = np; b.ti_ld = 0; }
             b.w = (const float*)p->d_scratch;
-            if (int rc = launch_conv_dx_mfma_bf16(code, b, near.n, st)) return rc;
+            if (int rc = launch_conv_dx_mfma_bf16(code, b, b.n_tiles, st)) return rc;
         } else if (near.n > 0) {
             if (int rc = pack_conv_weights(code, w, S_exp, Cin, Cout, true, (float*)p->d_scratch, st)) return rc;
             b.w = (const float*)p->d_scratch;
-            b.tile_win = nullptr;
+            b.win_level = nullptr;
             if (int rc = launch_conv_dx_mfma(code, b, near.n, st)) return rc;
         }
         if (int rc = guard.join()) return rc;

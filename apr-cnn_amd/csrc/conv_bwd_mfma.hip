@@ -649,7 +649,7 @@ template <typename T, class G>
 static int launch_dw(const ConvArgs<T>& a0, const TileList& tl, const WinLists* wl, int level_min, hipStream_t st) {
     const int code = G::KZ * 100 + G::KX * 10 + G::KY;
     const int64_t n_el = (int64_t)a0.Cout * a0.Cin * G::K;
-    if (a0.tile_win && wl) {
+    if (a0.win_level && wl) {
         if (wl->n_win <= 0) return 0;
         const DwWork k = dw_work(code, a0.Cout, a0.Cin, a0.S_exp, a0.Lc, *wl);
         if (int rc = launch_dw_kernel<T, G, true>(a0, k, 0, k.blk0[k.n_s], st)) return rc;

@@ -64,7 +64,7 @@ struct ConvArgs {
     // cells they would cover do not exist); a separate kernel adds their gradient (faces.hip)
     int dx_skip_faces;
     // window lists built once per APR and kept in the plan (kernels that do not scan)
-    const int* tile_win;                       // [n_tiles + 1] first stored window of every tile
+    const int* win_level;                      // level per stored window (null: no lists, the kernel scans)
     const int4* win;                           // per stored window: {first item, items, first column, columns}; the two
                                                // "first" fields are unsigned 32-bit offsets
     const int* l_item_idx; const unsigned short* l_item_pos;
@@ -175,8 +175,6 @@ struct ScanArgs {
     int tree_off, yn, y0;
     bool tree_from_x, out_tree;
     int z0, x0, zn, xn;             // tile origin and level extent (input-gradient scan only)
-    bool pool;                      // input-gradient scan: one pooled column per coarser particle (COL_BOX)
-    bool group;                     // input-gradient scan for lists: the columns of a coarser particle next to each other (see dx_group)
     bool skip_faces;                // input-gradient scan: no columns for coarser particles with cells outside the level
 };
 
@@ -276,10 +274,9 @@ constexpr unsigned COL_CELL = 0x0fffu;
 constexpr unsigned COL_SOLE = 0x2000u;    // input gradient: no other column, of this window or another, adds to this place
 constexpr unsigned COL_BOX = 0x4000u;
 constexpr unsigned COL_TREE = 0x8000u;
-// Columns of a coarser particle with all its cells inside the tile, in input-gradient lists: one per cell, next to each
+// Columns of a coarser particle with all its cells inside the tile, in input-gradient lists (lists.hip): one per cell, next to each
 // other from a multiple of their number on, all marked COL_BOX; the kernel adds them up across lanes and the first column
-// takes the sum to the particle.  They come first in a window's columns.  (A scan leaves them at the front of the column
-// arrays, nbox particles, and the other columns, ncol of them, at the back in reverse.)
+// takes the sum to the particle.  They come first in a window's columns.
 template <class G> __host__ __device__ constexpr int dx_group() { return G::TZ >= 2 ? 8 : 4; }
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v) {
@@ -350,7 +347,7 @@ __device__ __attribute__((noinline)) void scan_window_dx_impl(const ScanArgs a, 
                     if (outl) {
                         const int rank = __popcll(m & below_me);
                         const bool to_tree = src == 2 && !tree_from_x;
-                        const int at = a.group ? G::MAXCOL - 1 - (base + rank) : base + rank;
+                        const int at = base + rank;
                         sh.col_idx[at] = i + ((src == 2 && tree_from_x) ? (int)a.tree_off : 0);
                         // a place is a centre cell of one window of its own level; further columns come from windows one
                         // level finer, which see it as a coarser particle: none above the finest level, none for a tree node
@@ -366,43 +363,10 @@ __device__ __attribute__((noinline)) void scan_window_dx_impl(const ScanArgs a, 
                 const bool rows_full = (BOXZ == 1 || (z | 1) < a.zn) && (x | 1) < a.xn;
                 const bool first_row = (BOXZ == 1 || (z & 1) == 0) && (x & 1) == 0;
                 const bool ina = in && ya >= y0 && ya < y0 + G::TY;
-                const bool pooled = (a.pool || a.group) && rows_full && yb < yn;
+                const bool pooled = rows_full && yb < yn;
                 const bool keep = pooled || !a.skip_faces;
                 const bool oa = ina && keep && (!pooled || first_row);
                 const bool ob = in && keep && !pooled && yb >= y0 && yb < y0 + G::TY && yb < yn;
-                if (a.group) {
-                    const unsigned long long mg = __ballot(oa && pooled);
-                    if (mg) {
-                        constexpr int N = dx_group<G>();
-                        int base = 0;
-                        if (lane == 0) base = atomicAdd(&sh.nbox, __popcll(mg));
-                        base = __shfl(base, 0);
-                        if (oa && pooled) {
-                            const int at = (base + __popcll(mg & below_me)) * N;
-#pragma unroll
-                            for (int k = 0; k < N; ++k) {            // cells in the order z, x, y
-                                sh.col_idx[at + k] = i;
-                                sh.col_pos[at + k] = (unsigned short)(((r + (k >> 2) * G::RX + ((k >> 1) & 1)) * G::RS + (ya - lo) + (k & 1)) | COL_BOX);
-                            }
-                        }
-                    }
-                    const bool sa = oa && !pooled;
-                    const unsigned long long ma = __ballot(sa), mb = __ballot(ob);
-                    if (ma | mb) {
-                        int base = 0;
-                        if (lane == 0) base = atomicAdd(&sh.ncol, __popcll(ma) + __popcll(mb));
-                        base = __shfl(base, 0);
-                        if (sa) {
-                            const int at = G::MAXCOL - 1 - (base + __popcll(ma & below_me));
-                            sh.col_idx[at] = i; sh.col_pos[at] = (unsigned short)(r * G::RS + (ya - lo));
-                        }
-                        if (ob) {
-                            const int at = G::MAXCOL - 1 - (base + __popcll(ma) + __popcll(mb & below_me));
-                            sh.col_idx[at] = i; sh.col_pos[at] = (unsigned short)(r * G::RS + (yb - lo));
-                        }
-                    }
-                    continue;
-                }
                 const unsigned long long ma = __ballot(oa), mb = __ballot(ob);
                 if (ma | mb) {
                     int base = 0;
@@ -430,12 +394,12 @@ __device__ __attribute__((noinline)) void scan_window_dx_impl(const ScanArgs a, 
 
 template <class G, typename T>
 __device__ __forceinline__ void scan_window_dx(const ConvArgs<T>& a, int L, int z0, int x0, int y0, bool out_tree,
-                                               ConvShared<G>& sh, bool pool = true, bool group = false) {
+                                               ConvShared<G>& sh) {
     ScanArgs s;
     s.apr_y = a.apr.y; s.tree_y = a.tree.y; s.tree_off = (int)a.tree_off; s.yn = a.apr.y_num[L]; s.y0 = y0;
     s.tree_from_x = (L == a.Lc); s.out_tree = out_tree;
-    s.z0 = z0; s.x0 = x0; s.zn = a.apr.z_num[L]; s.xn = a.apr.x_num[L]; s.pool = pool; s.group = group;
-    s.skip_faces = (pool || group) && a.dx_skip_faces != 0;
+    s.z0 = z0; s.x0 = x0; s.zn = a.apr.z_num[L]; s.xn = a.apr.x_num[L];
+    s.skip_faces = a.dx_skip_faces != 0;
     scan_window_dx_impl<G>(s, sh);
 }
 

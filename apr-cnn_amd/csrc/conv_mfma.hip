@@ -270,8 +270,8 @@ __device__ __forceinline__ void mfma16_window(const ConvArgs<T>& a, int co0, int
 }
 
 // COH = 16-channel parts of the output block: 1 for layers of at most 16 output channels, 2 otherwise
-// LISTS: the windows of the tile come as precomputed lists from the plan (forward); otherwise the block scans
-// the access arrays itself (input gradient).
+// LISTS: one window of the precomputed lists of the plan (forward); otherwise the block scans the access arrays itself, all
+// windows of a row group (input gradient).
 // FUSE: built for the fused forward entry points (second input tensor, clamp at zero)
 template <typename T, class G, int COH, int MODE, bool LISTS, bool FUSE = false>
 __global__ void __launch_bounds__(G::NT)
@@ -285,7 +285,9 @@ conv_mfma16_kernel(const ConvArgs<T> a) {
     __shared__ float bias_l[16 * COH];
 
     if (MODE == 1 && a.redo && a.redo[0] == 0) return;          // only if the products of pieces gave a sum that is not finite
-    const ConvTile tile = a.tiles[blockIdx.x];
+    // a window of the lists, or a row group to scan
+    const int4 hd = LISTS ? a.win[blockIdx.x] : int4{};
+    const ConvTile tile = LISTS ? ConvTile{a.win_level[blockIdx.x], 0, 0, 0} : a.tiles[blockIdx.x];
     const int L = tile.level, z0 = tile.z0, x0 = tile.x0;
     const int co0 = blockIdx.y * 16 * COH;
     const int yn = a.apr.y_num[L];
@@ -317,21 +319,10 @@ conv_mfma16_kernel(const ConvArgs<T> a) {
 
     if constexpr (LISTS) {
         (void)z0; (void)x0; (void)yn; (void)out_tree;
-        __shared__ int4 hdr[16];              // headers of sixteen windows: one round trip instead of one per window
-        const int wb = a.tile_win[blockIdx.x], we = a.tile_win[blockIdx.x + 1];
-        for (int w = wb; w < we; ++w) {
-            const int win = w - wb;
-            if ((win & 15) == 0) {            // every wave is past the previous window's last barrier
-                if (threadIdx.x < 16 && w + (int)threadIdx.x < we) hdr[threadIdx.x] = a.win[w + threadIdx.x];
-                __syncthreads();
-            }
-            const int4 hd = hdr[win & 15];
-            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-            const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
-            const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
-            APRNET_WINDOW(gl)
-            __syncthreads();        // the next window rewrites the patch
-        }
+        const int win = 0, nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+        const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
+        const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
+        APRNET_WINDOW(gl)
     } else {
         __shared__ ConvShared<G> sh;
         open_segments<G, T>(a, L, z0, x0, sh);
@@ -366,27 +357,24 @@ conv_mfma16_redo_kernel(const ConvArgs<float> a, int n_tiles, int n_cb) {
     const int wave = threadIdx.x >> 6;
     for (int u = blockIdx.x; u < n_tiles * n_cb; u += gridDim.x) {              // uniform
         if (a.redo[split_mark(u)] == 0) continue;
-        const int tile = u % n_tiles, co0 = u / n_tiles * 16 * COH, L = a.tiles[tile].level;
+        const int w = u % n_tiles, co0 = u / n_tiles * 16 * COH, L = a.win_level[w];
         const float4* __restrict__ wl = reinterpret_cast<const float4*>(a.w_raw + (int64_t)min(a.S_exp - 1, a.Lc - L) * a.Cout * a.Cin * G::K);
         const bool tree_items = L < a.Lc;
         if (threadIdx.x < 16 * COH)                                            // (read behind the barriers of a window)
             bias_l[threadIdx.x] = (a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
-        const int wb = a.tile_win[tile], we = a.tile_win[tile + 1];
-        for (int w = wb; w < we; ++w) {
-            const int4 hd = a.win[w];
-            const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-            const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
-            const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
-            const int nblk = (nc + 15) >> 4, nb = wave < nblk ? (nblk - wave + G::NWAVE - 1) / G::NWAVE : 0;
-            switch (__builtin_amdgcn_readfirstlane(nb)) {
-                case 0: mfma16_window<float, G, CIB, COH, 0, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
-                case 1: mfma16_window<float, G, CIB, COH, 1, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
-                case 2: mfma16_window<float, G, CIB, COH, 2, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
-                case 3: mfma16_window<float, G, CIB, COH, 3, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
-                default: mfma16_window<float, G, CIB, COH, 4, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
-            }
-            __syncthreads();        // the next window rewrites the patch, the next tile the bias
+        const int4 hd = a.win[w];
+        const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+        const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
+        const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
+        const int nblk = (nc + 15) >> 4, nb = wave < nblk ? (nblk - wave + G::NWAVE - 1) / G::NWAVE : 0;
+        switch (__builtin_amdgcn_readfirstlane(nb)) {
+            case 0: mfma16_window<float, G, CIB, COH, 0, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+            case 1: mfma16_window<float, G, CIB, COH, 1, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+            case 2: mfma16_window<float, G, CIB, COH, 2, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+            case 3: mfma16_window<float, G, CIB, COH, 3, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
+            default: mfma16_window<float, G, CIB, COH, 4, 0, true, true>(a, co0, nc, nitem, tree_items, wave, wl, gl, patch, Wl, bias_l); break;
         }
+        __syncthreads();        // the next window rewrites the patch and the bias
     }
 }
 
@@ -778,7 +766,7 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
     }
 }
 
-// The windows of the tile come as precomputed lists from the plan.
+// A window of the precomputed lists of the plan per workgroup.
 // Two workgroups per CU (128 registers); the forward pass of layers of at most 16 outputs on regrouped input runs
 // three (80 registers, with spills): a third chain of windows per CU hides more of the memory round trips at the
 // start of every window than the spills cost (16->16 on the 23 M-particle APR 1.40 -> 1.28 ms; four workgroups at 64
@@ -793,8 +781,8 @@ conv_mfma_bf16_kernel(const ConvArgs<bf16_t> a) {
     __shared__ __attribute__((aligned(16))) uint4 Wl16[NSTEP * COH * 64];
     __shared__ float bias_l[16 * COH];
 
-    const ConvTile tile = a.tiles[blockIdx.x];
-    const int L = tile.level;
+    const int4 hd = a.win[blockIdx.x];
+    const int L = a.win_level[blockIdx.x];
     const int co0 = blockIdx.y * 16 * COH;
     const int s_idx = min(a.S_exp - 1, a.Lc - L);
     const int nq = (a.Cin + BF_CIB - 1) / BF_CIB;
@@ -807,7 +795,6 @@ conv_mfma_bf16_kernel(const ConvArgs<bf16_t> a) {
     if (threadIdx.x < 16 * COH)
         bias_l[threadIdx.x] = (MODE == 0 && a.bias && co0 + (int)threadIdx.x < a.Cout) ? a.bias[co0 + threadIdx.x] : 0.f;
 
-    __shared__ int4 hdr[16];                  // headers of sixteen windows: one round trip instead of one per window
     // tap offsets per step and lane group: a table in LDS costs one read per step and saves the registers of a
     // per-lane copy through the whole kernel (the 16-output form no longer spills inside its matrix phase)
     __shared__ int toff_l[NSTEP * 4];
@@ -833,28 +820,19 @@ conv_mfma_bf16_kernel(const ConvArgs<bf16_t> a) {
         }
         if (threadIdx.x < 4) head_b4[threadIdx.x] = (a.head_b && (int)threadIdx.x < a.head_C) ? a.head_b[threadIdx.x] : 0.f;
     }
-    const int wb = a.tile_win[blockIdx.x], we = a.tile_win[blockIdx.x + 1];
-    for (int w = wb; w < we; ++w) {
-        const int win = w - wb;
-        if ((win & 15) == 0) {                // every wave is past the previous window's last barrier
-            if (threadIdx.x < 16 && w + (int)threadIdx.x < we) hdr[threadIdx.x] = a.win[w + threadIdx.x];
-            __syncthreads();
-        }
-        const int4 hd = hdr[win & 15];
-        const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-        const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
-        const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
-        const int nblk = (nc + 15) >> 4;
-        const int first = (wave - (int)blockIdx.x - win) & (G::NWAVE - 1);
-        const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
-        switch (__builtin_amdgcn_readfirstlane(nb)) {
-            case 0: mfma_bf16_window<G, COH, 0, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-            case 1: mfma_bf16_window<G, COH, 1, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-            case 2: mfma_bf16_window<G, COH, 2, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-            case 3: mfma_bf16_window<G, COH, 3, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-            default: mfma_bf16_window<G, COH, 4, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-        }
-        __syncthreads();        // the next window rewrites the patch
+    __syncthreads();
+    const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+    const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
+    const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
+    const int nblk = (nc + 15) >> 4;
+    const int first = (wave - (int)blockIdx.x) & (G::NWAVE - 1);
+    const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
+    switch (__builtin_amdgcn_readfirstlane(nb)) {
+        case 0: mfma_bf16_window<G, COH, 0, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
+        case 1: mfma_bf16_window<G, COH, 1, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
+        case 2: mfma_bf16_window<G, COH, 2, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
+        case 3: mfma_bf16_window<G, COH, 3, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
+        default: mfma_bf16_window<G, COH, 4, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
     }
 }
 
@@ -870,16 +848,16 @@ bool conv_mfma_supported(int code) { return code == 333 || code == 133 || code =
 static int conv_taps(int code) { return code == 333 ? 27 : code == 133 ? 9 : 25; }
 static int conv_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
 
-// a.tile_win set: forward with the window lists of the plan; otherwise the kernel scans (always for the input gradient)
+// a.win_level set: forward with the window lists of the plan; otherwise the kernel scans (always for the input gradient)
 template <typename T, class G, int MODE>
 static int launch16(const ConvArgs<T>& a, int n_tiles, hipStream_t st) {
     const int coh = conv_coh(a.Cout);
     dim3 grid((unsigned)n_tiles, (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
     const bool fuse = MODE == 0 && (a.relu || a.x2);
-    if (MODE == 0 && a.tile_win && fuse) {
+    if (MODE == 0 && a.win_level && fuse) {
         if (coh == 1) hipLaunchKernelGGL((conv_mfma16_kernel<T, G, 1, 0, true, true>), grid, dim3(G::NT), 0, st, a);
         else hipLaunchKernelGGL((conv_mfma16_kernel<T, G, 2, 0, true, true>), grid, dim3(G::NT), 0, st, a);
-    } else if (MODE == 0 && a.tile_win) {
+    } else if (MODE == 0 && a.win_level) {
         if (coh == 1) hipLaunchKernelGGL((conv_mfma16_kernel<T, G, 1, 0, true>), grid, dim3(G::NT), 0, st, a);
         else hipLaunchKernelGGL((conv_mfma16_kernel<T, G, 2, 0, true>), grid, dim3(G::NT), 0, st, a);
     } else if (fuse) {
@@ -969,7 +947,7 @@ int launch_conv_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipS
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }
 // Input gradient with bfloat16 products: a.x / a.Cin describe the output gradient, a.Cout the layer's input channels,
-// a.w the transposed image of pack_conv_weights_bf16, a.tile_win ... the input-gradient lists of the plan.
+// a.w the transposed image of pack_conv_weights_bf16, a.win_level ... the input-gradient lists of the plan.
 int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st) {
     switch (code) {
         case 333: return launch_bf16<M333N>(a, n_tiles, st, true);

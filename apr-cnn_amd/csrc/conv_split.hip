@@ -169,7 +169,6 @@ struct SplitShared {
     uint4 w[split_steps<G>() * 3 * COH * 64];
     uint2 patch[3][G::CH_STRIDE];  // the three pieces of four channels, 8 bytes per cell
     float bias[16 * COH];
-    int4 hdr[16];                  // headers of sixteen windows: one round trip instead of one per window
     int2 toff[split_steps<G>() * 4];
 };
 template <class G, int COH>
@@ -194,7 +193,7 @@ __device__ __forceinline__ void store_items_split(const SplitItems<G>& R, int ni
 // MODE 0: forward, results stored (plus bias).  MODE 1: input gradient on the plan's input-gradient lists (items = output
 // gradient): the columns of a coarser particle are summed across lanes and the first one takes the sum along; a place that no
 // other column adds to takes a plain store, the others (one more column at most) an atomic addition.
-template <class G, int COH, int NB, int MODE, bool TIGHT>
+template <class G, int COH, int NB, int MODE>
 __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, int nc, int nitem, bool tree_items, int first,
                                              const uint4* __restrict__ wl, const WindowLists& gl, int* __restrict__ mark, SplitShared<G, COH>& sh) {
     constexpr int NSTEP = split_steps<G>(), NBA = NB > 0 ? NB : 1;
@@ -232,12 +231,9 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     }
     load_values_split<G>(a, 0, nitem, tree_items, R);
     // With 32 outputs a wave that holds two and more blocks of columns asks for the weights of a chunk in front of the barrier that ends the
-    // chunk before it, whose operands no longer need registers then; a wave with one block, as in sparse windows, has them to spare and asks
-    // together with the values.  32 -> 32 channels on 23 M particles 11.3 ms (always in front of the barrier 11.5, always with the values
-    // 11.8), 24 -> 32 on 4.9 M in sparse windows 1.98 (2.08, 2.11), 64 -> 64 on 8 M 18.9 (19.1, 20.0).  With 16 outputs and two workgroups
-    // per CU they travel with the values (16 -> 16 on 43 M 9.35 ms, in front of the barrier 9.65); with three (TIGHT) as with 32 outputs (9.1, always with
-    // the values 10.4).
-    constexpr bool LATE = (COH == 2 || TIGHT) && NB >= 2;
+    // chunk before it, whose operands no longer need registers then; a wave with one block has them to spare and asks together with the
+    // values (64 -> 64 channels on 8 M particles 18.9, always in front of the barrier 19.1, always with the values 20.0), as do the 16 outputs.
+    constexpr bool LATE = COH == 2 && NB >= 2;
     if constexpr (!LATE) load_weights(0);
     for (int i = threadIdx.x; i < 3 * G::CH_STRIDE / 2; i += G::NT) reinterpret_cast<uint4*>(sh.patch)[i] = make_uint4(0u, 0u, 0u, 0u);
     for (int ci0 = 0; ci0 < a.Cin; ci0 += SP_CIB) {
@@ -349,17 +345,17 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     }
 }
 
-// Two workgroups per CU.  TIGHT: three (80 registers, some of them spilled), which hide more of the round trips of sparse windows with 16
-// outputs (see SPLIT_SPARSE).
-template <class G, int COH, int MODE, bool TIGHT>
-__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(TIGHT ? 6 : 4, TIGHT ? 6 : 4)))
+// One window per workgroup, two workgroups per CU.  (Three with 80 registers, some of them spilled, took 3 to 10 % longer with 16 outputs on every
+// APR; eight windows one after the other, 32 -> 32 channels on 23 M particles 10.05 instead of 9.84 ms.)
+template <class G, int COH, int MODE>
+__global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 conv_split_kernel(const ConvArgs<float> a) {
     constexpr int NBW = 4, NSTEP = split_steps<G>();
     static_assert((G::MAXCOL + 15) / 16 <= G::NWAVE * NBW, "a window must fit the accumulators of the block");
     static_assert(G::RS == 64, "the plan's lists carry cells of rows of 64");
     __shared__ SplitShared<G, COH> sh;
-    const ConvTile tile = a.tiles[blockIdx.x];
-    const int L = tile.level;
+    const int4 hd = a.win[blockIdx.x];
+    const int L = a.win_level[blockIdx.x];
     const int co0 = blockIdx.y * 16 * COH;
     const int s_idx = min(a.S_exp - 1, a.Lc - L);
     const int nq = (a.Cin + SP_CIB - 1) / SP_CIB;
@@ -380,78 +376,56 @@ conv_split_kernel(const ConvArgs<float> a) {
         }
         sh.toff[threadIdx.x] = make_int2(o[0], o[1]);
     }
-    const int wb = a.tile_win[blockIdx.x], we = a.tile_win[blockIdx.x + 1];
-    for (int w = wb; w < we; ++w) {
-        const int win = w - wb;
-        if ((win & 15) == 0) {                // every wave is past the previous window's last barrier
-            if (threadIdx.x < 16 && w + (int)threadIdx.x < we) sh.hdr[threadIdx.x] = a.win[w + threadIdx.x];
-            __syncthreads();
-        }
-        const int4 hd = sh.hdr[win & 15];
-        const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
-        const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
-        const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
-        const int nblk = (nc + 15) >> 4;
-        const int first = (wave - (int)blockIdx.x - win) & (G::NWAVE - 1);
-        const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
-        switch (__builtin_amdgcn_readfirstlane(nb)) {
-            case 0: split_window<G, COH, 0, MODE, TIGHT>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            case 1: split_window<G, COH, 1, MODE, TIGHT>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            case 2: split_window<G, COH, 2, MODE, TIGHT>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            case 3: split_window<G, COH, 3, MODE, TIGHT>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-            default: split_window<G, COH, 4, MODE, TIGHT>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
-        }
-        __syncthreads();        // the next window rewrites the patch
+    __syncthreads();
+    const int nitem = __builtin_amdgcn_readfirstlane(hd.y), nc = __builtin_amdgcn_readfirstlane(hd.w);
+    const unsigned i0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.x), c0 = (unsigned)__builtin_amdgcn_readfirstlane(hd.z);
+    const WindowLists gl{a.l_item_idx + i0, a.l_item_pos + i0, a.l_col_idx + c0, a.l_col_pos + c0};
+    const int nblk = (nc + 15) >> 4;
+    const int first = (wave - (int)blockIdx.x) & (G::NWAVE - 1);
+    const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
+    switch (__builtin_amdgcn_readfirstlane(nb)) {
+        case 0: split_window<G, COH, 0, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+        case 1: split_window<G, COH, 1, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+        case 2: split_window<G, COH, 2, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+        case 3: split_window<G, COH, 3, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
+        default: split_window<G, COH, 4, MODE>(a, co0, nc, nitem, tree_items, first, wl, gl, a.redo, sh); break;
     }
 }
 
 using S333 = ConvGeom<3, 3, 3, 2, 4, 512, 64, 16>;
 using S155 = ConvGeom<1, 5, 5, 1, 8, 512, 64, 16>;
 
-// Fewer columns than this per window on average: three workgroups per CU for 16 outputs, which pay for their spills with round trips that they
-// hide; same sums.  3x3x3, three workgroups against two: 110 to 118 columns, 16 -> 16 channels on 43 M particles 9.1 and 9.37 ms, 32 -> 16 on 4.9 M
-// 1.77 and 1.86; 160 to 172, 16 -> 16 on 14 M 2.58 and 2.58, 32 -> 16 4.69 and 4.78; 245 to 288, 16 -> 16 on 13 M 2.08 and 1.97, 32 -> 16 on 1.7 M
-// 0.533 and 0.511.  1x5x5 always runs two (16 -> 16 on 2 M 0.63 ms, three 0.80).
-constexpr int SPLIT_SPARSE = 192;
 static int split_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
 static int split_nstep(int code) { return code == 333 ? split_steps<S333>() : split_steps<S155>(); }
 
 int launch_conv_redo(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);        // conv_mfma.hip
 
 template <class G, int MODE>
-static int launch_split(const ConvArgs<float>& a, int n_tiles, bool sparse, hipStream_t st) {
+static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     const int coh = split_coh(a.Cout), n_cb = (a.Cout + 16 * coh - 1) / (16 * coh);
     dim3 grid((unsigned)n_tiles, (unsigned)n_cb);
-    if constexpr (MODE == 0 && G::KZ > 1) {
-        if (coh == 1 && sparse) {
-            hipLaunchKernelGGL((conv_split_kernel<G, 1, 0, true>), grid, dim3(G::NT), 0, st, a);
-            APRNET_LAUNCH_CHECK("conv_split_kernel");
-            return 0;
-        }
-    }
-    if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1, MODE, false>), grid, dim3(G::NT), 0, st, a);
-    else hipLaunchKernelGGL((conv_split_kernel<G, 2, MODE, false>), grid, dim3(G::NT), 0, st, a);
+    if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1, MODE>), grid, dim3(G::NT), 0, st, a);
+    else hipLaunchKernelGGL((conv_split_kernel<G, 2, MODE>), grid, dim3(G::NT), 0, st, a);
     APRNET_LAUNCH_CHECK("conv_split_kernel");
     return 0;
 }
-// a.w, a.redo, a.xi, a.ti: what prepare_split made of the weights a.w_raw and of a.x, a.x2 and a.tree_data; a.tile_win ... the forward
+// a.w, a.redo, a.xi, a.ti: what prepare_split made of the weights a.w_raw and of a.x, a.x2 and a.tree_data; a.win_level ... the forward
 // lists of the plan
-int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, const WinLists& wl, hipStream_t st) {
-    const bool sparse = wl.n_cols < (int64_t)SPLIT_SPARSE * wl.n_win;
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     int rc;
     switch (code) {
-        case 333: rc = launch_split<S333, 0>(a, n_tiles, sparse, st); break;
-        case 155: rc = launch_split<S155, 0>(a, n_tiles, sparse, st); break;
+        case 333: rc = launch_split<S333, 0>(a, n_tiles, st); break;
+        case 155: rc = launch_split<S155, 0>(a, n_tiles, st); break;
         default: rc = fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
     }
     return rc ? rc : launch_conv_redo(code, a, n_tiles, st);
 }
 // Input gradient: a.x / a.xi / a.Cin describe the output gradient, a.Cout the layer's input channels, a.w the transposed image,
-// a.tile_win ... the input-gradient lists of the plan without the particles on far faces.  a.redo[0] is set if a sum is not finite.
+// a.win_level ... the input-gradient lists of the plan without the particles on far faces.  a.redo[0] is set if a sum is not finite.
 int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     switch (code) {
-        case 333: return launch_split<S333, 1>(a, n_tiles, false, st);
-        case 155: return launch_split<S155, 1>(a, n_tiles, false, st);
+        case 333: return launch_split<S333, 1>(a, n_tiles, st);
+        case 155: return launch_split<S155, 1>(a, n_tiles, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }

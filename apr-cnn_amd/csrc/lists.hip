@@ -3,132 +3,279 @@
 // patch, so the lists depend on the APR alone; every convolution call at that level delta reuses them and its
 // kernel neither searches the access arrays nor keeps list bookkeeping in LDS.
 //
-// Two passes over the tiles with the scanning code of conv_common.hpp: the first counts windows, items and
-// columns per tile, the host turns the counts into offsets, the second writes the lists in tile order.
+// Windows are cut from a compressed y axis.  A row group (2 x 4 rows, 1 x 8 for flat stencils) of a sparse APR has outputs at a part
+// of its y positions only, in thin shells around what is finely resolved: kept are the positions within the stencil's reach of an
+// output, one after the other, and the kept positions of all row groups of a level behind each other, with as many empty cells between
+// two groups as the stencil reaches.  Neighbours along y of an output are kept with it, so they are neighbours on the compressed
+// axis too, and what lies next to the end of a run there is a position that no output occupies.  A window is 62 (60) cells of that axis
+// and its halo, whatever row groups they come from; the kernels see cells only.
+// The kernels are bound by what a window costs whether it is full or not (lists, round trips, weights, barriers).  Windows of
+// 62 positions of one row group, as they were, held 173 outputs of 496 on average on the 23 M particles of a blob volume (134,000
+// windows, now 60,200 of 385), 118 on a sparse light-sheet one of 43 M (366,000, now 121,000 of 355), 311 on a dense one of 52 M (167,000, now
+// 121,000 of 428).  3x3x3 of fp32 features 32 -> 32 on the first 11.6 -> 9.7 ms, 16 -> 16 on the second 9.1 -> 7.0, a bfloat16 U-Net on the third
+// 58.4 -> 53.7.
+//
+// Three passes over the row groups: kept positions, then items and columns per window, then the lists; the host turns the counts into
+// offsets in between.
 #include "conv_common.hpp"
 
-#include <numeric>
+#include <cstring>
 
 namespace aprnet {
 
-// DX: lists of the input gradient (scan_window_dx, the columns of a coarser particle in groups) over the tiles within one row of an
-// output; windows without an output position are not stored.
-//
-// Forward lists keep the items that some output position of the window can reach through the stencil.  The scan
-// yields every particle and tree node of the staged rows, but a window of a coarser level often holds a handful of
-// output positions next to long runs of tree nodes standing for finely resolved regions: no output reads those, so
-// they are neither staged by the kernels nor needed in the mean-filled tree (need.hip).
-template <class G, bool DX>
-__global__ void __launch_bounds__(G::NT)
-build_lists_kernel(const ConvArgs<float> a, const int pass, int4* __restrict__ tile_counts, const int4* __restrict__ tile_off,
-                   int4* __restrict__ win, int* __restrict__ item_idx, unsigned short* __restrict__ item_pos,
-                   int* __restrict__ col_idx, unsigned short* __restrict__ col_pos) {
-    __shared__ ConvShared<G> sh;
-    __shared__ unsigned char reach[DX ? 4 : G::NROW * G::RS];   // cell -> an output position of its row lies within the y taps
-    __shared__ int kept;
-    static_assert((G::NROW * G::RS) % 4 == 0, "the reach map is cleared with 4-byte stores");
-    const ConvTile tile = a.tiles[blockIdx.x];
-    const int L = tile.level;
-    const int yn = a.apr.y_num[L];
-    const bool out_tree = (L == a.Lc) && (L < a.apr.level_max);
-    int nwin = 0, ni = 0, ncl = 0;
-    int4 off = make_int4(0, 0, 0, 0);
-    if (pass == 1) off = tile_off[blockIdx.x];
+struct ListArgs {
+    AccessDev apr, tree;
+    const ConvTile* tiles; int n_tiles;
+    int Lc; int64_t tree_off;
+    int skip_faces;                // input gradient: no columns for coarser particles that stick out of a far face
+    int words;                     // 64-bit words of a row's bit map, for the longest rows
+    int per_row;                   // a bit map per staged row fits LDS: items and columns are kept if an output lies in reach on three axes, not only along y
+    int* n_cells;                  // [n_tiles] pass 0: kept positions of a row group
+    const int* first_cell;         // [n_tiles] its first cell on the compressed axis of its level
+    int win0[MAX_LEVELS + 1], nwin[MAX_LEVELS + 1];          // windows of a level
+    int4* count;                   // [windows] pass 1: items, groups of columns (see dx_group), other columns
+    const int* slot0;              // [n_tiles] first entry in `share` of a row group, which has one per window it stages a cell of,
+    int4* share;                   // pass 1: the entries of other row groups before its own
+    const int4* off;               // [windows] pass 2: first item, first column, groups of columns, 1 if the window is stored
+    int* item_idx; unsigned short* item_pos; int* col_idx; unsigned short* col_pos;
+};
 
-    open_segments<G, float>(a, L, tile.z0, tile.x0, sh);
-    __syncthreads();
-    for (int y0 = 0; y0 < yn; y0 += G::TY) {
-        if constexpr (DX) scan_window_dx<G, float>(a, L, tile.z0, tile.x0, y0, out_tree, sh, false, true);
-        else scan_window<G, float>(a, L, y0, out_tree, sh);
-        __syncthreads();
-        const int nsum = DX ? dx_group<G>() * sh.nbox : 0;                   // columns of coarser particles, summed in groups: first
-        const int nc = nsum + sh.ncol, nitem = sh.nitem;
-        if (nc > 0 && (!DX || nitem > 0)) {
-            // list offsets are unsigned 32-bit numbers stored in the int fields of the header
-            const unsigned ib = (unsigned)off.y + (unsigned)ni, cb = (unsigned)off.z + (unsigned)ncl;
-            int nkeep = nitem;
-            if constexpr (DX) {
-                if (pass == 1)
-                    for (int i = threadIdx.x; i < nitem; i += G::NT) { item_idx[(size_t)ib + i] = sh.item_idx[i]; item_pos[(size_t)ib + i] = sh.item_pos[i]; }
-            } else {
-                for (int i = threadIdx.x; i < G::NROW * G::RS / 4; i += G::NT) reinterpret_cast<int*>(reach)[i] = 0;
-                if (threadIdx.x == 0) kept = 0;
-                __syncthreads();
-                for (int i = threadIdx.x; i < nc; i += G::NT) {
-                    const int cell = sh.col_pos[i] & COL_CELL, y = cell % G::RS, row = cell - y;
-                    for (int yy = max(y - G::HY, 0); yy <= min(y + G::HY, G::RS - 1); ++yy) reach[row + yy] = 1;
-                }
-                __syncthreads();
-                for (int i0 = 0; i0 < nitem; i0 += G::NT) {
-                    const int i = i0 + (int)threadIdx.x;
-                    bool keep = false;
-                    unsigned pos = 0;
-                    if (i < nitem) {
-                        pos = sh.item_pos[i];
-                        const int cell = pos & 0x0fffu, y = cell % G::RS, r = cell / G::RS, rz = r / G::RX, rx = r - rz * G::RX;
-                        const bool pair = (pos & ITEM_PAIR) != 0 && y + 1 < G::RS;
-                        for (int dz = -G::HZ; dz <= G::HZ; ++dz)
-                            for (int dx = -G::HX; dx <= G::HX; ++dx) {
-                                const int z2 = rz + dz, x2 = rx + dx;
-                                if (z2 < 0 || z2 >= G::RZ || x2 < 0 || x2 >= G::RX) continue;
-                                const int c2 = (z2 * G::RX + x2) * G::RS + y;
-                                keep = keep || reach[c2] != 0 || (pair && reach[c2 + 1] != 0);
-                            }
-                    }
-                    const unsigned long long m = __ballot(keep);
-                    int base = 0;
-                    if (lane_id() == 0 && m) base = atomicAdd(&kept, __popcll(m));
-                    base = __shfl(base, 0);
-                    if (keep && pass == 1) {
-                        const size_t dst = (size_t)ib + base + __popcll(m & ((1ull << lane_id()) - 1ull));
-                        item_idx[dst] = sh.item_idx[i]; item_pos[dst] = (unsigned short)pos;
-                    }
-                }
-                __syncthreads();
-                nkeep = kept;
-            }
-            if (pass == 1) {
-                if (threadIdx.x == 0) win[off.x + nwin] = make_int4((int)ib, nkeep, (int)cb, nc);
-                for (int i = threadIdx.x; i < nc; i += G::NT) {
-                    const int at = DX && i >= nsum ? G::MAXCOL - 1 - (i - nsum) : i;
-                    col_idx[(size_t)cb + i] = sh.col_idx[at]; col_pos[(size_t)cb + i] = sh.col_pos[at];
-                }
-            }
-            ++nwin; ni += nkeep; ncl += nc;
+// windows that a row group can stage a cell of: its cells and the halo, cut anywhere
+__host__ __device__ constexpr int list_windows(int words) { return words * 64 / 60 + 3; }
+__host__ __device__ constexpr int list_used_words(int words) { return (list_windows(words) * 3 + 1) / 2; }
+// word u of a bit map (p the one before, n the one after it), dilated by hy to either side
+__device__ __forceinline__ unsigned long long dilated(unsigned long long u, unsigned long long p, unsigned long long n, int hy) {
+    unsigned long long k = u;
+    for (int h = 1; h <= hy; ++h) k |= (u << h) | (u >> h) | (p >> (64 - h)) | (n << (64 - h));
+    return k;
+}
+
+// DX: lists of the input gradient: items are the output positions of the staged rows, columns every cell of the centre rows that some
+// source covers and an output reaches (the others' gradient is zero), those of a coarser particle in groups (dx_group).
+// PASS 0 counts kept positions, 1 items and columns, 2 writes them.
+template <class G, bool DX, int PASS>
+__global__ void __launch_bounds__(G::NT)
+build_lists_kernel(const ListArgs a) {
+    extern __shared__ unsigned long long maps[];
+    __shared__ int seg_b[G::NSEG], seg_e[G::NSEG];
+    __shared__ int total;
+    const ConvTile tile = a.tiles[blockIdx.x];
+    const int L = tile.level, yn = a.apr.y_num[L], zn = a.apr.z_num[L], xn = a.apr.x_num[L];
+    const bool out_tree = L == a.Lc && L < a.apr.level_max, tree_from_x = L == a.Lc;
+    const int W = (yn + 63) >> 6, lane = lane_id(), wave = threadIdx.x >> 6;
+    unsigned long long* keep = maps;                                     // [W] kept positions
+    unsigned long long* any = maps + a.words;                            // [W] positions with an output in some row
+    int* before = reinterpret_cast<int*>(maps + 2 * a.words);            // [W] kept positions in the words before
+    int* used = reinterpret_cast<int*>(maps + 3 * a.words);              // [windows of the group][3] entries so far (pass 2: and those of other groups before them)
+    unsigned long long* rows = maps + 3 * a.words + list_used_words(a.words);    // [NROW][W] outputs of a row (per_row)
+    unsigned long long* reach = rows + G::NROW * a.words;                // [NROW][W] positions of a row with an output in reach (per_row)
+
+    // ---- the rows of the group: particles of the level, of the coarser one, tree nodes
+    for (int s = threadIdx.x; s < G::NSEG; s += G::NT) {
+        const int r = s / 3, src = s - 3 * r, rz = r / G::RX, rx = r - rz * G::RX;
+        const int z = tile.z0 - G::HZ + rz, x = tile.x0 - G::HX + rx;
+        int b = 0, e = 0;
+        if (z >= 0 && z < zn && x >= 0 && x < xn && (src == 0 || (src == 1 ? L > a.apr.level_min : L < a.apr.level_max))) {
+            const AccessDev& acc = src == 2 ? a.tree : a.apr;
+            const uint64_t row = src == 1 ? acc.row(L - 1, z >> 1, x >> 1) : acc.row(L, z, x);
+            b = (int)acc.xz_end[row - 1]; e = (int)acc.xz_end[row];
         }
-        __syncthreads();
-        close_window<G>(sh);
-        __syncthreads();
+        seg_b[s] = b; seg_e[s] = e;
     }
-    if (pass == 0 && threadIdx.x == 0) tile_counts[blockIdx.x] = make_int4(nwin, ni, ncl, 0);
+    for (int i = threadIdx.x; i < W; i += G::NT) any[i] = 0;
+    if (a.per_row) for (int i = threadIdx.x; i < G::NROW * W; i += G::NT) rows[i] = 0;
+    __syncthreads();
+
+    // ---- outputs (of the centre rows, DX: of all staged ones), and the positions within the stencil's reach of one along y
+    auto centre = [](int r) { const int rz = r / G::RX, rx = r - rz * G::RX; return rz >= G::HZ && rz < G::HZ + G::TZ && rx >= G::HX && rx < G::HX + G::TX; };
+    for (int s = wave; s < G::NSEG; s += G::NWAVE) {
+        const int r = s / 3, src = s - 3 * r;
+        if (!(src == 0 || (src == 2 && out_tree)) || !(DX || centre(r))) continue;
+        const uint16_t* yv = src == 2 ? a.tree.y : a.apr.y;
+        for (int i = seg_b[s] + lane; i < seg_e[s]; i += 64) {
+            const int y = yv[i];
+            atomicOr(&any[y >> 6], 1ull << (y & 63));
+            if (a.per_row) atomicOr(&rows[r * W + (y >> 6)], 1ull << (y & 63));
+        }
+    }
+    __syncthreads();
+    for (int w = threadIdx.x; w < W; w += G::NT) {
+        unsigned long long k = dilated(any[w], w > 0 ? any[w - 1] : 0, w + 1 < W ? any[w + 1] : 0, G::HY);
+        // whole pairs 2y, 2y + 1, which a coarser particle covers; the added position has no output in reach and, like the last one of the run that
+        // it lies next to on the compressed axis, none on it
+        if (DX) k |= ((k & 0x5555555555555555ull) << 1) | ((k >> 1) & 0x5555555555555555ull);
+        if (w == W - 1 && (yn & 63)) k &= ~0ull >> (64 - (yn & 63));
+        keep[w] = k;
+    }
+    if (PASS > 0 && a.per_row)
+        for (int i = threadIdx.x; i < G::NROW * W; i += G::NT) {
+            const int r = i / W, w = i - r * W, rz = r / G::RX, rx = r - rz * G::RX;
+            unsigned long long u = 0, p = 0, n = 0;
+            for (int z2 = max(rz - G::HZ, 0); z2 <= min(rz + G::HZ, G::RZ - 1); ++z2)
+                for (int x2 = max(rx - G::HX, 0); x2 <= min(rx + G::HX, G::RX - 1); ++x2) {
+                    const unsigned long long* m = rows + (z2 * G::RX + x2) * W + w;
+                    u |= m[0];
+                    if (w > 0) p |= m[-1];
+                    if (w + 1 < W) n |= m[1];
+                }
+            reach[i] = dilated(u, p, n, G::HY);
+        }
+    __syncthreads();
+    if (wave == 0) {
+        int sum = 0;
+        for (int w0 = 0; w0 < W; w0 += 64) {
+            const int n = w0 + lane < W ? __popcll(keep[w0 + lane]) : 0;
+            int inc = n;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) { const int t = __shfl_up(inc, d); if (lane >= d) inc += t; }
+            if (w0 + lane < W) before[w0 + lane] = sum + inc - n;
+            sum += __shfl(inc, 63);
+        }
+        if (lane == 0) total = sum;
+    }
+    __syncthreads();
+    if constexpr (PASS == 0) {
+        if (threadIdx.x == 0) a.n_cells[blockIdx.x] = total;
+        return;
+    }
+    const int first = a.first_cell[blockIdx.x], win0 = a.win0[L], nwin = a.nwin[L];
+    auto kept = [&](int y) { return y >= 0 && y < yn && ((keep[y >> 6] >> (y & 63)) & 1ull) != 0; };
+    auto cell_of = [&](int y) { return first + before[y >> 6] + __popcll(keep[y >> 6] & ((1ull << (y & 63)) - 1ull)); };
+    // an output within the stencil's reach of position y of row r (whose position is kept)
+    auto reached = [&](int r, int y) { return !a.per_row || ((reach[r * W + (y >> 6)] >> (y & 63)) & 1ull) != 0; };
+    const int wf = max((first + G::HY - G::WY + G::TY) / G::TY, 0);        // first window that stages a cell of the group
+    const int nw = total > 0 ? min((first + total - 1 + G::HY) / G::TY, nwin - 1) - wf + 1 : 0;
+    int4* share = a.share + a.slot0[blockIdx.x];
+    for (int i = threadIdx.x; i < nw; i += G::NT) {
+        const int4 o = PASS == 2 ? share[i] : make_int4(0, 0, 0, 0);
+        used[3 * i] = o.x; used[3 * i + 1] = o.y; used[3 * i + 2] = o.z;
+    }
+    __syncthreads();
+    // One entry per lane with `has` to window w (of the level): place(number of the entry among those of `field` in that window)
+    auto append = [&](bool has, int w, int field, auto place) {
+        for (unsigned long long m = __ballot(has); m; m = __ballot(has)) {
+            const int lead = __ffsll(m) - 1, wl = __shfl(w, lead);
+            const unsigned long long mm = __ballot(has && w == wl);
+            int base = 0;
+            if (lane == lead) base = atomicAdd(&used[3 * (wl - wf) + field], __popcll(mm));
+            if constexpr (PASS == 2) base = __shfl(base, lead);
+            if (has && w == wl) {
+                if constexpr (PASS == 2) place(win0 + wl, base + __popcll(mm & ((1ull << lane) - 1ull)));
+                has = false;
+            }
+        }
+    };
+    // an item on cell c, and on c + 1 if it is a pair, for every window that stages one of the two
+    auto item = [&](bool has, int r, int c, bool pair, int idx, unsigned flags) {
+        const int lo = max((c + G::HY - G::WY + G::TY) / G::TY, 0), hi = min((c + (pair ? 1 : 0) + G::HY) / G::TY, nwin - 1);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            const int w = lo + k, p = c - (w * G::TY - G::HY);
+            const bool in = p >= 0 && p < G::WY, in2 = pair && p + 1 >= 0 && p + 1 < G::WY;
+            append(has && w <= hi && (in || in2), w, 0, [&](int win, int n) {
+                const int4 o = a.off[win];
+                if (!o.w) return;
+                a.item_idx[(size_t)(unsigned)o.x + n] = idx;
+                a.item_pos[(size_t)(unsigned)o.x + n] = (unsigned short)((r * G::RS + (in ? p : p + 1)) | flags | (in && in2 ? ITEM_PAIR : 0u));
+            });
+        }
+    };
+    auto column = [&](bool has, int r, int c, int idx, unsigned flags) {
+        const int w = c / G::TY;
+        append(has, w, 2, [&](int win, int n) {
+            const int4 o = a.off[win];
+            if (!o.w) return;
+            const size_t at = (size_t)(unsigned)o.y + (DX ? dx_group<G>() * o.z : 0) + n;
+            a.col_idx[at] = idx;
+            a.col_pos[at] = (unsigned short)((r * G::RS + c - w * G::TY + G::HY) | flags);
+        });
+    };
+    for (int s = wave; s < G::NSEG; s += G::NWAVE) {
+        const int r = s / 3, src = s - 3 * r, rz = r / G::RX, rx = r - rz * G::RX;
+        const int z = tile.z0 - G::HZ + rz, x = tile.x0 - G::HX + rx;
+        const bool mid = centre(r), is_out = src == 0 || (src == 2 && out_tree);
+        const uint16_t* yv = src == 2 ? a.tree.y : a.apr.y;
+        const int plus = src == 2 && tree_from_x ? (int)a.tree_off : 0;
+        for (int i0 = seg_b[s]; i0 < seg_e[s]; i0 += 64) {                // wave-uniform
+            const int i = i0 + lane;
+            const bool valid = i < seg_e[s];
+            const int y = valid ? (int)yv[i] : 0, ya = src == 1 ? 2 * y : y, yb = ya + 1;
+            const bool ka = valid && kept(ya), kb = src == 1 && valid && kept(yb);
+            const int ca = ka ? cell_of(ya) : 0, cb = kb ? cell_of(yb) : 0;
+            if constexpr (!DX) {
+                const bool need = (ka && reached(r, ya)) || (kb && reached(r, yb));
+                item(need, r, ka ? ca : cb, ka && kb, i + plus, src == 2 && !tree_from_x ? ITEM_TREE : 0u);
+                if (mid && is_out) column(valid, r, ca, i + plus, 0u);
+            } else {
+                if (is_out) item(valid, r, ca, false, i + plus, 0u);
+                if (!mid) continue;
+                if (src != 1) {
+                    // a place is a centre cell of one window of its own level; further columns come from windows one level finer, which see
+                    // it as a coarser particle: none above the finest level, none for a tree node
+                    const bool to_tree = src == 2 && !tree_from_x;
+                    column(ka && reached(r, ya), r, ca, i + plus, (to_tree ? COL_TREE : 0u) | (to_tree || tree_from_x ? COL_SOLE : 0u));
+                    continue;
+                }
+                constexpr int N = dx_group<G>(), BOXZ = G::TZ >= 2 ? 2 : 1;         // a flat tile sees one z-slice of the coarser particle
+                const bool rows_full = (BOXZ == 1 || (z | 1) < zn) && (x | 1) < xn;  // wave-uniform
+                const bool first_row = (BOXZ == 1 || (z & 1) == 0) && (x & 1) == 0;
+                const bool pooled = rows_full && yb < yn;
+                if (rows_full && first_row) {
+                    bool hit = false;
+                    if (pooled && ka)
+#pragma unroll
+                        for (int k = 0; k < N; ++k) hit = hit || reached(r + (k >> 2) * G::RX + ((k >> 1) & 1), ya + (k & 1));
+                    const int w = ca / G::TY;
+                    append(hit, w, 1, [&](int win, int n) {
+                        const int4 o = a.off[win];
+                        if (!o.w) return;
+#pragma unroll
+                        for (int k = 0; k < N; ++k) {                     // cells in the order z, x, y
+                            const size_t at = (size_t)(unsigned)o.y + N * n + k;
+                            a.col_idx[at] = i;
+                            a.col_pos[at] = (unsigned short)(((r + (k >> 2) * G::RX + ((k >> 1) & 1)) * G::RS + ca - w * G::TY + G::HY + (k & 1)) | COL_BOX);
+                        }
+                    });
+                }
+                if (!a.skip_faces) {
+                    column(ka && !pooled && reached(r, ya), r, ca, i, 0u);
+                    column(kb && !pooled && reached(r, yb), r, cb, i, 0u);
+                }
+            }
+        }
+    }
+    if constexpr (PASS == 1) {
+        __syncthreads();
+        for (int i = threadIdx.x; i < nw; i += G::NT) {
+            int* c = reinterpret_cast<int*>(a.count + win0 + wf + i);
+            int o[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) o[k] = used[3 * i + k] ? atomicAdd(c + k, used[3 * i + k]) : 0;
+            share[i] = make_int4(o[0], o[1], o[2], 0);
+        }
+    }
 }
 
 using L333 = ConvGeom<3, 3, 3, 2, 4, 512>;
 using L133 = ConvGeom<1, 3, 3, 1, 8, 512>;
 using L155 = ConvGeom<1, 5, 5, 1, 8, 512>;
 
-template <class G>
-static void launch_build(const ConvArgs<float>& a, int n_tiles, int pass, int4* counts, const int4* offs, const WinLists& wl,
-                         bool dx, hipStream_t st) {
-    if (dx)
-        hipLaunchKernelGGL((build_lists_kernel<G, true>), dim3((unsigned)n_tiles), dim3(G::NT), 0, st, a, pass, counts, offs,
-                           wl.d_win, wl.d_item_idx, wl.d_item_pos, wl.d_col_idx, wl.d_col_pos);
-    else
-        hipLaunchKernelGGL((build_lists_kernel<G, false>), dim3((unsigned)n_tiles), dim3(G::NT), 0, st, a, pass, counts, offs,
-                           wl.d_win, wl.d_item_idx, wl.d_item_pos, wl.d_col_idx, wl.d_col_pos);
+static size_t list_lds(int words, int rows) { return 8 * ((size_t)words * (3 + 2 * rows) + list_used_words(words)); }
+template <class G, bool DX>
+static void launch_build(const ListArgs& a, int pass, hipStream_t st) {
+    const size_t lds = list_lds(a.words, a.per_row ? G::NROW : 0);
+    if (pass == 0) hipLaunchKernelGGL((build_lists_kernel<G, DX, 0>), dim3((unsigned)a.n_tiles), dim3(G::NT), lds, st, a);
+    else if (pass == 1) hipLaunchKernelGGL((build_lists_kernel<G, DX, 1>), dim3((unsigned)a.n_tiles), dim3(G::NT), lds, st, a);
+    else hipLaunchKernelGGL((build_lists_kernel<G, DX, 2>), dim3((unsigned)a.n_tiles), dim3(G::NT), lds, st, a);
 }
-
-static void launch_build_code(int code, const ConvArgs<float>& a, int n_tiles, int pass, int4* counts, const int4* offs,
-                              const WinLists& wl, bool dx, hipStream_t st) {
-    if (code == 333) launch_build<L333>(a, n_tiles, pass, counts, offs, wl, dx, st);
-    else if (code == 133) launch_build<L133>(a, n_tiles, pass, counts, offs, wl, dx, st);
-    else launch_build<L155>(a, n_tiles, pass, counts, offs, wl, dx, st);
+static void launch_build_code(int code, const ListArgs& a, bool dx, int pass, hipStream_t st) {
+    if (code == 333) { if (dx) launch_build<L333, true>(a, pass, st); else launch_build<L333, false>(a, pass, st); }
+    else if (code == 133) { if (dx) launch_build<L133, true>(a, pass, st); else launch_build<L133, false>(a, pass, st); }
+    else { if (dx) launch_build<L155, true>(a, pass, st); else launch_build<L155, false>(a, pass, st); }
 }
 
 void free_lists(WinLists& wl) {
-    for (void* q : {(void*)wl.d_tile_win, (void*)wl.d_win, (void*)wl.d_item_idx, (void*)wl.d_item_pos, (void*)wl.d_col_idx,
-                    (void*)wl.d_col_pos})
-        if (q) (void)hipFree(q);
+    if (wl.d_block) (void)hipFree(wl.d_block);
     wl = WinLists{};
 }
 
@@ -150,52 +297,97 @@ int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, Win
     WinLists none{}; none.unavailable = true;
     p->lists[key] = none;             // replaced below when the build succeeds
     if (tl.n > 0) {
-        ConvArgs<float> a{};
-        a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.Lc = p->lc(level_delta); a.tree_off = p->tree_offset(a.Lc);
-        a.dx_skip_faces = dx == 2 ? 1 : 0;
-        int4* d_counts = nullptr; int4* d_offs = nullptr;
-        APRNET_HIP_CHECK(hipMalloc((void**)&d_counts, (size_t)tl.n * sizeof(int4)));
-        launch_build_code(code, a, tl.n, 0, d_counts, nullptr, wl, dx, st);
-        APRNET_LAUNCH_CHECK("build_lists_kernel (count)");
-        std::vector<int4> counts(tl.n), offs(tl.n);
+        const int HY = code == 155 ? 2 : 1, TY = 64 - 2 * HY, nrow = code == 333 ? L333::NROW : code == 133 ? L133::NROW : L155::NROW;
+        const int group = dx ? (code == 333 ? dx_group<L333>() : dx_group<L133>()) : 0;
+        ListArgs a{};
+        a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.n_tiles = tl.n; a.Lc = p->lc(level_delta); a.tree_off = p->tree_offset(a.Lc);
+        a.skip_faces = dx == 2 ? 1 : 0;
+        a.words = (p->apr.y_num[a.Lc] + 63) / 64;              // (no level is longer)
+        a.per_row = list_lds(a.words, nrow) <= 60 * 1024;
+        std::vector<void*> temps;                              // freed on every way out
+        struct Free { std::vector<void*>& t; ~Free() { for (void* q : t) (void)hipFree(q); } } guard{temps};
+        auto alloc = [&](void** q, size_t bytes) -> int { APRNET_HIP_CHECK(hipMalloc(q, std::max<size_t>(bytes, 16))); return 0; };
+        auto temp = [&](void** q, size_t bytes) -> int { const int rc = alloc(q, bytes); if (!rc) temps.push_back(*q); return rc; };
+        // kept positions of every row group -> its place on the compressed axis of its level, windows of the level
+        int* d_tile = nullptr;                                 // [3][n_tiles]
+        if (int rc = temp((void**)&d_tile, (size_t)tl.n * 3 * sizeof(int))) return rc;
+        a.n_cells = d_tile;
+        launch_build_code(code, a, dx != 0, 0, st);
+        APRNET_LAUNCH_CHECK("build_lists_kernel (positions)");
+        std::vector<int> cells(tl.n), place((size_t)2 * tl.n);
         APRNET_HIP_CHECK(hipStreamSynchronize(st));
-        APRNET_HIP_CHECK(hipMemcpy(counts.data(), d_counts, (size_t)tl.n * sizeof(int4), hipMemcpyDeviceToHost));
-        std::vector<int> tile_win(tl.n + 1);
-        int64_t nw = 0, ni = 0, nc = 0;
-        for (int t = 0; t < tl.n; ++t) {
-            offs[t] = make_int4((int)nw, (int)(uint32_t)ni, (int)(uint32_t)nc, 0);
-            tile_win[t] = (int)nw;
-            nw += counts[t].x; ni += counts[t].y; nc += counts[t].z;
+        APRNET_HIP_CHECK(hipMemcpy(cells.data(), a.n_cells, (size_t)tl.n * sizeof(int), hipMemcpyDeviceToHost));
+        int* first = place.data(), *slot0 = first + tl.n;
+        int64_t nw = 0, nslot = 0;
+        for (int l = MAX_LEVELS; l >= 0; --l) {                // tiles are sorted finest level first
+            int64_t c = 0;
+            for (int t = tl.level_begin[l]; t < tl.level_begin[l] + tl.level_count[l]; ++t) {
+                first[t] = (int)c; slot0[t] = (int)nslot;
+                c += (cells[t] + HY + 1) & ~1;                 // (even: pairs of cells stay in one window)
+                nslot += (cells[t] + 2 * HY) / TY + 2;         // windows that stage a cell of it, at most
+                if (c >= INT32_MAX - 65536 || nslot >= INT32_MAX - 65536) return fail(APRNET_ERR_UNSUPPORTED, "window lists: more than 2^31 positions");
+            }
+            a.win0[l] = (int)nw; a.nwin[l] = (int)((c + TY - 1) / TY);
+            nw += a.nwin[l];
         }
-        tile_win[tl.n] = (int)nw;
-        if (ni >= (int64_t)UINT32_MAX || nc >= (int64_t)UINT32_MAX || nw >= (int64_t)INT32_MAX) {
-            (void)hipFree(d_counts);
-            return fail(APRNET_ERR_UNSUPPORTED, "window lists: more than 2^32 entries");
-        }
-        wl.n_win = (int)nw; wl.n_items = ni; wl.n_cols = nc;
-        for (int l = MAX_LEVELS; l >= 0; --l) {        // tiles are sorted finest level first
-            if (tl.level_count[l] <= 0) continue;
-            const int fw = tile_win[tl.level_begin[l]], lw = tile_win[tl.level_begin[l] + tl.level_count[l]];
-            if (lw <= fw) continue;
-            wl.lv_first[wl.n_lv] = fw; wl.lv_level[wl.n_lv] = l;
-            for (int t = 0; t < tl.level_count[l]; ++t) wl.lv_cols[wl.n_lv] += counts[tl.level_begin[l] + t].z;
+        if (nw >= (int64_t)INT32_MAX) return fail(APRNET_ERR_UNSUPPORTED, "window lists: more than 2^31 windows");
+        APRNET_HIP_CHECK(hipMemcpy(d_tile + tl.n, place.data(), place.size() * sizeof(int), hipMemcpyHostToDevice));
+        a.first_cell = d_tile + tl.n; a.slot0 = d_tile + 2 * tl.n;
+        // items and columns per window -> offsets; windows without an output (or, input gradient, without a column) are not stored
+        std::vector<int4> cnt((size_t)nw, make_int4(0, 0, 0, 0)), off((size_t)nw), win;
+        if (int rc = temp((void**)&a.count, (size_t)(2 * nw + nslot) * sizeof(int4))) return rc;
+        int4* d_off = a.count + nw;
+        a.share = d_off + nw;
+        APRNET_HIP_CHECK(hipMemcpy(a.count, cnt.data(), (size_t)nw * sizeof(int4), hipMemcpyHostToDevice));
+        launch_build_code(code, a, dx != 0, 1, st);
+        APRNET_LAUNCH_CHECK("build_lists_kernel (count)");
+        APRNET_HIP_CHECK(hipStreamSynchronize(st));
+        APRNET_HIP_CHECK(hipMemcpy(cnt.data(), a.count, (size_t)nw * sizeof(int4), hipMemcpyDeviceToHost));
+        int64_t ni = 0, nc = 0;
+        for (int l = MAX_LEVELS; l >= 0; --l) {
+            const int w_first = (int)win.size();
+            const int64_t c_first = nc;
+            for (int w = a.win0[l]; w < a.win0[l] + a.nwin[l]; ++w) {
+                const int cols = group * cnt[w].y + cnt[w].z;
+                off[w] = make_int4(0, 0, 0, 0);
+                if (cols == 0 || cnt[w].x == 0) continue;
+                off[w] = make_int4((int)(uint32_t)ni, (int)(uint32_t)nc, cnt[w].y, 1);
+                win.push_back(make_int4((int)(uint32_t)ni, cnt[w].x, (int)(uint32_t)nc, cols));
+                ni += cnt[w].x; nc += cols;
+            }
+            if ((int)win.size() == w_first) continue;
+            wl.lv_first[wl.n_lv] = w_first; wl.lv_level[wl.n_lv] = l; wl.lv_cols[wl.n_lv] = nc - c_first;
             ++wl.n_lv;
         }
-        auto alloc = [&](void** q, size_t bytes) -> int { APRNET_HIP_CHECK(hipMalloc(q, std::max<size_t>(bytes, 16))); return 0; };
-        int rc = alloc((void**)&d_offs, (size_t)tl.n * sizeof(int4));
-        if (!rc) rc = alloc((void**)&wl.d_tile_win, tile_win.size() * sizeof(int));
-        if (!rc) rc = alloc((void**)&wl.d_win, (size_t)nw * sizeof(int4));
-        if (!rc) rc = alloc((void**)&wl.d_item_idx, (size_t)ni * sizeof(int));
-        if (!rc) rc = alloc((void**)&wl.d_item_pos, (size_t)ni * sizeof(unsigned short));
-        if (!rc) rc = alloc((void**)&wl.d_col_idx, (size_t)nc * sizeof(int));
-        if (!rc) rc = alloc((void**)&wl.d_col_pos, (size_t)nc * sizeof(unsigned short));
-        if (rc) { (void)hipFree(d_counts); if (d_offs) (void)hipFree(d_offs); free_lists(wl); return rc; }
-        APRNET_HIP_CHECK(hipMemcpy(d_offs, offs.data(), (size_t)tl.n * sizeof(int4), hipMemcpyHostToDevice));
-        APRNET_HIP_CHECK(hipMemcpy(wl.d_tile_win, tile_win.data(), tile_win.size() * sizeof(int), hipMemcpyHostToDevice));
-        launch_build_code(code, a, tl.n, 1, d_counts, d_offs, wl, dx, st);
-        APRNET_LAUNCH_CHECK("build_lists_kernel (fill)");
-        APRNET_HIP_CHECK(hipStreamSynchronize(st));
-        (void)hipFree(d_counts); (void)hipFree(d_offs);
+        if (ni >= (int64_t)UINT32_MAX || nc >= (int64_t)UINT32_MAX) return fail(APRNET_ERR_UNSUPPORTED, "window lists: more than 2^32 entries");
+        wl.n_win = (int)win.size(); wl.n_items = ni; wl.n_cols = nc;
+        std::vector<int> level;
+        level.reserve(win.size());
+        for (int k = 0; k < wl.n_lv; ++k) level.resize((size_t)(k + 1 < wl.n_lv ? wl.lv_first[k + 1] : wl.n_win), wl.lv_level[k]);
+        // one allocation for all of it
+        size_t at = 0;
+        auto part = [&](size_t bytes) { const size_t o = at; at = (at + bytes + 255) / 256 * 256; return o; };
+        const size_t o_win = part(win.size() * sizeof(int4)), o_level = part(level.size() * sizeof(int)), o_ii = part((size_t)ni * sizeof(int)),
+                     o_ci = part((size_t)nc * sizeof(int)), o_ip = part((size_t)ni * sizeof(unsigned short)), o_cp = part((size_t)nc * sizeof(unsigned short));
+        if (int rc = alloc(&wl.d_block, at)) return rc;
+        char* base = (char*)wl.d_block;
+        wl.d_win = (int4*)(base + o_win); wl.d_level = (int*)(base + o_level);
+        wl.d_item_idx = (int*)(base + o_ii); wl.d_col_idx = (int*)(base + o_ci);
+        wl.d_item_pos = (unsigned short*)(base + o_ip); wl.d_col_pos = (unsigned short*)(base + o_cp);
+        std::vector<char> head(o_ii);                          // headers and levels, in one copy
+        if (!win.empty()) {
+            std::memcpy(head.data() + o_win, win.data(), win.size() * sizeof(int4));
+            std::memcpy(head.data() + o_level, level.data(), level.size() * sizeof(int));
+        }
+        auto copy = [&](void* dst, const void* src, size_t bytes) -> int { if (bytes) APRNET_HIP_CHECK(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice)); return 0; };
+        int rc = copy(wl.d_block, head.data(), head.size());
+        if (!rc) rc = copy(d_off, off.data(), (size_t)nw * sizeof(int4));
+        if (rc) { free_lists(wl); return rc; }
+        a.off = d_off; a.item_idx = wl.d_item_idx; a.item_pos = wl.d_item_pos; a.col_idx = wl.d_col_idx; a.col_pos = wl.d_col_pos;
+        launch_build_code(code, a, dx != 0, 2, st);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(st);
+        if (e != hipSuccess) { free_lists(wl); return fail(APRNET_ERR_HIP, std::string("build_lists_kernel (fill): ") + hipGetErrorString(e)); }
     }
     p->lists[key] = wl;
     *out = wl;

@@ -7,7 +7,7 @@
 // of its y positions only, in thin shells around what is finely resolved: kept are the positions within the stencil's reach of an
 // output, one after the other, and the kept positions of all row groups of a level behind each other, with as many empty cells between
 // two groups as the stencil reaches.  Neighbours along y of an output are kept with it, so they are neighbours on the compressed
-// axis too, and what lies next to the end of a run there is a position that no output occupies.  A window is 62 (60) cells of that axis
+// axis too, and what lies next to the end of a run there is a position that no output occupies.  A window is up to 62 (60) cells of that axis
 // and its halo, whatever row groups they come from; the kernels see cells only.
 // The kernels are bound by what a window costs whether it is full or not (lists, round trips, weights, barriers).  Windows of
 // 62 positions of one row group, as they were, held 173 outputs of 496 on average on the 23 M particles of a blob volume (134,000
@@ -33,6 +33,8 @@ struct ListArgs {
     int* n_cells;                  // [n_tiles] pass 0: kept positions of a row group
     const int* first_cell;         // [n_tiles] its first cell on the compressed axis of its level
     int win0[MAX_LEVELS + 1], nwin[MAX_LEVELS + 1];          // windows of a level
+    int ty;                        // cells of a window without its halo
+    int used_words;                // 64-bit words of the counters of a row group's windows
     int4* count;                   // [windows] pass 1: items, groups of columns (see dx_group), other columns
     const int* slot0;              // [n_tiles] first entry in `share` of a row group, which has one per window it stages a cell of,
     int4* share;                   // pass 1: the entries of other row groups before its own
@@ -40,9 +42,6 @@ struct ListArgs {
     int* item_idx; unsigned short* item_pos; int* col_idx; unsigned short* col_pos;
 };
 
-// windows that a row group can stage a cell of: its cells and the halo, cut anywhere
-__host__ __device__ constexpr int list_windows(int words) { return words * 64 / 60 + 3; }
-__host__ __device__ constexpr int list_used_words(int words) { return (list_windows(words) * 3 + 1) / 2; }
 // word u of a bit map (p the one before, n the one after it), dilated by hy to either side
 __device__ __forceinline__ unsigned long long dilated(unsigned long long u, unsigned long long p, unsigned long long n, int hy) {
     unsigned long long k = u;
@@ -67,7 +66,7 @@ build_lists_kernel(const ListArgs a) {
     unsigned long long* any = maps + a.words;                            // [W] positions with an output in some row
     int* before = reinterpret_cast<int*>(maps + 2 * a.words);            // [W] kept positions in the words before
     int* used = reinterpret_cast<int*>(maps + 3 * a.words);              // [windows of the group][3] entries so far (pass 2: and those of other groups before them)
-    unsigned long long* rows = maps + 3 * a.words + list_used_words(a.words);    // [NROW][W] outputs of a row (per_row)
+    unsigned long long* rows = maps + 3 * a.words + a.used_words;    // [NROW][W] outputs of a row (per_row)
     unsigned long long* reach = rows + G::NROW * a.words;                // [NROW][W] positions of a row with an output in reach (per_row)
 
     // ---- the rows of the group: particles of the level, of the coarser one, tree nodes
@@ -143,8 +142,8 @@ build_lists_kernel(const ListArgs a) {
     auto cell_of = [&](int y) { return first + before[y >> 6] + __popcll(keep[y >> 6] & ((1ull << (y & 63)) - 1ull)); };
     // an output within the stencil's reach of position y of row r (whose position is kept)
     auto reached = [&](int r, int y) { return !a.per_row || ((reach[r * W + (y >> 6)] >> (y & 63)) & 1ull) != 0; };
-    const int wf = max((first + G::HY - G::WY + G::TY) / G::TY, 0);        // first window that stages a cell of the group
-    const int nw = total > 0 ? min((first + total - 1 + G::HY) / G::TY, nwin - 1) - wf + 1 : 0;
+    const int ty = a.ty, wf = max(first - G::HY, 0) / ty;        // first window that stages a cell of the group
+    const int nw = total > 0 ? min((first + total - 1 + G::HY) / ty, nwin - 1) - wf + 1 : 0;
     int4* share = a.share + a.slot0[blockIdx.x];
     for (int i = threadIdx.x; i < nw; i += G::NT) {
         const int4 o = PASS == 2 ? share[i] : make_int4(0, 0, 0, 0);
@@ -167,11 +166,11 @@ build_lists_kernel(const ListArgs a) {
     };
     // an item on cell c, and on c + 1 if it is a pair, for every window that stages one of the two
     auto item = [&](bool has, int r, int c, bool pair, int idx, unsigned flags) {
-        const int lo = max((c + G::HY - G::WY + G::TY) / G::TY, 0), hi = min((c + (pair ? 1 : 0) + G::HY) / G::TY, nwin - 1);
+        const int lo = max(c - G::HY, 0) / ty, hi = min((c + (pair ? 1 : 0) + G::HY) / ty, nwin - 1), wy = ty + 2 * G::HY;
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const int w = lo + k, p = c - (w * G::TY - G::HY);
-            const bool in = p >= 0 && p < G::WY, in2 = pair && p + 1 >= 0 && p + 1 < G::WY;
+            const int w = lo + k, p = c - (w * ty - G::HY);
+            const bool in = p >= 0 && p < wy, in2 = pair && p + 1 >= 0 && p + 1 < wy;
             append(has && w <= hi && (in || in2), w, 0, [&](int win, int n) {
                 const int4 o = a.off[win];
                 if (!o.w) return;
@@ -181,13 +180,13 @@ build_lists_kernel(const ListArgs a) {
         }
     };
     auto column = [&](bool has, int r, int c, int idx, unsigned flags) {
-        const int w = c / G::TY;
+        const int w = c / ty;
         append(has, w, 2, [&](int win, int n) {
             const int4 o = a.off[win];
             if (!o.w) return;
             const size_t at = (size_t)(unsigned)o.y + (DX ? dx_group<G>() * o.z : 0) + n;
             a.col_idx[at] = idx;
-            a.col_pos[at] = (unsigned short)((r * G::RS + c - w * G::TY + G::HY) | flags);
+            a.col_pos[at] = (unsigned short)((r * G::RS + c - w * ty + G::HY) | flags);
         });
     };
     for (int s = wave; s < G::NSEG; s += G::NWAVE) {
@@ -225,7 +224,7 @@ build_lists_kernel(const ListArgs a) {
                     if (pooled && ka)
 #pragma unroll
                         for (int k = 0; k < N; ++k) hit = hit || reached(r + (k >> 2) * G::RX + ((k >> 1) & 1), ya + (k & 1));
-                    const int w = ca / G::TY;
+                    const int w = ca / ty;
                     append(hit, w, 1, [&](int win, int n) {
                         const int4 o = a.off[win];
                         if (!o.w) return;
@@ -233,7 +232,7 @@ build_lists_kernel(const ListArgs a) {
                         for (int k = 0; k < N; ++k) {                     // cells in the order z, x, y
                             const size_t at = (size_t)(unsigned)o.y + N * n + k;
                             a.col_idx[at] = i;
-                            a.col_pos[at] = (unsigned short)(((r + (k >> 2) * G::RX + ((k >> 1) & 1)) * G::RS + ca - w * G::TY + G::HY + (k & 1)) | COL_BOX);
+                            a.col_pos[at] = (unsigned short)(((r + (k >> 2) * G::RX + ((k >> 1) & 1)) * G::RS + ca - w * ty + G::HY + (k & 1)) | COL_BOX);
                         }
                     });
                 }
@@ -260,10 +259,10 @@ using L333 = ConvGeom<3, 3, 3, 2, 4, 512>;
 using L133 = ConvGeom<1, 3, 3, 1, 8, 512>;
 using L155 = ConvGeom<1, 5, 5, 1, 8, 512>;
 
-static size_t list_lds(int words, int rows) { return 8 * ((size_t)words * (3 + 2 * rows) + list_used_words(words)); }
+static size_t list_lds(int words, int rows, int used_words) { return 8 * ((size_t)words * (3 + 2 * rows) + used_words); }
 template <class G, bool DX>
 static void launch_build(const ListArgs& a, int pass, hipStream_t st) {
-    const size_t lds = list_lds(a.words, a.per_row ? G::NROW : 0);
+    const size_t lds = list_lds(a.words, a.per_row ? G::NROW : 0, a.used_words);
     if (pass == 0) hipLaunchKernelGGL((build_lists_kernel<G, DX, 0>), dim3((unsigned)a.n_tiles), dim3(G::NT), lds, st, a);
     else if (pass == 1) hipLaunchKernelGGL((build_lists_kernel<G, DX, 1>), dim3((unsigned)a.n_tiles), dim3(G::NT), lds, st, a);
     else hipLaunchKernelGGL((build_lists_kernel<G, DX, 2>), dim3((unsigned)a.n_tiles), dim3(G::NT), lds, st, a);
@@ -277,6 +276,16 @@ static void launch_build_code(int code, const ListArgs& a, bool dx, int pass, hi
 void free_lists(WinLists& wl) {
     if (wl.d_block) (void)hipFree(wl.d_block);
     wl = WinLists{};
+}
+
+// Cells of a window without its halo: as many as the patch holds where that leaves a window for each of the 512 workgroups that the chip
+// holds, fewer otherwise, an even number of them.  Training step on two APRs of 338 k particles, whose coarser level deltas had 5 to 370
+// full windows, 11.5 -> 10.3 ms, group-normed fp32 U-Net on 2.7 M 5.31 -> 5.13.  (1024 windows 32 -> 32 channels on 320 k particles
+// 0.176 instead of 0.165 ms, 2048 0.209; down to 14 cells the step 10.3, to 6 11.4 ms; widths of 62, 30 and 14 only 10.75.)
+constexpr int WINDOWS_MIN = 512, CELLS_MIN = 22;
+static int window_cells(int64_t n_cells, int HY) {
+    const int widest = 64 - 2 * HY;
+    return (int)std::max<int64_t>(CELLS_MIN, std::min<int64_t>(widest, n_cells / WINDOWS_MIN & ~(int64_t)1));
 }
 
 // Lists of the forward convolution at `level_delta` for stencil `code` (333, 133, 155); `tl` must be the tile list
@@ -297,13 +306,13 @@ int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, Win
     WinLists none{}; none.unavailable = true;
     p->lists[key] = none;             // replaced below when the build succeeds
     if (tl.n > 0) {
-        const int HY = code == 155 ? 2 : 1, TY = 64 - 2 * HY, nrow = code == 333 ? L333::NROW : code == 133 ? L133::NROW : L155::NROW;
+        const int HY = code == 155 ? 2 : 1, nrow = code == 333 ? L333::NROW : code == 133 ? L133::NROW : L155::NROW;
         const int group = dx ? (code == 333 ? dx_group<L333>() : dx_group<L133>()) : 0;
         ListArgs a{};
         a.apr = p->dapr; a.tree = p->dtree; a.tiles = tl.d_tiles; a.n_tiles = tl.n; a.Lc = p->lc(level_delta); a.tree_off = p->tree_offset(a.Lc);
         a.skip_faces = dx == 2 ? 1 : 0;
         a.words = (p->apr.y_num[a.Lc] + 63) / 64;              // (no level is longer)
-        a.per_row = list_lds(a.words, nrow) <= 60 * 1024;
+        a.per_row = list_lds(a.words, nrow, 0) <= 48 * 1024;
         std::vector<void*> temps;                              // freed on every way out
         struct Free { std::vector<void*>& t; ~Free() { for (void* q : t) (void)hipFree(q); } } guard{temps};
         auto alloc = [&](void** q, size_t bytes) -> int { APRNET_HIP_CHECK(hipMalloc(q, std::max<size_t>(bytes, 16))); return 0; };
@@ -318,18 +327,23 @@ int get_lists(aprnet_plan* p, int level_delta, int code, const TileList& tl, Win
         APRNET_HIP_CHECK(hipStreamSynchronize(st));
         APRNET_HIP_CHECK(hipMemcpy(cells.data(), a.n_cells, (size_t)tl.n * sizeof(int), hipMemcpyDeviceToHost));
         int* first = place.data(), *slot0 = first + tl.n;
-        int64_t nw = 0, nslot = 0;
+        int64_t nw = 0, nslot = 0, n_cells = 0;
+        for (int t = 0; t < tl.n; ++t) n_cells += (cells[t] + HY + 1) & ~1;
+        a.ty = window_cells(n_cells, HY);
+        int most = 0;                                          // windows that stage a cell of one row group
         for (int l = MAX_LEVELS; l >= 0; --l) {                // tiles are sorted finest level first
             int64_t c = 0;
             for (int t = tl.level_begin[l]; t < tl.level_begin[l] + tl.level_count[l]; ++t) {
                 first[t] = (int)c; slot0[t] = (int)nslot;
                 c += (cells[t] + HY + 1) & ~1;                 // (even: pairs of cells stay in one window)
-                nslot += (cells[t] + 2 * HY) / TY + 2;         // windows that stage a cell of it, at most
+                const int n = (cells[t] + 2 * HY) / a.ty + 2;
+                nslot += n; most = std::max(most, n);
                 if (c >= INT32_MAX - 65536 || nslot >= INT32_MAX - 65536) return fail(APRNET_ERR_UNSUPPORTED, "window lists: more than 2^31 positions");
             }
-            a.win0[l] = (int)nw; a.nwin[l] = (int)((c + TY - 1) / TY);
+            a.win0[l] = (int)nw; a.nwin[l] = (int)((c + a.ty - 1) / a.ty);
             nw += a.nwin[l];
         }
+        a.used_words = (3 * most + 1) / 2;                     // (at most 65,536 positions in windows of 60: 13 KB; narrower ones of fewer cells)
         if (nw >= (int64_t)INT32_MAX) return fail(APRNET_ERR_UNSUPPORTED, "window lists: more than 2^31 windows");
         APRNET_HIP_CHECK(hipMemcpy(d_tile + tl.n, place.data(), place.size() * sizeof(int), hipMemcpyHostToDevice));
         a.first_cell = d_tile + tl.n; a.slot0 = d_tile + 2 * tl.n;

@@ -152,8 +152,8 @@ int pack_conv_weights(int code, const float* w, int S_exp, int Cm, int Ck, bool 
 
 size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
-int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
-                  const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
+int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx, int64_t nx, float* xi,
+                  hipStream_t st);
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
 static std::atomic<int> g_dw_split{1};       // and their weight gradient (conv_dw_split.hip), likewise
@@ -223,26 +223,21 @@ static int try_narrow(aprnet_plan* p, const ConvArgs<T>& a, int code, int d, con
     return launch_conv_narrow(code, b, wl, st);
 }
 
-// Work space of the forward pass on products of bfloat16 pieces: packed weights, the input and its mean tree in groups of four
-// channels.  0: the layer does not take that path.
-//  - fewer than SPLIT_MIN_CIN input channels: with 8 it is no faster (8 -> 16 channels on 320 k particles 0.080 against 0.078 ms,
-//    copies included).
-//  - 1x3x3: two steps of eight taps for nine, less than the copies cost (64 -> 64 channels on 70 k particles 107 against 98 us,
-//    on 320 k 346 against 352).
-//  - little work: one more launch than the fp32 kernel's, which also counts where the host is behind the device (3x3x3, split against
-//    fp32; 16 outputs: 70 k particles 45 and 46 us, 320 k 90 and 104; 32 outputs: 14 k particles x 16 channels 34 and 37, x 32 42
-//    and 54, 2 k x 32 30 and 32; 64 outputs: 2 k x 64 39 and 51 us).
-//    1x5x5 gains from less work on, but takes the same line: 4 k particles 16 -> 16 channels 35 and 42 us, 64 -> 64 115 and 163; 99 k 89 and
-//    114, 406 and 614; 2 M 423 and 497 us, 3.54 and 4.94 ms.
-//  - the 16-byte items are reached with 32-bit offsets: fewer than 2^28 particles.
+// Work space of the forward pass on products of bfloat16 pieces: packed weights and marks.  0: the layer does not take that path.
+//  - fewer than SPLIT_MIN_CIN input channels: half of an instruction's products are zero.
+//  - 1x3x3: two steps of eight taps for nine.
+//  - little work: one more launch than the fp32 kernel's, which also counts where the host is behind the device (3x3x3, pieces against
+//    fp32; 16 outputs: 90 k particles x 16 channels 50 and 48 us, x 32 70 and 65, 160 k x 16 58 and 58, 320 k 78 and 90; 32 outputs: 12 k
+//    x 16 34 and 36, x 32 43 and 49, 90 k 79 and 95; 64 outputs: 2 k x 64 62 and 74, 90 k 183 and 251 us).
+//    1x5x5 gains about as much (16 -> 16 channels on 80 k 44 and 43 us, on 230 k 54 and 58; 64 -> 64 on 20 k 68 and 86, on 1 M 1.21 and 1.64 ms).
+//  - values are reached with 32-bit offsets: fewer than 2^28 particles.
 constexpr int SPLIT_MIN_CIN = 16;
 static size_t split_align(size_t v) { return (v + 255) / 256 * 256; }
 static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx, int64_t nt) {
     if (!g_f32_split || g_conv_path == 1 || (code != 333 && code != 155) || Cin < SPLIT_MIN_CIN || nx >= (1ll << 28) || nt >= (1ll << 28)) return 0;
     if (g_f32_split == 1 && (double)nx * Cin * ((Cout + 15) / 16 * 16) < (Cout <= 16 ? 1 << 26 : 1 << 23)) return 0;
     if (conv_packed_split_bytes(code, S_exp, Cout, Cin) / 48 >= (1u << 29)) return 0;               // elements the packing kernel counts in 32 bits
-    if ((double)(Cin + 3) / 4 * (nx + nt) >= 1.6e10) return 0;                                   // 2^32 threads of the copies, four elements each
-    return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cout, Cin)) + (size_t)(Cin + 3) / 4 * (size_t)(nx + nt) * 16;
+    return split_mark_bytes() + split_align(conv_packed_split_bytes(code, S_exp, Cout, Cin));
 }
 
 // The same of the input gradient: packed weights and the output gradient in groups of four channels.
@@ -280,17 +275,12 @@ template <> int try_mfma<float>(aprnet_plan* p, const ConvArgs<float>& a, int co
     *done = true;
     ConvArgs<float> b = a;
     if (int rc = set_lists(p, d, code, tl, b, st)) return rc;
-    WinLists wl;
-    const size_t need = b.win_level && get_lists(p, d, code, tl, &wl, st) == 0 ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
+    const size_t need = b.win_level ? split_fwd_bytes(code, a.Cin, a.S_exp, a.Cout, a.x_count, a.t_count) : 0;
     if (need > 0 && ws && ws_bytes >= 0 && (size_t)ws_bytes >= need) {
-        // products of bfloat16 pieces on copies in groups of four channels, all in the caller's work space
-        const size_t wbytes = split_align(conv_packed_split_bytes(code, a.S_exp, a.Cout, a.Cin)), ng = (size_t)(a.Cin + 3) / 4;
+        // products of bfloat16 pieces: weights and marks in the caller's work space
         char* image = (char*)ws + split_mark_bytes();
-        float* xi = (float*)(image + wbytes), *ti = xi + ng * (size_t)a.x_count * 4;
-        if (int rc = prepare_split(code, a.w, a.S_exp, a.Cout, a.Cin, false, image, (int*)ws, a.x, a.ldx, a.x2, a.ldx2, a.c_split, a.x_count, xi,
-                                   a.tree_data, a.ldt, a.t_count, ti, st)) return rc;
+        if (int rc = prepare_split(code, a.w, a.S_exp, a.Cout, a.Cin, false, image, (int*)ws, nullptr, 0, 0, nullptr, st)) return rc;
         b.w_raw = a.w; b.w = (const float*)image; b.redo = (int*)ws;
-        b.xi = xi; b.ti = ti; b.xi_ld = a.x_count; b.ti_ld = a.t_count;
         TimedLaunch timed(st);
         return launch_conv_split(code, b, b.n_tiles, st);
     }

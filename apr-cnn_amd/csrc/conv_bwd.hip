@@ -269,8 +269,8 @@ size_t split_dx_bytes(int code, int Cin, int S_exp, int Cout, int64_t n);
 bool split_dw(int Cin, int Cout, int64_t n, int64_t ldx, int64_t ldt);
 size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
-int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
-                  const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st);
+int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx, int64_t nx, float* xi,
+                  hipStream_t st);
 int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
 int launch_conv_dw_split(int code, const ConvArgs<float>& a, const DwWork& k, int* mark, hipStream_t st);
 int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
@@ -350,15 +350,15 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
         float* gi = (float*)(image + (conv_packed_split_bytes(code, a.S_exp, a.Cin, a.Cout) + 255) / 256 * 256);
         mark = (int*)ws;
         redo = RedoClear{mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin};
-        if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, nullptr, 0, a.Cout, a.x_count, gi,
-                                   nullptr, 0, 0, nullptr, st)) return rc;
+        if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, a.x_count, gi, st)) return rc;
         e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
         e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
     }
+    const bool dw_pieces = pieces && wl && wl->n_win > 0 && split_dw(a.Cin, a.Cout, a.x_count, a.ldx, a.ldt);
     hipStream_t side = st;
     if (a.gx) if (int rc = fork_side(p, st, &side)) return rc;
     SideJoin guard(p, st, side);
-    if (pieces && wl && wl->n_win > 0 && split_dw(a.Cin, a.Cout, a.x_count, a.ldx, a.ldt)) {
+    if (dw_pieces) {
         c.xi = e.xi; c.xi_ld = e.xi_ld; c.redo = mark + 1;
         if (int rc = launch_conv_dw_split(code, c, dw_work(code, a.Cout, a.Cin, a.S_exp, a.Lc, *wl), mark + 1, side)) return rc;
     }

@@ -577,7 +577,8 @@ struct ItemRegs16 { intx4 v[IPT]; unsigned off[IPT]; unsigned short pos[IPT]; };
 
 // BIG: tensors of 2^28 elements and more per group, whose 16-byte items lie past 32-bit byte offsets: R.off keeps the
 // element index and the loads take 64-bit addresses (a lane without an item reads element 0; its value is never stored)
-template <class G, int IPT, bool BIG = false, class Lists>
+// SIZE: bytes of an item in the tensor that R.off reaches into
+template <class G, int IPT, bool BIG = false, int SIZE = 16, class Lists>
 __device__ __forceinline__ void fetch_slots16(const Lists& sh, int nitem, ItemRegs16<G, IPT>& R) {
     // unconditional buffer loads, results touched only after every round is issued (see fetch_slots)
     const __amdgpu_buffer_rsrc_t ri = __builtin_amdgcn_make_buffer_rsrc(const_cast<int*>(sh.item_idx), 0, nitem * 4, 0x00020000);
@@ -597,7 +598,7 @@ __device__ __forceinline__ void fetch_slots16(const Lists& sh, int nitem, ItemRe
     for (int k = 0; k < IPT; ++k) {
         const bool valid = (int)threadIdx.x + k * G::NT < nitem;
         R.pos[k] = valid ? (unsigned short)pos[k] : (unsigned short)0xffffu;
-        R.off[k] = BIG ? (valid ? (unsigned)idx[k] : 0u) : (valid ? (unsigned)idx[k] * 16u : BUF_OOB);
+        R.off[k] = BIG ? (valid ? (unsigned)idx[k] : 0u) : (valid ? (unsigned)idx[k] * (unsigned)SIZE : BUF_OOB);
     }
 }
 // Gather of one channel chunk into the patch.  Cells that no item covers keep the zeros written once

@@ -15,12 +15,11 @@
 // on 23 M particles.)  Values come from copies in groups of four channels, one 16-byte load per item; a value is split when it is
 // written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
 //
-// Measured against the fp32 instructions (3x3x3, the kernel alone): 23 M particles, 32 -> 32 channels 9.5 (12.5) ms, 16 -> 16
-// channels 3.4 (4.1) ms; 320 k particles, 64 -> 64 channels 0.51 (0.78) ms.
-// Input gradient, whole backward pass beside the weight gradient: 23 M particles, 32 -> 32 channels 38.3 (43.5) ms, 16 -> 16 14.1
-// (15.3) ms; the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
-// Bound by the barriers around the matrix phases of sparse windows and the LDS reads of the operands: 32 -> 32 channels, matrix pipes busy
-// 44 % of the launch, waves waiting for memory, LDS or a barrier 51 % of their cycles.
+// Measured against the fp32 instructions (3x3x3, whole forward pass): 23 M particles, 32 -> 32 channels 8.7 ms; 1 M, 32 -> 32 0.40 (0.52), 64 -> 64
+// 1.40 (1.78); 320 k, 16 -> 16 0.078 (0.090), 64 -> 64 0.46 (0.64).
+// Input gradient, whole backward pass with the weight gradient (conv_dw_split.hip): 1 M particles, 32 -> 32 channels 1.33 (1.84), 16 -> 16 0.48
+// (0.72); the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
+// Bound by the barriers around the matrix phases and the LDS reads of the operands.
 // Error against 64 bits (2-norm): 0.31 to 0.33 of the fp32 instructions' with N(0, 1) features, 0.31 to 0.35 with those after a ReLU, below theirs
 // also where few products are not zero, but for a single one (1.02; see split_window).
 //
@@ -93,19 +92,17 @@ __device__ __forceinline__ void pack_weights_split(const float* __restrict__ w, 
     }
 }
 
-// ---- input in groups of four channels: [Cin / 4][count][4] ---------------------------------------------------
-// out[q][i][c] = SPLIT_SCALE * channel 4 q + c of element i; channels from c_split on come from x2 (null: all from x), channels past C
-// are zeros.  A streaming pass (8 bytes per value), four elements per thread, all reads issued before the first is used.
+// ---- output gradient in groups of four channels: [C / 4][count][4] --------------------------------------------
+// out[q][i][c] = SPLIT_SCALE * channel 4 q + c of element i; channels past C are zeros.  A streaming pass (8 bytes per value), four
+// elements per thread, all reads issued before the first is used.
 constexpr int IG_E = 4;
-__device__ __forceinline__ void group4(const float* __restrict__ x, int64_t ldx, const float* __restrict__ x2, int64_t ldx2, int c_split, int C, int64_t count,
-                                       float4* __restrict__ out, unsigned block, int q) {
+__device__ __forceinline__ void group4(const float* __restrict__ x, int64_t ldx, int C, int64_t count, float4* __restrict__ out, unsigned block, int q) {
     constexpr int IG_TB = PREP_TB;
     const int64_t i0 = (int64_t)block * (IG_TB * IG_E) + threadIdx.x;
     float v[SP_CIB][IG_E];
 #pragma unroll
     for (int c = 0; c < SP_CIB; ++c) {
-        const int ch = min(q * SP_CIB + c, C - 1);
-        const float* p = (x2 != nullptr && ch >= c_split) ? x2 + (int64_t)(ch - c_split) * ldx2 : x + (int64_t)ch * ldx;
+        const float* p = x + (int64_t)min(q * SP_CIB + c, C - 1) * ldx;
 #pragma unroll
         for (int e = 0; e < IG_E; ++e) v[c][e] = p[min(i0 + e * IG_TB, count - 1)];
     }
@@ -122,46 +119,84 @@ __device__ __forceinline__ void group4(const float* __restrict__ x, int64_t ldx,
             dst[i0 + e * IG_TB] = make_float4(SPLIT_SCALE * v[0][e], SPLIT_SCALE * v[1][e], SPLIT_SCALE * v[2][e], SPLIT_SCALE * v[3][e]);
 }
 
-// What the convolution reads, in one launch: the first blocks pack the weights and clear the marks, the others copy the features (nbx
-// blocks per group of channels) and the tree (nbt).  (As three launches the copies of small layers cost more than the
-// convolution gained where the host is behind: a group-normed fp32 U-Net on a small crop 2.57 against 2.44 ms without.)
-struct SplitCopy { const float* x; int64_t ldx; const float* x2; int64_t ldx2; int c_split; int64_t count; float4* out; };
+// What the convolution reads, in one launch: the first blocks pack the weights and clear the marks, the others copy the output gradient (nbx
+// blocks per group of channels).
 template <int K>
 __global__ void __launch_bounds__(PREP_TB)
 split_prepare_kernel(const float* __restrict__ w, int S_exp, int Cm, int Ck, int COH, int transposed, uint4* __restrict__ image,
-                     int* __restrict__ marks, unsigned nb_pack, const SplitCopy fx, unsigned nbx, const SplitCopy ft, unsigned nbt) {
+                     int* __restrict__ marks, unsigned nb_pack, const float* __restrict__ x, int64_t ldx, int64_t count, float4* __restrict__ out, unsigned nbx) {
     unsigned b = blockIdx.x;
     if (b < nb_pack) { pack_weights_split<K>(w, S_exp, Cm, Ck, COH, transposed, image, marks, b, nb_pack); return; }
     b -= nb_pack;
-    const unsigned nq = (unsigned)(Ck + SP_CIB - 1) / SP_CIB;
-    if (b < nbx * nq) { group4(fx.x, fx.ldx, fx.x2, fx.ldx2, fx.c_split, Ck, fx.count, fx.out, b % nbx, (int)(b / nbx)); return; }
-    b -= nbx * nq;
-    group4(ft.x, ft.ldx, nullptr, 0, Ck, Ck, ft.count, ft.out, b % nbt, (int)(b / nbt));
+    group4(x, ldx, Ck, count, out, b % nbx, (int)(b / nbx));
 }
 
 template <class G> struct SplitItems : ItemRegs16<G, (G::MAXITEM + G::NT - 1) / G::NT> {
     static constexpr int IPT = (G::MAXITEM + G::NT - 1) / G::NT;
 };
-template <class G>
+// Forward: from the caller's channel planes, four loads per item, every plane at a scalar offset from the first one of the chunk, so that features
+// and tree take one descriptor each.  (One 16-byte load per item from copies in groups of four channels, made by a pass of 8 bytes per value:
+// 32 -> 32 channels on 23 M particles 9.5 instead of 8.7 ms, 16 -> 16 on 43 M 6.9 and 6.5, on 1 M 0.175 and 0.164, 64 -> 48 on 2 M 2.55 and 2.48.)
+// A chunk that takes channels of both tensors, or rows of 2^28 values and more, has a descriptor per plane.
+// Input gradient: from the copy of the output gradient, which the weight gradient reads too.
+template <class G, int MODE>
 __device__ __forceinline__ void load_values_split(const ConvArgs<float>& a, int q, int nitem, bool tree_items, SplitItems<G>& R) {
+    if constexpr (MODE == 0) {
+        const int c0 = q * SP_CIB, last = min(SP_CIB, a.Cin - c0) - 1;         // (a channel past the last one reads that one's plane; its weights are zero)
+        const bool second = a.x2 != nullptr && c0 >= a.c_split;
+        const float* xb = second ? a.x2 + (int64_t)(c0 - a.c_split) * a.ldx2 : a.x + (int64_t)c0 * a.ldx;
+        const int64_t ld = second ? a.ldx2 : a.ldx;
+        const bool both = a.x2 != nullptr && !second && c0 + last >= a.c_split;
+        if (both || ld >= (1ll << 28) || a.ldt >= (1ll << 28)) {               // uniform
+#pragma unroll
+            for (int c = 0; c < SP_CIB; ++c) {
+                const int ch = c0 + min(c, last);
+                const bool s2 = a.x2 != nullptr && ch >= a.c_split;
+                const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(s2 ? a.x2 + (int64_t)(ch - a.c_split) * a.ldx2 : a.x + (int64_t)ch * a.ldx),
+                                                                                    0, (int)(unsigned)(a.x_count * 4), 0x00020000);
+                const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.tree_data + (int64_t)ch * a.ldt), 0,
+                                                                                    tree_items ? (int)(unsigned)(a.t_count * 4) : 0, 0x00020000);
+#pragma unroll
+                for (int k = 0; k < SplitItems<G>::IPT; ++k) {
+                    if (k * G::NT >= nitem) break;          // wave-uniform
+                    if (R.pos[k] != 0xffffu && (R.pos[k] & ITEM_TREE) != 0) {
+                        R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rt, (int)R.off[k], 0, 0);
+                        asm volatile("" ::: "memory");
+                    } else R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, (int)R.off[k], 0, 0);
+                }
+            }
+            return;
+        }
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(xb), 0, (int)(unsigned)((last * ld + a.x_count) * 4), 0x00020000);
+        const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.tree_data + (int64_t)c0 * a.ldt), 0,
+                                                                            tree_items ? (int)(unsigned)((last * a.ldt + a.t_count) * 4) : 0, 0x00020000);
+#pragma unroll
+        for (int k = 0; k < SplitItems<G>::IPT; ++k) {
+            if (k * G::NT >= nitem) break;                  // wave-uniform
+            const bool item = R.pos[k] != 0xffffu;
+            const int off = item ? (int)R.off[k] : 0;       // (no item: a value that is not stored)
+            if (tree_items) {
+                if (item && (R.pos[k] & ITEM_TREE) != 0) {
+#pragma unroll
+                    for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rt, off, min(c, last) * (int)a.ldt * 4, 0);
+                    asm volatile("" ::: "memory");          // keeps the two branches from being merged into one load with a per-lane descriptor
+                } else {
+#pragma unroll
+                    for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, min(c, last) * (int)ld * 4, 0);
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, min(c, last) * (int)ld * 4, 0);
+            }
+        }
+        return;
+    }
     const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.xi + (int64_t)q * a.xi_ld * SP_CIB), 0,
                                                                         (int)(a.x_count * 16), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rt = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.ti + (int64_t)q * a.ti_ld * SP_CIB), 0,
-                                                                        tree_items ? (int)(a.t_count * 16) : 0, 0x00020000);
 #pragma unroll
     for (int k = 0; k < SplitItems<G>::IPT; ++k) {
-        if (k * G::NT >= nitem) break;                  // wave-uniform
-        const bool from_tree = (R.pos[k] & ITEM_TREE) != 0 && R.pos[k] != 0xffffu;
-        if (tree_items) {
-            if (from_tree) {
-                R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rt, (int)R.off[k], 0, 0);
-                asm volatile("" ::: "memory");          // keeps the two branches from being merged into one load with a per-lane descriptor
-            } else {
-                R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)R.off[k], 0, 0);
-            }
-        } else {
-            R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)R.off[k], 0, 0);
-        }
+        if (k * G::NT >= nitem) break;                      // wave-uniform
+        R.v[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)R.off[k], 0, 0);
     }
 }
 template <class G, int COH>
@@ -171,15 +206,16 @@ struct SplitShared {
     float bias[16 * COH];
     int2 toff[split_steps<G>() * 4];
 };
-template <class G, int COH>
+template <class G, int COH, int MODE>
 __device__ __forceinline__ void store_items_split(const SplitItems<G>& R, int nitem, SplitShared<G, COH>& sh) {
+    constexpr float S = MODE == 0 ? SPLIT_SCALE : 1.f;         // (the copy is scaled)
 #pragma unroll
     for (int k = 0; k < SplitItems<G>::IPT; ++k) {
         if (k * G::NT >= nitem) break;                  // wave-uniform
         if (R.pos[k] == 0xffffu) continue;
         uint2 p[3];
-        split_pair(__builtin_bit_cast(float, (int)R.v[k][0]), __builtin_bit_cast(float, (int)R.v[k][1]), p[0].x, p[1].x, p[2].x);
-        split_pair(__builtin_bit_cast(float, (int)R.v[k][2]), __builtin_bit_cast(float, (int)R.v[k][3]), p[0].y, p[1].y, p[2].y);
+        split_pair(S * __builtin_bit_cast(float, (int)R.v[k][0]), S * __builtin_bit_cast(float, (int)R.v[k][1]), p[0].x, p[1].x, p[2].x);
+        split_pair(S * __builtin_bit_cast(float, (int)R.v[k][2]), S * __builtin_bit_cast(float, (int)R.v[k][3]), p[0].y, p[1].y, p[2].y);
         const int c = R.pos[k] & ITEM_CELL;
 #pragma unroll
         for (int i = 0; i < 3; ++i) sh.patch[i][c] = p[i];
@@ -223,13 +259,13 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
 #pragma unroll
         for (int k = 0; k < WPT; ++k) wr[k] = __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(threadIdx.x + k * G::NT) * 16, 0, 0);
     };
-    fetch_slots16<G, SplitItems<G>::IPT>(gl, nitem, R);
+    fetch_slots16<G, SplitItems<G>::IPT, false, MODE == 0 ? 4 : 16>(gl, nitem, R);
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
         const int col = ((first + G::NWAVE * j) << 4) + (lane & 15);
         cell[j] = col < nc ? ((cell[j] & (int)COL_CELL) - G::TAP0) * 8 : 0;
     }
-    load_values_split<G>(a, 0, nitem, tree_items, R);
+    load_values_split<G, MODE>(a, 0, nitem, tree_items, R);
     // With 32 outputs a wave that holds two and more blocks of columns asks for the weights of a chunk in front of the barrier that ends the
     // chunk before it, whose operands no longer need registers then; a wave with one block has them to spare and asks together with the
     // values (64 -> 64 channels on 8 M particles 18.9, always in front of the barrier 19.1, always with the values 20.0), as do the 16 outputs.
@@ -239,7 +275,7 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
     for (int ci0 = 0; ci0 < a.Cin; ci0 += SP_CIB) {
         if constexpr (LATE) load_weights(ci0 / SP_CIB);
         __syncthreads();
-        store_items_split<G, COH>(R, nitem, sh);
+        store_items_split<G, COH, MODE>(R, nitem, sh);
 #pragma unroll
         for (int k = 0; k < WPT; ++k) {
             const int i = threadIdx.x + k * G::NT;
@@ -247,7 +283,7 @@ __device__ __forceinline__ void split_window(const ConvArgs<float>& a, int co0, 
         }
         __syncthreads();
         if (ci0 + SP_CIB < a.Cin) {
-            load_values_split<G>(a, ci0 / SP_CIB + 1, nitem, tree_items, R);
+            load_values_split<G, MODE>(a, ci0 / SP_CIB + 1, nitem, tree_items, R);
             if constexpr (!LATE) load_weights(ci0 / SP_CIB + 1);
         }
         if constexpr (NB > 0) {
@@ -409,8 +445,7 @@ static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     APRNET_LAUNCH_CHECK("conv_split_kernel");
     return 0;
 }
-// a.w, a.redo, a.xi, a.ti: what prepare_split made of the weights a.w_raw and of a.x, a.x2 and a.tree_data; a.win_level ... the forward
-// lists of the plan
+// a.w, a.redo: what prepare_split made of the weights a.w_raw; a.win_level ... the forward lists of the plan
 int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
     int rc;
     switch (code) {
@@ -435,16 +470,15 @@ size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck) {
     const int coh = split_coh(Cm);
     return (size_t)S_exp * ((Cm + 16 * coh - 1) / (16 * coh)) * ((Ck + SP_CIB - 1) / SP_CIB) * split_nstep(code) * 3 * coh * 64 * sizeof(uint4);
 }
-// Packed weights, cleared marks and copies of x (x2 from channel c_split on) and of the tree in groups of four channels:
-// [(Ck + 3) / 4][count][4] each.  Fewer than 2^28 elements and 2^32 threads (split_fwd_bytes).
-int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx,
-                  const float* x2, int64_t ldx2, int c_split, int64_t nx, float* xi, const float* tree, int64_t ldt, int64_t nt, float* ti, hipStream_t st) {
+// Packed weights, cleared marks and (xi not null) a copy of x in groups of four channels, [(Ck + 3) / 4][nx][4].  Fewer than 2^28 elements
+// and 2^32 threads (split_dx_bytes).
+int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx, int64_t nx, float* xi,
+                  hipStream_t st) {
     const size_t n = conv_packed_split_bytes(code, S_exp, Cm, Ck) / (3 * sizeof(uint4));
     const unsigned nb = (unsigned)std::min<size_t>((n + PREP_TB - 1) / PREP_TB, 2048), nq = (unsigned)(Ck + SP_CIB - 1) / SP_CIB;
-    const unsigned nbx = (unsigned)((nx + PREP_TB * IG_E - 1) / (PREP_TB * IG_E)), nbt = (unsigned)((nt + PREP_TB * IG_E - 1) / (PREP_TB * IG_E));
-    const SplitCopy fx{x, ldx, x2, ldx2, c_split, nx, (float4*)xi}, ft{tree, ldt, nullptr, 0, Ck, nt, (float4*)ti};
-#define APRNET_PREP(K) hipLaunchKernelGGL(split_prepare_kernel<K>, dim3(nb + nq * (nbx + nbt)), dim3(PREP_TB), 0, st, w, S_exp, Cm, Ck, split_coh(Cm), \
-                                          transposed ? 1 : 0, (uint4*)packed, marks, nb, fx, nbx, ft, nbt)
+    const unsigned nbx = xi ? (unsigned)((nx + PREP_TB * IG_E - 1) / (PREP_TB * IG_E)) : 0;
+#define APRNET_PREP(K) hipLaunchKernelGGL(split_prepare_kernel<K>, dim3(nb + nq * nbx), dim3(PREP_TB), 0, st, w, S_exp, Cm, Ck, split_coh(Cm), \
+                                          transposed ? 1 : 0, (uint4*)packed, marks, nb, x, ldx, nx, (float4*)xi, nbx)
     if (code == 333) APRNET_PREP(27); else APRNET_PREP(25);
 #undef APRNET_PREP
     APRNET_LAUNCH_CHECK("split_prepare_kernel");

@@ -238,7 +238,7 @@ APRNET_DECL(float, f32)
 APRNET_DECL(double, f64)
 
 /* No counterpart in the reference.  Stencil convolutions of fp32 features with an optional work space of the caller, in which the
- * forward pass keeps its packed weights and copies of its input and mean tree in groups of four channels: with at least
+ * forward pass keeps its packed weights (and marks of results that are not finite): with at least
  * aprnet_conv_ws_bytes_f32() bytes (16-byte aligned, contents irrelevant before and after) it multiplies pieces of the fp32 values on the
  * bfloat16 matrix instructions (every value as the exact sum of three bfloat16 numbers, all products above 2^-25 of the result,
  * fp32 sums: against 64 bits a third of the fp32 instructions' error on dense features, less than theirs on sparse ones, but for results

@@ -355,8 +355,13 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
         e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
     }
     const bool dw_pieces = pieces && wl && wl->n_win > 0 && split_dw(a.Cin, a.Cout, a.x_count, a.ldx, a.ldt);
+    // Two kernels on pieces that each fill the chip run one after the other: beside each other they read more past the caches (3x3x3, 9.8 M
+    // particles 32 -> 32 channels 12.6 and, on two streams, 13.8 ms, 16 -> 16 3.98 and 4.08; 1 M 64 -> 64 4.61 and 4.77, 16 -> 16 0.479
+    // and 0.494; on 320 k, 32 -> 32 0.500 and 0.512, 64 -> 64 1.63 and 1.60; on 90 k 16 -> 16 0.140 and 0.134, 64 -> 64 0.670 and 0.627;
+    // 1x5x5 1 M 16 -> 16 0.370 and 0.365, 3.9 M 64 -> 64 12.1 and 12.0).
+    const bool in_turn = dw_pieces && code == 333 && a.x_count >= 1 << 20;
     hipStream_t side = st;
-    if (a.gx) if (int rc = fork_side(p, st, &side)) return rc;
+    if (a.gx && !in_turn) if (int rc = fork_side(p, st, &side)) return rc;
     SideJoin guard(p, st, side);
     if (dw_pieces) {
         c.xi = e.xi; c.xi_ld = e.xi_ld; c.redo = mark + 1;

@@ -8,6 +8,23 @@ from pyapr.aprnet import cuda as aprnet
 from .unet_parts import BasicBlock, ConvBlock, DownConv, UpConv
 
 
+def _submodules(root):
+    """Every module below ``root`` once, as root.modules() has them but in another order: the generators of modules() nest, and its names are
+    made only to be dropped, 0.1 ms for the modules of a network, twice a call."""
+    seen, todo = {root}, [root]
+    while todo:
+        for m in todo.pop()._modules.values():
+            if m is not None and m not in seen:
+                seen.add(m)
+                todo.append(m)
+                yield m
+
+
+def _flag(m, name):
+    # getattr(m, name, True) past Module.__getattr__, which raises and formats an error for every module without the attribute
+    return m.__dict__[name] if name in m.__dict__ else getattr(type(m), name, True)
+
+
 class APRUNet(nn.Module):
     def __init__(self, in_channels, out_channels, depth=3, kernel_size=3, dims=3, activation=nn.ReLU,
                  n_filters_base=16, n_conv_per_block=2, n_stencils=2, decrement_stencils=False, num_groups=None,
@@ -53,13 +70,20 @@ class APRUNet(nn.Module):
         if torch.is_grad_enabled() or not x.is_cuda or x.dtype != torch.bfloat16 or x.size(1) > 3 \
                 or not getattr(self, "use_grouped", True):
             return False
-        blocks = [b for m in self.modules() if isinstance(m, ConvBlock) for b in m.blocks] + [st.reduce_ch for st in self.decoder]
+        blocks = [st.reduce_ch for st in self.decoder]
+        for m in _submodules(self):
+            if isinstance(m, ConvBlock):
+                blocks += m.blocks
+            if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks:
+                return False
+            if _flag(m, "increment_level_deltas") is not True or _flag(m, "decrement_level_deltas") is not True:
+                return False
         limits = grouped.limits()
         for b in blocks:
             if not isinstance(b.norm, nn.Identity) or type(b.activation) is not nn.ReLU:
                 return False
-            s_, cout, cin = b.conv.weight.shape[:3]
-            ks = tuple(b.conv.weight.shape[3:])
+            _, cout, cin, *ks = b.conv.weight.shape
+            ks = tuple(ks)
             if ks not in ((3, 3, 3), (1, 3, 3), (1, 5, 5), (1, 1, 1)) or cout % 8:
                 return False
             if ks == (1, 1, 1) and (cin % 8 or cin > limits["conv111_max_cin"]):
@@ -69,13 +93,6 @@ class APRUNet(nn.Module):
         hw = self.head.weight
         if tuple(hw.shape[3:]) != (1, 1, 1) or hw.shape[2] % 8 or hw.shape[2] > limits["conv111_max_cin"]:
             return False
-        for m in self.modules():
-            if m is self:
-                continue
-            if m._forward_hooks or m._forward_pre_hooks or m._backward_hooks:
-                return False
-            if getattr(m, "increment_level_deltas", True) is not True or getattr(m, "decrement_level_deltas", True) is not True:
-                return False
         return grouped.supported(aprs, [])
 
     def prepare_inference(self, aprs=None, levels=None):
@@ -132,11 +149,12 @@ class APRUNet(nn.Module):
             return _ops.restrict_kernel_forward(conv_module.weight.detach().float().contiguous(), levels), None
 
         def conv(bb, inp, second=None, coarse=None):
-            w = bb.conv.weight.detach().float()
-            bias = None if bb.conv.bias is None else bb.conv.bias.detach()
-            if tuple(w.shape[3:]) == (1, 1, 1):
-                return g8.conv111_forward(aprs, inp, w, level_deltas, bias, relu=True)
-            w, packed = restricted(bb.conv)
+            cm = bb.conv
+            weight, bias = cm.weight, cm.bias
+            bias = None if bias is None else bias.detach()
+            if tuple(weight.shape[3:]) == (1, 1, 1):
+                return g8.conv111_forward(aprs, inp, weight.detach().float(), level_deltas, bias, relu=True)
+            w, packed = restricted(cm)
             return g8.conv_forward(aprs, inp, w, level_deltas, bias, relu=True, x2=second, x2_coarse=coarse, packed=packed)
 
         def block(cb, inp, second=None):

@@ -8,6 +8,7 @@ Weight layouts: the ``cuda`` flavour uses [S, Cout, Cin, kz, kx, ky] (cuda/conv.
 kernels consume; the CPU-flavour names (``convolve333_forward`` ...) take [Cin, S, Cout, kz, kx, ky]
 (conv.py:164) and are permuted on the way in and out.
 """
+import contextlib
 import ctypes as C
 import warnings
 
@@ -65,12 +66,30 @@ def _plans(aprs, device):
     return [a.plan(device.index if device.index is not None else torch.cuda.current_device()) for a in aprs]
 
 
+_stay = contextlib.nullcontext()
+
+
+def _on(device):
+    """torch.cuda.device(device), without its two switches where that is the current device already."""
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index == torch.cuda.current_device():
+        return _stay
+    return torch.cuda.device(device)
+
+
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # the handle alone: torch.cuda.current_stream() makes an object and looks the device up twice, 3 us of a call's host time
+    return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def _ptr(t):
     return C.c_void_p(t.data_ptr())
+
+
+def _at(t, b):
+    """_ptr(t[b]) without the tensor in between"""
+    if b >= t.shape[0]:
+        raise IndexError(f"index {b} is out of bounds for dimension 0 with size {t.shape[0]}")
+    return C.c_void_p(t.data_ptr() + b * t.stride(0) * t.element_size())
 
 
 def _zero_tails(out, sizes):
@@ -115,7 +134,7 @@ def _restrict(weights, n_other, backward):
     s_in, cout, cin, kz, kx, ky = weights.shape
     out = torch.empty((n_other, cout, cin, kz, kx, ky), dtype=weights.dtype, device=weights.device)
     fn = getattr(_lib(), f"aprnet_restrict_kernel_{'bwd' if backward else 'fwd'}_{_sfx(weights)}")
-    with torch.cuda.device(weights.device):
+    with _on(weights.device):
         rc = fn(_ptr(weights), s_in, cout * cin, kz, kx, ky, n_other, _ptr(out), _stream())
     if rc:
         _raise(rc, "restrict_kernel failed")
@@ -203,7 +222,7 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
                 out[b, :, nb:] = (bias.clamp(min=0) if relu else bias).view(-1, 1)
     plans = _plans(aprs, x.device)
     sfx = _sfx(x, bf16=True)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         if sfx == "f32" and pieces and (kz, kx, ky) != (1, 1, 1):
             ld_tree = max(max(tree_parts(a, d[b]) for b, a in enumerate(aprs)), 1)
@@ -211,8 +230,8 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
             tree_ws, ws, ws_bytes = _workspace(cin * ld_tree * 4, max([lib.aprnet_conv_ws_bytes_f32(plans[b], d[b], kz, kx, ky, cin, s_exp, cout)
                                                                        for b in range(B)]), x.device)
             for b in range(B):
-                fu = _Fusion(_ptr(x2[b]) if x2 is not None else None, N, c2, 1 if relu else 0) if fused else None
-                rc = lib.aprnet_conv_fwd_ws_f32(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, c1, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N,
+                fu = _Fusion(_at(x2, b) if x2 is not None else None, N, c2, 1 if relu else 0) if fused else None
+                rc = lib.aprnet_conv_fwd_ws_f32(plans[b], d[b], kz, kx, ky, _at(x, b), N, c1, _ptr(weights), s_exp, cout, bptr, _at(out, b), N,
                                                 _ptr(tree_ws), ld_tree, C.byref(fu) if fused else None, ws, ws_bytes, st)
                 if rc:
                     _raise(rc, "conv_forward failed")
@@ -221,15 +240,15 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
             tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             fn = getattr(_lib(), "aprnet_conv_fwd_fused_" + sfx)
             for b in range(B):
-                fu = _Fusion(_ptr(x2[b]) if x2 is not None else None, N, c2, 1 if relu else 0)
-                rc = fn(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, c1, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N,
+                fu = _Fusion(_at(x2, b) if x2 is not None else None, N, c2, 1 if relu else 0)
+                rc = fn(plans[b], d[b], kz, kx, ky, _at(x, b), N, c1, _ptr(weights), s_exp, cout, bptr, _at(out, b), N,
                         _ptr(tree_ws), ld_tree, C.byref(fu), st)
                 if rc:
                     _raise(rc, "conv_forward failed")
         elif (kz, kx, ky) == (1, 1, 1):
             fn = getattr(_lib(), "aprnet_conv111_fwd_" + sfx)
             for b in range(B):
-                rc = fn(plans[b], d[b], _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N, st)
+                rc = fn(plans[b], d[b], _at(x, b), N, cin, _ptr(weights), s_exp, cout, bptr, _at(out, b), N, st)
                 if rc:
                     _raise(rc, "conv111_forward failed")
         else:
@@ -237,7 +256,7 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
             tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             fn = getattr(_lib(), "aprnet_conv_fwd_" + sfx)
             for b in range(B):
-                rc = fn(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout, bptr, _ptr(out[b]), N,
+                rc = fn(plans[b], d[b], kz, kx, ky, _at(x, b), N, cin, _ptr(weights), s_exp, cout, bptr, _at(out, b), N,
                         _ptr(tree_ws), ld_tree, st)
                 if rc:
                     _raise(rc, "conv_forward failed")
@@ -253,10 +272,10 @@ def channel_sum(x):
     lib = _lib()
     work = torch.empty(lib.aprnet_channel_sum_work_elems(C), dtype=acc, device=x.device)
     fn = getattr(lib, "aprnet_channel_sum_" + _sfx(x, bf16=True))
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         for b in range(B):
-            rc = fn(_ptr(x[b]), N, C, N, _ptr(out), 1 if b else 0, _ptr(work), st)
+            rc = fn(_at(x, b), N, C, N, _ptr(out), 1 if b else 0, _ptr(work), st)
             if rc:
                 _raise(rc, "channel_sum failed")
     return out
@@ -286,7 +305,7 @@ def row_moments(x):
     B, Cn, N = x.shape
     mean = torch.empty(B, Cn, dtype=torch.float64, device=x.device)
     m2 = torch.empty_like(mean)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = getattr(_lib(), "aprnet_row_moments_" + sfx)(_ptr(x), N, B * Cn, N, _ptr(mean), _ptr(m2),
                                                           _ptr(_norm_work(B * Cn, x.device)), _stream())
     if rc:
@@ -320,7 +339,7 @@ def norm_coeffs_forward(shape, groups, eps, row_mean, row_m2, given, gamma, beta
     if given is None:
         sets = [torch.empty(Cn if groups == 0 else (B, groups), dtype=torch.float32, device=device) for _ in range(2)]
     gamma, beta = _f32_or_none(gamma, Cn, "weight"), _f32_or_none(beta, Cn, "bias")
-    with torch.cuda.device(device):
+    with _on(device):
         rc = _lib().aprnet_norm_coeffs_fwd(B, Cn, groups, N, float(eps), _optr(row_mean), _optr(row_m2), _optr(gm), _optr(gv),
                                            _optr(gamma), _optr(beta), *[_ptr(t) for t in out],
                                            _optr(sets[0] if sets else None), _optr(sets[1] if sets else None), _stream())
@@ -337,7 +356,7 @@ def norm_coeffs_backward(shape, groups, own_stats, sum_g, sum_gx, gamma, rstd32,
     gg = torch.empty(Cn, dtype=torch.float32, device=dev) if want_gamma else None
     gb = torch.empty(Cn, dtype=torch.float32, device=dev) if want_beta else None
     gamma = _f32_or_none(gamma, Cn, "weight")
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _lib().aprnet_norm_coeffs_bwd(B, Cn, groups, N, 1 if own_stats else 0, _ptr(sum_g), _ptr(sum_gx), _optr(gamma),
                                            _ptr(_rowvec(rstd32, B * Cn, "rstd")), _ptr(a), _ptr(b), _ptr(c), _optr(gg), _optr(gb),
                                            _stream())
@@ -351,7 +370,7 @@ def norm_apply(x, mean, scale, shift, relu):
     sfx = _norm_sfx(x, "input")
     B, Cn, N = x.shape
     y = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = getattr(_lib(), "aprnet_norm_apply_" + sfx)(_ptr(x), N, B * Cn, N, _ptr(_rowvec(mean, B * Cn, "mean")),
                                                          _ptr(_rowvec(scale, B * Cn, "scale")), _ptr(_rowvec(shift, B * Cn, "shift")),
                                                          1 if relu else 0, _ptr(y), N, _stream())
@@ -369,7 +388,7 @@ def norm_backward_sums(gy, x, y, mean, rstd):
     B, Cn, N = x.shape
     s_g = torch.empty(B, Cn, dtype=torch.float64, device=x.device)
     s_gx = torch.empty_like(s_g)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = getattr(_lib(), "aprnet_norm_bwd_sums_" + sfx)(_ptr(gy), N, _ptr(x), N, None if y is None else _ptr(y), N, B * Cn, N,
                                                             _ptr(_rowvec(mean, B * Cn, "mean")), _ptr(_rowvec(rstd, B * Cn, "rstd")),
                                                             _ptr(s_g), _ptr(s_gx), _ptr(_norm_work(B * Cn, x.device)), _stream())
@@ -387,7 +406,7 @@ def norm_backward_apply(gy, x, y, mean, rstd, a, b, c):
     B, Cn, N = x.shape
     gx = torch.empty_like(x)
     rows = B * Cn
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         rc = getattr(_lib(), "aprnet_norm_bwd_apply_" + sfx)(_ptr(gy), N, _ptr(x), N, None if y is None else _ptr(y), N, rows, N,
                                                              _ptr(_rowvec(mean, rows, "mean")), _ptr(_rowvec(rstd, rows, "rstd")),
                                                              _ptr(_rowvec(a, rows, "a")), _ptr(_rowvec(b, rows, "b")),
@@ -413,7 +432,7 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
     gx = None if skip_gx else torch.empty_like(x)
     if gx is not None:
         _zero_tails(gx, sizes)
-    gxp = (lambda b: None) if skip_gx else (lambda b: _ptr(gx[b]))
+    gxp = (lambda b: None) if skip_gx else (lambda b: _at(gx, b))
     plans = _plans(aprs, x.device)
     if x.dtype == torch.bfloat16:
         # bfloat16 features and output gradient; weights and their gradient in fp32, fp32 accumulation
@@ -422,11 +441,11 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
         weights = weights.float()
         gw = torch.zeros_like(weights)
         if (kz, kx, ky) == (1, 1, 1):
-            with torch.cuda.device(x.device):
+            with _on(x.device):
                 st = _stream()
                 for b in range(B):
-                    rc = _lib().aprnet_conv111_bwd_bf16(plans[b], d[b], _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout,
-                                                        _ptr(grad_output[b]), grad_output.size(2), _ptr(gx[b]), N, _ptr(gw), st)
+                    rc = _lib().aprnet_conv111_bwd_bf16(plans[b], d[b], _at(x, b), N, cin, _ptr(weights), s_exp, cout,
+                                                        _at(grad_output, b), grad_output.size(2), _at(gx, b), N, _ptr(gw), st)
                     if rc:
                         _raise(rc, "conv111_backward failed")
             return [gx, gw]
@@ -434,11 +453,11 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
         tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
         gtree_ws = None if skip_gx else torch.empty((cin, ld_tree), dtype=torch.float32, device=x.device)
         gx32_ws = None if skip_gx else torch.empty((cin, N), dtype=torch.float32, device=x.device)
-        with torch.cuda.device(x.device):
+        with _on(x.device):
             st = _stream()
             for b in range(B):
-                rc = _lib().aprnet_conv_bwd_bf16(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout,
-                                                 _ptr(grad_output[b]), grad_output.size(2), gxp(b), N, _ptr(gw),
+                rc = _lib().aprnet_conv_bwd_bf16(plans[b], d[b], kz, kx, ky, _at(x, b), N, cin, _ptr(weights), s_exp, cout,
+                                                 _at(grad_output, b), grad_output.size(2), gxp(b), N, _ptr(gw),
                                                  _ptr(tree_ws), ld_tree, None if skip_gx else _ptr(gx32_ws), N,
                                                  None if skip_gx else _ptr(gtree_ws), ld_tree, st)
                 if rc:
@@ -446,13 +465,13 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
         return [gx, gw]
     gw = torch.zeros_like(weights)
     sfx = _sfx(x)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         if (kz, kx, ky) == (1, 1, 1):
             fn = getattr(_lib(), "aprnet_conv111_bwd_" + sfx)
             for b in range(B):
-                rc = fn(plans[b], d[b], _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout, _ptr(grad_output[b]),
-                        grad_output.size(2), _ptr(gx[b]), N, _ptr(gw), st)
+                rc = fn(plans[b], d[b], _at(x, b), N, cin, _ptr(weights), s_exp, cout, _at(grad_output, b),
+                        grad_output.size(2), _at(gx, b), N, _ptr(gw), st)
                 if rc:
                     _raise(rc, "conv111_backward failed")
         else:
@@ -466,8 +485,8 @@ def conv_backward(aprs, x, weights, grad_output, level_delta, need_input_grad=Tr
             else:
                 tree_ws = torch.empty((cin, ld_tree), dtype=x.dtype, device=x.device)
             for b in range(B):
-                rc = fn(plans[b], d[b], kz, kx, ky, _ptr(x[b]), N, cin, _ptr(weights), s_exp, cout,
-                        _ptr(grad_output[b]), grad_output.size(2), gxp(b), N, _ptr(gw),
+                rc = fn(plans[b], d[b], kz, kx, ky, _at(x, b), N, cin, _ptr(weights), s_exp, cout,
+                        _at(grad_output, b), grad_output.size(2), gxp(b), N, _ptr(gw),
                         _ptr(tree_ws), ld_tree, None if skip_gx else _ptr(gtree_ws), ld_tree, *extra, st)
                 if rc:
                     _raise(rc, "conv_backward failed")
@@ -492,10 +511,10 @@ def maxpool_forward(aprs, x, level_delta, pad_value=-1e17):
             idx[b, :, nb:] = 0
     plans = _plans(aprs, x.device)
     fn = getattr(_lib(), "aprnet_maxpool_fwd_" + _sfx(x, bf16=True))
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(x[b]), N, Cn, _ptr(out[b]), n_out, _ptr(idx[b]), n_out, st)
+            rc = fn(plans[b], d[b], _at(x, b), N, Cn, _at(out, b), n_out, _at(idx, b), n_out, st)
             if rc:
                 _raise(rc, "maxpool_forward failed")
     return [out, idx]
@@ -512,10 +531,10 @@ def maxpool_backward(aprs, grad_output, max_indices, level_delta):
     _zero_tails(gx, sizes)
     plans = _plans(aprs, grad_output.device)
     fn = getattr(_lib(), "aprnet_maxpool_bwd_" + _sfx(grad_output, bf16=True))
-    with torch.cuda.device(grad_output.device):
+    with _on(grad_output.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(grad_output[b]), n_out, Cn, _ptr(gx[b]), n_in, _ptr(max_indices[b]),
+            rc = fn(plans[b], d[b], _at(grad_output, b), n_out, Cn, _at(gx, b), n_in, _at(max_indices, b),
                     max_indices.size(2), st)
             if rc:
                 _raise(rc, "maxpool_backward failed")
@@ -536,10 +555,10 @@ def upsample_const_forward(aprs, x, level_delta):
     _zero_tails(out, sizes)
     plans = _plans(aprs, x.device)
     fn = getattr(_lib(), "aprnet_upsample_fwd_" + _sfx(x, bf16=True))
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(x[b]), N, Cn, _ptr(out[b]), n_out, st)
+            rc = fn(plans[b], d[b], _at(x, b), N, Cn, _at(out, b), n_out, st)
             if rc:
                 _raise(rc, "upsample_const_forward failed")
     return out
@@ -555,10 +574,10 @@ def upsample_const_backward(aprs, grad_output, level_delta):
     _zero_tails(gx, sizes)
     plans = _plans(aprs, grad_output.device)
     fn = getattr(_lib(), "aprnet_upsample_bwd_" + _sfx(grad_output, bf16=True))
-    with torch.cuda.device(grad_output.device):
+    with _on(grad_output.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(grad_output[b]), n_out, Cn, _ptr(gx[b]), n_in, st)
+            rc = fn(plans[b], d[b], _at(grad_output, b), n_out, Cn, _at(gx, b), n_in, st)
             if rc:
                 _raise(rc, "upsample_const_backward failed")
     return gx
@@ -592,10 +611,10 @@ def reconstruct_forward(aprs, x, level_delta):
     plane = shape[0] * shape[1] * shape[2]
     plans = _plans(aprs, x.device)
     fn = getattr(_lib(), "aprnet_reconstruct_fwd_" + _sfx(x, bf16=True))
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(x[b]), N, Cn, _ptr(out[b]), plane, st)
+            rc = fn(plans[b], d[b], _at(x, b), N, Cn, _at(out, b), plane, st)
             if rc:
                 _raise(rc, "reconstruct_forward failed")
     return out
@@ -613,10 +632,10 @@ def reconstruct_backward(aprs, grad_output, level_delta):
     plane = grad_output[0, 0].numel()
     plans = _plans(aprs, grad_output.device)
     fn = getattr(_lib(), "aprnet_reconstruct_bwd_" + _sfx(grad_output, bf16=True))
-    with torch.cuda.device(grad_output.device):
+    with _on(grad_output.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(grad_output[b]), plane, Cn, _ptr(gx[b]), n, st)
+            rc = fn(plans[b], d[b], _at(grad_output, b), plane, Cn, _at(gx, b), n, st)
             if rc:
                 _raise(rc, "reconstruct_backward failed")
     return gx
@@ -635,10 +654,10 @@ def sample_particles_forward(aprs, img, level_delta):
     plane = img[0, 0].numel()
     plans = _plans(aprs, img.device)
     fn = getattr(_lib(), "aprnet_sample_particles_fwd_" + _sfx(img, bf16=True))
-    with torch.cuda.device(img.device):
+    with _on(img.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(img[b]), plane, Cn, _ptr(out[b]), n, st)
+            rc = fn(plans[b], d[b], _at(img, b), plane, Cn, _at(out, b), n, st)
             if rc:
                 _raise(rc, "sample_particles_forward failed")
     return out
@@ -654,10 +673,10 @@ def sample_particles_backward(aprs, grad_output, level_delta):
     plane = shape[0] * shape[1] * shape[2]
     plans = _plans(aprs, grad_output.device)
     fn = getattr(_lib(), "aprnet_sample_particles_bwd_" + _sfx(grad_output, bf16=True))
-    with torch.cuda.device(grad_output.device):
+    with _on(grad_output.device):
         st = _stream()
         for b in range(B):
-            rc = fn(plans[b], d[b], _ptr(grad_output[b]), N, Cn, _ptr(gimg[b]), plane, st)
+            rc = fn(plans[b], d[b], _at(grad_output, b), N, Cn, _at(gimg, b), plane, st)
             if rc:
                 _raise(rc, "sample_particles_backward failed")
     return gimg

@@ -9,7 +9,7 @@ import ctypes as C
 import torch
 
 from . import _ops
-from ._ops import _check_input, _deltas, _lib, _plans, _ptr, _raise, _stream, number_particles, tree_parts
+from ._ops import _at, _check_input, _deltas, _lib, _on, _plans, _ptr, _raise, _stream, number_particles, tree_parts
 
 MAX_PARTICLES = (1 << 31) - 1
 
@@ -47,10 +47,10 @@ def regroup(x):
         raise TypeError("grouped features are bfloat16")
     B, Cn, N = x.shape
     out = torch.empty((B, (Cn + 7) // 8, N, 8), dtype=x.dtype, device=x.device)
-    with torch.cuda.device(x.device):
+    with _on(x.device):
         st = _stream()
         for b in range(B):
-            rc = _lib().aprnet_regroup8_bf16(_ptr(x[b]), N, Cn, N, _ptr(out[b]), N, st)
+            rc = _lib().aprnet_regroup8_bf16(_at(x, b), N, Cn, N, _at(out, b), N, st)
             if rc:
                 _raise(rc, "regroup failed")
     return Grouped(out)
@@ -61,21 +61,21 @@ def ungroup(g, channels=None):
     B, G, N, _ = g.data.shape
     Cn = channels or G * 8
     out = torch.empty((B, Cn, N), dtype=g.data.dtype, device=g.data.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         st = _stream()
         for b in range(B):
-            rc = _lib().aprnet_ungroup8_bf16(_ptr(g.data[b]), N, Cn, N, _ptr(out[b]), N, st)
+            rc = _lib().aprnet_ungroup8_bf16(_at(g.data, b), N, Cn, N, _at(out, b), N, st)
             if rc:
                 _raise(rc, "ungroup failed")
     return out
 
 
 def _fusion(x2, b, N, c2, relu, x2_coarse):
-    fu = _ops._Fusion(_ptr(x2.data[b]) if x2 is not None else None, N, c2, 1 if relu else 0)
+    fu = _ops._Fusion(_at(x2.data, b) if x2 is not None else None, N, c2, 1 if relu else 0)
     if x2_coarse is not None:
         if x2 is None or x2_coarse.channels != c2 or x2_coarse.data.shape[0] != x2.data.shape[0]:
             raise ValueError("x2_coarse goes with a second input of the same batch size and channel count")
-        fu.x2_coarse, fu.ld_coarse = _ptr(x2_coarse.data[b]), x2_coarse.data.shape[2]
+        fu.x2_coarse, fu.ld_coarse = _at(x2_coarse.data, b), x2_coarse.data.shape[2]
     return fu
 
 
@@ -88,7 +88,7 @@ def pack_weights(weights):
         return None
     _check_input(weights, "weights")
     out = torch.empty(nbytes, dtype=torch.uint8, device=weights.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         rc = _lib().aprnet_conv_pack_bf16(kz, kx, ky, _ptr(weights), s_exp, cout, cin, _ptr(out), _stream())
         if rc:
             _raise(rc, "conv_pack failed")
@@ -144,12 +144,12 @@ def conv_forward(aprs, x, weights, level_delta, bias=None, relu=False, x2=None, 
     tree_ws = torch.empty((cin if planes_in else cin // 8, ld_tree, 1 if planes_in else 8), dtype=torch.bfloat16, device=xd.device)
     plans = _plans(aprs, xd.device)
     image = None if planes_in else _image(packed, weights, xd.device)
-    with torch.cuda.device(xd.device):
+    with _on(xd.device):
         st = _stream()
         for b in range(B):
             fu = _fusion(x2, b, N, c2, relu, x2_coarse)
-            rc = _lib().aprnet_conv_fwd_packed_bf16l(plans[b], d[b], kz, kx, ky, _ptr(xd[b]), N, c1, 0 if planes_in else 1, _ptr(weights),
-                                                     image, s_exp, cout, None if bias is None else _ptr(bias), _ptr(out[b]), N,
+            rc = _lib().aprnet_conv_fwd_packed_bf16l(plans[b], d[b], kz, kx, ky, _at(xd, b), N, c1, 0 if planes_in else 1, _ptr(weights),
+                                                     image, s_exp, cout, None if bias is None else _ptr(bias), _at(out, b), N,
                                                     1 if grouped_output else 0, _ptr(tree_ws), ld_tree, C.byref(fu), st)
             if rc:
                 _raise(rc, "conv_forward failed")
@@ -193,13 +193,13 @@ def conv_head_forward(aprs, x, weights, level_delta, bias, head_weights, head_bi
     tree_ws = torch.empty((cin // 8, ld_tree, 8), dtype=torch.bfloat16, device=out.device)
     plans = _plans(aprs, out.device)
     image = _image(packed, weights, out.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         st = _stream()
         for b in range(B):
             fu = _fusion(x2, b, N, c2, relu, x2_coarse)
-            rc = _lib().aprnet_conv_fwd_head_packed_bf16g(plans[b], d[b], kz, kx, ky, _ptr(x.data[b]), N, c1, _ptr(weights), image, s_exp, cout,
+            rc = _lib().aprnet_conv_fwd_head_packed_bf16g(plans[b], d[b], kz, kx, ky, _at(x.data, b), N, c1, _ptr(weights), image, s_exp, cout,
                                                    None if bias is None else _ptr(bias), _ptr(tree_ws), ld_tree, C.byref(fu),
-                                                   _ptr(hw), hs, hc, None if hb is None else _ptr(hb), _ptr(out[b]), N, st)
+                                                   _ptr(hw), hs, hc, None if hb is None else _ptr(hb), _at(out, b), N, st)
             if rc:
                 _raise(rc, "conv_head_forward failed")
     return out
@@ -228,11 +228,11 @@ def conv111_forward(aprs, x, weights, level_delta, bias=None, relu=False, groupe
             else:
                 out[b, :, nb:] = pad.to(torch.bfloat16).view(-1, 1)
     plans = _plans(aprs, out.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         st = _stream()
         for b in range(B):
-            rc = _lib().aprnet_conv111_fwd_bf16g(plans[b], d[b], _ptr(x.data[b]), N, cin, _ptr(weights), s, cout,
-                                                 None if bias is None else _ptr(bias), 1 if relu else 0, _ptr(out[b]), N,
+            rc = _lib().aprnet_conv111_fwd_bf16g(plans[b], d[b], _at(x.data, b), N, cin, _ptr(weights), s, cout,
+                                                 None if bias is None else _ptr(bias), 1 if relu else 0, _at(out, b), N,
                                                  1 if grouped_output else 0, st)
             if rc:
                 _raise(rc, "conv111_forward failed")
@@ -250,10 +250,10 @@ def maxpool_forward(aprs, x, level_delta):
         if nb < n_out:
             out[b, :, nb:, :] = 0
     plans = _plans(aprs, out.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         st = _stream()
         for b in range(B):
-            rc = _lib().aprnet_maxpool_fwd_bf16g(plans[b], d[b], _ptr(x.data[b]), N, G * 8, _ptr(out[b]), n_out, st)
+            rc = _lib().aprnet_maxpool_fwd_bf16g(plans[b], d[b], _at(x.data, b), N, G * 8, _at(out, b), n_out, st)
             if rc:
                 _raise(rc, "maxpool_forward failed")
     return Grouped(out)
@@ -271,10 +271,10 @@ def upsample_const_forward(aprs, x, level_delta):
         if nb < n_out:
             out[b, :, nb:, :] = 0
     plans = _plans(aprs, out.device)
-    with torch.cuda.device(out.device):
+    with _on(out.device):
         st = _stream()
         for b in range(B):
-            rc = _lib().aprnet_upsample_fwd_bf16g(plans[b], d[b], _ptr(x.data[b]), N, G * 8, _ptr(out[b]), n_out, st)
+            rc = _lib().aprnet_upsample_fwd_bf16g(plans[b], d[b], _at(x.data, b), N, G * 8, _at(out, b), n_out, st)
             if rc:
                 _raise(rc, "upsample_const_forward failed")
     return Grouped(out)

@@ -35,6 +35,19 @@ __device__ __forceinline__ uint4* g8_at(bf16_t* base, int64_t ld, int q, int64_t
     return reinterpret_cast<uint4*>(base) + (int64_t)q * ld + i;
 }
 
+// Groups of a thread in the kernels that walk the child table: all of them, so that the table is read once, halved while fewer than SPLIT_THREADS
+// threads would remain (the chip holds 2^19 at a time).  A thread's groups are a serial chain, each waiting for its own loads: in a network of 16 to
+// 128 channels on 1.3 M particles a fill took 8.3 us with one thread for all groups and 5.1 split, a pool 11.8 and 7.6, an upsample 9.5 and
+// 8.0, the network 0.92 and 0.835 ms.  Limits of 2^17, 2^18, 2^20, 2^21: 0.842, 0.835, 0.842, 0.839, and on 210 M particles 53.7, 53.7,
+// 54.0, 53.9 ms (2^19: 53.7).
+constexpr int64_t SPLIT_THREADS = (int64_t)1 << 19;
+static int groups_per_thread(int64_t n, int G) {
+    int gpt = G;
+    if (G > 65535) return gpt;          // a grid's second dimension
+    while (gpt > 1 && n * ((G + gpt - 1) / gpt) < SPLIT_THREADS) gpt = (gpt + 1) / 2;
+    return gpt;
+}
+
 // ---------------------------------------------------------------------------- planes <-> groups
 // out[q][i][c] = x[8 q + c][i]; channels past C read as zeros
 __global__ void regroup8_kernel(const bf16_t* __restrict__ x, int64_t ldx, int C, int64_t n, bf16_t* __restrict__ out, int64_t ldo) {
@@ -98,21 +111,22 @@ __device__ __forceinline__ void fill_node_g8(const int32_t* children, int64_t n_
 
 __global__ void __launch_bounds__(GTB)
 fill_tree_level_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t t_begin, int64_t t_end, const bf16_t* __restrict__ x,
-                          int64_t ldx, bf16_t* __restrict__ tree, int64_t ldt, int64_t tree_off, int from_x, int tree_first, int G) {
+                          int64_t ldx, bf16_t* __restrict__ tree, int64_t ldt, int64_t tree_off, int from_x, int tree_first, int G, int gpt) {
     const int64_t t = t_begin + (int64_t)blockIdx.x * GTB + threadIdx.x;
     if (t >= t_end) return;
-    for (int q = 0; q < G; ++q) fill_node_g8(children, n_tree, t, x, ldx, tree, ldt, tree_off, from_x, tree_first, q);
+    const int q1 = min(G, ((int)blockIdx.y + 1) * gpt);
+    for (int q = blockIdx.y * gpt; q < q1; ++q) fill_node_g8(children, n_tree, t, x, ldx, tree, ldt, tree_off, from_x, tree_first, q);
 }
 
 __global__ void __launch_bounds__(GTB)
 fill_tree_list_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, const int32_t* __restrict__ nodes, int64_t count,
                          const bf16_t* __restrict__ x, int64_t ldx, bf16_t* __restrict__ tree, int64_t ldt, int64_t tree_off, int from_x,
-                         int tree_first, int G) {
+                         int tree_first, int G, int gpt) {
     const int64_t i = (int64_t)blockIdx.x * GTB + threadIdx.x;
     if (i >= count) return;
     const int64_t t = nodes[i];
-    // every channel group of the node in one thread: the list entry and the child table are read once
-    for (int q = 0; q < G; ++q) fill_node_g8(children, n_tree, t, x, ldx, tree, ldt, tree_off, from_x, tree_first, q);
+    const int q1 = min(G, ((int)blockIdx.y + 1) * gpt);
+    for (int q = blockIdx.y * gpt; q < q1; ++q) fill_node_g8(children, n_tree, t, x, ldx, tree, ldt, tree_off, from_x, tree_first, q);
 }
 
 constexpr int G_MAX_COARSE = 12;
@@ -199,13 +213,16 @@ int fill_tree_mean_g8(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx,
         if (e <= b) continue;
         const int from_x = (l + 1 == Lc);
         if (need && need->cnt[l] == 0) continue;
+        const int64_t n = need && !need->whole[l] ? need->cnt[l] : e - b;
+        const int gpt = groups_per_thread(n, G);
+        const dim3 grid((unsigned)((n + GTB - 1) / GTB), (unsigned)((G + gpt - 1) / gpt));
         if (need && !need->whole[l])
-            hipLaunchKernelGGL(fill_tree_list_g8_kernel, dim3((unsigned)((need->cnt[l] + GTB - 1) / GTB)), dim3(GTB), 0, st,
+            hipLaunchKernelGGL(fill_tree_list_g8_kernel, grid, dim3(GTB), 0, st,
                                p->d_children, p->n_tree, need->d_nodes + need->off[l], need->cnt[l], x, ldx, tree, ldt,
-                               from_x ? p->tree_offset(Lc) : 0, from_x, from_x && !particles_first, G);
+                               from_x ? p->tree_offset(Lc) : 0, from_x, from_x && !particles_first, G, gpt);
         else
-            hipLaunchKernelGGL(fill_tree_level_g8_kernel, dim3((unsigned)((e - b + GTB - 1) / GTB)), dim3(GTB), 0, st, p->d_children,
-                               p->n_tree, b, e, x, ldx, tree, ldt, from_x ? p->tree_offset(Lc) : 0, from_x, from_x && !particles_first, G);
+            hipLaunchKernelGGL(fill_tree_level_g8_kernel, grid, dim3(GTB), 0, st, p->d_children,
+                               p->n_tree, b, e, x, ldx, tree, ldt, from_x ? p->tree_offset(Lc) : 0, from_x, from_x && !particles_first, G, gpt);
     }
     int l_read = p->tree.level_min;          // with a need list: down to the coarsest level that is read (see fill_tree_mean_needed)
     if (need) while (l_read <= l_coarse && need->cnt[l_read] == 0) ++l_read;
@@ -256,18 +273,19 @@ int tree_of_upsampled_g8(const aprnet_plan* p, int d, const bf16_t* z, int64_t l
 // downsampled particles, strict >, start value -1e17 (maxpool.hpp:51, 88-143).
 __global__ void __launch_bounds__(GTB)
 maxpool_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t n_copy, int64_t n_out, int64_t t_begin,
-                  const bf16_t* __restrict__ x, int64_t ldx, int G, bf16_t* __restrict__ y, int64_t ldy, int64_t in_tree_off) {
+                  const bf16_t* __restrict__ x, int64_t ldx, int G, int gpt, bf16_t* __restrict__ y, int64_t ldy, int64_t in_tree_off) {
     const int64_t i = (int64_t)blockIdx.x * GTB + threadIdx.x;
     if (i >= n_out) return;
+    const int q0 = blockIdx.y * gpt, q1 = min(G, q0 + gpt);
     if (i < n_copy) {
-        for (int q = 0; q < G; ++q) *g8_at(y, ldy, q, i) = *g8_at(x, ldx, q, i);
+        for (int q = q0; q < q1; ++q) *g8_at(y, ldy, q, i) = *g8_at(x, ldx, q, i);
         return;
     }
     const int64_t t = t_begin + (i - n_copy);
-    int32_t ch[8];                        // read once for all channel groups
+    int32_t ch[8];                        // read once for the groups of the thread
 #pragma unroll
     for (int s = 0; s < 8; ++s) ch[s] = children[(int64_t)s * n_tree + t];
-    for (int q = 0; q < G; ++q) {
+    for (int q = q0; q < q1; ++q) {
         uint4 raw[8];                     // unconditional loads, as in fill_node_g8
 #pragma unroll
         for (int s = 0; s < 8; ++s)
@@ -294,11 +312,12 @@ maxpool_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t 
 // in memory, so the lanes of a wave write whole lines (one lane per parent would fill every other 16 bytes of them).
 __global__ void __launch_bounds__(GTB)
 upsample_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t n_copy, int64_t n_in, int64_t t_begin,
-                   const bf16_t* __restrict__ src, int64_t lds, int G, bf16_t* __restrict__ dst, int64_t ldd, int64_t out_tree_off) {
+                   const bf16_t* __restrict__ src, int64_t lds, int G, int gpt, bf16_t* __restrict__ dst, int64_t ldd, int64_t out_tree_off) {
     const int64_t j = (int64_t)blockIdx.x * GTB + threadIdx.x;
     const int64_t n_par = n_in - n_copy;
+    const int q0 = blockIdx.y * gpt, q1 = min(G, q0 + gpt);
     if (j < n_copy) {                     // copied positions: one lane each
-        for (int q = 0; q < G; ++q) *g8_at(dst, ldd, q, j) = *g8_at(src, lds, q, j);
+        for (int q = q0; q < q1; ++q) *g8_at(dst, ldd, q, j) = *g8_at(src, lds, q, j);
         return;
     }
     const int64_t k = j - n_copy;
@@ -311,7 +330,7 @@ upsample_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t
         const int32_t c = children[(int64_t)(2 * p + dy) * n_tree + t];
         at[p] = c >= 0 ? (int64_t)c : (c != NO_CHILD ? out_tree_off + ~c : -1);
     }
-    for (int q = 0; q < G; ++q) {
+    for (int q = q0; q < q1; ++q) {
         const uint4 v = *g8_at(src, lds, q, i);
 #pragma unroll
         for (int p = 0; p < 4; ++p)
@@ -542,8 +561,9 @@ int aprnet_maxpool_fwd_bf16g(const aprnet_plan* p, int d, const uint16_t* x, int
     if (C <= 0 || n_out <= 0) return 0;
     if (ldy < n_out || ldx < p->number_parts(d)) return fail(APRNET_ERR_INVALID_ARGUMENT, "maxpool_forward: row shorter than the particle count");
     APRNET_HIP_CHECK(hipSetDevice(p->device));
-    hipLaunchKernelGGL(maxpool_g8_kernel, dim3((unsigned)((n_out + GTB - 1) / GTB)), dim3(GTB), 0, (hipStream_t)st,
-                       p->d_children, p->n_tree, n_copy, n_out, p->tree.level_begin(Lc - 1), (const bf16_t*)x, ldx, C / 8, (bf16_t*)y, ldy,
+    const int G = C / 8, gpt = groups_per_thread(n_out, G);
+    hipLaunchKernelGGL(maxpool_g8_kernel, dim3((unsigned)((n_out + GTB - 1) / GTB), (unsigned)((G + gpt - 1) / gpt)), dim3(GTB), 0, (hipStream_t)st,
+                       p->d_children, p->n_tree, n_copy, n_out, p->tree.level_begin(Lc - 1), (const bf16_t*)x, ldx, G, gpt, (bf16_t*)y, ldy,
                        p->tree_offset(Lc));
     APRNET_LAUNCH_CHECK("maxpool_g8_kernel");
     return 0;
@@ -558,8 +578,9 @@ int aprnet_upsample_fwd_bf16g(const aprnet_plan* p, int d, const uint16_t* x, in
     if (ldx < n_in || ldy < p->number_parts(d - 1)) return fail(APRNET_ERR_INVALID_ARGUMENT, "upsample_const_forward: row shorter than the particle count");
     APRNET_HIP_CHECK(hipSetDevice(p->device));
     const int64_t n_thr = n_copy + 2 * (n_in - n_copy);
-    hipLaunchKernelGGL(upsample_g8_kernel, dim3((unsigned)((n_thr + GTB - 1) / GTB)), dim3(GTB), 0, (hipStream_t)st,
-                       p->d_children, p->n_tree, n_copy, n_in, p->tree.level_begin(Lc), (const bf16_t*)x, ldx, C / 8, (bf16_t*)y, ldy,
+    const int G = C / 8, gpt = groups_per_thread(n_thr, G);
+    hipLaunchKernelGGL(upsample_g8_kernel, dim3((unsigned)((n_thr + GTB - 1) / GTB), (unsigned)((G + gpt - 1) / gpt)), dim3(GTB), 0, (hipStream_t)st,
+                       p->d_children, p->n_tree, n_copy, n_in, p->tree.level_begin(Lc), (const bf16_t*)x, ldx, G, gpt, (bf16_t*)y, ldy,
                        p->tree_offset(Lc + 1));
     APRNET_LAUNCH_CHECK("upsample_g8_kernel");
     return 0;

@@ -56,6 +56,25 @@ def test_tree_fill_pool_upsample_equal_the_plane_kernels():
     assert torch.equal(g8.ungroup(up), _ops.upsample_const_forward(aprs, ref, ld + 1))
 
 
+@pytest.mark.parametrize("groups", [1, 3, 5, 61], ids=["one", "three", "five", "several-per-thread"])
+def test_channel_groups_split_over_threads(groups):
+    """One group per thread where nodes are few, several (a last thread with fewer) where nodes x groups fill the chip."""
+    C = 8 * groups
+    aprs, ld = [apr_cases.random_apr((96, 96, 96), 21, 0.5) if groups > 8 else apr_cases.get("3d_s")], torch.zeros(1, dtype=torch.int32)
+    x = torch.randn(1, C, aprs[0].total_number_particles(), device=DEV).to(torch.bfloat16)
+    g = g8.regroup(x)
+    lib, st = _native.hip(), torch.cuda.current_stream().cuda_stream
+    nt, n = _ops.tree_parts(aprs[0], 0), x.shape[2]
+    tp = torch.zeros(C, nt, dtype=torch.bfloat16, device=DEV)
+    tg = torch.zeros(groups, nt, 8, dtype=torch.bfloat16, device=DEV)
+    assert lib.aprnet_fill_tree_mean_bf16(aprs[0].plan(0), 0, x[0].data_ptr(), n, C, tp.data_ptr(), nt, st) == 0
+    assert lib.aprnet_fill_tree_mean_bf16g(aprs[0].plan(0), 0, g.data[0].data_ptr(), n, C, tg.data_ptr(), nt, st) == 0
+    assert torch.equal(tg.permute(0, 2, 1).reshape(C, nt), tp)
+    pooled, (ref, _) = g8.maxpool_forward(aprs, g, ld), _ops.maxpool_forward(aprs, x, ld, 0.0)
+    assert torch.equal(g8.ungroup(pooled), ref)
+    assert torch.equal(g8.ungroup(g8.upsample_const_forward(aprs, pooled, ld + 1)), _ops.upsample_const_forward(aprs, ref, ld + 1))
+
+
 @pytest.mark.parametrize("ksize", [(3, 3, 3), (1, 3, 3), (1, 5, 5)], ids=["333", "133", "155"])
 @pytest.mark.parametrize("c1,c2,cout", [(16, 0, 16), (8, 24, 40), (32, 0, 8), (32, 32, 64), (64, 0, 72), (8, 0, 16)])
 def test_grouped_convolution_equals_the_plane_kernel(c1, c2, cout, ksize):

@@ -535,9 +535,8 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
     const bool flat = (kz == 1);
     TileList tl, near;
     if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &tl, st)) return rc;
-    NeedLists need_store;            // (a regrouped copy carries the unfilled nodes along unread)
+    NeedLists need_store;
     const NeedLists* nodes = needed_nodes(p, d, code, tl, st, &need_store);
-    if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, nodes)) return rc;
     if (int rc = get_tiles(p, d, flat ? 1 : 2, flat ? 8 : 4, &near, st, 1)) return rc;
     bool g4 = false;                 // the work spaces hold groups of four channels (grad_groups.hip)
     if (tl.n > 0) {
@@ -575,8 +574,9 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         const size_t wbytes = near.n == 0 ? 0 : align(b.win_level ? conv_packed_bf16_bytes(code, S_exp, Cin, Cout)
                                                                  : conv_packed_floats(code, S_exp, Cin, Cout, true) * sizeof(float));
         const size_t gybytes = align(ngo * (size_t)np * 16);
-        const int chunk = gx ? dw_copy_channels(Cin, np, nt, gybytes) : (Cin + 15) / 16 * 16;
-        const size_t ngc = std::min<size_t>(ngi, chunk / 8), xbytes = align(ngc * (size_t)np * 16), tbytes = align(ngc * (size_t)nt * 16);
+        const bool tree_g8 = tree_ws_grouped(Cin, tree_ws);          // the tree is made of the regrouped features, in its work space
+        const int chunk = gx ? dw_copy_channels(Cin, np, tree_g8 ? 0 : nt, gybytes) : (Cin + 15) / 16 * 16;
+        const size_t ngc = std::min<size_t>(ngi, chunk / 8), xbytes = align(ngc * (size_t)np * 16), tbytes = tree_g8 ? 0 : align(ngc * (size_t)nt * 16);
         const bool regroup = bf16_math() && bf16_regroup() && np < (1ll << 28) && nt < (1ll << 28);
         const bool regroup_gy = regroup && gybytes <= ((size_t)32 << 30);
         WinLists wl;
@@ -603,6 +603,8 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
             if (rc) return rc;
         }
         if (pbytes && !dw_g8) set_dw_partials(p, need, code, a);
+        if (!dw_g8 || !tree_g8)
+            if (int rc = fill_tree_for_conv(p, d, x, ldx, Cin, tree_ws, ldt, st, nodes)) return rc;
         if (gx && !g4) {
             fill2d<float>(gx32_ws, ldgx32, np, Cin, 0.f, st);
             fill2d<float>(gtree_ws, ldgt, nt, Cin, 0.f, st);
@@ -614,11 +616,12 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         SideJoin guard(p, st, side);
         if (dw_g8) {
             bf16_t* xi = (bf16_t*)((char*)gyi + gybytes);
-            bf16_t* ti = (bf16_t*)((char*)xi + xbytes);
             for (int c0 = 0; c0 < Cin; c0 += chunk) {
                 const int c = std::min(chunk, Cin - c0);
                 if (int rc = interleave8_bf16(x + (int64_t)c0 * ldx, ldx, nullptr, 0, c, c, np, xi, side)) return rc;
-                if (int rc = interleave8_bf16(tree_ws + (int64_t)c0 * ldt, ldt, nullptr, 0, c, c, nt, ti, side)) return rc;
+                bf16_t* ti = tree_g8 ? tree_ws + (int64_t)c0 * nt : (bf16_t*)((char*)xi + xbytes);
+                if (int rc = tree_g8 ? fill_tree_mean_g8(p, d, xi, np, c, ti, nt, side, nodes)
+                                     : interleave8_bf16(tree_ws + (int64_t)c0 * ldt, ldt, nullptr, 0, c, c, nt, ti, side)) return rc;
                 if (int rc = launch_conv_dw_g8(code, xi, np, np, ti, nt, nt, gyi, np, np, c, c0, Cin, Cout, S_exp, a.Lc, wl,
                                                (float*)((char*)p->d_scratch + need), pbytes, gw, side)) return rc;
             }

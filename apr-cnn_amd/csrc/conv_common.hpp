@@ -613,4 +613,9 @@ __device__ __forceinline__ void stage_values(const ConvArgs<T>& a, int ci0, int 
     store_items<G, T, CIB>(R, nitem, patch);
 }
 
+int fill_tree_mean_g8(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx, int C, bf16_t* tree, int64_t ldt, hipStream_t st,
+                      const NeedLists* need, bool particles_first = false);
+// A bfloat16 tree work space of C channel planes has room for the tree in groups of eight channels, 16 bytes an access
+inline bool tree_ws_grouped(int C, const bf16_t* tree_ws) { return C % 8 == 0 && ((uintptr_t)tree_ws & 15) == 0; }
+
 }  // namespace aprnet

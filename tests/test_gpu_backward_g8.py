@@ -1,5 +1,7 @@
 """The backward pass of the stencil convolutions on copies grouped by eight channels (bfloat16 features): sizes at the
 edges of the kernels' blocks (16 input / 16 or 32 output channels, 32 columns per product, 256 columns per staged group)."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -243,3 +245,38 @@ def test_copies_of_a_large_layer_are_made_in_parts(cin, cout):
     finally:
         lib.aprnet_set_conv_path(8)
     assert float((gw - planes).abs().max()) <= 1e-4 * float(planes.abs().max())
+
+
+@pytest.mark.parametrize("fill", [16, 17], ids=["needed-nodes", "whole-tree"])
+@pytest.mark.parametrize("ksize,c1,c2", [((3, 3, 3), 8, 0), ((1, 3, 3), 12, 12), ((1, 5, 5), 40, 0), ((3, 3, 3), 16, 24)])
+def test_tree_made_of_the_regrouped_features(ksize, c1, c2, fill):
+    """A 16-byte aligned tree work space takes the tree in groups of eight channels, made of the regrouped features; any other one the planes'
+    tree, regrouped.  Same bits in the output and in both gradients, also where the rows of the work space are longer than the tree."""
+    lib, st, cin, cout = _native.hip(), torch.cuda.current_stream().cuda_stream, c1 + c2, 16
+    apr, d = apr_cases.get("3d_t" if ksize[0] == 3 else "2d_t"), 0
+    n, nt = _ops.number_particles(apr, d), _ops.tree_parts(apr, d)
+    g = torch.Generator().manual_seed(cin)
+    x = torch.randn(cin, n, generator=g).to(torch.bfloat16).to(DEV)
+    gy = torch.randn(cout, n, generator=g).to(torch.bfloat16).to(DEV)
+    S = apr.level_max() - apr.level_min() + 1
+    w = (torch.randn(S, cout, cin, *ksize, generator=g) * 0.1).to(DEV)
+    results = []
+    try:
+        assert lib.aprnet_set_conv_path(fill) == 0
+        for shift in (0, 1):                                       # elements, 2 bytes each
+            ldt = nt + 3
+            tree = torch.full((cin * ldt + 8,), float("nan"), dtype=torch.bfloat16, device=DEV)[shift:]
+            assert (tree.data_ptr() % 16 == 0) == (shift == 0)
+            y, gx = torch.zeros(cout, n, dtype=torch.bfloat16, device=DEV), torch.zeros_like(x)
+            gw = torch.zeros_like(w)
+            gx32, gt = torch.zeros(cin, n, device=DEV), torch.zeros(cin, nt, device=DEV)
+            fu = _ops._Fusion(x[c1:].data_ptr() if c2 else None, n, c2, 0)
+            assert lib.aprnet_conv_fwd_fused_bf16(apr.plan(0), d, *ksize, x.data_ptr(), n, c1, w.data_ptr(), S, cout, None, y.data_ptr(), n,
+                                                  tree.data_ptr(), ldt, C.byref(fu), st) == 0, lib.aprnet_last_error()
+            assert lib.aprnet_conv_bwd_bf16(apr.plan(0), d, *ksize, x.data_ptr(), n, cin, w.data_ptr(), S, cout, gy.data_ptr(), n, gx.data_ptr(), n,
+                                            gw.data_ptr(), tree.data_ptr(), ldt, gx32.data_ptr(), n, gt.data_ptr(), nt, st) == 0, lib.aprnet_last_error()
+            results.append([t.float().cpu() for t in (y, gx, gw)])
+    finally:
+        lib.aprnet_set_conv_path(16)
+    for a, b in zip(*results):
+        assert torch.isfinite(a).all() and torch.equal(a, b)

@@ -176,6 +176,8 @@ int bf16_math() { return g_bf16_math; }
 int bf16_regroup() { return g_bf16_regroup; }
 static std::atomic<int> g_bwd_overlap{1};    // backward: weight gradient on a second stream next to the input gradient
 int backward_overlap() { return g_bwd_overlap; }
+static std::atomic<int> g_wide{0};           // bfloat16 kernels on regrouped input: 64 outputs per workgroup (conv_mfma.hip, WIDE_WINDOWS)
+int conv_wide_mode() { return g_wide; }
 static std::atomic<int> g_bwd_deterministic{1};   // backward: weight gradient summed in a fixed order (partial sums per workgroup) instead of atomics
 int bwd_deterministic() { return g_bwd_deterministic; }
 
@@ -678,6 +680,7 @@ int aprnet_set_conv_path(int path) {
     if (path == 12 || path == 13) { g_narrow = path == 12; return 0; }
     if (path == 14 || path == 15) { g_big_addr = path == 15; return 0; }
     if (path == 16 || path == 17) { g_need_fill = path == 16; return 0; }
+    if (path >= 24 && path <= 26) { g_wide = path - 24; return 0; }
     if (path >= 21 && path <= 23) { g_dw_split = path == 21 ? 1 : path == 22 ? 0 : 2; return 0; }
     if (path >= 18 && path <= 20) { g_f32_split = path == 18 ? 1 : path == 19 ? 0 : 2; return 0; }
     if (path != 0 && path != 1)
@@ -688,7 +691,8 @@ int aprnet_set_conv_path(int path) {
                                                  "14 / 15 (grouped bfloat16 forward: 32-bit offsets where they suffice / 64-bit addresses always), "
                                                  "16 / 17 (tree fill before a forward convolution: the nodes it reads / every node), "
                                                  "18 / 19 / 20 (fp32 features with a work space: products of bfloat16 pieces where faster / fp32 matrix instructions / pieces at any size), "
-                                                 "21 / 22 / 23 (the same for the weight gradient beside an input gradient on pieces)");
+                                                 "21 / 22 / 23 (the same for the weight gradient beside an input gradient on pieces), "
+                                                 "24 / 25 / 26 (bfloat16, flat stencils, more than 32 outputs: 64 per workgroup from a number of windows on / always / never)");
     g_conv_path = path;
     return 0;
 }

@@ -553,7 +553,7 @@ template <class G, int COH, int NB, bool FUSE, int MODE, bool IL, bool BIG, bool
 __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int co0, int nc, int nitem, bool tree_items, int first,
                                                  const uint4* __restrict__ wl, const Lists& sh,
                                                  uint4* __restrict__ patch16, uint4* __restrict__ Wl16,
-                                                 const float* __restrict__ bias_l, const int* __restrict__ toff_l,
+                                                 const float* __restrict__ bias_l, const int* __restrict__ toff_l, int wl_range,
                                                  const uint4* __restrict__ head_a = nullptr, const float* __restrict__ head_b4 = nullptr) {
     constexpr int NSTEP = bf16_steps<G>();
     const int lane = lane_id();
@@ -590,12 +590,18 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
     constexpr int WPT = (W16 + G::NT - 1) / G::NT;
     typename std::conditional<IL, ItemRegs16<G, ItemRegs<G, bf16_t, BF_CIB>::IPT>, ItemRegs<G, bf16_t, BF_CIB>>::type R;
     intx4w wr[WPT];                    // unconditional buffer loads, see the fp32 kernel
+    // The image holds blocks of 32 outputs (16 for layers of at most 16); a workgroup of 64 takes its second half from the next block, or zeros
+    // where there is none (wl_range ends in front of it).
+    const int wl_block = COH == 4 ? (a.Cin + BF_CIB - 1) / BF_CIB * NSTEP * 128 * 16 : 0;
 #define APRNET_LOAD_WEIGHTS(q)                                                                     \
     {                                                                                              \
         const __amdgpu_buffer_rsrc_t rw_ = __builtin_amdgcn_make_buffer_rsrc(                      \
-            const_cast<uint4*>(wl + (int64_t)(q) * W16), 0, W16 * 16, 0x00020000);                 \
-        _Pragma("unroll") for (int k = 0; k < WPT; ++k)                                            \
-            wr[k] = __builtin_amdgcn_raw_buffer_load_b128(rw_, (int)(threadIdx.x + k * G::NT) * 16, 0, 0); \
+            const_cast<uint4*>(wl + (int64_t)(q) * (COH == 4 ? W16 / 2 : W16)), 0, COH == 4 ? wl_range : W16 * 16, 0x00020000); \
+        _Pragma("unroll") for (int k = 0; k < WPT; ++k) {                                          \
+            const int i = threadIdx.x + k * G::NT;                                                 \
+            const int at = COH == 4 ? ((i >> 8) * 128 + (i & 127)) * 16 + ((i >> 7) & 1) * wl_block : i * 16; \
+            wr[k] = __builtin_amdgcn_raw_buffer_load_b128(rw_, COH == 4 && i >= W16 ? BUF_OOB : at, 0, 0); \
+        }                                                                                          \
     }
 #define APRNET_STORE_WEIGHTS()                                                                     \
     _Pragma("unroll") for (int k = 0; k < WPT; ++k) {                                              \
@@ -624,7 +630,7 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
             else load_values<G, bf16_t, BF_CIB>(a, ci0 + BF_CIB, nitem, tree_items, R, 0, std::bool_constant<FUSE>{});
             APRNET_LOAD_WEIGHTS(ci0 / BF_CIB + 1)
         }
-#pragma unroll
+#pragma unroll (COH == 4 ? 1 : NSTEP)          // (see WIDE_WINDOWS)
         for (int st = 0; st < NSTEP; ++st) {
             bf16x8 av[COH];
 #pragma unroll
@@ -787,8 +793,10 @@ conv_mfma_bf16_kernel(const ConvArgs<bf16_t> a) {
     const int s_idx = min(a.S_exp - 1, a.Lc - L);
     const int nq = (a.Cin + BF_CIB - 1) / BF_CIB;
     // a.w carries the packed bfloat16 image
-    const uint4* __restrict__ wl = reinterpret_cast<const uint4*>(a.w) +
-                                   ((int64_t)s_idx * gridDim.y + blockIdx.y) * nq * (NSTEP * COH * 64);
+    constexpr int COH_IMG = COH == 4 ? 2 : COH;
+    const int nb_img = COH == 4 ? (a.Cout + 31) >> 5 : (int)gridDim.y, b_img = blockIdx.y * (COH / COH_IMG);
+    const uint4* __restrict__ wl = reinterpret_cast<const uint4*>(a.w) + ((int64_t)s_idx * nb_img + b_img) * nq * (NSTEP * COH_IMG * 64);
+    const int wl_range = COH == 4 ? (b_img + 1 < nb_img ? nq + 1 : 1) * NSTEP * 128 * 16 : 0;
     const int wave = threadIdx.x >> 6;
     const bool tree_items = MODE == 0 && L < a.Lc;       // the output gradient has no tree part
 
@@ -828,11 +836,11 @@ conv_mfma_bf16_kernel(const ConvArgs<bf16_t> a) {
     const int first = (wave - (int)blockIdx.x) & (G::NWAVE - 1);
     const int nb = first < nblk ? (nblk - first + G::NWAVE - 1) / G::NWAVE : 0;
     switch (__builtin_amdgcn_readfirstlane(nb)) {
-        case 0: mfma_bf16_window<G, COH, 0, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-        case 1: mfma_bf16_window<G, COH, 1, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-        case 2: mfma_bf16_window<G, COH, 2, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-        case 3: mfma_bf16_window<G, COH, 3, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
-        default: mfma_bf16_window<G, COH, 4, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, head_a, head_b4); break;
+        case 0: mfma_bf16_window<G, COH, 0, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, wl_range, head_a, head_b4); break;
+        case 1: mfma_bf16_window<G, COH, 1, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, wl_range, head_a, head_b4); break;
+        case 2: mfma_bf16_window<G, COH, 2, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, wl_range, head_a, head_b4); break;
+        case 3: mfma_bf16_window<G, COH, 3, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, wl_range, head_a, head_b4); break;
+        default: mfma_bf16_window<G, COH, 4, FUSE, MODE, IL, BIG, HEAD>(a, co0, nc, nitem, tree_items, first, wl, gl, patch16, Wl16, bias_l, toff_l, wl_range, head_a, head_b4); break;
     }
 }
 
@@ -904,10 +912,30 @@ int launch_conv_mfma(int code, const ConvArgs<float>& a, int n_tiles, hipStream_
 int launch_conv_mfma(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st) { return launch16_code<bf16_t, 0>(code, a, n_tiles, st); }
 
 // bfloat16 features, bfloat16 contraction (a.w = image of pack_conv_weights_bf16)
+// Workgroups of 64 outputs instead of 32, for layers of more than 32 outputs and flat stencils on regrouped input: LDS bounds the kernel (1.07
+// reads of 1 KB for a product of 2 cycles per CU; of the 3.8 ms of 1x5x5 64 -> 64 on 15.4 M particles they are 3.0), and twice the products per
+// cell read, and a patch staged once instead of twice, take a third of it away; what is left is hidden less well, with 64 sums a lane and none of a
+// step's reads hoisted into the one before (unrolled, the 128 registers spill).  Forward 3.80 -> 3.58 ms, forward and backward 18.2 -> 17.6; 1x3x3
+// on 3.8 M, forward, 1.29 -> 1.10.  It halves the workgroups: 1x5x5 on 0.24 M 0.111 and 0.117 ms.
+// 3x3x3 spills all the same: 64 -> 64 on 5.5 M 2.03 -> 1.89, but forward and backward on 1.2 M 2.12 and 2.15, and a U-Net's layers, with a ReLU, on
+// 4.2 M and 0.5 M particles are 0.2 ms slower together.
+constexpr int WIDE_WINDOWS = 2048;
+int conv_wide_mode();           // 0 the rule, 1 always, 2 never
 template <class G>
 static int launch_bf16(const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st, bool dx = false) {
     const int coh = conv_coh(a.Cout);
     dim3 grid((unsigned)n_tiles, (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
+    if constexpr (G::KZ == 1) {
+        const int wide = conv_wide_mode();
+        if (a.xi != nullptr && !a.big && !a.head_w && a.Cout > 32 && wide != 2 && (wide == 1 || n_tiles >= WIDE_WINDOWS)) {
+            grid.y = (unsigned)((a.Cout + 63) / 64);
+            if (dx) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, false, 1, true>), grid, dim3(G::NT), 0, st, a);
+            else if (a.relu) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, true, 0, true>), grid, dim3(G::NT), 0, st, a);
+            else hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, false, 0, true>), grid, dim3(G::NT), 0, st, a);
+            APRNET_LAUNCH_CHECK("conv_mfma_bf16_kernel");
+            return 0;
+        }
+    }
     if (dx && a.xi != nullptr) {           // regrouped output gradient
         if (coh == 1) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 1, false, 1, true>), grid, dim3(G::NT), 0, st, a);
         else hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 2, false, 1, true>), grid, dim3(G::NT), 0, st, a);

@@ -368,3 +368,32 @@ def test_unet_grouped_limits_fall_back_to_the_plane_path():
         model.encoder[1].pool.increment_level_deltas = True
         del model.use_grouped                              # a whole-model pickle from before the attribute existed
         assert model._grouped_ok(x, [apr])
+
+
+@pytest.mark.parametrize("ksize", [(1, 3, 3), (1, 5, 5)], ids=["133", "155"])
+@pytest.mark.parametrize("cin,cout", [(8, 33), (24, 48), (16, 64), (64, 72), (8, 128)])
+def test_workgroups_of_64_outputs(cin, cout, ksize):
+    """Against those of 32: the same bits forward (the same products in the same order), grouped and on planes, with and without ReLU; the input
+    gradient, whose additions to coarser particles come in any order, within the fp32 sums' own error (2^-17 of the largest value, for sums of some 64
+    terms) and one step of bfloat16 (2^-7 of a value at most), for a sum that this error takes across the middle between two of them."""
+    aprs, ld, x, g = _batch(cin, seed=6)
+    levels = max(a.level_max() - a.level_min() + 1 for a in aprs)
+    w = (torch.randn(levels, cout, cin, *ksize, generator=g) * 0.1).to(DEV)
+    bias = torch.randn(cout, generator=g).to(DEV)
+    # the input gradient's outputs are the layer's inputs
+    xt = torch.randn(2, cout, x.shape[2], generator=g).to(torch.bfloat16).to(DEV)
+    wt = (torch.randn(levels, cin, cout, *ksize, generator=g) * 0.1).to(DEV)
+    lib, results = _native.hip(), []
+    try:
+        for path in (25, 26):
+            assert lib.aprnet_set_conv_path(path) == 0
+            out = [_ops.conv_forward(aprs, x, w, ld, bias, relu=True), _ops.conv_forward(aprs, x, w, ld, bias)]
+            if cout % 8 == 0:
+                out.append(g8.ungroup(g8.conv_forward(aprs, g8.regroup(x), w, ld, bias, relu=True)))
+            results.append((out, _ops.conv_backward(aprs, xt, wt, x, ld)[0].float()))
+    finally:
+        lib.aprnet_set_conv_path(24)
+    for a, b in zip(results[0][0], results[1][0]):
+        assert torch.equal(a, b)
+    a, b = results[0][1], results[1][1]
+    assert bool(((a - b).abs() <= 2 ** -7 * b.abs() + 2 ** -17 * b.abs().max()).all())

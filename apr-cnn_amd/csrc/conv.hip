@@ -243,7 +243,7 @@ static size_t split_fwd_bytes(int code, int Cin, int S_exp, int Cout, int64_t nx
 }
 
 // The same of the input gradient: packed weights and the output gradient in groups of four channels.
-// Next to the weight gradient, which bounds many of these calls, it gains less by it (whole backward pass, split against fp32:
+// Next to a weight gradient on fp32 instructions, which bounds many of these calls, it gains less by it (whole backward pass, split against fp32:
 // 3x3x3 16 -> 16 channels on 70 k particles 152 and 159 us, on 320 k 319 and 353; 32 -> 32 on 14 k 144 and 142, on 70 k 242
 // and 266; 64 -> 64 on 14 k 212 and 220; 128 -> 128 on 2 k 218 and 278; 1x5x5 16 -> 16 on 14 k 139 and 119, on 70 k 142
 // and 157, 64 -> 64 on 14 k 209 and 209).

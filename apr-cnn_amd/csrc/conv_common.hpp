@@ -4,7 +4,8 @@
 // Work decomposition.  One workgroup owns a row group of one level: TZ x TX sparse rows
 // (z0..z0+TZ-1, x0..x0+TX-1) and walks along y in windows of TY output cells.  For each window it
 // stages the isotropic neighbourhood of the group, (TZ+KZ-1) x (TX+KX-1) rows of WY = TY+KY-1 = 64
-// cells, into LDS.  A staged row is the union of three sorted sparse sources
+// cells, into LDS.  (With the window lists of a plan it computes one window of a compressed y axis, whose cells may come from several
+// row groups: lists.hip.)  A staged row is the union of three sorted sparse sources
 // (helpers.hpp:358-420):
 //     0  particles of the same level            row (L,   z,   x)
 //     1  particles one level coarser, each      row (L-1, z/2, x/2)   -> cells 2y, 2y+1

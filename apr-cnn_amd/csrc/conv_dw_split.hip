@@ -17,6 +17,8 @@
 // Measured against the fp32 instructions (conv_bwd_mfma.hip), backward pass with the input gradient beside it, ms: 3x3x3, 9.8 M particles
 // 32 -> 32 channels 14.0 (15.0), 16 -> 16 4.7 (5.6); 2.9 M sparse ones 24 -> 48 6.6 (8.8); 2.2 M dense ones 64 -> 64 9.8 (10.6); 320 k
 // 32 -> 32 0.59 (0.73); 12 k 128 -> 128 0.58 (0.67); 1x5x5 64 -> 64 on 3.9 M 12.8 (17.4).  Error against 64 bits 0.3 to 0.6 of theirs.
+// (On the windows of one row group that the plan's lists held then.  With those of the compressed axis, lists.hip, and the gradients in turn
+// where each fills the chip, conv_bwd.hip: 12.6, 3.98, 5.7, 9.1, 0.51, 0.48 and 12.0; the kernel alone 6.4 of the first.)
 // Bound by waiting, not by a unit: 32 -> 32 on 9.8 M, alone, matrix pipes busy 20 % of the launch, vector ALU and LDS 30 % each, a
 // window takes lists, values, two rounds of staging and of products in turn, and two workgroups per CU overlap them in part.  What was
 // tried: sixteen waves with both chunks staged at once and every load a window ahead 14.7 ms (one workgroup per CU, its phases in

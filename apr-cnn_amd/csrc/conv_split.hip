@@ -12,8 +12,8 @@
 // 4 pairs of taps x 4 channels, so both operands are pieces as they lie there and a step of eight taps takes six instructions.  (With
 // 16-byte cells {x1, x2} and weights {w1, w1}, {w2, w2}, {w3, w1} a step of four taps takes three, one eighth fewer over
 // the 27 taps, but the doubled weights cost 24 register moves per step and wave: 10.1 against 9.1 ms for 32 -> 32 channels
-// on 23 M particles.)  Values come from copies in groups of four channels, one 16-byte load per item; a value is split when it is
-// written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
+// on 23 M particles.)  Values come from the caller's planes (input gradient: from a copy of the output gradient in groups of four
+// channels, see load_values_split); a value is split when it is written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
 //
 // Measured against the fp32 instructions (3x3x3, whole forward pass): 23 M particles, 32 -> 32 channels 8.7 ms; 1 M, 32 -> 32 0.40 (0.52), 64 -> 64
 // 1.40 (1.78); 320 k, 16 -> 16 0.078 (0.090), 64 -> 64 0.46 (0.64).

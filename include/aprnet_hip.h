@@ -18,7 +18,8 @@
  *    size, the image size) before anything is launched: a shorter row is APRNET_ERR_INVALID_ARGUMENT with
  *    both numbers in the message, as the reference refuses tensors whose shape does not match (conv.hpp:63-66).
  *  - Work-space contents: the stencil convolutions fill the mean tree in `tree_ws` only at the nodes their
- *    kernels read (the others keep what the buffer held); callers must not rely on it afterwards.
+ *    kernels read (the others keep what the buffer held), bfloat16 ones also in groups of eight channels; callers must
+ *    not rely on it afterwards.
  *  - `level_delta` d is the number of finest levels pooled away (helpers.hpp:86-117);
  *    Lc = level_max - d.  A feature vector at d holds aprnet_number_parts(plan, d) values.
  *  - No function allocates caller-visible memory; work space is passed in.  Kernels are enqueued

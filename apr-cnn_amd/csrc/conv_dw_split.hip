@@ -240,7 +240,7 @@ conv_dw_split_kernel(const ConvArgs<float> a, const DwWork wk, int* __restrict__
     auto load_x = [&](const int q, const int nitem, const bool tree_items, const Slots& s, Values& v) {
         int plane[SP_CIB];          // (a channel past the last one reads the last one's plane; what it gives is not kept)
 #pragma unroll
-        for (int c = 0; c < SP_CIB; ++c) plane[c] = 4 * min(q * SP_CIB + c, a.Cin - 1 - ci0);
+        for (int c = 0; c < SP_CIB; ++c) plane[c] = min(q * SP_CIB + c, a.Cin - 1 - ci0);
 #pragma unroll
         for (int k = 0; k < S::IPT; ++k) {
             if (k * G::NT >= nitem) break;                                // wave-uniform
@@ -248,15 +248,15 @@ conv_dw_split_kernel(const ConvArgs<float> a, const DwWork wk, int* __restrict__
             if (tree_items) {                                            // (see load_values of conv_common.hpp)
                 if (s.pos[k] & (int)ITEM_TREE) {
 #pragma unroll
-                    for (int c = 0; c < SP_CIB; ++c) v.x[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rt, off, plane[c] * (int)a.ldt, 0);
+                    for (int c = 0; c < SP_CIB; ++c) v.x[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rt, off, plane_offset(plane[c], a.ldt), 0);
                     asm volatile("" ::: "memory");
                 } else {
 #pragma unroll
-                    for (int c = 0; c < SP_CIB; ++c) v.x[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, plane[c] * (int)a.ldx, 0);
+                    for (int c = 0; c < SP_CIB; ++c) v.x[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, plane_offset(plane[c], a.ldx), 0);
                 }
             } else {
 #pragma unroll
-                for (int c = 0; c < SP_CIB; ++c) v.x[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, plane[c] * (int)a.ldx, 0);
+                for (int c = 0; c < SP_CIB; ++c) v.x[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, plane_offset(plane[c], a.ldx), 0);
             }
         }
     };

@@ -178,15 +178,15 @@ __device__ __forceinline__ void load_values_split(const ConvArgs<float>& a, int 
             if (tree_items) {
                 if (item && (R.pos[k] & ITEM_TREE) != 0) {
 #pragma unroll
-                    for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rt, off, min(c, last) * (int)a.ldt * 4, 0);
+                    for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rt, off, plane_offset(min(c, last), a.ldt), 0);
                     asm volatile("" ::: "memory");          // keeps the two branches from being merged into one load with a per-lane descriptor
                 } else {
 #pragma unroll
-                    for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, min(c, last) * (int)ld * 4, 0);
+                    for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, plane_offset(min(c, last), ld), 0);
                 }
             } else {
 #pragma unroll
-                for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, min(c, last) * (int)ld * 4, 0);
+                for (int c = 0; c < SP_CIB; ++c) R.v[k][c] = __builtin_amdgcn_raw_buffer_load_b32(rx, off, plane_offset(min(c, last), ld), 0);
             }
         }
         return;

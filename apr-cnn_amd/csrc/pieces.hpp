@@ -31,4 +31,10 @@ __device__ __forceinline__ void split_pair(float a, float b, unsigned& p1, unsig
     p3 = split_round(ra - split_lo(p2), rb - split_hi(p2));
 }
 
+// Bytes from a plane of `ld` fp32 values to the one `planes` further on, for the scalar offset of a buffer load, which is an unsigned 32-bit
+// number: a signed product overflows from 2^31 bytes on, two planes of 2^28 values or seven of 77 million.
+__host__ __device__ constexpr int plane_offset(int planes, int64_t ld) { return (int)(4u * (unsigned)planes * (unsigned)ld); }
+// the largest ones that the rules of the two kernels let through: eight planes of fewer than 2^27 values, four of fewer than 2^28
+static_assert((unsigned)plane_offset(7, (1 << 27) - 1) == 3758096356u && (unsigned)plane_offset(3, (1 << 28) - 1) == 3221225460u, "wraps nowhere");
+
 }  // namespace aprnet

@@ -1,5 +1,6 @@
 """Stencil convolution of fp32 features on products of bfloat16 pieces, against the oracle in float64, the fp32 matrix
 instructions and the scanning kernels."""
+import ctypes as C
 
 import pytest
 import torch
@@ -531,3 +532,66 @@ def test_weight_gradient_under_capture(dw_path):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out.nan_to_num(), want.nan_to_num()) and torch.equal(out.isnan(), want.isnan())
+
+
+# ---- rows of many values: the planes of a group of channels are reached from the first one with unsigned 32-bit offsets
+def planes(x, ld):
+    """[C, n] -> the same values in rows of ``ld``, with 4 GiB of memory in front of them: an offset that wraps lands in there."""
+    t = torch.empty((1 << 30) + x.shape[0] * ld, device=DEV)[1 << 30:].as_strided(x.shape, (ld, 1))
+    return t.copy_(x)
+
+
+@pytest.mark.parametrize("c2", [0, 8, 6], ids=["one-tensor", "two-tensors", "a-group-of-both"])
+@pytest.mark.parametrize("ld", [200_000_000, (1 << 28) - 1, 1 << 28])
+def test_forward_of_long_rows(path, ld, c2):
+    """Offsets past 2^31 bytes and, from rows of 2^28 values on, a descriptor per plane: the bits that compact rows give."""
+    path(20)
+    lib, st, cin, cout = _native.hip(), torch.cuda.current_stream().cuda_stream, 16, 16
+    x, aprs, _, w_exp = _conv_case([("3d_s", 0)], (3, 3, 3), 2, cin, cout, torch.float32)
+    apr, xd, w = aprs[0], x[0].to(DEV), layer(w_exp)
+    n, nt, c1 = _ops.number_particles(apr, 0), _ops.tree_parts(apr, 0), cin - c2
+    xd = xd[:, :n].contiguous()
+    out = []
+    try:
+        for lx, lt in ((n, nt), (ld, ld)):
+            tree = planes(torch.zeros(cin, nt, device=DEV), lt)
+            a, b = planes(xd[:c1], lx), planes(xd[c1:], lx) if c2 else None
+            y = torch.empty(cout, n, device=DEV)
+            ws_bytes = lib.aprnet_conv_ws_bytes_f32(apr.plan(0), 0, 3, 3, 3, cin, w.shape[0], cout)
+            assert ws_bytes > 0
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=DEV)
+            fu = _ops._Fusion(b.data_ptr() if c2 else None, lx, c2, 0)
+            assert lib.aprnet_conv_fwd_ws_f32(apr.plan(0), 0, 3, 3, 3, a.data_ptr(), lx, c1, w.data_ptr(), w.shape[0], cout, None, y.data_ptr(), n,
+                                              tree.data_ptr(), lt, C.byref(fu), ws.data_ptr(), ws_bytes, st) == 0, lib.aprnet_last_error()
+            out.append(y)
+            del tree, a, b
+        assert torch.equal(*out)
+    finally:
+        torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("ld", [100_000_000, (1 << 27) - 1, 1 << 27])
+def test_weight_gradient_of_long_rows(dw_path, ld):
+    """The same with eight planes per workgroup; rows of 2^27 values and more are left to the fp32 instructions."""
+    lib, st, cin, cout = _native.hip(), torch.cuda.current_stream().cuda_stream, 16, 16
+    x, aprs, _, w_exp, gy = _dw_case([("3d_s", 0)], (3, 3, 3), cin, cout)
+    apr, w = aprs[0], layer(w_exp)
+    n, nt = _ops.number_particles(apr, 0), _ops.tree_parts(apr, 0)
+    xd, gd = x[0, :, :n].contiguous().to(DEV), gy[0, :, :n].contiguous().to(DEV)
+    out = []
+    try:
+        for lx, lt, p in ((n, nt, 23 if ld < 1 << 27 else 22), (ld, ld, 23)):
+            dw_path(p)
+            a, tree = planes(xd, lx), planes(torch.zeros(cin, nt, device=DEV), lt)
+            gx, gw, gt = torch.empty(cin, n, device=DEV), torch.zeros_like(w), torch.empty(cin, nt, device=DEV)
+            ws_bytes = lib.aprnet_conv_bwd_ws_bytes_f32(apr.plan(0), 0, 3, 3, 3, cin, w.shape[0], cout)
+            assert ws_bytes > 0
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=DEV)
+            assert lib.aprnet_conv_bwd_ws_f32(apr.plan(0), 0, 3, 3, 3, a.data_ptr(), lx, cin, w.data_ptr(), w.shape[0], cout, gd.data_ptr(), n,
+                                              gx.data_ptr(), n, gw.data_ptr(), tree.data_ptr(), lt, gt.data_ptr(), nt, ws.data_ptr(), ws_bytes, st) == 0, \
+                lib.aprnet_last_error()
+            out.append(gw)
+            del a, tree
+        assert torch.equal(*out)
+    finally:
+        torch.cuda.empty_cache()

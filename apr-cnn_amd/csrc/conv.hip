@@ -176,7 +176,7 @@ int bf16_math() { return g_bf16_math; }
 int bf16_regroup() { return g_bf16_regroup; }
 static std::atomic<int> g_bwd_overlap{1};    // backward: weight gradient on a second stream next to the input gradient
 int backward_overlap() { return g_bwd_overlap; }
-static std::atomic<int> g_wide{0};           // bfloat16 kernels on regrouped input: 64 outputs per workgroup (conv_mfma.hip, WIDE_WINDOWS)
+static std::atomic<int> g_wide{0};           // bfloat16 kernels on regrouped input: 64 outputs per workgroup (conv_mfma.hip, wide_outputs)
 int conv_wide_mode() { return g_wide; }
 static std::atomic<int> g_bwd_deterministic{1};   // backward: weight gradient summed in a fixed order (partial sums per workgroup) instead of atomics
 int bwd_deterministic() { return g_bwd_deterministic; }
@@ -692,7 +692,7 @@ int aprnet_set_conv_path(int path) {
                                                  "16 / 17 (tree fill before a forward convolution: the nodes it reads / every node), "
                                                  "18 / 19 / 20 (fp32 features with a work space: products of bfloat16 pieces where faster / fp32 matrix instructions / pieces at any size), "
                                                  "21 / 22 / 23 (the same for the weight gradient beside an input gradient on pieces), "
-                                                 "24 / 25 / 26 (bfloat16, flat stencils, more than 32 outputs: 64 per workgroup from a number of windows on / always / never)");
+                                                 "24 / 25 / 26 (bfloat16, flat stencils, more than 32 outputs: 64 per workgroup where that is faster / always / never)");
     g_conv_path = path;
     return 0;
 }

@@ -630,7 +630,7 @@ __device__ __forceinline__ void mfma_bf16_window(const ConvArgs<bf16_t>& a, int 
             else load_values<G, bf16_t, BF_CIB>(a, ci0 + BF_CIB, nitem, tree_items, R, 0, std::bool_constant<FUSE>{});
             APRNET_LOAD_WEIGHTS(ci0 / BF_CIB + 1)
         }
-#pragma unroll (COH == 4 ? 1 : NSTEP)          // (see WIDE_WINDOWS)
+#pragma unroll (COH == 4 ? 1 : NSTEP)          // (see wide_outputs)
         for (int st = 0; st < NSTEP; ++st) {
             bf16x8 av[COH];
 #pragma unroll
@@ -916,10 +916,26 @@ int launch_conv_mfma(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream
 // reads of 1 KB for a product of 2 cycles per CU; of the 3.8 ms of 1x5x5 64 -> 64 on 15.4 M particles they are 3.0), and twice the products per
 // cell read, and a patch staged once instead of twice, take a third of it away; what is left is hidden less well, with 64 sums a lane and none of a
 // step's reads hoisted into the one before (unrolled, the 128 registers spill).  Forward 3.80 -> 3.58 ms, forward and backward 18.2 -> 17.6; 1x3x3
-// on 3.8 M, forward, 1.29 -> 1.10.  It halves the workgroups: 1x5x5 on 0.24 M 0.111 and 0.117 ms.
+// on 3.8 M, forward, 1.29 -> 1.10.
 // 3x3x3 spills all the same: 64 -> 64 on 5.5 M 2.03 -> 1.89, but forward and backward on 1.2 M 2.12 and 2.15, and a U-Net's layers, with a ReLU, on
 // 4.2 M and 0.5 M particles are 0.2 ms slower together.
-constexpr int WIDE_WINDOWS = 2048;
+//
+// Not where the last workgroup would do half of its products for outputs that are not there (a rest of 1 to 32 above a multiple of 64): 1x5x5,
+// 32 against 64 per workgroup, 64 -> 72 channels forward on 14.3 M particles 6.09 and 6.79 ms, on 1.1 M 0.443 and 0.499, -> 96 6.32 and
+// 6.88, -> 160 9.96 and 10.12; input gradient of 72 inputs, whole backward pass, 15.28 and 16.08.  With two blocks of 64, -> 104 7.89 and 7.00,
+// -> 128 8.14 and 7.40.  1x3x3 has nine taps a cell read for 25 and gains by the half as well (72 on 14.3 M 3.99 and 3.85, 96 4.26 and 4.00), forward from
+// more windows on: 72 on 0.9 M particles (2100 windows) 0.248 and 0.254, on 1.1 M (2600) 0.300 and 0.304, on 1.3 M (2950) 0.351 and 0.347.
+// Windows: it halves the workgroups.  1x5x5 64 -> 64 forward on 0.085 M (550 windows) 0.0640 and 0.0647, on 0.75 M (1880) 0.237 and 0.231; its
+// input gradient beside the weight gradient, whole backward pass, on 0.9 M (2400) 0.785 and 0.811, on 1.1 M (2940) 0.938 and 0.943, on
+// 1.4 M (3780) 1.188 and 1.187, of 40 inputs 0.617 and 0.619, 0.727 and 0.705, 0.922 and 0.897.
+constexpr int WIDE_WINDOWS = 2048, WIDE_WINDOWS_MORE = 2816;
+constexpr bool wide_outputs(int KX, int Cout, int n_win, bool dx) {
+    const bool rest = (Cout + 31) / 32 % 2 != 0;
+    return Cout > 32 && !(KX == 5 && rest) && n_win >= ((KX == 5 ? dx : rest && !dx) ? WIDE_WINDOWS_MORE : WIDE_WINDOWS);
+}
+static_assert(!wide_outputs(5, 32, 1 << 20, false) && wide_outputs(5, 33, 1 << 20, false) && wide_outputs(5, 64, 2048, false) && !wide_outputs(5, 64, 2047, false), "one block");
+static_assert(!wide_outputs(5, 65, 1 << 20, false) && !wide_outputs(5, 96, 1 << 20, true) && wide_outputs(5, 97, 1 << 20, false) && !wide_outputs(5, 160, 1 << 20, false), "no half block");
+static_assert(wide_outputs(3, 96, 2816, false) && !wide_outputs(3, 96, 2815, false) && wide_outputs(3, 96, 2048, true) && !wide_outputs(5, 64, 2815, true), "more windows");
 int conv_wide_mode();           // 0 the rule, 1 always, 2 never
 template <class G>
 static int launch_bf16(const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st, bool dx = false) {
@@ -927,7 +943,7 @@ static int launch_bf16(const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st, b
     dim3 grid((unsigned)n_tiles, (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
     if constexpr (G::KZ == 1) {
         const int wide = conv_wide_mode();
-        if (a.xi != nullptr && !a.big && !a.head_w && a.Cout > 32 && wide != 2 && (wide == 1 || n_tiles >= WIDE_WINDOWS)) {
+        if (a.xi != nullptr && !a.big && !a.head_w && wide != 2 && (wide == 1 ? a.Cout > 32 : wide_outputs(G::KX, a.Cout, n_tiles, dx))) {
             grid.y = (unsigned)((a.Cout + 63) / 64);
             if (dx) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, false, 1, true>), grid, dim3(G::NT), 0, st, a);
             else if (a.relu) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, true, 0, true>), grid, dim3(G::NT), 0, st, a);

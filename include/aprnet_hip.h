@@ -130,7 +130,7 @@ int aprnet_profile_enable(int on);
  * where that is faster (default), 19 = fp32 matrix instructions, 20 = products of pieces at any size; 21, 22 and 23 = the same for
  * the weight gradient of a backward pass whose input gradient is made of pieces (aprnet_conv_bwd_ws_f32).
  * And for bfloat16 layers of flat stencils and more than 32 outputs (input gradients: inputs) on regrouped features: 24 = 64 of them per
- * workgroup where the windows are many (default), 25 = always, 26 = 32.
+ * workgroup where that is faster (default), 25 = always, 26 = 32.
  * All are HIP kernels; the switch
  * exists so that tests can cover them and memory-bound callers can do without the lists. */
 int aprnet_set_conv_path(int path);

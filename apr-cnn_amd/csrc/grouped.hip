@@ -35,18 +35,23 @@ __device__ __forceinline__ uint4* g8_at(bf16_t* base, int64_t ld, int q, int64_t
     return reinterpret_cast<uint4*>(base) + (int64_t)q * ld + i;
 }
 
-// Groups of a thread in the kernels that walk the child table: all of them, so that the table is read once, halved while fewer than SPLIT_THREADS
-// threads would remain (the chip holds 2^19 at a time).  A thread's groups are a serial chain, each waiting for its own loads: in a network of 16 to
-// 128 channels on 1.3 M particles a fill took 8.3 us with one thread for all groups and 5.1 split, a pool 11.8 and 7.6, an upsample 9.5 and
-// 8.0, the network 0.92 and 0.835 ms.  Limits of 2^17, 2^18, 2^20, 2^21: 0.842, 0.835, 0.842, 0.839, and on 210 M particles 53.7, 53.7,
-// 54.0, 53.9 ms (2^19: 53.7).
-constexpr int64_t SPLIT_THREADS = (int64_t)1 << 19;
-static int groups_per_thread(int64_t n, int G) {
+// Groups of a thread in the kernels that walk the child table: all of them, so that the table is read once, halved while fewer than `threads`
+// would remain.  A thread's groups are a serial chain, each waiting for its own loads: in a network of 16 to 128 channels on 1.3 M
+// particles a fill took 8.3 us with one thread for all groups and 5.1 split, a pool 11.8 and 7.6, an upsample 9.5 and 8.0, the network 0.92 and 0.835 ms.
+// Fills gain up to 2^19 threads, what the chip holds at a time (1.3 M particles of 32 channels 44.9 -> 37.7 us, of 256 279 -> 186 and, with limits of
+// 2^17 and 2^18, 204 and 192; 2^20 and 2^21: the network 0.842 and 0.839 ms).  A pool or upsample moves little more than the table it reads again: past 2^17 threads
+// splitting costs it, at 2^19 a pool to 0.21 M outputs of 16 channels 8.0 us instead of 7.1, to 0.36 M 11.7 and 11.3, an upsample of 64 channels to
+// 0.92 M particles 24.8 and 21.6, of 16 to 1.3 M 11.4 and 10.0 (some gain: a pool to 0.15 M of 16 channels 4.8 and 5.5).
+// The loops over a thread's groups start at zero, from addresses moved to its first one: counted from that one, a pool of 128 channels to
+// 0.36 M outputs took 100 instead of 93 us, split or not.
+constexpr int64_t FILL_THREADS = (int64_t)1 << 19, MOVE_THREADS = (int64_t)1 << 17;
+static constexpr int groups_per_thread(int64_t n, int G, int64_t threads) {
     int gpt = G;
     if (G > 65535) return gpt;          // a grid's second dimension
-    while (gpt > 1 && n * ((G + gpt - 1) / gpt) < SPLIT_THREADS) gpt = (gpt + 1) / 2;
+    while (gpt > 1 && n * ((G + gpt - 1) / gpt) < threads) gpt = (gpt + 1) / 2;
     return gpt;
 }
+static_assert(groups_per_thread(145197, 32, MOVE_THREADS) == 32 && groups_per_thread(69318, 8, MOVE_THREADS) == 4 && groups_per_thread(69318, 8, FILL_THREADS) == 1, "see above");
 
 // ---------------------------------------------------------------------------- planes <-> groups
 // out[q][i][c] = x[8 q + c][i]; channels past C read as zeros
@@ -214,7 +219,7 @@ int fill_tree_mean_g8(const aprnet_plan* p, int d, const bf16_t* x, int64_t ldx,
         const int from_x = (l + 1 == Lc);
         if (need && need->cnt[l] == 0) continue;
         const int64_t n = need && !need->whole[l] ? need->cnt[l] : e - b;
-        const int gpt = groups_per_thread(n, G);
+        const int gpt = groups_per_thread(n, G, FILL_THREADS);
         const dim3 grid((unsigned)((n + GTB - 1) / GTB), (unsigned)((G + gpt - 1) / gpt));
         if (need && !need->whole[l])
             hipLaunchKernelGGL(fill_tree_list_g8_kernel, grid, dim3(GTB), 0, st,
@@ -276,16 +281,17 @@ maxpool_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t 
                   const bf16_t* __restrict__ x, int64_t ldx, int G, int gpt, bf16_t* __restrict__ y, int64_t ldy, int64_t in_tree_off) {
     const int64_t i = (int64_t)blockIdx.x * GTB + threadIdx.x;
     if (i >= n_out) return;
-    const int q0 = blockIdx.y * gpt, q1 = min(G, q0 + gpt);
+    const int q0 = blockIdx.y * gpt, nq = min(gpt, G - q0);
+    x += (int64_t)q0 * ldx * 8; y += (int64_t)q0 * ldy * 8;      // (loops from zero on, see groups_per_thread)
     if (i < n_copy) {
-        for (int q = q0; q < q1; ++q) *g8_at(y, ldy, q, i) = *g8_at(x, ldx, q, i);
+        for (int q = 0; q < nq; ++q) *g8_at(y, ldy, q, i) = *g8_at(x, ldx, q, i);
         return;
     }
     const int64_t t = t_begin + (i - n_copy);
     int32_t ch[8];                        // read once for the groups of the thread
 #pragma unroll
     for (int s = 0; s < 8; ++s) ch[s] = children[(int64_t)s * n_tree + t];
-    for (int q = q0; q < q1; ++q) {
+    for (int q = 0; q < nq; ++q) {
         uint4 raw[8];                     // unconditional loads, as in fill_node_g8
 #pragma unroll
         for (int s = 0; s < 8; ++s)
@@ -315,9 +321,10 @@ upsample_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t
                    const bf16_t* __restrict__ src, int64_t lds, int G, int gpt, bf16_t* __restrict__ dst, int64_t ldd, int64_t out_tree_off) {
     const int64_t j = (int64_t)blockIdx.x * GTB + threadIdx.x;
     const int64_t n_par = n_in - n_copy;
-    const int q0 = blockIdx.y * gpt, q1 = min(G, q0 + gpt);
+    const int q0 = blockIdx.y * gpt, nq = min(gpt, G - q0);
+    src += (int64_t)q0 * lds * 8; dst += (int64_t)q0 * ldd * 8;
     if (j < n_copy) {                     // copied positions: one lane each
-        for (int q = q0; q < q1; ++q) *g8_at(dst, ldd, q, j) = *g8_at(src, lds, q, j);
+        for (int q = 0; q < nq; ++q) *g8_at(dst, ldd, q, j) = *g8_at(src, lds, q, j);
         return;
     }
     const int64_t k = j - n_copy;
@@ -330,7 +337,7 @@ upsample_g8_kernel(const int32_t* __restrict__ children, int64_t n_tree, int64_t
         const int32_t c = children[(int64_t)(2 * p + dy) * n_tree + t];
         at[p] = c >= 0 ? (int64_t)c : (c != NO_CHILD ? out_tree_off + ~c : -1);
     }
-    for (int q = q0; q < q1; ++q) {
+    for (int q = 0; q < nq; ++q) {
         const uint4 v = *g8_at(src, lds, q, i);
 #pragma unroll
         for (int p = 0; p < 4; ++p)
@@ -561,7 +568,7 @@ int aprnet_maxpool_fwd_bf16g(const aprnet_plan* p, int d, const uint16_t* x, int
     if (C <= 0 || n_out <= 0) return 0;
     if (ldy < n_out || ldx < p->number_parts(d)) return fail(APRNET_ERR_INVALID_ARGUMENT, "maxpool_forward: row shorter than the particle count");
     APRNET_HIP_CHECK(hipSetDevice(p->device));
-    const int G = C / 8, gpt = groups_per_thread(n_out, G);
+    const int G = C / 8, gpt = groups_per_thread(n_out, G, MOVE_THREADS);
     hipLaunchKernelGGL(maxpool_g8_kernel, dim3((unsigned)((n_out + GTB - 1) / GTB), (unsigned)((G + gpt - 1) / gpt)), dim3(GTB), 0, (hipStream_t)st,
                        p->d_children, p->n_tree, n_copy, n_out, p->tree.level_begin(Lc - 1), (const bf16_t*)x, ldx, G, gpt, (bf16_t*)y, ldy,
                        p->tree_offset(Lc));
@@ -578,7 +585,7 @@ int aprnet_upsample_fwd_bf16g(const aprnet_plan* p, int d, const uint16_t* x, in
     if (ldx < n_in || ldy < p->number_parts(d - 1)) return fail(APRNET_ERR_INVALID_ARGUMENT, "upsample_const_forward: row shorter than the particle count");
     APRNET_HIP_CHECK(hipSetDevice(p->device));
     const int64_t n_thr = n_copy + 2 * (n_in - n_copy);
-    const int G = C / 8, gpt = groups_per_thread(n_thr, G);
+    const int G = C / 8, gpt = groups_per_thread(n_thr, G, MOVE_THREADS);
     hipLaunchKernelGGL(upsample_g8_kernel, dim3((unsigned)((n_thr + GTB - 1) / GTB), (unsigned)((G + gpt - 1) / gpt)), dim3(GTB), 0, (hipStream_t)st,
                        p->d_children, p->n_tree, n_copy, n_in, p->tree.level_begin(Lc), (const bf16_t*)x, ldx, G, gpt, (bf16_t*)y, ldy,
                        p->tree_offset(Lc + 1));

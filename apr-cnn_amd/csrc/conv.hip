@@ -138,7 +138,7 @@ template <> struct Chunk<double> { static constexpr int c333 = 4, c133 = 8,  c15
 bool conv_mfma_supported(int code);
 int launch_conv_mfma(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
 int launch_conv_mfma(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
-int launch_conv_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
+int launch_conv_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_win, hipStream_t st);
 size_t conv_packed_bf16_bytes(int code, int S_exp, int Cout, int Cin);
 int pack_conv_weights_bf16(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, hipStream_t st, bool transposed = false);
 int interleave8_bf16(const bf16_t* x, int64_t ldx, const bf16_t* x2, int64_t ldx2, int c_split, int C, int64_t count, bf16_t* out,
@@ -154,7 +154,7 @@ size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
 int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx, int64_t nx, float* xi,
                   hipStream_t st);
-int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_win, hipStream_t st);
 static std::atomic<int> g_f32_split{1};      // fp32 features: products of bfloat16 pieces (conv_split.hip) 1 = where faster, 2 = at any size, 0 = never
 static std::atomic<int> g_dw_split{1};       // and their weight gradient (conv_dw_split.hip), likewise
 

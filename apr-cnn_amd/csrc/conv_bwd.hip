@@ -271,9 +271,9 @@ size_t split_mark_bytes();
 size_t conv_packed_split_bytes(int code, int S_exp, int Cm, int Ck);
 int prepare_split(int code, const float* w, int S_exp, int Cm, int Ck, bool transposed, void* packed, int* marks, const float* x, int64_t ldx, int64_t nx, float* xi,
                   hipStream_t st);
-int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);
+int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_win, hipStream_t st);
 int launch_conv_dw_split(int code, const ConvArgs<float>& a, const DwWork& k, int* mark, hipStream_t st);
-int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st);
+int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_win, hipStream_t st);
 size_t conv_packed_bf16_bytes(int code, int S_exp, int Cout, int Cin);
 int pack_conv_weights_bf16(int code, const float* w, int S_exp, int Cout, int Cin, void* packed, hipStream_t st, bool transposed);
 int interleave8_bf16(const bf16_t* x, int64_t ldx, const bf16_t* x2, int64_t ldx2, int c_split, int C, int64_t count, bf16_t* out,
@@ -352,7 +352,7 @@ template <> int try_mfma_bwd<float>(aprnet_plan* p, const ConvArgs<float>& a, co
         redo = RedoClear{mark, a.gx, a.ldgx, a.x_count, a.gtree, a.ldgt, a.t_count, a.Cin};
         if (int rc = prepare_split(code, a.w, a.S_exp, a.Cin, a.Cout, true, image, mark, a.gy, a.ldy, a.x_count, gi, st)) return rc;
         e.x = a.gy; e.ldx = a.ldy; e.Cin = a.Cout; e.Cout = a.Cin; e.w = (const float*)image; e.bias = nullptr; e.redo = mark;
-        e.xi = gi; e.xi_ld = a.x_count; e.ti = gi; e.ti_ld = 0; e.t_count = 0;
+        e.xi = gi; e.xi_ld = a.x_count;
     }
     const bool dw_pieces = pieces && wl && wl->n_win > 0 && split_dw(a.Cin, a.Cout, a.x_count, a.ldx, a.ldt);
     // Two kernels on pieces that each fill the chip run one after the other: beside each other they read more past the caches (3x3x3, 9.8 M

@@ -414,7 +414,7 @@ __device__ __forceinline__ void close_window(ConvShared<G>& sh) {
 struct RedoClear { const int* mark; float* gx; int64_t ldgx, n; float* gtree; int64_t ldgt, nt; int C; };
 
 // Marks of a forward launch on products of bfloat16 pieces (conv_split.hip), set where a result is not finite: word 0 = any, the others
-// one per tile and block of output channels, several of them to a word where there are more (all of these are then computed again).
+// one per window and block of output channels, several of them to a word where there are more (all of these are then computed again).
 constexpr unsigned SPLIT_MARKS = 4096;
 __device__ __forceinline__ unsigned split_mark(unsigned unit) { return 1 + unit % (SPLIT_MARKS - 1); }
 

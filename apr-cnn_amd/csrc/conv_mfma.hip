@@ -342,22 +342,22 @@ conv_mfma16_kernel(const ConvArgs<T> a) {
 #undef APRNET_WINDOW
 }
 
-// The marked tiles of a forward launch on products of bfloat16 pieces (conv_split.hip), on the fp32 instructions and bit for bit
-// what conv_mfma16_kernel gives.  Persistent workgroups, which end at once where nothing is marked.  With a NaN in every tile: 32 -> 32
+// The marked windows (times blocks of outputs) of a forward launch on products of bfloat16 pieces (conv_split.hip), on the fp32 instructions and bit for bit
+// what conv_mfma16_kernel gives.  Persistent workgroups, which end at once where nothing is marked.  With a NaN in every window: 32 -> 32
 // channels on 320 k particles 0.67 ms in all (finite features 0.22; one thread per column, a channel staged at a time 9.7), on 9.8 M 13.8
 // (4.8; 202).
 template <class G, int COH>
 __global__ void __launch_bounds__(G::NT) __attribute__((amdgpu_waves_per_eu(FWD_WAVES, FWD_WAVES)))
-conv_mfma16_redo_kernel(const ConvArgs<float> a, int n_tiles, int n_cb) {
+conv_mfma16_redo_kernel(const ConvArgs<float> a, int n_win, int n_cb) {
     constexpr int CIB = FWD_CIB;
     __shared__ float patch[CIB * G::CH_STRIDE];
     __shared__ __attribute__((aligned(16))) float Wl[CIB * G::K * 16 * COH];
     __shared__ float bias_l[16 * COH];
     if (a.redo[0] == 0) return;
     const int wave = threadIdx.x >> 6;
-    for (int u = blockIdx.x; u < n_tiles * n_cb; u += gridDim.x) {              // uniform
+    for (int u = blockIdx.x; u < n_win * n_cb; u += gridDim.x) {              // uniform
         if (a.redo[split_mark(u)] == 0) continue;
-        const int w = u % n_tiles, co0 = u / n_tiles * 16 * COH, L = a.win_level[w];
+        const int w = u % n_win, co0 = u / n_win * 16 * COH, L = a.win_level[w];
         const float4* __restrict__ wl = reinterpret_cast<const float4*>(a.w_raw + (int64_t)min(a.S_exp - 1, a.Lc - L) * a.Cout * a.Cin * G::K);
         const bool tree_items = L < a.Lc;
         if (threadIdx.x < 16 * COH)                                            // (read behind the barriers of a window)
@@ -857,6 +857,7 @@ static int conv_taps(int code) { return code == 333 ? 27 : code == 133 ? 9 : 25;
 static int conv_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
 
 // a.win_level set: forward with the window lists of the plan; otherwise the kernel scans (always for the input gradient)
+// n_tiles: windows of the lists, or row groups to scan
 template <typename T, class G, int MODE>
 static int launch16(const ConvArgs<T>& a, int n_tiles, hipStream_t st) {
     const int coh = conv_coh(a.Cout);
@@ -888,20 +889,20 @@ static int launch16_code(int code, const ConvArgs<T>& a, int n_tiles, hipStream_
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }
 
-// The tiles that a.redo marks (a.w_raw: the weights, not packed; forward lists of the plan)
+// What a.redo marks (a.w_raw: the weights, not packed; forward lists of the plan)
 template <class G>
-static int launch_redo(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+static int launch_redo(const ConvArgs<float>& a, int n_win, hipStream_t st) {
     const int coh = conv_coh(a.Cout), n_cb = (a.Cout + 16 * coh - 1) / (16 * coh);
-    const dim3 grid((unsigned)std::min<int64_t>((int64_t)n_tiles * n_cb, 768));         // three workgroups on each of 256 CUs
-    if (coh == 1) hipLaunchKernelGGL((conv_mfma16_redo_kernel<G, 1>), grid, dim3(G::NT), 0, st, a, n_tiles, n_cb);
-    else hipLaunchKernelGGL((conv_mfma16_redo_kernel<G, 2>), grid, dim3(G::NT), 0, st, a, n_tiles, n_cb);
+    const dim3 grid((unsigned)std::min<int64_t>((int64_t)n_win * n_cb, 768));         // three workgroups on each of 256 CUs
+    if (coh == 1) hipLaunchKernelGGL((conv_mfma16_redo_kernel<G, 1>), grid, dim3(G::NT), 0, st, a, n_win, n_cb);
+    else hipLaunchKernelGGL((conv_mfma16_redo_kernel<G, 2>), grid, dim3(G::NT), 0, st, a, n_win, n_cb);
     APRNET_LAUNCH_CHECK("conv_mfma16_redo_kernel");
     return 0;
 }
-int launch_conv_redo(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+int launch_conv_redo(int code, const ConvArgs<float>& a, int n_win, hipStream_t st) {
     switch (code) {
-        case 333: return launch_redo<M333N>(a, n_tiles, st);
-        case 155: return launch_redo<M155N>(a, n_tiles, st);
+        case 333: return launch_redo<M333N>(a, n_win, st);
+        case 155: return launch_redo<M155N>(a, n_win, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }
@@ -938,12 +939,12 @@ static_assert(!wide_outputs(5, 65, 1 << 20, false) && !wide_outputs(5, 96, 1 << 
 static_assert(wide_outputs(3, 96, 2816, false) && !wide_outputs(3, 96, 2815, false) && wide_outputs(3, 96, 2048, true) && !wide_outputs(5, 64, 2815, true), "more windows");
 int conv_wide_mode();           // 0 the rule, 1 always, 2 never
 template <class G>
-static int launch_bf16(const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st, bool dx = false) {
+static int launch_bf16(const ConvArgs<bf16_t>& a, int n_win, hipStream_t st, bool dx = false) {
     const int coh = conv_coh(a.Cout);
-    dim3 grid((unsigned)n_tiles, (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
+    dim3 grid((unsigned)n_win, (unsigned)((a.Cout + 16 * coh - 1) / (16 * coh)));
     if constexpr (G::KZ == 1) {
         const int wide = conv_wide_mode();
-        if (a.xi != nullptr && !a.big && !a.head_w && wide != 2 && (wide == 1 ? a.Cout > 32 : wide_outputs(G::KX, a.Cout, n_tiles, dx))) {
+        if (a.xi != nullptr && !a.big && !a.head_w && wide != 2 && (wide == 1 ? a.Cout > 32 : wide_outputs(G::KX, a.Cout, n_win, dx))) {
             grid.y = (unsigned)((a.Cout + 63) / 64);
             if (dx) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, false, 1, true>), grid, dim3(G::NT), 0, st, a);
             else if (a.relu) hipLaunchKernelGGL((conv_mfma_bf16_kernel<G, 4, true, 0, true>), grid, dim3(G::NT), 0, st, a);
@@ -982,21 +983,21 @@ static int launch_bf16(const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st, b
     APRNET_LAUNCH_CHECK("conv_mfma_bf16_kernel");
     return 0;
 }
-int launch_conv_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st) {
+int launch_conv_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_win, hipStream_t st) {
     switch (code) {
-        case 333: return launch_bf16<M333N>(a, n_tiles, st);
-        case 133: return launch_bf16<M133N>(a, n_tiles, st);
-        case 155: return launch_bf16<M155N>(a, n_tiles, st);
+        case 333: return launch_bf16<M333N>(a, n_win, st);
+        case 133: return launch_bf16<M133N>(a, n_win, st);
+        case 155: return launch_bf16<M155N>(a, n_win, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }
 // Input gradient with bfloat16 products: a.x / a.Cin describe the output gradient, a.Cout the layer's input channels,
 // a.w the transposed image of pack_conv_weights_bf16, a.win_level ... the input-gradient lists of the plan.
-int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_tiles, hipStream_t st) {
+int launch_conv_dx_mfma_bf16(int code, const ConvArgs<bf16_t>& a, int n_win, hipStream_t st) {
     switch (code) {
-        case 333: return launch_bf16<M333N>(a, n_tiles, st, true);
-        case 133: return launch_bf16<M133N>(a, n_tiles, st, true);
-        case 155: return launch_bf16<M155N>(a, n_tiles, st, true);
+        case 333: return launch_bf16<M333N>(a, n_win, st, true);
+        case 133: return launch_bf16<M133N>(a, n_win, st, true);
+        case 155: return launch_bf16<M155N>(a, n_win, st, true);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }

@@ -13,7 +13,7 @@
 // 16-byte cells {x1, x2} and weights {w1, w1}, {w2, w2}, {w3, w1} a step of four taps takes three, one eighth fewer over
 // the 27 taps, but the doubled weights cost 24 register moves per step and wave: 10.1 against 9.1 ms for 32 -> 32 channels
 // on 23 M particles.)  Values come from the caller's planes (input gradient: from a copy of the output gradient in groups of four
-// channels, see load_values_split); a value is split when it is written to LDS.  Lists, tiles, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
+// channels, see load_values_split); a value is split when it is written to LDS.  Lists, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
 //
 // Measured against the fp32 instructions (3x3x3, whole forward pass): 23 M particles, 32 -> 32 channels 8.7 ms; 1 M, 32 -> 32 0.40 (0.52), 64 -> 64
 // 1.40 (1.78); 320 k, 16 -> 16 0.078 (0.090), 64 -> 64 0.46 (0.64).
@@ -25,7 +25,7 @@
 //
 // Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
 // NaN), and values of 2^111 and more, or sums of 2^95 and more, are infinite for these kernels (see SPLIT_SCALE).  Where a result comes
-// out infinite or NaN its tile is marked, and the fp32 instructions compute the marked tiles again (conv_mfma16_redo_kernel; as a call
+// out infinite or NaN its window and block of outputs are marked, and the fp32 instructions compute what is marked again (conv_mfma16_redo_kernel; as a call
 // inside this kernel a second pass cost registers: 16 -> 16 channels on 23 M particles 3.47 instead of 3.26 ms); an
 // input gradient that holds one is made again from the start by the fp32 kernel.  Small values keep all their bits: features of 1e-37
 // come out with 0.4 of the fp32 instructions' error (split without SPLIT_SCALE, 510 times that error).
@@ -434,33 +434,33 @@ using S155 = ConvGeom<1, 5, 5, 1, 8, 512, 64, 16>;
 static int split_coh(int Cm) { return Cm <= 16 ? 1 : 2; }
 static int split_nstep(int code) { return code == 333 ? split_steps<S333>() : split_steps<S155>(); }
 
-int launch_conv_redo(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st);        // conv_mfma.hip
+int launch_conv_redo(int code, const ConvArgs<float>& a, int n_win, hipStream_t st);        // conv_mfma.hip
 
 template <class G, int MODE>
-static int launch_split(const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+static int launch_split(const ConvArgs<float>& a, int n_win, hipStream_t st) {
     const int coh = split_coh(a.Cout), n_cb = (a.Cout + 16 * coh - 1) / (16 * coh);
-    dim3 grid((unsigned)n_tiles, (unsigned)n_cb);
+    dim3 grid((unsigned)n_win, (unsigned)n_cb);
     if (coh == 1) hipLaunchKernelGGL((conv_split_kernel<G, 1, MODE>), grid, dim3(G::NT), 0, st, a);
     else hipLaunchKernelGGL((conv_split_kernel<G, 2, MODE>), grid, dim3(G::NT), 0, st, a);
     APRNET_LAUNCH_CHECK("conv_split_kernel");
     return 0;
 }
 // a.w, a.redo: what prepare_split made of the weights a.w_raw; a.win_level ... the forward lists of the plan
-int launch_conv_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+int launch_conv_split(int code, const ConvArgs<float>& a, int n_win, hipStream_t st) {
     int rc;
     switch (code) {
-        case 333: rc = launch_split<S333, 0>(a, n_tiles, st); break;
-        case 155: rc = launch_split<S155, 0>(a, n_tiles, st); break;
+        case 333: rc = launch_split<S333, 0>(a, n_win, st); break;
+        case 155: rc = launch_split<S155, 0>(a, n_win, st); break;
         default: rc = fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
     }
-    return rc ? rc : launch_conv_redo(code, a, n_tiles, st);
+    return rc ? rc : launch_conv_redo(code, a, n_win, st);
 }
 // Input gradient: a.x / a.xi / a.Cin describe the output gradient, a.Cout the layer's input channels, a.w the transposed image,
 // a.win_level ... the input-gradient lists of the plan without the particles on far faces.  a.redo[0] is set if a sum is not finite.
-int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_tiles, hipStream_t st) {
+int launch_conv_dx_split(int code, const ConvArgs<float>& a, int n_win, hipStream_t st) {
     switch (code) {
-        case 333: return launch_split<S333, 1>(a, n_tiles, st);
-        case 155: return launch_split<S155, 1>(a, n_tiles, st);
+        case 333: return launch_split<S333, 1>(a, n_win, st);
+        case 155: return launch_split<S155, 1>(a, n_win, st);
     }
     return fail(APRNET_ERR_UNSUPPORTED, "no matrix-core kernel for this stencil");
 }

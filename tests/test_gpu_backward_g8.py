@@ -248,12 +248,14 @@ def test_copies_of_a_large_layer_are_made_in_parts(cin, cout):
 
 
 @pytest.mark.parametrize("fill", [16, 17], ids=["needed-nodes", "whole-tree"])
+@pytest.mark.parametrize("d", [0, 1, 2])
 @pytest.mark.parametrize("ksize,c1,c2", [((3, 3, 3), 8, 0), ((1, 3, 3), 12, 12), ((1, 5, 5), 40, 0), ((3, 3, 3), 16, 24)])
-def test_tree_made_of_the_regrouped_features(ksize, c1, c2, fill):
+def test_tree_made_of_the_regrouped_features(ksize, c1, c2, d, fill):
     """A 16-byte aligned tree work space takes the tree in groups of eight channels, made of the regrouped features; any other one the planes'
-    tree, regrouped.  Same bits in the output and in the weight gradient, also where the rows of the work space are longer than the tree."""
+    tree, regrouped.  Same bits in the output and in the weight gradient, also where the rows of the work space are longer than the tree, and
+    at the level deltas at which downsampled particles come first in a node's sum."""
     lib, st, cin, cout = _native.hip(), torch.cuda.current_stream().cuda_stream, c1 + c2, 16
-    apr, d = apr_cases.get("3d_t" if ksize[0] == 3 else "2d_t"), 0
+    apr = apr_cases.get("3d_t" if ksize[0] == 3 else "2d_t")
     n, nt = _ops.number_particles(apr, d), _ops.tree_parts(apr, d)
     g = torch.Generator().manual_seed(cin)
     x = torch.randn(cin, n, generator=g).to(torch.bfloat16).to(DEV)

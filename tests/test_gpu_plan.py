@@ -136,3 +136,30 @@ def test_partial_sums_of_a_very_wide_layer_stay_within_their_limit():
         torch.cuda.synchronize()
         used.append(free - torch.cuda.mem_get_info()[0])
     assert used[1] <= 32 * c * c * 27 * 4 + (64 << 20)               # (lists and tables of 18 k particles, in whole pages)
+
+
+def test_input_gradient_captured_before_the_table_of_parents_is_there():
+    """bfloat16 features, eight channels: the first eager backward pass builds the plan's table of parents, a capture must not.  The pass it
+    records instead works on channel planes; small whole numbers, so that every replay gives the eager pass's bits, whichever way that goes."""
+    from pyapr import _native
+    apr = apr_cases.random_apr((33, 29, 37), 23, density=0.02)
+    apr.init_cuda()
+    n, levels = apr.total_number_particles(), apr.level_max() - apr.level_min() + 1
+    ld, g = torch.zeros(1, dtype=torch.int32), torch.Generator().manual_seed(0)
+    rand = lambda c: torch.randint(-3, 4, (1, c, n), generator=g).to(torch.bfloat16).to(DEV)
+    w = torch.randint(-2, 3, (levels, 16, 8, 3, 3, 3), generator=g).float().to(DEV)
+    x, gy = rand(8), rand(16)
+    _ops.conv_backward([apr], rand(5), w[:, :, :5].contiguous(), gy, ld)          # tiles, lists and nodes; five channels need no table
+    assert _native.hip().aprnet_plan_reserve(apr.plan(0), 64 << 20, None) == 0
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        gx, gw = _ops.conv_backward([apr], x, w, gy, ld)
+    assert b"table of parents" in _native.hip().aprnet_last_error()               # asked for and refused
+    for k in range(3):
+        x.copy_(rand(8)); gy.copy_(rand(16))
+        want = _ops.conv_backward([apr], x, w, gy, ld) if k else None             # from the second replay on the table is there
+        graph.replay()
+        torch.cuda.synchronize()
+        if want is None: want = _ops.conv_backward([apr], x, w, gy, ld)
+        assert torch.equal(gx, want[0]) and torch.equal(gw, want[1]) and float(gx.float().abs().max()) > 0

@@ -226,7 +226,11 @@ static int try_narrow(aprnet_plan* p, const ConvArgs<T>& a, int code, int d, con
 }
 
 // Work space of the forward pass on products of bfloat16 pieces: packed weights and marks.  0: the layer does not take that path.
-//  - fewer than SPLIT_MIN_CIN input channels: half of an instruction's products are zero.
+//  - fewer than SPLIT_MIN_CIN input channels.  The line was drawn when the kernel read copies of features and tree, whose cost these layers did not win
+//    back (8 -> 16 channels 0.080 and 0.078 ms); without copies pieces are ahead there too, by less with 16 outputs (fp32 instructions and pieces, 3x3x3,
+//    1 M particles: 4 -> 16 0.082 and 0.080 ms, 8 -> 16 0.113 and 0.106, 8 -> 32 0.168 and 0.137, 12 -> 32 0.224 and 0.170; 0.16 M: 8 -> 16 0.044 and
+//    0.044, 8 -> 32 0.055 and 0.049), and so are input gradients of 4 to 12 outputs (1 M, whole backward pass, 16 -> 8 0.59 and 0.42, 32 -> 8 1.07 and
+//    0.67).  It has not been moved since.
 //  - 1x3x3: two steps of eight taps for nine.
 //  - little work: one more launch than the fp32 kernel's, which also counts where the host is behind the device (3x3x3, pieces against
 //    fp32; 16 outputs: 90 k particles x 16 channels 50 and 48 us, x 32 70 and 65, 160 k x 16 58 and 58, 320 k 78 and 90; 32 outputs: 12 k

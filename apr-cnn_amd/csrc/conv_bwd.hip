@@ -611,6 +611,8 @@ int conv_bwd_bf16(const aprnet_plan* cp, int d, int kz, int kx, int ky, const bf
         }
         bf16_t* gyi = (bf16_t*)((char*)p->d_scratch + wbytes);
         if (dw_g8 || dx_g8) if (int rc = interleave8_bf16(gy, ldy, nullptr, 0, Cout, Cout, np, gyi, st)) return rc;
+        // side by side at any size (in turn, forward and backward: 3x3x3 64 -> 64 channels on 1.2 M particles 2.03 instead of 2.12 ms, on 5.5 M 9.53
+        // and 9.45, 1x5x5 64 -> 64 on 15.4 M 18.5 and 18.2)
         hipStream_t side = st;
         if (near.n > 0) if (int rc = fork_side(p, st, &side)) return rc;
         SideJoin guard(p, st, side);

@@ -12,11 +12,12 @@
 // 4 pairs of taps x 4 channels, so both operands are pieces as they lie there and a step of eight taps takes six instructions.  (With
 // 16-byte cells {x1, x2} and weights {w1, w1}, {w2, w2}, {w3, w1} a step of four taps takes three, one eighth fewer over
 // the 27 taps, but the doubled weights cost 24 register moves per step and wave: 10.1 against 9.1 ms for 32 -> 32 channels
-// on 23 M particles.)  Values come from the caller's planes (input gradient: from a copy of the output gradient in groups of four
+// on 23 M particles, with the windows of one row group that the lists held then.)  Values come from the caller's planes (input gradient: from a copy of the output gradient in groups of four
 // channels, see load_values_split); a value is split when it is written to LDS.  Lists, work split and epilogue are those of the fp32 kernel (conv_mfma.hip).
 //
-// Measured against the fp32 instructions (3x3x3, whole forward pass): 23 M particles, 32 -> 32 channels 8.7 ms; 1 M, 32 -> 32 0.40 (0.52), 64 -> 64
-// 1.40 (1.78); 320 k, 16 -> 16 0.078 (0.090), 64 -> 64 0.46 (0.64).
+// Measured against the fp32 instructions (3x3x3, whole forward pass, tree fill included): 23 M particles, 32 -> 32 channels 9.1 ms (11.0), of which
+// this kernel 8.3; 1 M, 32 -> 32 0.40 (0.52), 64 -> 64 1.40 (1.78); 320 k, 16 -> 16 0.075 (0.085), 64 -> 64 0.46 (0.64).  1x5x5 64 -> 64 on 23 M
+// 31.4 (38.4).  Pairs of times further down were taken when a variant was tried, each pair on one state of the kernel and of the lists.
 // Input gradient, whole backward pass with the weight gradient (conv_dw_split.hip): 1 M particles, 32 -> 32 channels 1.33 (1.84), 16 -> 16 0.48
 // (0.72); the fp32 kernel scans the access arrays and stages box sums, this one reads lists kept with the plan.
 // Bound by the barriers around the matrix phases and the LDS reads of the operands.
@@ -26,7 +27,7 @@
 // Infinities: where x or w is infinite the pieces of the other operand decide the result (infinity times a zero piece is
 // NaN), and values of 2^111 and more, or sums of 2^95 and more, are infinite for these kernels (see SPLIT_SCALE).  Where a result comes
 // out infinite or NaN its window and block of outputs are marked, and the fp32 instructions compute what is marked again (conv_mfma16_redo_kernel; as a call
-// inside this kernel a second pass cost registers: 16 -> 16 channels on 23 M particles 3.47 instead of 3.26 ms); an
+// inside this kernel a second pass cost registers: 16 -> 16 channels on 23 M particles 3.47 instead of 3.26 ms then); an
 // input gradient that holds one is made again from the start by the fp32 kernel.  Small values keep all their bits: features of 1e-37
 // come out with 0.4 of the fp32 instructions' error (split without SPLIT_SCALE, 510 times that error).
 #include "pieces.hpp"

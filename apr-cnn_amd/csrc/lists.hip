@@ -12,8 +12,8 @@
 // The kernels are bound by what a window costs whether it is full or not (lists, round trips, weights, barriers).  Windows of
 // 62 positions of one row group, as they were, held 173 outputs of 496 on average on the 23 M particles of a blob volume (134,000
 // windows, now 60,200 of 385), 118 on a sparse light-sheet one of 43 M (366,000, now 121,000 of 355), 311 on a dense one of 52 M (167,000, now
-// 121,000 of 428).  3x3x3 of fp32 features 32 -> 32 on the first 11.6 -> 9.7 ms, 16 -> 16 on the second 9.1 -> 7.0, a bfloat16 U-Net on the third
-// 58.4 -> 53.7.
+// 121,000 of 428).  By the windows alone, whole passes: 3x3x3 of fp32 features 32 -> 32 on the first 11.6 -> 9.7 ms, 16 -> 16 on the second 9.1 -> 7.0, a
+// bfloat16 U-Net on the third 58.4 -> 53.7.
 //
 // Three passes over the row groups: kept positions, then items and columns per window, then the lists; the host turns the counts into
 // offsets in between.
@@ -279,9 +279,13 @@ void free_lists(WinLists& wl) {
 }
 
 // Cells of a window without its halo: as many as the patch holds where that leaves a window for each of the 512 workgroups that the chip
-// holds, fewer otherwise, an even number of them.  Training step on two APRs of 338 k particles, whose coarser level deltas had 5 to 370
+// holds, fewer otherwise, an even number of them; one width for all levels of a list, by their cells together.  Training step on two APRs of 338 k particles, whose coarser level deltas had 5 to 370
 // full windows, 11.5 -> 10.3 ms, group-normed fp32 U-Net on 2.7 M 5.31 -> 5.13.  (1024 windows 32 -> 32 channels on 320 k particles
 // 0.176 instead of 0.165 ms, 2048 0.209; down to 14 cells the step 10.3, to 6 11.4 ms; widths of 62, 30 and 14 only 10.75.)
+// One list serves layers of any width, and the line is drawn for few blocks of channels.  Kernels with many, whose workgroups fill the chip on fuller
+// windows, pay for narrow ones: weight gradients without an input gradient on lists of 11 to 31 thousand cells, 64 -> 128 channels 1x5x5 on 0.04 M
+// particles 365 us with full windows of one row group, 475 with these, 315 with full ones; 1 -> 16 on bfloat16 38, 44 and 38.  256 windows instead of
+// 512 mend a third of these calls, the step above 10.1 instead of 10.3, but 16 and 32 outputs lose (U-Net on 2.7 M 5.10 and 5.22, 32 -> 32 on 0.16 M 0.095 and 0.101).
 constexpr int WINDOWS_MIN = 512, CELLS_MIN = 22;
 static int window_cells(int64_t n_cells, int HY) {
     const int widest = 64 - 2 * HY;

@@ -37,7 +37,7 @@ __device__ __forceinline__ uint4* g8_at(bf16_t* base, int64_t ld, int q, int64_t
 
 // Groups of a thread in the kernels that walk the child table: all of them, so that the table is read once, halved while fewer than `threads`
 // would remain.  A thread's groups are a serial chain, each waiting for its own loads: in a network of 16 to 128 channels on 1.3 M
-// particles a fill took 8.3 us with one thread for all groups and 5.1 split, a pool 11.8 and 7.6, an upsample 9.5 and 8.0, the network 0.92 and 0.835 ms.
+// particles, all three split up to 2^19 threads, a fill took 5.1 us instead of 8.3, a pool 7.6 (11.8), an upsample 8.0 (9.5), the network 0.835 ms (0.92).
 // Fills gain up to 2^19 threads, what the chip holds at a time (1.3 M particles of 32 channels 44.9 -> 37.7 us, of 256 279 -> 186 and, with limits of
 // 2^17 and 2^18, 204 and 192; 2^20 and 2^21: the network 0.842 and 0.839 ms).  A pool or upsample moves little more than the table it reads again: past 2^17 threads
 // splitting costs it, at 2^19 a pool to 0.21 M outputs of 16 channels 8.0 us instead of 7.1, to 0.36 M 11.7 and 11.3, an upsample of 64 channels to
